@@ -166,6 +166,11 @@ int blr_blast_q_fwd(const void* x, int64_t ldx,
  * quantizer).                                                                                */
 int blr_quantize_sym(const void* w, int dtype, int64_t outer, int64_t reduce, int64_t inner,
                      int bits, void* codes, void* scales, void* stream);
+/* The same quantizer for a factor stored with the reduced axis contiguous, w (outer, inner, reduce): codes and scales
+ * come out in the same order as above, codes (outer, reduce, inner[/2]), so that U (b, q, r) of the bmm names is packed
+ * without a transposed copy of it.  bits = 4 needs an even `inner`.                                              */
+int blr_quantize_sym_t(const void* w, int dtype, int64_t outer, int64_t reduce, int64_t inner,
+                       int bits, void* codes, void* scales, void* stream);
 
 /* ---- Monarch ------------------------------------------------------------------------------
  * w1 (b, in_f/b, rank) with pre-permuted columns (reference layer.py:221-224), w2 per

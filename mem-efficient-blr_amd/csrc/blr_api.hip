@@ -37,81 +37,7 @@ int device_cus() {
 static int elt_size(int dtype) { return dtype == BLR_F32 ? 4 : 2; }
 static bool dtype_ok(int dtype) { return dtype == BLR_F16 || dtype == BLR_BF16 || dtype == BLR_F32; }
 
-// ---- quantizer --------------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ float ld_f32(const T* p, int64_t i) { return TypeTraits<T>::to_f32(p[i]); }
-
-__device__ __forceinline__ int quant_code(float w, float s, float qmax) {
-  float q = rintf(__fdiv_rn(w, s));
-  q = fminf(fmaxf(q, -qmax), qmax);
-  return (int)q;
-}
-__device__ __forceinline__ float make_scale(float amax, float qmax, f16* store) {
-  f16 s16 = (f16)__fdiv_rn(amax, qmax);
-  if ((float)s16 == 0.0f) s16 = (f16)1.0f;
-  *store = s16;
-  return (float)s16;
-}
-
-// inner == 1: one workgroup per channel row, max over the contiguous axis.
-template <typename T>
-__global__ __launch_bounds__(256) void quant_rows_kernel(const T* __restrict__ w, int64_t reduce, int bits,
-                                                         uint8_t* __restrict__ codes, f16* __restrict__ scales) {
-  __shared__ float s_max[4];
-  __shared__ float s_scale;
-  const int64_t row = blockIdx.x;
-  const T* wr = w + row * reduce;
-  float amax = 0.0f;
-  for (int64_t k = threadIdx.x; k < reduce; k += 256) amax = fmaxf(amax, fabsf(ld_f32(wr, k)));
-  for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
-  if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = amax;
-  __syncthreads();
-  const float qmax = bits == 8 ? 127.0f : 7.0f;
-  if (threadIdx.x == 0) {
-    float m = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
-    s_scale = make_scale(m, qmax, &scales[row]);
-  }
-  __syncthreads();
-  const float s = s_scale;
-  if (bits == 8) {
-    int8_t* c = reinterpret_cast<int8_t*>(codes) + row * reduce;
-    for (int64_t k = threadIdx.x; k < reduce; k += 256) c[k] = (int8_t)quant_code(ld_f32(wr, k), s, qmax);
-  } else {
-    uint8_t* c = codes + row * (reduce / 2);
-    for (int64_t k = threadIdx.x; k < reduce / 2; k += 256) {
-      int lo = quant_code(ld_f32(wr, 2 * k), s, qmax), hi = quant_code(ld_f32(wr, 2 * k + 1), s, qmax);
-      c[k] = (uint8_t)((lo & 0xF) | ((hi & 0xF) << 4));
-    }
-  }
-}
-
-// inner > 1: thread per inner column (or column pair for int4), max over the strided axis.
-template <typename T>
-__global__ __launch_bounds__(256) void quant_cols_kernel(const T* __restrict__ w, int64_t reduce, int64_t inner, int bits,
-                                                         uint8_t* __restrict__ codes, f16* __restrict__ scales) {
-  const int64_t o = blockIdx.y;
-  const int per = bits == 8 ? 1 : 2;
-  const int64_t c0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * per;
-  if (c0 >= inner) return;
-  const T* wo = w + o * reduce * inner;
-  const float qmax = bits == 8 ? 127.0f : 7.0f;
-  float amax[2] = {0.0f, 0.0f};
-  for (int64_t k = 0; k < reduce; ++k)
-    for (int u = 0; u < per; ++u) amax[u] = fmaxf(amax[u], fabsf(ld_f32(wo, k * inner + c0 + u)));
-  float s[2];
-  for (int u = 0; u < per; ++u) s[u] = make_scale(amax[u], qmax, &scales[o * inner + c0 + u]);
-  if (bits == 8) {
-    int8_t* c = reinterpret_cast<int8_t*>(codes) + o * reduce * inner;
-    for (int64_t k = 0; k < reduce; ++k) c[k * inner + c0] = (int8_t)quant_code(ld_f32(wo, k * inner + c0), s[0], qmax);
-  } else {
-    uint8_t* c = codes + o * reduce * (inner / 2);
-    for (int64_t k = 0; k < reduce; ++k) {
-      int lo = quant_code(ld_f32(wo, k * inner + c0), s[0], qmax), hi = quant_code(ld_f32(wo, k * inner + c0 + 1), s[1], qmax);
-      c[k * (inner / 2) + c0 / 2] = (uint8_t)((lo & 0xF) | ((hi & 0xF) << 4));
-    }
-  }
-}
-
+// ---- expansion of codes for the tiled kernels -----------------------------------------------------
 // codes (rows, cols) -> T; scale index = (row / rows_per_scale_block) * cols + col when per_col, else row.
 // cols % 8 == 0: a thread expands 8 consecutive codes (8 or 4 bytes in, 16 bytes out).
 template <typename T>
@@ -145,19 +71,6 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
     }
     *reinterpret_cast<V8*>(&out[idx]) = o;
   }
-}
-
-template <typename T>
-static int quantize_t(const void* w, int64_t outer, int64_t reduce, int64_t inner, int bits, void* codes, void* scales, hipStream_t st) {
-  if (inner == 1) {
-    hipLaunchKernelGGL(quant_rows_kernel<T>, dim3((unsigned)outer), dim3(256), 0, st, (const T*)w, reduce, bits, (uint8_t*)codes, (f16*)scales);
-  } else {
-    int per = bits == 8 ? 1 : 2;
-    dim3 grid((unsigned)cdiv(cdiv(inner, per), 256), (unsigned)outer);
-    hipLaunchKernelGGL(quant_cols_kernel<T>, grid, dim3(256), 0, st, (const T*)w, reduce, inner, bits, (uint8_t*)codes, (f16*)scales);
-  }
-  BLR_CHECK_LAUNCH("quantize");
-  return BLR_OK;
 }
 
 // ---- fused output stage ------------------------------------------------------------------------------
@@ -633,10 +546,15 @@ int blr_quantize_sym(const void* w, int dtype, int64_t outer, int64_t reduce, in
   if (!w || !codes || !scales) { set_error("quantize: null pointer"); return BLR_ERR_BAD_ARG; }
   if (outer <= 0 || reduce <= 0 || inner <= 0 || (bits != 8 && bits != 4) || !dtype_ok(dtype)) { set_error("quantize: bad argument"); return BLR_ERR_BAD_ARG; }
   if (bits == 4 && ((inner == 1 ? reduce : inner) % 2)) { set_error("quantize: int4 needs an even contiguous axis"); return BLR_ERR_BAD_SHAPE; }
-  hipStream_t st = (hipStream_t)stream;
-  if (dtype == BLR_F32) return quantize_t<float>(w, outer, reduce, inner, bits, codes, scales, st);
-  if (dtype == BLR_F16) return quantize_t<f16>(w, outer, reduce, inner, bits, codes, scales, st);
-  return quantize_t<bf16>(w, outer, reduce, inner, bits, codes, scales, st);
+  return quantize_launch(w, dtype, outer, reduce, inner, bits, codes, scales, (hipStream_t)stream);
+}
+
+int blr_quantize_sym_t(const void* w, int dtype, int64_t outer, int64_t reduce, int64_t inner,
+                       int bits, void* codes, void* scales, void* stream) {
+  if (!w || !codes || !scales) { set_error("quantize: null pointer"); return BLR_ERR_BAD_ARG; }
+  if (outer <= 0 || reduce <= 0 || inner <= 0 || (bits != 8 && bits != 4) || !dtype_ok(dtype)) { set_error("quantize: bad argument"); return BLR_ERR_BAD_ARG; }
+  if (bits == 4 && inner % 2) { set_error("quantize: int4 needs an even contiguous axis"); return BLR_ERR_BAD_SHAPE; }
+  return quantize_t_launch(w, dtype, outer, reduce, inner, bits, codes, scales, (hipStream_t)stream);
 }
 
 // ---- Monarch --------------------------------------------------------------------------------------

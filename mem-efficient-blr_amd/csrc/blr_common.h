@@ -139,6 +139,12 @@ __device__ __forceinline__ void side_prep_item(const SidePrep& s, int64_t idx) {
   }
 }
 
+// ---- weight quantizer (blr_quant.hip) ---------------------------------------------------
+// w (outer, reduce, inner) contiguous; codes in the same order, scales (outer, inner).
+int quantize_launch(const void* w, int dtype, int64_t outer, int64_t reduce, int64_t inner, int bits, void* codes, void* scales, hipStream_t st);
+// w (outer, inner, reduce) contiguous; the same codes and scales, i.e. transposed on the way: codes (outer, reduce, inner).
+int quantize_t_launch(const void* w, int dtype, int64_t outer, int64_t reduce, int64_t inner, int bits, void* codes, void* scales, hipStream_t st);
+
 // ---- tiled GEMM (blr_gemm.hip) ----------------------------------------------------------
 enum { EPI_PLAIN = 0, EPI_MONARCH_SCATTER = 1 };
 struct GemmArgs {

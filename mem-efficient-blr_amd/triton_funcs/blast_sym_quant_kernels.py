@@ -72,7 +72,18 @@ def quantize_blast_factors(U, V, bits=8):
 
     The codes of U are stored transposed, (b, r, q[/2]) - the order the kernels stream them in
     (output channel contiguous, like V); ``QuantFactor.shape`` keeps the logical (b, q, r)."""
-    uc, us = quantize_sym(U.transpose(1, 2).contiguous(), 1, bits)
+    L.require_gpu(U, V)
+    assert bits in (8, 4)
+    U = U.contiguous()
+    b, q, r = U.shape
+    if bits == 8:
+        uc = torch.empty((b, r, q), dtype=torch.int8, device=U.device)
+    else:
+        assert q % 2 == 0, "int4 packing needs an even last axis"
+        uc = torch.empty((b, r, q // 2), dtype=torch.uint8, device=U.device)
+    us = torch.empty((b, q), dtype=torch.float16, device=U.device)
+    rc = L.lib().blr_quantize_sym_t(U.data_ptr(), L.dtype_code(U.dtype), b, r, q, bits, uc.data_ptr(), us.data_ptr(), L.stream_ptr(U.device))
+    L.check(rc, "blr_quantize_sym_t")
     vc, vs = quantize_sym(V, 1, bits)
     return QuantFactor(uc, us, bits, tuple(U.shape)), QuantFactor(vc, vs, bits, tuple(V.shape))
 

@@ -29,6 +29,26 @@ def test_quantizer_codes_bit_exact(shape, axis, bits):
         np.testing.assert_array_equal(O.unpack_int4(codes.cpu().numpy()), rc)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [8, 4])
+# tiles of the turning kernel are 128 channels x 64 values, its loads four values; the column kernel's pieces four columns
+@pytest.mark.parametrize("b,p,q,r", [(2, 1, 2, 2), (2, 37, 126, 62), (3, 64, 130, 66), (2, 33, 256, 64), (2, 300, 136, 264), (16, 40, 8, 1030)])
+def test_packed_factors_codes_bit_exact(b, p, q, r, bits, dtype):
+    from triton_funcs import blast_sym_quant_kernels as Q
+    g = torch.Generator().manual_seed(b * p + q * r)
+    U = (torch.randn(b, q, r, generator=g) / 8).to(dtype)
+    V = (torch.randn(b, p, r, generator=g) / 8).to(dtype)
+    U[0, 1] = 0.0                      # an all-zero channel of each factor, and values that sit exactly between two codes
+    V[1, :, 0] = 0.0
+    U[1, 0] = torch.arange(r).remainder(15).sub(7).add(0.5).clamp(max=7).to(dtype)
+    say(f"[case] packed factors bits={bits} {dtype} b={b} p={p} q={q} r={r}")
+    Uq, Vq = Q.quantize_blast_factors(U.cuda(), V.cuda(), bits)
+    for got, (codes, scales), turned in ((Uq, O.quantize_sym(U.float().numpy(), 2, bits), True), (Vq, O.quantize_sym(V.float().numpy(), 1, bits), False)):
+        c = got.codes.cpu().numpy() if bits == 8 else O.unpack_int4(got.codes.cpu().numpy())
+        np.testing.assert_array_equal(c.transpose(0, 2, 1) if turned else c, codes)
+        np.testing.assert_array_equal(got.scales.cpu().numpy(), scales)
+
+
 def test_quantizer_half_inputs_and_ties():
     from triton_funcs import blast_sym_quant_kernels as Q
     # values that land exactly on .5 after scaling: scale = 1/127*127 ... use amax = 127 -> scale 1
