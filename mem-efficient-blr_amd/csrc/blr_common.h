@@ -87,7 +87,7 @@ void epilogue_taken();
 // Every run-time switch of the library (blr_set_option): each starts from the environment variable of its name, read once, and
 // is range-checked where it is set.  The first six pick the GEMM variant, the rest switch a kernel family off (0) so that the
 // call falls through to the next one that serves it - for A/B measurements and as a way out should a kernel misbehave.
-enum { OPT_GEMM_RING = 0, OPT_GEMM_RING_TILE, OPT_GEMM_RING_PER_CU, OPT_GEMM_RING_WAVES, OPT_GEMM_RING_BK, OPT_GEMM_SPLITK,
+enum { OPT_GEMM_RING = 0, OPT_GEMM_RING_TILE, OPT_GEMM_RING_PER_CU, OPT_GEMM_RING_WAVES, OPT_GEMM_RING_BK, OPT_GEMM_SPLITK, OPT_GEMM_MID,
        OPT_DECODE2, OPT_DECODE3, OPT_DECODE_PAIR, OPT_DECODE_ROWS, OPT_DENSE_SLAB, OPT_DENSE_ROWS, OPT_BLAST_MIXU, OPT_BLAST_ONE, OPT_BLAST_YMIXW, OPT_COUNT };
 int option_value(int id, int dflt);             // the option's value, or dflt when it is unset
 // true when p is aligned to `bytes`.
@@ -174,6 +174,12 @@ struct GemmArgs {
 };
 // dtype: blr_dtype.  Returns blr_status.
 int gemm_launch(const GemmArgs& a, int dtype, hipStream_t st);
+// Kernels for products that do not fill the chip with the large tiles (blr_gemm_mid.hip; the ring kinds live in blr_gemm.hip).
+enum { MID_32_64 = 0, MID_32_64_DEEP, MID_64_64, MID_64_64_DEEP, MID_64_128, MID_RING_128, MID_RING_128_TWO, MID_RING_256_SLICES, MID_KINDS };
+struct MidPlan { int kind, slices, kc; };       // kind < 0: none of them takes the product; kc: k per slice
+MidPlan gemm_mid_plan(int M, int N, int K, int batch, bool ring, bool mid, bool slices);
+bool gemm_mid_ok(const GemmArgs& a);            // whether the operands suit kinds MID_32_64 .. MID_64_128
+int gemm_mid_launch(const GemmArgs& a, int kind, bool partial, int dtype, hipStream_t st);
 // Scratch a plain single GEMM M x N x K of dtype wants in GemmArgs::splitk_ws so that a problem with few output tiles and
 // a long reduction can be cut along K to fill the chip (fp32 partial results, summed in a fixed order).  0: no split.
 size_t gemm_splitk_bytes(int M, int N, int K, int dtype);

@@ -10,8 +10,10 @@
 #include <cstdlib>
 #include <mutex>
 #include <set>
+#include <type_traits>
 #include "blr_common.h"
 #include "blr_decode.h"
+#include "blr_gemm_dev.h"
 #include "blr_ring_dev.h"
 
 namespace blr {
@@ -156,69 +158,6 @@ struct KnStage {
     }
   }
 };
-
-__device__ __forceinline__ int64_t epi_offset(const GemmArgs& g, int bt, int m, int n) {
-  if (g.epi == EPI_MONARCH_SCATTER) {
-    int dst_blk = n / g.per, j = n - dst_blk * g.per;
-    return (int64_t)dst_blk * g.sL + (int64_t)m * g.ldc + (int64_t)bt * g.per + j;
-  }
-  return (int64_t)bt * g.sC + (int64_t)m * g.ldc + (int64_t)n * g.cn;
-}
-
-// Fused output stage (kernels instantiated with EP): bias (indexed by the element's offset inside its row of C) and
-// activation are applied to the rounded result on its way out, like the separate kernels of the callers would.  The
-// plain instantiations do not contain this code: it costs registers that the main loops need.
-template <typename T>
-__device__ __forceinline__ T ep_value(const GemmArgs& g, T r, int64_t in_row, int row) {
-  float v = TypeTraits<T>::to_f32(r);
-  if (g.bias) v += TypeTraits<T>::to_f32(reinterpret_cast<const T*>(g.bias)[in_row]);
-  v = apply_act(v, g.act);
-  if (g.gate || g.resid) {
-    v = TypeTraits<T>::to_f32(TypeTraits<T>::from_f32(v));                    // what a separate gate / residual kernel would read
-    if (g.gate) v *= TypeTraits<T>::to_f32(reinterpret_cast<const T*>(g.gate)[(int64_t)(row / g.gate_rows) * g.ld_gate + in_row]);
-    if (g.resid) v += TypeTraits<T>::to_f32(reinterpret_cast<const T*>(g.resid)[(int64_t)row * g.ld_resid + in_row]);
-  }
-  return TypeTraits<T>::from_f32(v);
-}
-
-// eight consecutive outputs; their offset inside the row is a multiple of 8, so the bias comes as one 16-byte load
-template <typename T>
-__device__ __forceinline__ typename TypeTraits<T>::vec8 ep_vector(const GemmArgs& g, typename TypeTraits<T>::vec8 r, int64_t in_row, int row) {
-  using V8 = typename TypeTraits<T>::vec8;
-  V8 bv;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) bv[e] = (T)0.0f;
-  if (g.bias) bv = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.bias) + in_row);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) r[e] = TypeTraits<T>::from_f32(apply_act(TypeTraits<T>::to_f32(r[e]) + TypeTraits<T>::to_f32(bv[e]), g.act));
-  if (g.gate || g.resid) {                      // one row of gate per group of gate_rows rows of C
-    V8 gv, rv;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { gv[e] = (T)1.0f; rv[e] = (T)0.0f; }
-    if (g.gate) gv = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.gate) + (int64_t)(row / g.gate_rows) * g.ld_gate + in_row);
-    if (g.resid) rv = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.resid) + (int64_t)row * g.ld_resid + in_row);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = TypeTraits<T>::from_f32(TypeTraits<T>::to_f32(r[e]) * TypeTraits<T>::to_f32(gv[e]) + TypeTraits<T>::to_f32(rv[e]));
-  }
-  return r;
-}
-
-// Second tile of a pair: (r + bias) rounded to T, times the first tile's result, which the same thread stored at `c` before.
-template <typename T>
-__device__ __forceinline__ typename TypeTraits<T>::vec8 ep_pair_up(const GemmArgs& g, typename TypeTraits<T>::vec8 r, int64_t in_row, const T* c) {
-  using V8 = typename TypeTraits<T>::vec8;
-  V8 bv;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) bv[e] = (T)0.0f;
-  if (g.bias) bv = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.bias) + in_row);
-  const V8 gv = *reinterpret_cast<const V8*>(c);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const T up = TypeTraits<T>::from_f32(TypeTraits<T>::to_f32(r[e]) + TypeTraits<T>::to_f32(bv[e]));
-    r[e] = TypeTraits<T>::from_f32(TypeTraits<T>::to_f32(gv[e]) * TypeTraits<T>::to_f32(up));
-  }
-  return r;
-}
 
 template <typename T, int BM, int BN, bool B_KN, int PD, bool EP = false>
 __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemmArgs g, int tiles_m, int tiles_n, int a_vec, int b_vec, int c_vec,
@@ -1130,48 +1069,44 @@ static int launch_mfma(const GemmArgs& g, hipStream_t st) {
 }
 
 // The ring kernels take plain row-major output and 16-byte friendly operands whose per-lane byte offsets fit 32 bits.
-// out[m, n] = sum over slices s of P[s][m][n] (fp32, fixed order), rounded once to T; 8 columns per thread
-template <typename T>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ P, T* __restrict__ C, int M, int N, int64_t ldc, int splits) {
+// out[m, n] = sum over slices s of P[s][m][n] (fp32, fixed order), rounded once to T, then the fused output stage if there is one;
+// 8 columns per thread, the slices asked for four at a time
+template <typename T, bool EP>
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ P, GemmArgs g, int splits) {
   using V8 = typename TypeTraits<T>::vec8;
   const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int vpr = N >> 3;
-  if (v >= (int64_t)M * vpr) return;
+  const int vpr = g.N >> 3;
+  if (v >= (int64_t)g.M * vpr) return;
   const int m = (int)(v / vpr), n = (int)(v - (int64_t)m * vpr) * 8;
-  float acc[8];
+  const int64_t slice = (int64_t)g.M * g.N;
+  const float* p = P + (int64_t)m * g.N + n;
+  f32x4 s0 = {0, 0, 0, 0}, s1 = {0, 0, 0, 0};
+  for (int s = 0; s < splits; s += 4) {
+    f32x4 a[4], b[4];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
-  for (int s = 0; s < splits; ++s) {
-    const float4* p = reinterpret_cast<const float4*>(P + ((int64_t)s * M + m) * N + n);
-    const float4 a = p[0], b = p[1];
-    acc[0] += a.x; acc[1] += a.y; acc[2] += a.z; acc[3] += a.w;
-    acc[4] += b.x; acc[5] += b.y; acc[6] += b.z; acc[7] += b.w;
+    for (int e = 0; e < 4; ++e) {                    // (slices past the last are fetched again and not added)
+      const float* q = p + (int64_t)min(s + e, splits - 1) * slice;
+      a[e] = *reinterpret_cast<const f32x4*>(q); b[e] = *reinterpret_cast<const f32x4*>(q + 4);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (s + e < splits) { s0 += a[e]; s1 += b[e]; }
   }
   V8 o;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) o[e] = TypeTraits<T>::from_f32(acc[e]);
-  *reinterpret_cast<V8*>(&C[(int64_t)m * ldc + n]) = o;
+  for (int e = 0; e < 4; ++e) { o[e] = TypeTraits<T>::from_f32(s0[e]); o[4 + e] = TypeTraits<T>::from_f32(s1[e]); }
+  if (EP) o = ep_vector<T>(g, o, n, m);
+  *reinterpret_cast<V8*>(&reinterpret_cast<T*>(g.C)[(int64_t)m * g.ldc + n]) = o;
 }
 
-// How many slices a plain single GEMM is cut into along K: only when 256 x 128 tiles leave at least half of the compute
-// units idle and every slice keeps at least 512 values of k (slices are multiples of 32).
-static int splitk_plan(int M, int N, int K, int* kc_out) {
-  const int cus = device_cus() > 0 ? device_cus() : 256;
-  const int64_t tiles = cdiv(M, 256) * cdiv(N, 128);
-  if (M < 96 || N % 8 || K % 8 || tiles * 2 > cus) return 1;
-  int splits = (int)std::min<int64_t>(8, cus / tiles);
-  while (splits > 1 && K / splits < 512) --splits;
-  if (splits <= 1) return 1;
-  const int kc = (int)cdiv(cdiv(K, splits), 32) * 32;
-  splits = (int)cdiv(K, kc);
-  if (kc_out) *kc_out = kc;
-  return splits;
-}
-
-size_t gemm_splitk_bytes(int M, int N, int K, int dtype) {
-  if (dtype != BLR_F16 && dtype != BLR_BF16) return 0;
-  const int splits = splitk_plan(M, N, K, nullptr);
-  return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+template <typename T>
+static int splitk_reduce_launch(const GemmArgs& g, int splits, hipStream_t st) {
+  const dim3 grid((unsigned)cdiv((int64_t)g.M * (g.N / 8), 256));
+  const float* P = reinterpret_cast<const float*>(g.splitk_ws);
+  if (g.bias || g.act || g.gate || g.resid) hipLaunchKernelGGL((splitk_reduce_kernel<T, true>), grid, dim3(256), 0, st, P, g, splits);
+  else hipLaunchKernelGGL((splitk_reduce_kernel<T, false>), grid, dim3(256), 0, st, P, g, splits);
+  BLR_CHECK_LAUNCH("splitk_reduce");
+  return BLR_OK;
 }
 
 static bool ring_ok(const GemmArgs& g) {
@@ -1269,6 +1204,14 @@ static int launch_ring64(const GemmArgs& g, hipStream_t st) {
   return BLR_OK;
 }
 
+size_t gemm_splitk_bytes(int M, int N, int K, int dtype) {
+  if ((dtype != BLR_F16 && dtype != BLR_BF16) || M < 96 || N % 8 || K % 8 || K < 64) return 0;
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  if (cdiv(M, 128) * cdiv(N, 128) > cus) return 0;
+  const MidPlan pl = gemm_mid_plan(M, N, K, 1, true, true, true);
+  return pl.slices > 1 ? (size_t)pl.slices * M * N * sizeof(float) : 0;
+}
+
 template <typename T>
 static int pick_mfma(const GemmArgs& g, hipStream_t st) {
   // Bigger tiles do more MFMA work per LDS byte (the 2x2 wave grid reads 0.5 fragments per MFMA at
@@ -1282,23 +1225,29 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
   // BLR_GEMM_RING_WAVES = 4 or 8 the workgroup size of the two larger ones - options that tests switch with
   // blr_set_option).
   const int ring = option_value(OPT_GEMM_RING, 1);
-  if (ring > 0 && ring_ok(g) && g.epi == EPI_PLAIN && g.splitk_ws && g.batch == 1 && g.cn == 1 && !g.sat8 && !g.bias && !g.act && !g.gate && !g.resid) {
-    // few tiles, long reduction: slices of K as the batch of the partial-sum kernel, then one pass that adds them up
-    int kc = 0;
-    const int splits = option_value(OPT_GEMM_SPLITK, 1) == 0 ? 1 : splitk_plan(g.M, g.N, g.K, &kc);
-    if (splits > 1 && g.splitk_bytes >= (size_t)splits * g.M * g.N * sizeof(float) && aligned(g.splitk_ws, 16)) {
+  // Products with at most one 128 x 128 tile per compute unit: smaller tiles, and slices of a long reduction, by the estimates of
+  // blr_gemm_mid.hip.  BLR_GEMM_MID = 0 switches that off, 2 .. 6 asks for one of its five tiles wherever the operands allow it.
+  const int mid = option_value(OPT_GEMM_MID, 1);
+  if (mid > 1 && gemm_mid_ok(g)) return gemm_mid_launch(g, mid - 2, false, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16, st);
+  const int64_t r128_all = cdiv(g.M, 128) * cdiv(g.N, 128) * g.batch;
+  if (mid == 1 && ring == 1 && r128_all <= cus && option_value(OPT_GEMM_RING_TILE, 0) == 0) {
+    constexpr int dt = std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16;
+    const bool rk = g.cn == 1 && g.M >= 96 && g.K >= 64 && ring_ok(g), mk = gemm_mid_ok(g);
+    bool cut = option_value(OPT_GEMM_SPLITK, 1) != 0 && rk && mk && g.epi == EPI_PLAIN && g.splitk_ws && aligned(g.splitk_ws, 16) && g.batch == 1 && !g.sat8 && !g.pair;
+    MidPlan pl = gemm_mid_plan(g.M, g.N, g.pair ? 2 * g.K : g.K, g.batch, rk, mk, cut);
+    if (pl.slices > 1 && g.splitk_bytes < (size_t)pl.slices * g.M * g.N * sizeof(float)) pl = gemm_mid_plan(g.M, g.N, g.K, g.batch, rk, mk, false);
+    if (pl.slices > 1) {                             // slices of K as the batch of a kernel that leaves partial sums
       GemmArgs p = g;
-      p.batch = splits; p.kc = kc;
-      p.sA = kc; p.sB = g.b_kn ? (int64_t)kc * g.ldb : kc;
+      p.batch = pl.slices; p.kc = pl.kc;
+      p.sA = pl.kc; p.sB = g.b_kn ? (int64_t)pl.kc * g.ldb : pl.kc;
       p.C = g.splitk_ws; p.ldc = g.N; p.sC = (int64_t)g.M * g.N;
-      int rc = launch_ring<T, 256, 128, false, 4, true>(p, st);
-      if (rc) return rc;
-      const int64_t vecs = (int64_t)g.M * (g.N / 8);
-      hipLaunchKernelGGL((splitk_reduce_kernel<T>), dim3((unsigned)cdiv(vecs, 256)), dim3(256), 0, st,
-                         reinterpret_cast<const float*>(g.splitk_ws), reinterpret_cast<T*>(g.C), g.M, g.N, g.ldc, splits);
-      BLR_CHECK_LAUNCH("splitk_reduce");
-      return BLR_OK;
+      p.bias = nullptr; p.act = 0; p.gate = nullptr; p.resid = nullptr;
+      const int rc = pl.kind == MID_RING_256_SLICES ? launch_ring<T, 256, 128, false, 4, true>(p, st) : gemm_mid_launch(p, pl.kind, true, dt, st);
+      return rc ? rc : splitk_reduce_launch<T>(g, pl.slices, st);
     }
+    if (pl.kind == MID_RING_128) return launch_ring64<T, 128, 128, 4, 3, 1>(g, st);
+    if (pl.kind == MID_RING_128_TWO) return launch_ring64<T, 128, 128, 4, 2, 2>(g, st);
+    if (pl.kind >= 0) return gemm_mid_launch(g, pl.kind, false, dt, st);
   }
   if (g.pair && (!ring_ok(g) || g.epi != EPI_PLAIN || g.cn != 1 || g.sat8 || g.gate || g.resid || g.pair_dA % 8 || g.pair_dB % 8 || g.pair_dbias % 8 || !aligned(g.C, 16))) {
     set_error("gemm: a pair of tiles (SiLU-gated halves) needs 16-byte aligned operands, K and the half width multiples of 8, a plain row-major output");

@@ -1,0 +1,87 @@
+"""GPU parity of the small-tile GEMM kernels (products that do not fill the chip), each of the five tiles at the edges of its tiles, of
+its stages of 64 k and of its groups of stages, and of reductions cut into slices.
+
+Bound per element: one rounding of the result to its type, and fp32 accumulation in any order (K roundings of 2^-24 of
+sum |x| |w|, K being generous)."""
+import pytest
+import torch
+
+from gpu_util import say, ulp
+
+pytestmark = pytest.mark.gpu
+
+
+def _bound(ref, mag, k, dtype):
+    return 0.5 * torch.from_numpy(ulp(ref.cpu().numpy(), dtype)).to(ref.device) * 1.01 + k * 2.0 ** -24 * mag
+
+
+def _check(out, x, w, dtype, what):
+    ref, mag = x.double() @ w.double(), x.double().abs() @ w.double().abs()
+    err = (out.double().reshape(ref.shape) - ref).abs()
+    assert torch.isfinite(out).all(), what
+    bad = err > _bound(ref, mag, x.shape[-1], dtype)
+    assert not bad.any(), f"{what}: {int(bad.sum())} of {bad.numel()} outside, worst {float(err[bad].max())}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tile", [2, 3, 4, 5, 6])
+# rows, columns, k: tiles are 32 or 64 rows by 64 or 128 columns, a wave group's stage is 64 k, up to four groups take turns
+@pytest.mark.parametrize("m,n,k", [(17, 8, 8), (31, 72, 64), (65, 136, 72), (130, 64, 328), (33, 264, 1016), (200, 56, 2560), (64, 128, 192)])
+def test_mid_tiles(m, n, k, tile, dtype):
+    from triton_funcs import _lib as L, dense_kernels as D, blast_kernels as B
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).to(dtype)
+    w = (torch.randn(k, n, device="cuda", generator=g) / k ** 0.5).to(dtype)
+    say(f"[case] mid tile {tile} {dtype} m={m} n={n} k={k}")
+    with L.options(BLR_GEMM_MID=tile, BLR_DENSE_ROWS=0):
+        _check(D.triton_dense_fp16(x, w, {"algo": L.ALGO_TILED}), x, w, dtype, "dense (k, n)")
+        # batched, both weight orders: BLAST's two products through the names that return the intermediates' arithmetic unfused
+        b = 2
+        V = (torch.randn(b, k // b if k % 16 == 0 else k, 16, device="cuda", generator=g) / k ** 0.5).to(dtype)
+        xb = torch.randn(1, m, b * V.shape[1], device="cuda", generator=g).to(dtype)
+        S = torch.zeros(16, b, b, device="cuda", dtype=dtype)
+        S[:, 0, 0] = S[:, 1, 1] = 1.0                            # no mixing: out_i = (x_i V_i) U_i^T
+        U = (torch.randn(b, n, 16, device="cuda", generator=g) / 4).to(dtype)
+        with L.options(BLR_DECODE_ROWS=0, BLR_BLAST_ONE=0, BLR_BLAST_MIXU=0):
+            out = B.triton_blast_bmm_fp16(xb, U, V, S, {"algo": L.ALGO_TILED})
+        p = V.shape[1]
+        for i in range(b):
+            y = (xb[0, :, i * p:(i + 1) * p].double() @ V[i].double())
+            mag = (xb[0, :, i * p:(i + 1) * p].double().abs() @ V[i].double().abs()) @ U[i].double().abs().t().contiguous()
+            ref = y.to(dtype).double() @ U[i].double().t().contiguous()
+            err = (out[0, :, i * n:(i + 1) * n].double() - ref).abs()
+            # y and z are rounded to dtype on the way (each may fall on the other side of a tie: one unit of y)
+            unit = torch.from_numpy(ulp(y.cpu().numpy(), dtype)).to(y.device) @ U[i].double().abs().t().contiguous()
+            assert (err <= _bound(ref, mag, p + 16, dtype) + unit).all(), (i, float(err.max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("act", [None, "silu", "silu_mul"])
+@pytest.mark.parametrize("m,n,k", [(130, 80, 8672), (257, 144, 4104), (150, 688, 10600), (279, 768, 768), (129, 3200, 9120)])
+def test_long_reductions_by_estimate(m, n, k, act, dtype):
+    """Shapes that the estimate cuts into slices (and two that it does not), plain and with an output stage."""
+    from triton_funcs import _lib as L, dense_kernels as D
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).to(dtype)
+    w = (torch.randn(k, n, device="cuda", generator=g) / k ** 0.5).to(dtype)
+    bias = torch.randn(n, device="cuda", generator=g).to(dtype) if act else None
+    say(f"[case] slices {dtype} m={m} n={n} k={k} act={act}")
+    with L.fused_epilogue(bias, act):
+        out = D.triton_dense_fp16(x, w)
+    if act is None:
+        return _check(out, x, w, dtype, "dense in slices")
+    ref, mag = x.double() @ w.double(), x.double().abs() @ w.double().abs()
+    pre = _bound(ref, mag, k, dtype)                              # what the rounded product may be off by
+    v = ref + bias.double()
+    silu = lambda t: t * torch.sigmoid(t)
+    if act == "silu":
+        want, slack = silu(v), 1.1 * pre                          # |silu'| <= 1.1
+    else:
+        h = n // 2
+        want = silu(v[:, :h]) * v[:, h:]
+        step = lambda t: torch.from_numpy(ulp(t.cpu().numpy(), dtype)).to(t.device)
+        slack = (1.1 * pre[:, :h] + 0.5 * step(silu(v[:, :h]))) * v[:, h:].abs() * 1.1 + (pre[:, h:] + 0.5 * step(v[:, h:])) * silu(v[:, :h]).abs() * 1.1
+    err = (out.double() - want).abs()
+    # the activation's exponential and reciprocal are good to a few units of fp32
+    lim = 0.51 * torch.from_numpy(ulp(want.cpu().numpy(), dtype)).to(want.device) + slack + 1e-5 * want.abs()
+    assert (err <= lim).all(), float((err / lim).max())
