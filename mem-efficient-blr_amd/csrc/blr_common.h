@@ -178,8 +178,10 @@ int gemm_launch(const GemmArgs& a, int dtype, hipStream_t st);
 enum { MID_32_64 = 0, MID_32_64_DEEP, MID_64_64, MID_64_64_DEEP, MID_64_128, MID_RING_128, MID_RING_128_TWO, MID_RING_256_SLICES, MID_KINDS };
 struct MidPlan { int kind, slices, kc; };       // kind < 0: none of them takes the product; kc: k per slice
 MidPlan gemm_mid_plan(int M, int N, int K, int batch, bool ring, bool mid, bool slices);
-bool gemm_mid_ok(const GemmArgs& a);            // whether the operands suit kinds MID_32_64 .. MID_64_128
+bool gemm_mid_ok(const GemmArgs& a, int dtype); // whether the operands suit kinds MID_32_64 .. MID_64_128, or the fp32 kernels
 int gemm_mid_launch(const GemmArgs& a, int kind, bool partial, int dtype, hipStream_t st);
+int gemm_mid_f32_slices(int M, int N, int K);   // slices that the reduction of a single fp32 product is worth cutting into
+int gemm_mid_f32_launch(const GemmArgs& a, bool partial, hipStream_t st);
 // Scratch a plain single GEMM M x N x K of dtype wants in GemmArgs::splitk_ws so that a problem with few output tiles and
 // a long reduction can be cut along K to fill the chip (fp32 partial results, summed in a fixed order).  0: no split.
 size_t gemm_splitk_bytes(int M, int N, int K, int dtype);

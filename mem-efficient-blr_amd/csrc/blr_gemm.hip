@@ -6,7 +6,7 @@
 // fragment reads bank-conflict free).  Activations and (b,q,r)-style weights are K-contiguous
 // and copied straight in; (k, n)-ordered weights (n contiguous - the layout most of the
 // reference's kernel names use) are transposed in registers on their way into LDS.
-// fp32: plain FMA tiles, used only by the *_fp32 verification names.
+// fp32: the kernels of blr_gemm_mid.hip, plain FMA tiles where the operands are not aligned to 16 bytes.
 #include <cstdlib>
 #include <mutex>
 #include <set>
@@ -972,7 +972,7 @@ __global__ __launch_bounds__(NWV * 64, (NWV / 4) * PER_CU) void gemm_ring64_kern
   TRG(4);
 }
 
-// ---- fp32 verification GEMM: 64x64 tile, 16x16 threads, 4x4 outputs per thread ---------------
+// ---- fp32 GEMM for operands without 16-byte alignment: 64x64 tile, 16x16 threads, 4x4 outputs per thread (the others: blr_gemm_mid.hip) ----
 template <bool B_KN>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs g, int tiles_m) {
   __shared__ float as[16][64 + 1];
@@ -1073,7 +1073,7 @@ static int launch_mfma(const GemmArgs& g, hipStream_t st) {
 // 8 columns per thread, the slices asked for four at a time
 template <typename T, bool EP>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ P, GemmArgs g, int splits) {
-  using V8 = typename TypeTraits<T>::vec8;
+  typedef T V8 __attribute__((ext_vector_type(8)));
   const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int vpr = g.N >> 3;
   if (v >= (int64_t)g.M * vpr) return;
@@ -1095,7 +1095,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
   V8 o;
 #pragma unroll
   for (int e = 0; e < 4; ++e) { o[e] = TypeTraits<T>::from_f32(s0[e]); o[4 + e] = TypeTraits<T>::from_f32(s1[e]); }
-  if (EP) o = ep_vector<T>(g, o, n, m);
+  if constexpr (EP) o = ep_vector<T>(g, o, n, m);
   *reinterpret_cast<V8*>(&reinterpret_cast<T*>(g.C)[(int64_t)m * g.ldc + n]) = o;
 }
 
@@ -1103,8 +1103,11 @@ template <typename T>
 static int splitk_reduce_launch(const GemmArgs& g, int splits, hipStream_t st) {
   const dim3 grid((unsigned)cdiv((int64_t)g.M * (g.N / 8), 256));
   const float* P = reinterpret_cast<const float*>(g.splitk_ws);
-  if (g.bias || g.act || g.gate || g.resid) hipLaunchKernelGGL((splitk_reduce_kernel<T, true>), grid, dim3(256), 0, st, P, g, splits);
-  else hipLaunchKernelGGL((splitk_reduce_kernel<T, false>), grid, dim3(256), 0, st, P, g, splits);
+  const bool ep = g.bias || g.act || g.gate || g.resid;
+  if constexpr (sizeof(T) == 2) {
+    if (ep) hipLaunchKernelGGL((splitk_reduce_kernel<T, true>), grid, dim3(256), 0, st, P, g, splits);
+  }
+  if (!ep) hipLaunchKernelGGL((splitk_reduce_kernel<T, false>), grid, dim3(256), 0, st, P, g, splits);
   BLR_CHECK_LAUNCH("splitk_reduce");
   return BLR_OK;
 }
@@ -1205,6 +1208,10 @@ static int launch_ring64(const GemmArgs& g, hipStream_t st) {
 }
 
 size_t gemm_splitk_bytes(int M, int N, int K, int dtype) {
+  if (dtype == BLR_F32) {
+    const int s = K % 4 || N % 8 ? 1 : gemm_mid_f32_slices(M, N, K);
+    return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+  }
   if ((dtype != BLR_F16 && dtype != BLR_BF16) || M < 96 || N % 8 || K % 8 || K < 64) return 0;
   const int cus = device_cus() > 0 ? device_cus() : 256;
   if (cdiv(M, 128) * cdiv(N, 128) > cus) return 0;
@@ -1228,11 +1235,11 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
   // Products with at most one 128 x 128 tile per compute unit: smaller tiles, and slices of a long reduction, by the estimates of
   // blr_gemm_mid.hip.  BLR_GEMM_MID = 0 switches that off, 2 .. 6 asks for one of its five tiles wherever the operands allow it.
   const int mid = option_value(OPT_GEMM_MID, 1);
-  if (mid > 1 && gemm_mid_ok(g)) return gemm_mid_launch(g, mid - 2, false, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16, st);
+  if (mid > 1 && gemm_mid_ok(g, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16)) return gemm_mid_launch(g, mid - 2, false, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16, st);
   const int64_t r128_all = cdiv(g.M, 128) * cdiv(g.N, 128) * g.batch;
   if (mid == 1 && ring == 1 && r128_all <= cus && option_value(OPT_GEMM_RING_TILE, 0) == 0) {
     constexpr int dt = std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16;
-    const bool rk = g.cn == 1 && g.M >= 96 && g.K >= 64 && ring_ok(g), mk = gemm_mid_ok(g);
+    const bool rk = g.cn == 1 && g.M >= 96 && g.K >= 64 && ring_ok(g), mk = gemm_mid_ok(g, dt);
     bool cut = option_value(OPT_GEMM_SPLITK, 1) != 0 && rk && mk && g.epi == EPI_PLAIN && g.splitk_ws && aligned(g.splitk_ws, 16) && g.batch == 1 && !g.sat8 && !g.pair;
     MidPlan pl = gemm_mid_plan(g.M, g.N, g.pair ? 2 * g.K : g.K, g.batch, rk, mk, cut);
     if (pl.slices > 1 && g.splitk_bytes < (size_t)pl.slices * g.M * g.N * sizeof(float)) pl = gemm_mid_plan(g.M, g.N, g.K, g.batch, rk, mk, false);
@@ -1337,6 +1344,18 @@ int gemm_launch(const GemmArgs& g, int dtype, hipStream_t st) {
   }
   if (dtype == BLR_F16) return pick_mfma<f16>(g, st);
   if (dtype == BLR_BF16) return pick_mfma<bf16>(g, st);
+  if (dtype == BLR_F32 && option_value(OPT_GEMM_MID, 1) && gemm_mid_ok(g, BLR_F32)) {
+    const bool cut = option_value(OPT_GEMM_SPLITK, 1) && g.splitk_ws && g.batch == 1 && g.cn == 1 && g.epi == EPI_PLAIN && !g.sat8 && g.N % 8 == 0 && aligned(g.splitk_ws, 16) &&
+                     aligned(g.C, 32) && g.ldc % 8 == 0 && !g.bias && !g.act && !g.gate && !g.resid;
+    const int s = cut ? gemm_mid_f32_slices(g.M, g.N, g.K) : 1;
+    if (s <= 1 || g.splitk_bytes < (size_t)s * g.M * g.N * sizeof(float)) return gemm_mid_f32_launch(g, false, st);
+    GemmArgs p = g;
+    p.batch = s; p.kc = (int)(cdiv(cdiv(g.K, s), 32) * 32);
+    p.sA = p.kc; p.sB = g.b_kn ? (int64_t)p.kc * g.ldb : p.kc;
+    p.C = g.splitk_ws; p.ldc = g.N; p.sC = (int64_t)g.M * g.N;
+    const int rc = gemm_mid_f32_launch(p, true, st);
+    return rc ? rc : splitk_reduce_launch<float>(g, s, st);
+  }
   if (dtype == BLR_F32) {
     int tiles_m = (int)cdiv(g.M, 64), tiles_n = (int)cdiv(g.N, 64);
     dim3 grid(tiles_m * tiles_n, g.batch);

@@ -20,9 +20,26 @@
 namespace blr {
 namespace {
 
+// What differs between the 2-byte types and fp32: a stage is 128 bytes of k (64 or 32 values), a chunk 16 bytes (8 or 4).  fp32 runs
+// on v_mfma_f32_32x32x2_f32 (fp32 products and sums; 256 flop per clock and compute unit, twice what the vector units do without
+// packed instructions): product e of a sub-step takes value e of the lanes' chunks, so lane half h adds k = 4 (2 q + h) + e.
+template <typename T> struct MidType {
+  using V = typename TypeTraits<T>::vec8;
+  static __device__ __forceinline__ f32x16 mul(V b, V a, f32x16 c) { return TypeTraits<T>::mfma32(b, a, c); }
+};
+template <> struct MidType<float> {
+  using V = f32x4;
+  static __device__ __forceinline__ f32x16 mul(V b, V a, f32x16 c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_32x32x2f32(b[e], a[e], c, 0, 0, 0);
+    return c;
+  }
+};
+
 // (k, n) stage: position of 16-byte chunk c of row k is c ^ mid_swz(k): the four rows that a transposing read touches then lie in
 // four different 32-byte groups of banks
-template <int BN> __device__ __forceinline__ int mid_swz(int k) { return BN == 32 ? ((k >> 1) & 1) << 1 : (k & 3) << 1; }
+// (fp32 reads single values, neighbouring lanes along n: nothing to spread)
+template <typename T, int BN> __device__ __forceinline__ int mid_swz(int k) { return sizeof(T) == 4 ? 0 : BN == 32 ? ((k >> 1) & 1) << 1 : (k & 3) << 1; }
 
 template <int BM, int BN, int KG, int NST>
 constexpr size_t mid_lds_bytes() {
@@ -46,8 +63,9 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
   constexpr int WGN = BN / 32 / TN, WPG = (BM / 32 / TM) * WGN, NT = WPG * KG * 64;
   constexpr int CH = TM * TN == 1 ? 2 : 1;                           // a single 32 x 32 block: even and odd sub-steps as two chains
   constexpr int GSTG = (BM + BN) * 128, LA = BM / 8, LPW = (LA + BN / 8) / WPG;
-  constexpr int RB = BN * 2, CPR = BN / 8, RPI = 1024 / RB;          // (k, n) operand: bytes and chunks of a k row, rows per load
-  using V8 = typename TypeTraits<T>::vec8;
+  constexpr int ES = sizeof(T), KS = 128 / ES, CE = 16 / ES;         // bytes of a value, k per stage, values per chunk
+  constexpr int RB = BN * ES, CPR = RB / 16, RPI = 1024 / RB;        // (k, n) operand: bytes and chunks of a k row, rows per load
+  using V8 = typename MidType<T>::V;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -56,7 +74,8 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
   const int tiles = tiles_m * tiles_n;
   int u = blockIdx.x;
   if (u < side_wgs) {                                                // the first workgroups carry the side job, if there is one
-    for (int64_t idx = (int64_t)u * NT + tid; idx < g.side.items; idx += (int64_t)side_wgs * NT) side_prep_item<T>(g.side, idx);
+    if constexpr (ES == 2)
+      for (int64_t idx = (int64_t)u * NT + tid; idx < g.side.items; idx += (int64_t)side_wgs * NT) side_prep_item<T>(g.side, idx);
     return;
   }
   u -= side_wgs;
@@ -67,31 +86,31 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
   const int m0 = (ut % tiles_m) * BM, n0 = (ut / tiles_m) * BN;
 
   const int Kloc = PARTIAL ? min(g.kc, g.K - bt * g.kc) : g.K;
-  const int KT = (Kloc + 63) >> 6, ktail = Kloc & 63;                // a partial last stage holds ktail k, a multiple of 8
+  const int KT = (Kloc + KS - 1) / KS, ktail = Kloc % KS;             // a partial last stage holds ktail k, whole chunks
   const int mine = KT > kg ? (KT - kg + KG - 1) / KG : 0;            // stages of this group
   const int steps = (KT + KG - 1) / KG;
 
-  const char* Ab0 = reinterpret_cast<const char*>(g.A) + (int64_t)bt * g.sA * 2;
-  const char* Bb0 = reinterpret_cast<const char*>(g.B) + (int64_t)bt * g.sB * 2;
+  const char* Ab0 = reinterpret_cast<const char*>(g.A) + (int64_t)bt * g.sA * ES;
+  const char* Bb0 = reinterpret_cast<const char*>(g.B) + (int64_t)bt * g.sB * ES;
   T* C = reinterpret_cast<T*>(g.C);
 
   // load li of this wave: rows 8 idx .. of A for idx = li * WPG + w < LA, else instruction idx - LA of the B stage
   const int r8 = lane >> 3, c8 = (lane & 7) ^ r8;
-  const int cmax = max((ktail >> 3) - 1, 0), rmax = max(ktail - 1, 0);
+  const int cmax = max(ktail / CE - 1, 0), rmax = max(ktail - 1, 0);
   const uint32_t tail_kc = (uint32_t)((c8 - min(c8, cmax)) * 16);    // what to step back by in a partial stage, to re-fetch valid values
   uint32_t off[LPW], tail[LPW];
 #pragma unroll
   for (int li = 0; li < LPW; ++li) {
     const int idx = li * WPG + w;
     if (idx < LA) {
-      off[li] = (uint32_t)(min(m0 + idx * 8 + r8, g.M - 1) * g.lda * 2 + c8 * 16);
+      off[li] = (uint32_t)(min(m0 + idx * 8 + r8, g.M - 1) * g.lda * ES + c8 * 16);
       tail[li] = tail_kc;
     } else if (B_KN) {
-      const int krow = (idx - LA) * RPI + lane / CPR, chunk = (lane % CPR) ^ mid_swz<BN>(krow);
-      off[li] = (uint32_t)(krow * g.ldb * 2 + min(n0 + chunk * 8, g.N - 8) * 2);
-      tail[li] = (uint32_t)((krow - min(krow, rmax)) * g.ldb * 2);
+      const int krow = (idx - LA) * RPI + lane / CPR, chunk = (lane % CPR) ^ mid_swz<T, BN>(krow);
+      off[li] = (uint32_t)(krow * g.ldb * ES + min(n0 + chunk * CE, g.N - CE) * ES);
+      tail[li] = (uint32_t)((krow - min(krow, rmax)) * g.ldb * ES);
     } else {
-      off[li] = (uint32_t)(min(n0 + (idx - LA) * 8 + r8, g.N - 1) * g.ldb * 2 + c8 * 16);
+      off[li] = (uint32_t)(min(n0 + (idx - LA) * 8 + r8, g.N - 1) * g.ldb * ES + c8 * 16);
       tail[li] = tail_kc;
     }
   }
@@ -107,9 +126,11 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
   }
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    if (B_KN) {
+    if (B_KN && ES == 4) {
+      rowB[j] = (uint32_t)(BM * 128 + half * 4 * RB + ((wn * TN + j) * 32 + (lane & 31)) * 4);
+    } else if (B_KN) {
       const int g4 = lane >> 4, i16 = lane & 15, chunk = (wn * TN + j) * 4 + (g4 & 1) * 2 + ((i16 & 3) >> 1);
-      rowB[j] = (uint32_t)(BM * 128 + ((g4 >> 1) * 8 + (i16 >> 2)) * RB + (i16 & 1) * 8 + ((chunk ^ mid_swz<BN>(i16 >> 2)) << 4));
+      rowB[j] = (uint32_t)(BM * 128 + ((g4 >> 1) * 8 + (i16 >> 2)) * RB + (i16 & 1) * 8 + ((chunk ^ mid_swz<T, BN>(i16 >> 2)) << 4));
     } else {
       const int rb = (wn * TN + j) * 32 + (lane & 31);
       rowB[j] = (uint32_t)(BM * 128 + ((rb >> 3) << 10) + ((rb & 7) << 7));
@@ -119,15 +140,16 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
   for (int q = 0; q < 4; ++q) xo[q] = (uint32_t)(((2 * q + half) ^ (lane & 7)) << 4);
 
   constexpr int NV = (BM * BN / 8 + NT - 1) / NT;                    // 8-column pieces of the tile per thread
-  V8 first[NV];                                                      // a pair: silu(first tile), kept for the second
+  typedef T out8 __attribute__((ext_vector_type(8)));
+  out8 first[NV];                                                    // a pair: silu(first tile), kept for the second
   const int halves = (EP && !PARTIAL && g.pair) ? 2 : 1;
   for (int hf = 0; hf < halves; ++hf) {
-    const char* Ab = Ab0 + (int64_t)hf * g.pair_dA * 2;
-    const char* Bb = Bb0 + (int64_t)hf * g.pair_dB * 2;
+    const char* Ab = Ab0 + (int64_t)hf * g.pair_dA * ES;
+    const char* Bb = Bb0 + (int64_t)hf * g.pair_dB * ES;
     auto issue = [&](int step, int li) {                             // load li of this group's stage number `step`
       const int s = step * KG + kg, slot = step % NST;
       const bool partial = ktail && s == KT - 1, isA = li * WPG + w < LA;
-      const char* base = isA ? Ab + (int64_t)s * 128 : Bb + (B_KN ? (int64_t)s * 64 * g.ldb * 2 : (int64_t)s * 128);
+      const char* base = isA ? Ab + (int64_t)s * 128 : Bb + (B_KN ? (int64_t)s * KS * g.ldb * ES : (int64_t)s * 128);
       ring_load_lds(base, off[li] - (partial ? tail[li] : 0u), lds0 + slot * GSTG + li * (WPG * 1024));
     };
     f32x16 acc[CH][TM][TN];
@@ -147,7 +169,10 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
       for (int i = 0; i < TM; ++i) af[set][q][i] = *reinterpret_cast<const V8*>(st + rowA[i] + xo[q]);
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        if (B_KN) {
+        if constexpr (B_KN && ES == 4) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bf[set][q][j][e] = *reinterpret_cast<const float*>(st + rowB[j] + (q * 8 + e) * RB);
+        } else if constexpr (B_KN) {
           union { V8 v; s16x4 h[2]; } x;
           x.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(st + rowB[j] + (q * 16) * RB));
           x.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(st + rowB[j] + (q * 16 + 4) * RB));
@@ -161,17 +186,17 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
       if (!(ktail && t * KG + kg == KT - 1)) return;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if ((2 * q + half) * 8 >= ktail)
+        if ((2 * q + half) * CE >= ktail)
 #pragma unroll
           for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) af[set][q][i][e] = (T)0.0f;
+            for (int e = 0; e < CE; ++e) af[set][q][i][e] = (T)0.0f;
     };
     auto products = [&](int q, int set) {                            // (operands swapped: a lane gets runs of four columns of a row)
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[q % CH][i][j] = TypeTraits<T>::mfma32(bf[set][q][j], af[set][q][i], acc[q % CH][i][j]);
+        for (int j = 0; j < TN; ++j) acc[q % CH][i][j] = MidType<T>::mul(bf[set][q][j], af[set][q][i], acc[q % CH][i][j]);
     };
     constexpr int AHEAD = PIPE ? NST : NST - 1;                      // stages asked for before the loop
 #pragma unroll
@@ -259,8 +284,8 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
     if (PARTIAL || c_vec) {
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
-        const int v = tid + n * NT, row = v / CPR, col = (v % CPR) * 8, gr = m0 + row, gc = n0 + col;
-        if (v >= BM * CPR || gr >= g.M || gc >= g.N) continue;
+        const int v = tid + n * NT, row = v / (BN / 8), col = (v % (BN / 8)) * 8, gr = m0 + row, gc = n0 + col;
+        if (v >= BM * BN / 8 || gr >= g.M || gc >= g.N) continue;
         f32x4 s0 = {0, 0, 0, 0}, s1 = {0, 0, 0, 0};
 #pragma unroll
         for (int k = 0; k < KG; ++k) {
@@ -273,23 +298,23 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
           *reinterpret_cast<f32x4*>(P + 4) = s1;
           continue;
         }
-        V8 o;
+        out8 o;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           o[e] = TypeTraits<T>::from_f32(g.sat8 ? sat8_rne(s0[e]) : s0[e]);
           o[4 + e] = TypeTraits<T>::from_f32(g.sat8 ? sat8_rne(s1[e]) : s1[e]);
         }
         const int64_t in_row = (int64_t)bt * g.sC + gc;
-        if (EP) {
+        if constexpr (EP && ES == 2) {
           if (hf == 0) o = ep_vector<T>(g, o, in_row, gr);
           else o = ep_pair_up<T>(g, o, in_row + g.pair_dbias, reinterpret_cast<const T*>(&first[n]));
           if (hf + 1 < halves) { first[n] = o; continue; }
         }
         if (g.epi == EPI_MONARCH_SCATTER) {
           const int d = gc / g.per;
-          *reinterpret_cast<V8*>(&C[(int64_t)d * g.sL + (int64_t)gr * g.ldc + (int64_t)bt * g.per + (gc - d * g.per)]) = o;
+          *reinterpret_cast<out8*>(&C[(int64_t)d * g.sL + (int64_t)gr * g.ldc + (int64_t)bt * g.per + (gc - d * g.per)]) = o;
         } else {
-          *reinterpret_cast<V8*>(&C[in_row + (int64_t)gr * g.ldc]) = o;
+          *reinterpret_cast<out8*>(&C[in_row + (int64_t)gr * g.ldc]) = o;
         }
       }
     } else {
@@ -333,11 +358,11 @@ int launch_mid(const GemmArgs& g, hipStream_t st) {
     }
   }
   // 8-column pieces of the result as one store
-  int c_vec = g.cn == 1 && g.N % 8 == 0 && aligned(g.C, 16) && g.ldc % 8 == 0 && g.sC % 8 == 0 &&
+  int c_vec = (sizeof(T) == 2 || !ep) && g.cn == 1 && g.N % 8 == 0 && aligned(g.C, 8 * sizeof(T)) && g.ldc % 8 == 0 && g.sC % 8 == 0 &&
               (!g.bias || aligned(g.bias, 16)) && (!g.gate || (aligned(g.gate, 16) && g.ld_gate % 8 == 0)) && (!g.resid || (aligned(g.resid, 16) && g.ld_resid % 8 == 0)) &&
               (g.epi == EPI_PLAIN || (g.per % 8 == 0 && g.sL % 8 == 0));
   int per_xcd = (int)cdiv(total, 8), side_wgs = 0;
-  if (!PARTIAL && g.side.items > 0 && g.side_taken) side_wgs = (int)std::min<int64_t>(cdiv(cdiv(g.side.items, NT), 8) * 8, 4096);
+  if (!PARTIAL && sizeof(T) == 2 && g.side.items > 0 && g.side_taken) side_wgs = (int)std::min<int64_t>(cdiv(cdiv(g.side.items, NT), 8) * 8, 4096);
   GemmArgs ga = g;
   void* args[] = {&ga, &tiles_m, &tiles_n, &per_xcd, &c_vec, &side_wgs};
   hipError_t e = hipLaunchKernel(fn, dim3((unsigned)(per_xcd * 8 + side_wgs)), dim3(NT), args, lds, st);
@@ -413,18 +438,45 @@ MidPlan gemm_mid_plan(int M, int N, int K, int batch, bool ring, bool mid, bool 
   return best;
 }
 
-bool gemm_mid_ok(const GemmArgs& g) {
-  if (g.N < 8 || g.K < 8 || g.K % 8 || (g.b_kn && g.N % 8)) return false;
+bool gemm_mid_ok(const GemmArgs& g, int dtype) {
+  const int es = dtype == BLR_F32 ? 4 : 2, ce = 16 / es;            // values per 16-byte chunk
+  if (g.N < ce || g.K < ce || g.K % ce || (g.b_kn && g.N % ce)) return false;
   if (g.epi != EPI_PLAIN && (g.bias || g.act || g.gate || g.resid)) return false;
-  if (!aligned(g.A, 16) || !aligned(g.B, 16) || g.lda % 8 || g.sA % 8 || g.ldb % 8 || g.sB % 8) return false;
-  if (g.pair && (g.cn != 1 || g.pair_dA % 8 || g.pair_dB % 8 || g.pair_dbias % 8 || g.N % 8 || !aligned(g.C, 16) || g.ldc % 8 || g.sC % 8 || (g.bias && !aligned(g.bias, 16)) || g.epi != EPI_PLAIN)) return false;
+  if (!aligned(g.A, 16) || !aligned(g.B, 16) || g.lda % ce || g.sA % ce || g.ldb % ce || g.sB % ce) return false;
+  if (g.pair && (es == 4 || g.cn != 1 || g.pair_dA % 8 || g.pair_dB % 8 || g.pair_dbias % 8 || g.N % 8 || !aligned(g.C, 16) || g.ldc % 8 || g.sC % 8 || (g.bias && !aligned(g.bias, 16)) || g.epi != EPI_PLAIN)) return false;
   const int64_t lim = (int64_t)1 << 32;                               // per-lane offsets are 32 bits
-  return (int64_t)(g.M - 1) * g.lda * 2 + 128 < lim && (g.b_kn ? 63 * g.ldb * 2 + (int64_t)g.N * 2 < lim : (int64_t)(g.N - 1) * g.ldb * 2 + 128 < lim);
+  return (int64_t)(g.M - 1) * g.lda * es + 128 < lim && (g.b_kn ? 63 * g.ldb * es + (int64_t)g.N * es < lim : (int64_t)(g.N - 1) * g.ldb * es + 128 < lim);
 }
 
 int gemm_mid_launch(const GemmArgs& g, int kind, bool partial, int dtype, hipStream_t st) {
   if (partial) return dtype == BLR_F16 ? mid_kind_launch<f16, true>(g, kind, st) : mid_kind_launch<bf16, true>(g, kind, st);
   return dtype == BLR_F16 ? mid_kind_launch<f16, false>(g, kind, st) : mid_kind_launch<bf16, false>(g, kind, st);
+}
+
+// fp32 at every size.  The matrix pipe bounds it: a compute unit adds 64 columns x 32 rows x 1000 k in 6.7 us, so a reduction on few
+// tiles is cut into slices while that saves more than the launch that adds them costs.  Against the 64 x 64 kernel on the vector
+// units that is still there for operands without 16-byte alignment: 128 x 128 x 192 25 -> 6 us, 35 x 768 x 3072 325 -> 11 us,
+// 1024 x 22016 x 4096 3886 -> 1492 us (47 -> 124 TFLOP/s of the 154 that a library product of 8192 cubed reaches).
+int gemm_mid_f32_slices(int M, int N, int K) {
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  const int64_t tiles = cdiv(M, 32) * cdiv(N, 64);
+  int best = 1;
+  float t_best = 1e30f;
+  for (int s = 1; s <= 16 && (s == 1 || (tiles * s <= cus && K / s >= 128)); ++s) {
+    const float t = 6.7e-3f * K / s + (s > 1 ? 2.5f + 2.f * s * M * N * 1e-6f : 0.f);
+    if (t < t_best) { t_best = t; best = s; }
+  }
+  return best > 1 ? (int)cdiv(K, cdiv(cdiv(K, best), 32) * 32) : 1;
+}
+
+int gemm_mid_f32_launch(const GemmArgs& g, bool partial, hipStream_t st) {
+  if (partial) return launch_mid<float, 32, 64, 1, 1, 4, 3, false, true>(g, st);
+  const int cus = device_cus() > 0 ? device_cus() : 256, mid = option_value(OPT_GEMM_MID, 1);
+  // 64 x 64 tiles halve the operand traffic and run two workgroups per compute unit (1024 x 22016 x 4096: 124 TFLOP/s against 94);
+  // with less than three for every four compute units the smaller tile spreads further (753 x 1152 x 1152, 216 tiles: 26.6 against
+  // 30.8 us; 128 x 3072 x 768, 96 tiles: 18.6 against 12.3 us)
+  if (mid == 3 || (mid == 1 && cdiv(g.M, 64) * cdiv(g.N, 64) * g.batch * 4 < 3 * cus)) return launch_mid<float, 32, 64, 1, 1, 4, 3, false, false>(g, st);
+  return launch_mid<float, 64, 64, 1, 1, 2, 2, false, false>(g, st);
 }
 
 }  // namespace blr

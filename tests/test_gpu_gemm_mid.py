@@ -55,6 +55,31 @@ def test_mid_tiles(m, n, k, tile, dtype):
             assert (err <= _bound(ref, mag, p + 16, dtype) + unit).all(), (i, float(err.max()))
 
 
+@pytest.mark.parametrize("tile", [1, 3, 5])
+# fp32 stages hold 32 k; the last two are cut into slices (only by the estimate, tile 1), 6 columns go to the kernel for unaligned operands
+@pytest.mark.parametrize("m,n,k", [(1, 8, 4), (31, 72, 36), (65, 136, 100), (33, 6, 64), (100, 64, 1028), (35, 768, 3072), (64, 8, 5000)])
+def test_fp32(m, n, k, tile):
+    from triton_funcs import _lib as L, dense_kernels as D, monarch_kernels as Mo
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+    x, w = torch.randn(m, k, device="cuda", generator=g), torch.randn(k, n, device="cuda", generator=g) / k ** 0.5
+    say(f"[case] fp32 tile {tile} m={m} n={n} k={k}")
+    with L.options(BLR_GEMM_MID=tile):
+        out = D.triton_dense_fp32(x, w)
+        ref, mag = x.double() @ w.double(), x.double().abs() @ w.double().abs()
+        # fp32 sums in any order: k roundings of 2^-24 of sum |x| |w|, and one of the result
+        assert ((out.double() - ref).abs() <= (k + 1) * 2.0 ** -24 * mag).all()
+        # the scatter of Monarch's first product and its interleaved result
+        w1, w2 = torch.randn(2, k, 8, device="cuda", generator=g) / k ** 0.5, torch.randn(2, n, 8, device="cuda", generator=g)
+        xm = torch.randn(1, m, 2 * k, device="cuda", generator=g)
+        got, out1, pre = Mo.triton_monarch_right_fp32(xm, w1, w2)
+        p1 = torch.stack([xm[0, :, i * k:(i + 1) * k].double() @ w1[i].double() for i in range(2)])
+        m1 = torch.stack([xm[0, :, i * k:(i + 1) * k].double().abs() @ w1[i].double().abs() for i in range(2)])
+        assert ((pre.double() - p1).abs() <= (k + 1) * 2.0 ** -24 * m1).all()
+        o2 = torch.stack([out1[i].double() @ w2[i].double().t().contiguous() for i in range(2)], dim=-1).reshape(m, -1)
+        m2 = torch.stack([out1[i].double().abs() @ w2[i].double().abs().t().contiguous() for i in range(2)], dim=-1).reshape(m, -1)
+        assert ((got[0].double() - o2).abs() <= 9 * 2.0 ** -24 * m2).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("act", [None, "silu", "silu_mul"])
 @pytest.mark.parametrize("m,n,k", [(130, 80, 8672), (257, 144, 4104), (150, 688, 10600), (279, 768, 768), (129, 3200, 9120)])
