@@ -269,6 +269,12 @@ int blr_blast_fwd_ep2(const void* x, int64_t ldx, const void* U, const void* V, 
                       int dtype, int u_layout, int s_layout, int algo,
                       void* ws, size_t ws_bytes, void* stream, const void* bias, int act,
                       const void* gate, int gate_rows, int64_t ld_gate, const void* resid, int64_t ld_resid);
+int blr_blast_q_fwd_ep2(const void* x, int64_t ldx, const void* u_codes, const void* u_scales,
+                        const void* v_codes, const void* v_scales, const void* S,
+                        void* out, int64_t ldo, int M, int in_f, int out_f, int b, int r,
+                        int dtype, int bits, int algo,
+                        void* ws, size_t ws_bytes, void* stream, const void* bias, int act,
+                        const void* gate, int gate_rows, int64_t ld_gate, const void* resid, int64_t ld_resid);
 int blr_monarch_fwd_ep2(const void* x, int64_t ldx, const void* w1, const void* w2,
                         void* out, int64_t ldo, int M, int in_f, int out_f, int b, int rank,
                         int dtype, int w2_layout, int out_order, int algo,

@@ -1,6 +1,6 @@
-"""Build libblr.so (the HIP kernels and their C ABI) for gfx950, in-tree, and the stand-alone probes under probes/.
+"""Build libblr.so (the HIP kernels and their C ABI) for gfx950, in-tree, the shims' native call path and the stand-alone probes.
 
-    python build.py            # -> lib/libblr.so next to this file, probes/<name> next to probes/<name>.hip
+    python build.py            # -> lib/libblr.so, lib/_blr_host.so next to this file, probes/<name> next to probes/<name>.hip
 
 Plain hipcc, no build system.  Objects are compiled in parallel, then linked.
 """
@@ -48,6 +48,17 @@ def build(verbose=True):
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", so])
     if verbose:
         print(f"built {so}")
+    # the native call path of the Python shims: host code against this torch's headers, no device code
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    host = os.path.join(HERE, "lib", "_blr_host.so")
+    out = _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", "-Wno-deprecated-declarations",
+                f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
+                os.path.join(HERE, "csrc", "blr_host.cpp"), "-o", host,
+                f"-L{root}/lib", "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10_hip", "-lc10"])
+    if verbose:
+        print(out.strip() or f"built {host}")
     # the stand-alone probes (not part of the library): built next to their sources so that they compile as long as the tree does
     probes = [n[:-4] for n in sorted(os.listdir(os.path.join(HERE, "probes"))) if n.endswith(".hip")]
     with ThreadPoolExecutor(max_workers=max(1, len(probes))) as ex:

@@ -499,7 +499,7 @@ int blr_blast_q_fwd(const void* x, int64_t ldx, const void* u_codes, const void*
   // rows of codes that are not whole 16-byte pieces (r = 1488 at 4 bits: 744 bytes) are served by the three-launch path only,
   // whose lanes fetch 8 columns (8 or 4 bytes) at a time
   const bool whole16 = ((int64_t)r * bits) % 128 == 0 && ((int64_t)(out_f / b) * bits) % 128 == 0;
-  if (ldx < in_f || ldo < out_f) { set_error("blast_q: leading dimension too small"); return BLR_ERR_BAD_ARG; }
+  if (ldx < in_f || ldo < (silu_mul_armed() ? out_f / 2 : out_f)) { set_error("blast_q: leading dimension too small"); return BLR_ERR_BAD_ARG; }
   if (!aligned(u_codes, 16) || !aligned(v_codes, 16)) { set_error("blast_q: code buffers must be 16-byte aligned"); return BLR_ERR_BAD_ARG; }
   hipStream_t st = (hipStream_t)stream;
   const bool phase_engine = algo == BLR_ALGO_STREAM || algo == BLR_ALGO_STREAM_SPLIT;
@@ -800,6 +800,16 @@ int blr_blast_fwd_ep2(const void* x, int64_t ldx, const void* U, const void* V, 
                       const void* gate, int gate_rows, int64_t ld_gate, const void* resid, int64_t ld_resid) {
   return with_epilogue(BLR_OP_BLAST, b, bias, act, out, ldo, M, out_f, dtype, ws, ws_bytes, stream, [&](void* o, int64_t ld, size_t wsb) {
     return blr_blast_fwd(x, ldx, U, V, S, o, ld, nullptr, nullptr, M, in_f, out_f, b, r, dtype, u_layout, s_layout, algo, ws, wsb, stream);
+  }, {gate, gate_rows, ld_gate, resid, ld_resid});
+}
+
+int blr_blast_q_fwd_ep2(const void* x, int64_t ldx, const void* u_codes, const void* u_scales,
+                        const void* v_codes, const void* v_scales, const void* S,
+                        void* out, int64_t ldo, int M, int in_f, int out_f, int b, int r,
+                        int dtype, int bits, int algo, void* ws, size_t ws_bytes, void* stream, const void* bias, int act,
+                        const void* gate, int gate_rows, int64_t ld_gate, const void* resid, int64_t ld_resid) {
+  return with_epilogue(BLR_OP_BLAST, b, bias, act, out, ldo, M, out_f, dtype, ws, ws_bytes, stream, [&](void* o, int64_t ld, size_t wsb) {
+    return blr_blast_q_fwd(x, ldx, u_codes, u_scales, v_codes, v_scales, S, o, ld, M, in_f, out_f, b, r, dtype, bits, algo, ws, wsb, stream);
   }, {gate, gate_rows, ld_gate, resid, ld_resid});
 }
 

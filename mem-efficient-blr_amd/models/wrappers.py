@@ -20,6 +20,9 @@ import math
 import torch
 import torch.nn as nn
 
+from triton_funcs import _lib as L
+from triton_funcs.blast_sym_quant_kernels import QuantFactor
+
 
 def resolve(func_path):
     module_name, func_name = func_path.rsplit(".", 1)
@@ -49,15 +52,26 @@ class _StructuredLinear(nn.Module):
     def _param(self, shape, fan_in):
         return nn.Parameter(torch.randn(shape, device=self.device, dtype=torch.float32).mul_(1.0 / math.sqrt(fan_in)).to(self.dtype))
 
+    def _stage(self):
+        """The output stage to hand to the kernel (bias, act, gate, gate_rows, residual), or None; takes a gate / residual that the
+        caller has armed."""
+        bias, act = self._parameters["bias"], self.fused_act
+        outer = getattr(L._ep_state, "outer", None)
+        if bias is None and act is None and outer is None:
+            return None
+        if act not in L.ACTS:
+            raise L.BlrError(f"unknown activation {act!r}")
+        if outer is None:
+            return bias, L.ACTS[act], None, 0, None
+        L._ep_state.outer = None
+        return (bias, L.ACTS[act]) + outer
+
     def _call(self, *args):
         """The forward function; library kernels take bias and activation into their output stage."""
-        if not self.fuses:
+        stage = self._stage() if self.fuses else None
+        if stage is None:
             return self.func(*args), False
-        from triton_funcs import _lib as L
-        if self.bias is None and self.fused_act is None and getattr(L._ep_state, "outer", None) is None:
-            return self.func(*args), False
-        with L.fused_epilogue(self.bias, self.fused_act):          # (also picks up a gate / residual armed by the caller)
-            return self.func(*args), True
+        return self.func.with_epilogue(*args, stage), True
 
     def _finish(self, out, fused=False):
         if isinstance(out, tuple):                     # torch baselines and the *_fp32 names: (out, intermediates...)
@@ -93,7 +107,8 @@ class BlastLinear(_StructuredLinear):
             self.S = self._param((b, b, rank), 1)
 
     def forward(self, x):
-        return self._finish(*self._call(x, self.U, self.V, self.S))
+        p = self._parameters
+        return self._finish(*self._call(x, p["U"], p["V"], p["S"]))
 
     def extra_repr(self):
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "
@@ -132,13 +147,11 @@ class QuantBlastLinear(BlastLinear):
 
     @property
     def Uq(self):
-        from triton_funcs.blast_sym_quant_kernels import QuantFactor
-        return QuantFactor(self.u_codes, self.u_scales, self.bits, self._u_shape)
+        return QuantFactor(self._buffers["u_codes"], self._buffers["u_scales"], self.bits, self._u_shape)
 
     @property
     def Vq(self):
-        from triton_funcs.blast_sym_quant_kernels import QuantFactor
-        return QuantFactor(self.v_codes, self.v_scales, self.bits, self._v_shape)
+        return QuantFactor(self._buffers["v_codes"], self._buffers["v_scales"], self.bits, self._v_shape)
 
     def get_extra_state(self):
         return {"format": self.PACK_FORMAT, "bits": self.bits, "u_shape": list(self._u_shape), "v_shape": list(self._v_shape)}
@@ -163,7 +176,13 @@ class QuantBlastLinear(BlastLinear):
         super()._load_from_state_dict(state_dict, prefix, local_metadata, strict, missing_keys, unexpected_keys, error_msgs)
 
     def forward(self, x):
-        return self._finish(self.func(x, self.Uq, self.Vq, self.S))
+        args = (x, self.Uq, self.Vq, self._parameters["S"])
+        bias = self._parameters["bias"]
+        if (bias is not None or self.fused_act is not None) and not self.is_compiled and self.fused_act in L.ACTS:
+            out = self.func.with_epilogue(*args, (bias, L.ACTS[self.fused_act], None, 0, None))
+            if out is not None:
+                return out
+        return self._finish(self.func(*args))
 
 
 class MonarchLinear(_StructuredLinear):
@@ -181,7 +200,8 @@ class MonarchLinear(_StructuredLinear):
             self.w2_bfly = self._param((b, s, rank), rank)
 
     def forward(self, x):
-        return self._finish(*self._call(x, self.w1_bfly, self.w2_bfly))
+        p = self._parameters
+        return self._finish(*self._call(x, p["w1_bfly"], p["w2_bfly"]))
 
     def extra_repr(self):
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "
@@ -200,8 +220,8 @@ class LowRankLinear(_StructuredLinear):
             self.U = self._param((out_features, rank), rank)
 
     def forward(self, x):
-        out, fused = self._call(x, self.V, self.U)
-        if self.kind == "triton" and not isinstance(out, tuple):   # the kernel returns (N, out_f): restore the leading dims
+        out, fused = self._call(x, self._parameters["V"], self._parameters["U"])
+        if not fused and self.kind == "triton" and not isinstance(out, tuple):   # the kernel returns (N, out_f): restore the leading dims
             out = out.reshape(*x.shape[:-1], out.shape[-1])
         return self._finish(out, fused)
 
@@ -216,8 +236,8 @@ class DenseLinear(_StructuredLinear):
         self.W = self._param(shape, in_features)
 
     def forward(self, x):
-        out, fused = self._call(x, self.W)
-        if self.kind == "triton" and not isinstance(out, tuple):
+        out, fused = self._call(x, self._parameters["W"])
+        if not fused and self.kind == "triton" and not isinstance(out, tuple):
             out = out.reshape(*x.shape[:-1], out.shape[-1])
         return self._finish(out, fused)
 

@@ -7,12 +7,15 @@ fails, the caller gets an exception.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
+import warnings
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
+HOST_PATH = os.path.join(_HERE, "..", "lib", "_blr_host.so")
 LIB_PATH = os.environ.get("BLR_LIB", os.path.join(_HERE, "..", "lib", "libblr.so"))
 
 # enums of include/blr.h
@@ -52,6 +55,7 @@ _SIGNATURES = {
     "blr_low_rank_fwd_ep": (_i, [_vp, _i64, _vp, _vp, _vp, _i64] + [_i] * 6 + [_vp, _sz, _vp, _vp, _i]),
     "blr_dense_fwd_ep": (_i, [_vp, _i64, _vp, _vp, _i64] + [_i] * 5 + [_vp, _sz, _vp, _vp, _i]),
     "blr_blast_fwd_ep2": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _i64] + [_i] * 9 + [_vp, _sz, _vp, _vp, _i, _vp, _i, _i64, _vp, _i64]),
+    "blr_blast_q_fwd_ep2": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64] + [_i] * 8 + [_vp, _sz, _vp, _vp, _i, _vp, _i, _i64, _vp, _i64]),
     "blr_monarch_fwd_ep2": (_i, [_vp, _i64, _vp, _vp, _vp, _i64] + [_i] * 9 + [_vp, _sz, _vp, _vp, _i, _vp, _i, _i64, _vp, _i64]),
     "blr_low_rank_fwd_ep2": (_i, [_vp, _i64, _vp, _vp, _vp, _i64] + [_i] * 6 + [_vp, _sz, _vp, _vp, _i, _vp, _i, _i64, _vp, _i64]),
     "blr_dense_fwd_ep2": (_i, [_vp, _i64, _vp, _vp, _i64] + [_i] * 5 + [_vp, _sz, _vp, _vp, _i, _vp, _i, _i64, _vp, _i64]),
@@ -94,6 +98,35 @@ def lib():
                     fn.restype, fn.argtypes = res, args
                 _lib = handle
     return _lib
+
+
+# The native call path (lib/_blr_host.so): what the shims do per call - shape checks, workspace, allocation, stream - without
+# Python in between.  It takes the regular calls and declines (None) the rest, which then go through the code below.  It is bound
+# to one build of torch; where it is missing or does not load, every call takes the Python path.
+_host = None
+
+
+def _load_host():
+    global _host
+    handle = lib()
+    with _lock:
+        if _host is None:
+            _host = False
+            if os.path.exists(HOST_PATH):
+                try:
+                    spec = importlib.util.spec_from_file_location("_blr_host", os.path.abspath(HOST_PATH))
+                    mod = importlib.util.module_from_spec(spec)
+                    spec.loader.exec_module(mod)
+                    mod.bind({n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value for n in _SIGNATURES}, BlrError)
+                    _host = mod
+                except (ImportError, OSError) as e:
+                    warnings.warn(f"{HOST_PATH} does not load ({e}): calls take the slower Python path")
+    return _host
+
+
+def call_path():
+    """The native call path, or something false: not there, or debug checks are on (they follow every call from Python)."""
+    return False if _debug_checks else _host if _host is not None else _load_host()
 
 
 ERR_TIMEOUT = -7
@@ -175,8 +208,13 @@ _workspaces = {}
 def workspace(device, nbytes, algo=ALGO_AUTO, M=None, dtype=None):
     streaming = algo in (ALGO_STREAM, ALGO_STREAM_SPLIT) or (
         algo == ALGO_AUTO and M is not None and M <= 16 and dtype != F32)
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(device).cuda_stream, "stream" if streaming else "scratch")
+    index, stream = device.index if device.index is not None else torch.cuda.current_device(), torch.cuda.current_stream(device).cuda_stream
+    host = _host if _host is not None else _load_host()
+    if host:                                           # one set of workspaces for both paths: the streaming ones carry state
+        ws = host.workspace(index, stream, int(nbytes), int(streaming))
+        ws._blr_streaming = streaming
+        return ws
+    key = (index, stream, "stream" if streaming else "scratch")
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         size = max(int(nbytes), 1 << 20)
@@ -255,6 +293,26 @@ class fused_epilogue:
         return False
 
 
+class armed:
+    """with armed(ep): the output stage `ep` (bias, act code, gate, gate_rows, residual) for the calls of the block."""
+
+    def __init__(self, ep):
+        self.ep = ep
+
+    def __enter__(self):
+        self.prev = getattr(_ep_state, "ep", None)
+        _ep_state.ep = self.ep
+
+    def __exit__(self, *exc):
+        _ep_state.ep = self.prev
+        return False
+
+
+def armed_epilogue():
+    """The output stage that the active context arms on this thread, as (bias, act, gate, gate_rows, residual), or None."""
+    return getattr(_ep_state, "ep", None)
+
+
 def ep_out_features(ep, out_f):
     """Columns of the result: out_f, or out_f / 2 under the gated activation (silu(gate) * up over a fused gate|up projection)."""
     return out_f // 2 if ep is not None and ep[1] == ACT_SILU_MUL else out_f
@@ -278,7 +336,9 @@ def pending_epilogue(out_f, dtype, device):
         bias = bias.detach().to(device=device, dtype=dtype).contiguous()
     extra = [None, 0, 0, None, 0]
     if gate is not None:
-        gate = gate.detach().to(device=device, dtype=dtype).reshape(-1, out_f).contiguous()
+        gate = gate.detach().to(device=device, dtype=dtype).reshape(-1, out_f)
+        if gate.stride(-1) != 1:
+            gate = gate.contiguous()
         extra[0:3] = [gate.data_ptr(), gate_rows, gate.stride(0)]
     if resid is not None:
         resid = resid.detach().to(device=device, dtype=dtype).reshape(-1, out_f)

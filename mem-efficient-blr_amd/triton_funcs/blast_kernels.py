@@ -89,11 +89,21 @@ def _blast(name, x, U, V, S, u_layout, s_layout, algo, want_intermediates):
 
 
 def _fp16(name, x, U, V, S, config, u_layout, s_layout):
+    host = L.call_path()
+    if host:
+        out = host.blast(name, _last_config, x, U, V, S, u_layout, s_layout, 0 if config is None else _algo_from(config), 0, L.armed_epilogue())
+        if out is not None:
+            return out
     assert x.dtype in (torch.float16, torch.bfloat16), "the *_fp16 names take fp16 or bf16 tensors"
     return _blast(name, x, U, V, S, u_layout, s_layout, _algo_from(config), False)[0]
 
 
 def _fp32(name, x, U, V, S, u_layout, s_layout):
+    host = L.call_path()
+    if host:
+        out = host.blast(name, _last_config, x, U, V, S, u_layout, s_layout, L.ALGO_TILED, 1, None)
+        if out is not None:
+            return out
     assert x.dtype == torch.float32                   # reference launcher asserts float32
     return _blast(name, x, U, V, S, u_layout, s_layout, L.ALGO_TILED, True)
 
@@ -140,6 +150,26 @@ def triton_blast_bmm_fp32(x, U, V, S):
 
 def triton_blast_bmm_fp16(x, U, V, S, config=(None, None, None)):
     return _fp16("triton_blast_bmm_fp16", x, U, V, S, config, L.U_QR, L.S_RIJ)
+
+
+# -- the wrapper modules' way in: the same call with its output stage (bias, act, gate, gate_rows, residual) as an argument ---------
+def _with_epilogue(func, u_layout, s_layout):
+    name = func.__name__
+
+    def call(x, U, V, S, ep):
+        host = L.call_path()
+        if host:
+            out = host.blast(name, _last_config, x, U, V, S, u_layout, s_layout, 0, 0, ep)
+            if out is not None:
+                return out
+        with L.armed(ep):
+            return func(x, U, V, S)
+    func.with_epilogue = call
+
+
+for _f in (triton_blast_partial_fp16, triton_blast_partial_grouped_fp16, triton_blast_partial_grouped_persistent_fp16, triton_blast_full_fp16):
+    _with_epilogue(_f, L.U_RQ, L.S_JIR)
+_with_epilogue(triton_blast_bmm_fp16, L.U_QR, L.S_RIJ)
 
 
 # -- tuning records (picklable; None until the function has run) ------------------------------------

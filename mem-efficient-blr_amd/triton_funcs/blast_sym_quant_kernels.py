@@ -115,6 +115,11 @@ def _blast_bmm_i8act(x, U, V, S):
 
 
 def triton_blast_bmm_int8_fp16(x, U, V, S, config=(None, None, None)):
+    host = L.call_path()
+    if host:
+        out = host.blast_q("triton_blast_bmm_int8_fp16", _last_config, x, U, V, S, int(config.get("algo", L.ALGO_AUTO)) if isinstance(config, dict) else 0, None)
+        if out is not None:
+            return out
     if isinstance(U, torch.Tensor) and isinstance(V, torch.Tensor):
         return _blast_bmm_i8act(x, U, V, S)
     if not (isinstance(U, QuantFactor) and isinstance(V, QuantFactor)):
@@ -149,6 +154,17 @@ def triton_blast_bmm_int8_fp16(x, U, V, S, config=(None, None, None)):
 def triton_blast_bmm_int4_fp16(x, U, V, S, config=(None, None, None)):
     assert isinstance(U, QuantFactor) and U.bits == 4
     return triton_blast_bmm_int8_fp16(x, U, V, S, config)
+
+
+def _with_epilogue(x, U, V, S, ep):
+    """The wrapper modules' way in: the output stage (bias, act, gate, gate_rows, residual) as an argument.  None where only the
+    plain call is to be had."""
+    host = L.call_path()
+    return host.blast_q("triton_blast_bmm_int8_fp16", _last_config, x, U, V, S, 0, ep) if host else None
+
+
+triton_blast_bmm_int8_fp16.with_epilogue = _with_epilogue
+triton_blast_bmm_int4_fp16.with_epilogue = _with_epilogue
 
 
 def get_triton_blast_bmm_xv_int8_fp16_config():

@@ -16,6 +16,11 @@ _last_config = {}
 
 
 def _dense(name, x, w, algo):
+    host = L.call_path()
+    if host:
+        out = host.dense(name, _last_config, x, w, algo, int(name == "triton_dense_fp32"), 0, L.armed_epilogue())
+        if out is not None:
+            return out
     L.require_gpu(x, w)
     assert x.shape[-1] == w.shape[0], "Incompatible dimensions"
     assert w.is_contiguous(), "Matrix W must be contiguous"
@@ -48,6 +53,21 @@ def triton_dense_fp16(x, w, config=None):
     assert x.dtype in (torch.float16, torch.bfloat16)
     algo = int(config.get("algo", L.ALGO_AUTO)) if isinstance(config, dict) else L.ALGO_AUTO
     return _dense("triton_dense_fp16", x, w, algo)
+
+
+def _with_epilogue(x, w, ep):
+    """The wrapper modules' way in: the output stage (bias, act, gate, gate_rows, residual) as an argument, leading sizes kept."""
+    host = L.call_path()
+    if host:
+        out = host.dense("triton_dense_fp16", _last_config, x, w, 0, 0, 1, ep)
+        if out is not None:
+            return out
+    with L.armed(ep):
+        out = triton_dense_fp16(x, w)
+    return out.reshape(*x.shape[:-1], out.shape[-1])
+
+
+triton_dense_fp16.with_epilogue = _with_epilogue
 
 
 def _probe(x, w):

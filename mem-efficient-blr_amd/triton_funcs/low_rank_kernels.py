@@ -16,6 +16,11 @@ _last_config = {}
 
 
 def _low_rank(name, x, a, b, algo, want_z):
+    host = L.call_path()
+    if host:
+        got = host.low_rank(name, _last_config, x, a, b, algo, int(want_z), 0, None if want_z else L.armed_epilogue())
+        if got is not None:
+            return got if want_z else (got, None)
     L.require_gpu(x, a, b)
     assert x.shape[-1] == a.shape[0] and a.shape[1] == b.shape[0], "Incompatible dimensions"
     assert a.is_contiguous(), "Matrix A must be contiguous"
@@ -51,6 +56,21 @@ def triton_low_rank_fp16(x, a, b, config=None):
     assert x.dtype in (torch.float16, torch.bfloat16)
     algo = int(config.get("algo", L.ALGO_AUTO)) if isinstance(config, dict) else L.ALGO_AUTO
     return _low_rank("triton_low_rank_fp16", x, a, b, algo, False)[0]
+
+
+def _with_epilogue(x, a, b, ep):
+    """The wrapper modules' way in: the output stage (bias, act, gate, gate_rows, residual) as an argument, leading sizes kept."""
+    host = L.call_path()
+    if host:
+        out = host.low_rank("triton_low_rank_fp16", _last_config, x, a, b, 0, 0, 1, ep)
+        if out is not None:
+            return out
+    with L.armed(ep):
+        out = triton_low_rank_fp16(x, a, b)
+    return out.reshape(*x.shape[:-1], out.shape[-1])
+
+
+triton_low_rank_fp16.with_epilogue = _with_epilogue
 
 
 def _probe(x, a, b):

@@ -35,6 +35,11 @@ def _algo_from(config):
 
 
 def _monarch(name, x, w1, w2, w2_layout, out_order, algo, want_out1):
+    host = L.call_path()
+    if host:
+        got = host.monarch(name, _last_config, x, w1, w2, w2_layout, out_order, algo, int(want_out1), None if want_out1 else L.armed_epilogue())
+        if got is not None:
+            return got if want_out1 else (got, None)
     L.require_gpu(x, w1, w2)
     k, p, q = w1.shape
     if w2_layout == L.W2_SR:
@@ -95,7 +100,7 @@ def triton_monarch_right_fp32(x, w1_bfly, w2_bfly_t):
 
 def triton_monarch_right_fp16(x, w1_bfly, w2_bfly_t, config=None):
     assert x.dtype in (torch.float16, torch.bfloat16)
-    return _monarch("triton_monarch_right_fp16", x, w1_bfly, w2_bfly_t, L.W2_SR, L.OUT_INTERLEAVED, _algo_from(config), False)[0]
+    return _monarch("triton_monarch_right_fp16", x, w1_bfly, w2_bfly_t, L.W2_SR, L.OUT_INTERLEAVED, 0 if config is None else _algo_from(config), False)[0]
 
 
 def triton_monarch_right_ideal_fp32(x, w1_bfly, w2_bfly_t):
@@ -118,6 +123,26 @@ def triton_monarch_right_left_fp32(x, w1_bfly, w2_bfly):
 def triton_monarch_right_left_fp16(x, w1_bfly, w2_bfly, config=(None, None)):
     assert x.dtype in (torch.float16, torch.bfloat16)
     return _monarch("triton_monarch_right_left_fp16", x, w1_bfly, w2_bfly, L.W2_RS, L.OUT_INTERLEAVED, _algo_from(config), False)[0]
+
+
+# the wrapper modules' way in: the same call with its output stage (bias, act, gate, gate_rows, residual) as an argument
+def _with_epilogue(func, w2_layout, out_order):
+    name = func.__name__
+
+    def call(x, w1, w2, ep):
+        host = L.call_path()
+        if host:
+            out = host.monarch(name, _last_config, x, w1, w2, w2_layout, out_order, 0, 0, ep)
+            if out is not None:
+                return out
+        with L.armed(ep):
+            return func(x, w1, w2)
+    func.with_epilogue = call
+
+
+_with_epilogue(triton_monarch_right_fp16, L.W2_SR, L.OUT_INTERLEAVED)
+_with_epilogue(triton_monarch_right_ideal_fp16, L.W2_SR, L.OUT_BLOCKED)
+_with_epilogue(triton_monarch_right_left_fp16, L.W2_RS, L.OUT_INTERLEAVED)
 
 
 def get_triton_monarch_right_fp16_config():
