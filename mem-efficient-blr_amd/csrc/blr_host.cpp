@@ -43,7 +43,8 @@ struct Api {
 PyObject* blr_error = nullptr;                     // triton_funcs._lib.BlrError
 
 // ---- workspaces: one per (device, stream, kind), kept until the process ends (the shims' contract; see _lib.workspace) -------
-std::map<std::tuple<int, void*, bool>, at::Tensor> workspaces;    // (only touched with the interpreter lock held)
+// Only touched with the interpreter lock held, and never destroyed: the process may end after the device runtime did.
+auto& workspaces = *new std::map<std::tuple<int, void*, bool>, at::Tensor>;
 
 const at::Tensor& workspace(const at::Device& dev, void* stream, size_t bytes, bool streaming) {
   at::Tensor& ws = workspaces[{dev.index(), stream, streaming}];
@@ -53,7 +54,8 @@ const at::Tensor& workspace(const at::Device& dev, void* stream, size_t bytes, b
 }
 
 // ---- what a call looks at ---------------------------------------------------------------------------------------------------
-const at::Tensor* tensor(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+// (plain tensors and parameters: a subclass may mean something else by its data)
+const at::Tensor* tensor(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
 
 int dtype_code(at::ScalarType t) { return t == at::kHalf ? BLR_F16 : t == at::kBFloat16 ? BLR_BF16 : t == at::kFloat ? BLR_F32 : -1; }
 
@@ -120,7 +122,7 @@ at::Tensor result(const at::Tensor& x, bool lead, int64_t M, int64_t columns) {
 
 // The record that get_*_config() hands out: made anew only when something about the call changed.
 struct Record {
-  PyObject* made = nullptr;                        // the dict in `rec` that these values describe (borrowed; compared, never read)
+  PyObject* made = nullptr;                        // the dict in `rec` that these values describe (held, so that its address stays its own)
   int64_t v[8] = {};
 };
 std::map<std::pair<PyObject*, PyObject*>, Record> records;
@@ -137,10 +139,11 @@ bool record(PyObject* rec, PyObject* name, const at::Tensor& x, const char* cons
   for (int i = 0; ok && i < n; ++i) ok = put(keys[i], PyLong_FromLongLong(v[i]));
   if (ok && dtype) ok = put("dtype", PyUnicode_FromString(x.scalar_type() == at::kHalf ? "torch.float16" : x.scalar_type() == at::kBFloat16 ? "torch.bfloat16" : "torch.float32"));
   ok = ok && PyDict_SetItem(rec, name, d) == 0;
+  Py_XDECREF(r.made);
   r.made = ok ? d : nullptr;
   for (int i = 0; i < n; ++i) r.v[i] = v[i];
   r.v[7] = t;
-  Py_DECREF(d);
+  if (!ok) Py_DECREF(d);
   return ok;
 }
 
