@@ -307,6 +307,13 @@ int blr_blast_fwd_static(const void* x, int64_t ldx, const void* U, const void* 
                          void* out, int64_t ldo, int M, int in_f, int out_f, int b, int r,
                          int dtype, int u_layout, int s_layout, void* stream);
 
+/* ---- between the linears of a DiT block ----------------------------------------------------------
+ * out = (1 + scale[g]) * LayerNorm(x) + shift[g], g = row / rows_per_group, LayerNorm without an affine part (reference
+ * DiT/models.py:19-20, 120-121).  x, out: (rows, cols) contiguous; shift, scale: one row per group, ld_* apart (column chunks of
+ * the adaLN projection).  f16 / bf16, cols % 8 == 0, cols <= 2048, 16-byte aligned; else BLR_ERR_UNSUPPORTED.  fp32 inside.  */
+int blr_ln_modulate(const void* x, const void* shift, int64_t ld_shift, const void* scale, int64_t ld_scale, void* out,
+                    int rows, int cols, int rows_per_group, float eps, int dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

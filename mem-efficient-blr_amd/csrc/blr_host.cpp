@@ -10,6 +10,7 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -38,6 +39,7 @@ struct Api {
   decltype(&blr_dense_fwd) dense;
   decltype(&blr_dense_fwd_ep2) dense_ep;
   decltype(&blr_ep_workspace_bytes) ep_ws;
+  decltype(&blr_ln_modulate) ln_modulate;
   decltype(&blr_last_error) last_error;
 } api = {};
 PyObject* blr_error = nullptr;                     // triton_funcs._lib.BlrError
@@ -363,6 +365,47 @@ PyObject* dense(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// The entries below stand in for torch operators, which autograd, autocast, transforms and dispatch modes see: a call that any of
+// those has a part in is left to torch.
+bool torch_modes_off() {
+  const auto tls = c10::impl::tls_local_dispatch_key_set();
+  return (tls.included_ - c10::default_included_set).empty() && !at::autocast::is_autocast_enabled(at::kCUDA);
+}
+bool plain(const at::Tensor& t) {
+  return t.is_cuda() && t.layout() == at::kStrided && !(at::GradMode::is_enabled() && t.requires_grad()) && !t._fw_grad(0).defined() &&
+         !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                                   c10::DispatchKey::Functionalize, c10::DispatchKey::Negative, c10::DispatchKey::Conjugate, c10::DispatchKey::ZeroTensor}));
+}
+bool aligned16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+// ln_modulate(x, shift, scale, eps): x (images, tokens, columns), shift and scale (images, columns) or column chunks of a wider matrix
+PyObject* ln_modulate(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  ENTER(4)
+  const at::Tensor *x = tensor(args[0]), *sh = tensor(args[1]), *sc = tensor(args[2]);
+  const double eps = PyFloat_AsDouble(args[3]);
+  if (PyErr_Occurred() || !x || !sh || !sc || !torch_modes_off() || !plain(*x) || !plain(*sh) || !plain(*sc)) DECLINE;
+  const int dt = dtype_code(x->scalar_type());
+  if ((dt != BLR_F16 && dt != BLR_BF16) || x->dim() != 3 || x->numel() == 0 || !x->is_contiguous() || !aligned16(*x)) DECLINE;
+  const int64_t B = x->size(0), N = x->size(1), C = x->size(2);
+  if (C % 8 || C > 2048 || B * N > INT32_MAX) DECLINE;
+  for (const at::Tensor* t : {sh, sc})
+    if (t->scalar_type() != x->scalar_type() || t->device() != x->device() || t->dim() != 2 || t->size(0) != B || t->size(1) != C || t->stride(1) != 1 ||
+        t->stride(0) < C || t->stride(0) % 8 || !aligned16(*t)) DECLINE;
+  const c10::OptionalDeviceGuard guard(x->device());
+  at::Tensor out = empty(*x, {B, N, C});
+  const void *xp = x->data_ptr(), *shp = sh->data_ptr(), *scp = sc->data_ptr();
+  const int64_t lsh = sh->stride(0), lsc = sc->stride(0);
+  void* st = (void*)c10::hip::getCurrentHIPStream(x->device().index()).stream();
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = api.ln_modulate(xp, shp, lsh, scp, lsc, out.data_ptr(), (int)(B * N), (int)C, (int)N, (float)eps, dt, st);
+  Py_END_ALLOW_THREADS
+  static PyObject* const name = PyUnicode_InternFromString("ln_modulate");
+  if (rc) return failed(name, rc);
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
 // workspace(device index, stream, bytes, streaming)
 PyObject* py_workspace(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   ENTER(4)
@@ -388,7 +431,7 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                   get("blr_monarch_workspace_bytes", api.monarch_ws) && get("blr_monarch_fwd", api.monarch) && get("blr_monarch_fwd_ep2", api.monarch_ep) &&
                   get("blr_low_rank_workspace_bytes", api.low_rank_ws) && get("blr_low_rank_fwd", api.low_rank) && get("blr_low_rank_fwd_ep2", api.low_rank_ep) &&
                   get("blr_dense_workspace_bytes", api.dense_ws) && get("blr_dense_fwd", api.dense) && get("blr_dense_fwd_ep2", api.dense_ep) &&
-                  get("blr_ep_workspace_bytes", api.ep_ws) && get("blr_last_error", api.last_error);
+                  get("blr_ep_workspace_bytes", api.ep_ws) && get("blr_ln_modulate", api.ln_modulate) && get("blr_last_error", api.last_error);
   if (!ok) { PyErr_SetString(PyExc_ValueError, "an entry point of libblr.so is missing"); return nullptr; }
   Py_INCREF(args[1]);
   Py_XDECREF(blr_error);
@@ -404,6 +447,7 @@ PyMethodDef methods[] = {
     {"blast_q", (PyCFunction)(void*)blast_q, METH_FASTCALL, nullptr},
     {"monarch", (PyCFunction)(void*)monarch, METH_FASTCALL, nullptr},
     {"low_rank", (PyCFunction)(void*)low_rank, METH_FASTCALL, nullptr},
+    {"ln_modulate", (PyCFunction)(void*)ln_modulate, METH_FASTCALL, nullptr},
     {"dense", (PyCFunction)(void*)dense, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_blr_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

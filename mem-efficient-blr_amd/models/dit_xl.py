@@ -13,6 +13,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from triton_funcs import _lib as L
 from utils import replace_linear_with_custom
 
 
@@ -21,13 +22,30 @@ def modulate(x, shift, scale):
     return torch.addcmul(shift.unsqueeze(1), x, (1 + scale).unsqueeze(1))
 
 
+def _bare(module, kind):
+    """Whether calling `module` is `kind`'s own forward and nothing else."""
+    m = nn.modules.module
+    return (type(module) is kind and "forward" not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
+            and not m._global_forward_hooks and not m._global_forward_pre_hooks)
+
+
+def _norm_modulate(norm, x, shift, scale):
+    """modulate(norm(x), shift, scale): one kernel where norm is a bare LayerNorm without an affine part and nothing but the result is
+    wanted (inference on the GPU), torch's operators otherwise."""
+    if x.is_cuda and _bare(norm, nn.LayerNorm) and norm.weight is None and norm.bias is None and norm.normalized_shape == x.shape[-1:]:
+        host = L.call_path()
+        out = host.ln_modulate(x, shift, scale, norm.eps) if host else None
+        if out is not None:
+            return out
+    return modulate(norm(x), shift, scale)
+
+
 def _gated(linear, h, gate, residual):
     """residual + gate.unsqueeze(1) * linear(h) (reference DiT/models.py:120-121).  A structured linear that fuses its output stage
     does the whole update while it writes its result; anything else gets one elementwise pass."""
     if gate is None:
         return linear(h)
     if getattr(linear, "fuses", False):
-        from triton_funcs import _lib as L
         with L.gate_residual(gate, h.shape[1], residual):
             return linear(h).reshape(residual.shape)
     return torch.addcmul(residual, gate.unsqueeze(1), linear(h))
@@ -88,8 +106,8 @@ class DiTBlock(nn.Module):
     def forward(self, x, c):
         s1, c1, g1, s2, c2, g2 = self.adaLN_modulation(c).chunk(6, dim=1)
         # gate and residual (reference DiT/models.py:120-121) in one elementwise pass each
-        x = self.attn(modulate(self.norm1(x), s1, c1), gate=g1, residual=x)
-        x = self.mlp(modulate(self.norm2(x), s2, c2), gate=g2, residual=x)
+        x = self.attn(_norm_modulate(self.norm1, x, s1, c1), gate=g1, residual=x)
+        x = self.mlp(_norm_modulate(self.norm2, x, s2, c2), gate=g2, residual=x)
         return x
 
 
@@ -102,7 +120,7 @@ class FinalLayer(nn.Module):
 
     def forward(self, x, c):
         shift, scale = self.adaLN_modulation(c).chunk(2, dim=1)
-        return self.linear(modulate(self.norm_final(x), shift, scale))
+        return self.linear(_norm_modulate(self.norm_final, x, shift, scale))
 
 
 def sincos_2d(dim, grid):

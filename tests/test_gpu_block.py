@@ -1,0 +1,60 @@
+"""The kernels between the linears of a DiT block against torch in 64 bits, and which calls are left to torch."""
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from gpu_util import say
+
+pytestmark = pytest.mark.gpu
+
+HALF = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}       # one rounding of a result, relatively
+
+
+def _host():
+    from triton_funcs import _lib as L
+    host = L.call_path()
+    assert host, "the native call path did not load"
+    return host
+
+
+# columns: one piece of a lane, the edges of its pieces per lane, the most; rows that do not fill a workgroup
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("images,tokens,cols", [(1, 1, 8), (3, 5, 504), (2, 64, 512), (1, 7, 520), (16, 256, 1152), (5, 3, 1544), (1, 2, 2048)])
+def test_ln_modulate(images, tokens, cols, dtype):
+    say(f"[case] ln_modulate {images} x {tokens} x {cols} {dtype}")
+    x = (torch.randn(images, tokens, cols, device="cuda") * 2 + 1).to(dtype)
+    mod = torch.randn(images, 3 * cols, device="cuda").to(dtype)
+    shift, scale, _ = mod.chunk(3, dim=1)
+    got = _host().ln_modulate(x, shift, scale, 1e-6)
+    ref = F.layer_norm(x.double(), (cols,), eps=1e-6) * (1 + scale.double().unsqueeze(1)) + shift.double().unsqueeze(1)
+    # fp32 inside: a few 2^-24 of the terms before the sum with the shift may cancel them, then one rounding
+    slack = 2.0 ** -20 * (ref.abs() + shift.double().abs().unsqueeze(1) + 1)
+    assert ((got.double() - ref).abs() <= HALF[dtype] * ref.abs() + slack).all()
+
+
+def test_ln_modulate_is_left_to_torch():
+    """fp32, odd columns, gradients, autocast, transforms, a norm with hooks: as before."""
+    from models import dit_xl as D
+    h = _host()
+    x, s = torch.randn(2, 4, 64, device="cuda").half(), torch.randn(2, 64, device="cuda").half()
+    assert h.ln_modulate(x, s, s, 1e-6) is not None
+    assert h.ln_modulate(x.float(), s.float(), s.float(), 1e-6) is None
+    assert h.ln_modulate(x[..., :60], s[:, :60], s[:, :60], 1e-6) is None
+    assert h.ln_modulate(x.transpose(0, 1), s[:, :], s, 1e-6) is None
+    assert h.ln_modulate(x.clone().requires_grad_(), s, s, 1e-6) is None
+    with torch.no_grad():
+        assert h.ln_modulate(x.clone().requires_grad_(), s, s, 1e-6) is not None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert h.ln_modulate(x, s, s, 1e-6) is None
+    norm = nn.LayerNorm(64, elementwise_affine=False, eps=1e-6)
+    want = D.modulate(norm(x), s, s)
+    got = torch.func.vmap(lambda xx, ss: D._norm_modulate(norm, xx[None], ss[None], ss[None])[0])(x, s)
+    assert torch.allclose(got.float(), want.float(), atol=2e-2)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x.float().half(), torch.ones_like(x))
+        assert h.ln_modulate(dual, s, s, 1e-6) is None
+    seen = []
+    norm.register_forward_hook(lambda *a: seen.append(1))
+    D._norm_modulate(norm, x, s, s)
+    assert seen
