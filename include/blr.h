@@ -313,6 +313,10 @@ int blr_blast_fwd_static(const void* x, int64_t ldx, const void* U, const void* 
  * the adaLN projection).  f16 / bf16, cols % 8 == 0, cols <= 2048, 16-byte aligned; else BLR_ERR_UNSUPPORTED.  fp32 inside.  */
 int blr_ln_modulate(const void* x, const void* shift, int64_t ld_shift, const void* scale, int64_t ld_scale, void* out,
                     int rows, int cols, int rows_per_group, float eps, int dtype, void* stream);
+/* out = softmax(q k^T / sqrt(head_dim)) v per image and head, no mask.  qkv (images, tokens, 3, heads, head_dim) contiguous, as the
+ * qkv linear leaves it; out (images, tokens, heads, head_dim).  f16 / bf16, heads of 64 or 72 values, 16-byte aligned; else
+ * BLR_ERR_UNSUPPORTED.                                                                              */
+int blr_attention_qkv(const void* qkv, void* out, int images, int tokens, int heads, int head_dim, int dtype, void* stream);
 
 #ifdef __cplusplus
 }

@@ -40,6 +40,7 @@ struct Api {
   decltype(&blr_dense_fwd_ep2) dense_ep;
   decltype(&blr_ep_workspace_bytes) ep_ws;
   decltype(&blr_ln_modulate) ln_modulate;
+  decltype(&blr_attention_qkv) attention;
   decltype(&blr_last_error) last_error;
 } api = {};
 PyObject* blr_error = nullptr;                     // triton_funcs._lib.BlrError
@@ -406,6 +407,30 @@ PyObject* ln_modulate(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// attention(qkv, heads): qkv (images, tokens, 3 * columns) as the qkv linear leaves it; (images, tokens, columns)
+PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  ENTER(2)
+  const at::Tensor* x = tensor(args[0]);
+  const int64_t H = PyLong_AsLong(args[1]);
+  if (PyErr_Occurred() || !x || H < 1 || !torch_modes_off() || !plain(*x)) DECLINE;
+  const int dt = dtype_code(x->scalar_type());
+  if ((dt != BLR_F16 && dt != BLR_BF16) || x->dim() != 3 || x->numel() == 0 || !x->is_contiguous() || !aligned16(*x) || x->size(2) % (3 * H)) DECLINE;
+  const int64_t B = x->size(0), N = x->size(1), D = x->size(2) / (3 * H);
+  if ((D != 64 && D != 72) || N > (1 << 20) || B * H > INT32_MAX / ((N + 127) / 128)) DECLINE;
+  const c10::OptionalDeviceGuard guard(x->device());
+  at::Tensor out = empty(*x, {B, N, H * D});
+  const void* xp = x->data_ptr();
+  void* st = (void*)c10::hip::getCurrentHIPStream(x->device().index()).stream();
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = api.attention(xp, out.data_ptr(), (int)B, (int)N, (int)H, (int)D, dt, st);
+  Py_END_ALLOW_THREADS
+  static PyObject* const name = PyUnicode_InternFromString("attention");
+  if (rc) return failed(name, rc);
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
 // workspace(device index, stream, bytes, streaming)
 PyObject* py_workspace(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   ENTER(4)
@@ -431,7 +456,8 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                   get("blr_monarch_workspace_bytes", api.monarch_ws) && get("blr_monarch_fwd", api.monarch) && get("blr_monarch_fwd_ep2", api.monarch_ep) &&
                   get("blr_low_rank_workspace_bytes", api.low_rank_ws) && get("blr_low_rank_fwd", api.low_rank) && get("blr_low_rank_fwd_ep2", api.low_rank_ep) &&
                   get("blr_dense_workspace_bytes", api.dense_ws) && get("blr_dense_fwd", api.dense) && get("blr_dense_fwd_ep2", api.dense_ep) &&
-                  get("blr_ep_workspace_bytes", api.ep_ws) && get("blr_ln_modulate", api.ln_modulate) && get("blr_last_error", api.last_error);
+                  get("blr_ep_workspace_bytes", api.ep_ws) && get("blr_ln_modulate", api.ln_modulate) &&
+                  get("blr_attention_qkv", api.attention) && get("blr_last_error", api.last_error);
   if (!ok) { PyErr_SetString(PyExc_ValueError, "an entry point of libblr.so is missing"); return nullptr; }
   Py_INCREF(args[1]);
   Py_XDECREF(blr_error);
@@ -448,6 +474,7 @@ PyMethodDef methods[] = {
     {"monarch", (PyCFunction)(void*)monarch, METH_FASTCALL, nullptr},
     {"low_rank", (PyCFunction)(void*)low_rank, METH_FASTCALL, nullptr},
     {"ln_modulate", (PyCFunction)(void*)ln_modulate, METH_FASTCALL, nullptr},
+    {"attention", (PyCFunction)(void*)attention, METH_FASTCALL, nullptr},
     {"dense", (PyCFunction)(void*)dense, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_blr_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -75,9 +75,18 @@ class Attention(nn.Module):
     def forward(self, x, gate=None, residual=None):
         """attention(x), or residual + gate * attention(x) with the update done by the last linear's output stage."""
         B, N, C = x.shape
-        qkv = self.qkv(x).reshape(B, N, 3, self.heads, C // self.heads).permute(2, 0, 3, 1, 4)
+        return _gated(self.proj, self._attend(self.qkv(x), B, N, C), gate, residual)
+
+    def _attend(self, qkv, B, N, C):
+        """Attention over the packed qkv, (B, N, C): the library's kernel at inference with heads it has, torch's otherwise."""
+        if qkv.is_cuda and qkv.shape == (B, N, 3 * C):
+            host = L.call_path()
+            o = host.attention(qkv, self.heads) if host else None
+            if o is not None:
+                return o
+        qkv = qkv.reshape(B, N, 3, self.heads, C // self.heads).permute(2, 0, 3, 1, 4)
         o = F.scaled_dot_product_attention(qkv[0], qkv[1], qkv[2])
-        return _gated(self.proj, o.transpose(1, 2).reshape(B, N, C), gate, residual)
+        return o.transpose(1, 2).reshape(B, N, C)
 
 
 class Mlp(nn.Module):

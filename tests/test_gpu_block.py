@@ -58,3 +58,63 @@ def test_ln_modulate_is_left_to_torch():
     norm.register_forward_hook(lambda *a: seen.append(1))
     D._norm_modulate(norm, x, s, s)
     assert seen
+
+
+def _attention64(qkv, heads):
+    B, N, C3 = qkv.shape
+    q, k, v = qkv.double().cpu().reshape(B, N, 3, heads, C3 // 3 // heads).permute(2, 0, 3, 1, 4)
+    p = torch.softmax(q @ k.transpose(-1, -2) * q.shape[-1] ** -0.5, dim=-1)
+    return (p @ v).transpose(1, 2).reshape(B, N, C3 // 3), (p @ v.abs()).transpose(1, 2).reshape(B, N, C3 // 3)
+
+
+def _close(got, ref, mag, half, slack):
+    """The result's rounding (half a place; at least half of fp16's smallest value, 2^-25), and the probabilities': each is off by at
+    most half a place, their errors add up to at most that of p |v|; slack * p |v| for the exponentials' arguments in fp32."""
+    err, bound = (got - ref).abs(), half * (ref.abs() + 1.01 * mag) + slack * mag + 2.0 ** -25
+    at = (err - bound).argmax()
+    assert (err <= bound).all(), (got.flatten()[at], ref.flatten()[at], mag.flatten()[at], err.flatten()[at], bound.flatten()[at])
+
+
+# tokens: one, the edges of a wave's queries, of a step of keys and of a workgroup's queries, several steps
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim", [64, 72])
+@pytest.mark.parametrize("images,heads,tokens", [(1, 1, 1), (2, 3, 31), (1, 2, 33), (3, 16, 64), (1, 5, 65), (2, 2, 127), (1, 1, 129), (2, 16, 256), (1, 3, 700)])
+def test_attention(images, heads, tokens, dim, dtype):
+    say(f"[case] attention {images} x {heads} x {tokens} x {dim} {dtype}")
+    qkv = (torch.randn(images, tokens, 3 * heads * dim, device="cuda") * 1.5).to(dtype)
+    got = _host().attention(qkv, heads).double().cpu()
+    ref, mag = _attention64(qkv, heads)
+    _close(got, ref, mag, HALF[dtype], 2.0 ** -16)
+
+
+def test_attention_large_scores_and_infinities():
+    """Scores far apart (the running maximum moves, exponentials underflow), and a key of minus infinity takes no part."""
+    heads, dim, n = 2, 72, 200
+    qkv = torch.randn(1, n, 3 * heads * dim, device="cuda").half()
+    qkv[:, :, : heads * dim] *= 12
+    qkv[:, :, heads * dim: 2 * heads * dim] *= torch.linspace(0.1, 4, n, device="cuda")[None, :, None].half()
+    ref, mag = _attention64(qkv, heads)
+    got = _host().attention(qkv, heads).double().cpu()
+    _close(got, ref, mag, 2.0 ** -11, 2.0 ** -14)
+    # the first value of every query is positive and of one key minus infinity
+    qkv[:, :, 0] = qkv[:, :, dim] = 1.0
+    for key in (0, 63, 64, 199):
+        one = qkv.clone()
+        one[0, key, heads * dim] = one[0, key, heads * dim + dim] = -float("inf")
+        ref, mag = _attention64(one, heads)
+        got = _host().attention(one, heads).double().cpu()
+        assert torch.isfinite(got).all()
+        _close(got, ref, mag, 2.0 ** -11, 2.0 ** -14)
+
+
+def test_attention_is_left_to_torch():
+    h = _host()
+    x = torch.randn(2, 8, 3 * 2 * 64, device="cuda").half()
+    assert h.attention(x, 2) is not None
+    assert h.attention(x.float(), 2) is None
+    assert h.attention(x, 4) is None                                 # heads of 32
+    assert h.attention(x, 5) is None
+    assert h.attention(x.transpose(0, 1), 2) is None
+    assert h.attention(x.clone().requires_grad_(), 2) is None
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert h.attention(x, 2) is None
