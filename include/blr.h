@@ -317,6 +317,10 @@ int blr_ln_modulate(const void* x, const void* shift, int64_t ld_shift, const vo
  * qkv linear leaves it; out (images, tokens, heads, head_dim).  f16 / bf16, heads of 64 or 72 values, 16-byte aligned; else
  * BLR_ERR_UNSUPPORTED.                                                                              */
 int blr_attention_qkv(const void* qkv, void* out, int images, int tokens, int heads, int head_dim, int dtype, void* stream);
+/* out = silu(c) W^T + bias (reference DiT/models.py:113-116, adaLN_modulation) for at most 16 rows of c, ldc apart; W (out_f, in_f) as
+ * nn.Linear keeps it, bias (out_f) or NULL, out (rows, out_f).  f16 / bf16, in_f and ldc % 8 == 0, out_f % 4 == 0, c and W 16-byte
+ * aligned; else BLR_ERR_UNSUPPORTED.                                                                */
+int blr_silu_linear(const void* c, int64_t ldc, const void* W, const void* bias, void* out, int rows, int out_f, int in_f, int dtype, void* stream);
 
 #ifdef __cplusplus
 }

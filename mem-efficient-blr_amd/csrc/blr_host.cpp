@@ -41,6 +41,7 @@ struct Api {
   decltype(&blr_ep_workspace_bytes) ep_ws;
   decltype(&blr_ln_modulate) ln_modulate;
   decltype(&blr_attention_qkv) attention;
+  decltype(&blr_silu_linear) silu_linear;
   decltype(&blr_last_error) last_error;
 } api = {};
 PyObject* blr_error = nullptr;                     // triton_funcs._lib.BlrError
@@ -431,6 +432,31 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// silu_linear(c, weight, bias): c (rows, in), weight (out, in) and bias (out) or None as an nn.Linear holds them
+PyObject* silu_linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  ENTER(3)
+  const at::Tensor *c = tensor(args[0]), *W = tensor(args[1]), *b = args[2] == Py_None ? nullptr : tensor(args[2]);
+  if (!c || !W || (!b && args[2] != Py_None) || !torch_modes_off() || !plain(*c) || !plain(*W) || (b && !plain(*b))) DECLINE;
+  const int dt = dtype_code(c->scalar_type());
+  if ((dt != BLR_F16 && dt != BLR_BF16) || c->dim() != 2 || !weight(W, *c, 2) || (b && !weight(b, *c, 1))) DECLINE;
+  const int64_t M = c->size(0), K = c->size(1), N = W->size(0);
+  if (M < 1 || M > 16 || K < 8 || K % 8 || K > INT32_MAX || N < 4 || N % 4 || N > INT32_MAX - 16 || W->size(1) != K || (b && b->numel() != N)) DECLINE;
+  if (c->stride(1) != 1 || (M > 1 && (c->stride(0) < K || c->stride(0) % 8)) || !aligned16(*c) || !aligned16(*W)) DECLINE;
+  const c10::OptionalDeviceGuard guard(c->device());
+  at::Tensor out = empty(*c, {M, N});
+  const void *cp = c->data_ptr(), *wp = W->data_ptr(), *bp = b ? b->data_ptr() : nullptr;
+  const int64_t ld = M > 1 ? c->stride(0) : K;
+  void* st = (void*)c10::hip::getCurrentHIPStream(c->device().index()).stream();
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = api.silu_linear(cp, ld, wp, bp, out.data_ptr(), (int)M, (int)N, (int)K, dt, st);
+  Py_END_ALLOW_THREADS
+  static PyObject* const name = PyUnicode_InternFromString("silu_linear");
+  if (rc) return failed(name, rc);
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
 // workspace(device index, stream, bytes, streaming)
 PyObject* py_workspace(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   ENTER(4)
@@ -457,7 +483,7 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                   get("blr_low_rank_workspace_bytes", api.low_rank_ws) && get("blr_low_rank_fwd", api.low_rank) && get("blr_low_rank_fwd_ep2", api.low_rank_ep) &&
                   get("blr_dense_workspace_bytes", api.dense_ws) && get("blr_dense_fwd", api.dense) && get("blr_dense_fwd_ep2", api.dense_ep) &&
                   get("blr_ep_workspace_bytes", api.ep_ws) && get("blr_ln_modulate", api.ln_modulate) &&
-                  get("blr_attention_qkv", api.attention) && get("blr_last_error", api.last_error);
+                  get("blr_attention_qkv", api.attention) && get("blr_silu_linear", api.silu_linear) && get("blr_last_error", api.last_error);
   if (!ok) { PyErr_SetString(PyExc_ValueError, "an entry point of libblr.so is missing"); return nullptr; }
   Py_INCREF(args[1]);
   Py_XDECREF(blr_error);
@@ -475,6 +501,7 @@ PyMethodDef methods[] = {
     {"low_rank", (PyCFunction)(void*)low_rank, METH_FASTCALL, nullptr},
     {"ln_modulate", (PyCFunction)(void*)ln_modulate, METH_FASTCALL, nullptr},
     {"attention", (PyCFunction)(void*)attention, METH_FASTCALL, nullptr},
+    {"silu_linear", (PyCFunction)(void*)silu_linear, METH_FASTCALL, nullptr},
     {"dense", (PyCFunction)(void*)dense, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_blr_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

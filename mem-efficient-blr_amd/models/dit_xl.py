@@ -40,6 +40,16 @@ def _norm_modulate(norm, x, shift, scale):
     return modulate(norm(x), shift, scale)
 
 
+def _conditioned(proj, c):
+    """proj(c) of an adaLN projection Sequential(SiLU, Linear): one kernel for the few rows of c at inference on the GPU."""
+    if c.is_cuda and _bare(proj, nn.Sequential) and len(proj) == 2 and _bare(proj[0], nn.SiLU) and not proj[0].inplace and _bare(proj[1], nn.Linear):
+        host = L.call_path()
+        out = host.silu_linear(c, proj[1].weight, proj[1].bias) if host else None
+        if out is not None:
+            return out
+    return proj(c)
+
+
 def _gated(linear, h, gate, residual):
     """residual + gate.unsqueeze(1) * linear(h) (reference DiT/models.py:120-121).  A structured linear that fuses its output stage
     does the whole update while it writes its result; anything else gets one elementwise pass."""
@@ -113,7 +123,7 @@ class DiTBlock(nn.Module):
         self.adaLN_modulation = nn.Sequential(nn.SiLU(), nn.Linear(hidden, 6 * hidden))
 
     def forward(self, x, c):
-        s1, c1, g1, s2, c2, g2 = self.adaLN_modulation(c).chunk(6, dim=1)
+        s1, c1, g1, s2, c2, g2 = _conditioned(self.adaLN_modulation, c).chunk(6, dim=1)
         # gate and residual (reference DiT/models.py:120-121) in one elementwise pass each
         x = self.attn(_norm_modulate(self.norm1, x, s1, c1), gate=g1, residual=x)
         x = self.mlp(_norm_modulate(self.norm2, x, s2, c2), gate=g2, residual=x)
@@ -128,7 +138,7 @@ class FinalLayer(nn.Module):
         self.adaLN_modulation = nn.Sequential(nn.SiLU(), nn.Linear(hidden, 2 * hidden))
 
     def forward(self, x, c):
-        shift, scale = self.adaLN_modulation(c).chunk(2, dim=1)
+        shift, scale = _conditioned(self.adaLN_modulation, c).chunk(2, dim=1)
         return self.linear(_norm_modulate(self.norm_final, x, shift, scale))
 
 

@@ -66,6 +66,7 @@ _SIGNATURES = {
     "blr_blast_fwd_static": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _i64] + [_i] * 8 + [_vp]),
     "blr_ln_modulate": (_i, [_vp, _vp, _i64, _vp, _i64, _vp, _i, _i, _i, _c.c_float, _i, _vp]),
     "blr_attention_qkv": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _vp]),
+    "blr_silu_linear": (_i, [_vp, _i64, _vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "blr_probe_dst_words": (_i, []),
     "blr_stream_probe": (_i, [_vp, _sz, _vp, _vp]),
     "blr_mfma_probe": (_i, [_i, _i, _i, _vp, _vp]),

@@ -118,3 +118,46 @@ def test_attention_is_left_to_torch():
     assert h.attention(x.clone().requires_grad_(), 2) is None
     with torch.autocast("cuda", dtype=torch.float16):
         assert h.attention(x, 2) is None
+
+
+# rows: one, the most; columns: less than a workgroup's, its edges, several; inputs: one piece, waves without work, more than one batch a wave
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,out_f,in_f", [(1, 4, 8), (16, 12, 24), (3, 16, 32), (5, 20, 136), (16, 6912, 1152), (2, 2304, 1160), (7, 68, 2600)])
+def test_silu_linear(rows, out_f, in_f, dtype):
+    say(f"[case] silu_linear {rows} x {in_f} -> {out_f} {dtype}")
+    lin = nn.Linear(in_f, out_f, device="cuda", dtype=dtype)
+    c = (torch.randn(rows, 2 * in_f, device="cuda") * 2).to(dtype)[:, :in_f]
+    s = F.silu(c.float()).to(dtype).double()
+    for bias in (lin.bias, None):
+        with torch.no_grad():
+            got = _host().silu_linear(c, lin.weight, bias).double()
+        w = lin.weight.double()
+        ref, mag = s @ w.t(), s.abs() @ w.abs().t()
+        if bias is not None:
+            ref = ref + bias.double()
+        # the result's rounding; a silu that the kernel's exponential puts on the other side of a tie is off by a whole place, at worst
+        # everywhere; fp16's smallest values
+        assert ((got - ref).abs() <= HALF[dtype] * (ref.abs() + 2 * mag) + 2.0 ** -16 * mag + 2.0 ** -25).all()
+
+
+def test_silu_linear_is_left_to_torch():
+    from models import dit_xl as D
+    h = _host()
+    proj = nn.Sequential(nn.SiLU(), nn.Linear(64, 96)).cuda().half()
+    lin, c = proj[1], torch.randn(4, 64, device="cuda").half()
+    with torch.no_grad():
+        assert h.silu_linear(c, lin.weight, lin.bias) is not None
+        assert h.silu_linear(c.float(), lin.weight, lin.bias) is None
+        assert h.silu_linear(torch.cat([c] * 5), lin.weight, lin.bias) is None              # 20 rows
+        assert h.silu_linear(c, lin.weight.t().contiguous().t(), lin.bias) is None
+        assert h.silu_linear(c.t().contiguous().t(), lin.weight, lin.bias) is None
+        assert h.silu_linear(c, lin.weight, lin.bias.float()) is None
+        assert torch.allclose(D._conditioned(proj, c).float(), proj(c).float(), atol=2e-2)
+        seen = []
+        hook = lin.register_forward_hook(lambda *a: seen.append(1))
+        D._conditioned(proj, c)
+        assert seen
+        hook.remove()
+    assert h.silu_linear(c, lin.weight, lin.bias) is None                                    # the weight wants a gradient
+    D._conditioned(proj, c).sum().backward()
+    assert lin.weight.grad is not None
