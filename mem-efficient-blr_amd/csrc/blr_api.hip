@@ -329,18 +329,43 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
   else { si = (int64_t)b * r; sj = r; sr = 1; }
   int rc = 1;
   int mixu_prepared = 0;
-  // A few dozen rows are still a weight-streaming problem: 256-row tiles would leave most compute units without one and the
-  // others with a long stream each (4096 -> 4096 at 17 rows: 36 us through the tiles, 12 us at 16 rows through the few-row
-  // kernels).  Up to 128 rows the three launches of the few-row path run over tiles of 16 rows with the weights held in registers
-  // (at 128 rows 32 / 44 / 43 us against 39 / 48 / 56 us through the tiles on the three Llama-7B layers).
-  constexpr int rows_max_m = 128;
-  if (M <= rows_max_m && !y_out && !z_out && !sat8 && fused <= 0 && dtype != BLR_F32 && !silu_mul_armed()) {
-    StreamBlastArgs s = {};
-    s.x = x; s.ldx = ldx; s.U = U; s.V = V; s.S = S; s.out = out; s.ldo = ldo;
-    s.M = M; s.in_f = in_f; s.out_f = out_f; s.b = b; s.r = r;
-    s.dtype = dtype; s.u_layout = u_layout; s.s_layout = s_layout; s.wbits = 16;
-    rc = decode_rows_launch(s, ws, ws_bytes, st);
-    if (rc != 1) return rc;
+  // Few rows and small ranks (blast_by_three): both products on the kernels for problems that do not fill the chip, which give a
+  // 16-block layer of a thousand columns one to several hundred small workgroups where the fused kernels below have 4 .. 32, and
+  // the mix as a launch of its own in between.  The cost of that launch goes with M r; up to where it lies below what the fused
+  // kernel of the shape gains by not having it, measured over the layers of the configurations at 17 .. 1024 rows:
+  //   17 .. 128 rows, any rank: 1152 -> 3456, r = 288 at 17 / 61 / 128 rows 20.4 / 21.3 / 22.6 us (fused) and 13.8 / 19.2 / 28.1
+  //   (tiles of 16 rows, as with codes) against 9.9 / 11.5 / 12.3; 4096 -> 22016, r = 1024 22.8 / 31.7 / 43.7 against 21.4 / 22.2 / 28.3;
+  //   S with the rank contiguous: to M r = 2^18 (2048 -> 8192, r = 512 at 512 rows 34.9 against 31.1 us, at 768 rows 39.4 against 42.4),
+  //   3/4 of that where output blocks are narrow (1152 -> 1152, r = 288 at 512 rows 27.3 against 23.4, at 768 rows 27.1 against 28.0);
+  //   S (r, i, j): the same, but with input blocks that the fused first half takes as they are 80 x 1024 (1152 -> 3456, r = 288 at
+  //   256 rows 18.3 against 17.0, at 384 rows 19.6 against 21.3; 2048 -> 8192, r = 768 at 144 rows 23.6 against 24.7).
+  // Longer calls of tiny ranks are left to the fused kernels, which were fitted there.
+  const bool narrow_out = b == 16 && Q % 8 == 0 && Q <= 80 && r % 32 == 0 && !silu_mul_armed();
+  const int64_t by_three = narrow_out ? 3 << 16 : sr != 1 && P <= 128 ? 80 << 10 : 1 << 18;
+  const bool few = M <= 128 || (M <= 2048 && (int64_t)M * r <= by_three);
+  if (few && !y_out && !z_out && !sat8 && fused <= 0 && dtype != BLR_F32 && option_value(OPT_DECODE_ROWS, 1)) {
+    if (M > 16) {
+      GemmArgs g1 = {}, g2 = {};
+      g1.A = x; g1.lda = ldx; g1.sA = P; g1.B = V; g1.ldb = r; g1.sB = (int64_t)P * r; g1.b_kn = 1;
+      g1.C = Y; g1.ldc = r; g1.sC = (int64_t)M * r; g1.cn = 1; g1.M = M; g1.N = r; g1.K = P; g1.batch = b;
+      g2.A = Z; g2.lda = r; g2.sA = (int64_t)M * r; g2.B = U;
+      g2.b_kn = u_layout == BLR_U_RQ; g2.ldb = g2.b_kn ? Q : r; g2.sB = (int64_t)r * Q;
+      g2.C = out; g2.ldc = ldo; g2.sC = Q; g2.cn = 1; g2.M = M; g2.N = Q; g2.K = r; g2.batch = b;
+      if (!(silu_mul_armed() && b % 2) && option_value(OPT_GEMM_MID, 1) && gemm_mid_ok(g1, dtype) && gemm_mid_ok(g2, dtype)) {
+        if ((rc = gemm_launch(g1, dtype, st)) || (rc = rows_mix_launch(Y, S, Z, M, b, r, s_layout, dtype, st))) return rc;
+        attach_epilogue(g2);
+        if (g2.pair) { g2.batch = b / 2; g2.pair_dA = (int64_t)(b / 2) * g2.sA; g2.pair_dB = (int64_t)(b / 2) * g2.sB; g2.pair_dbias = (int64_t)(b / 2) * Q; }
+        return gemm_launch(g2, dtype, st);
+      }
+    } else if (!silu_mul_armed()) {                  // (a tiled call of a handful of rows: weight streaming)
+      StreamBlastArgs s = {};
+      s.x = x; s.ldx = ldx; s.U = U; s.V = V; s.S = S; s.out = out; s.ldo = ldo;
+      s.M = M; s.in_f = in_f; s.out_f = out_f; s.b = b; s.r = r;
+      s.dtype = dtype; s.u_layout = u_layout; s.s_layout = s_layout; s.wbits = 16;
+      rc = decode_rows_launch(s, ws, ws_bytes, st);
+      if (rc != 1) return rc;
+    }
+    rc = 1;
   }
   // Nobody asked for Y: x V and the mix can run as one launch with Y kept inside the compute units (BLR_ALGO_FUSED).  Chosen
   // by itself only for narrow input blocks: the fused kernel re-reads V once per 32 rows, and from about 128 columns per
@@ -559,18 +584,6 @@ int blr_quantize_sym_t(const void* w, int dtype, int64_t outer, int64_t reduce, 
 }
 
 // ---- Monarch --------------------------------------------------------------------------------------
-// Monarch at 17..128 rows through the few-row kernels: bytes of their intermediates - the first product's output (in slices
-// of the input blocks when those are deeper than 1024 rows, as decode_rows_launch cuts them) and the permuted z.
-static size_t monarch_rows_bytes(int M, int in_f, int b, int rank, int dtype) {
-  if (M <= 16 || M > 128 || dtype == BLR_F32 || b < 2 || in_f % b || rank % b) return 0;
-  const int P = in_f / b;
-  int mks = 1;
-  if (P > 1024)
-    for (int ks = (P + 1023) / 1024; ks <= 8; ++ks)
-      if (P % ks == 0 && (P / ks) % 8 == 0) { mks = ks; break; }
-  return align_up((size_t)b * mks * M * rank * (mks > 1 ? 4 : 2), 256) + align_up((size_t)b * M * rank * 2, 256);   // slices: fp32 partial sums
-}
-
 size_t blr_monarch_workspace_bytes(int M, int in_f, int out_f, int b, int rank, int dtype, int algo) {
   if (M <= 0 || b <= 0 || rank <= 0) return 0;
   int a = resolve_algo(algo, M, dtype, false);
@@ -579,8 +592,7 @@ size_t blr_monarch_workspace_bytes(int M, int in_f, int out_f, int b, int rank, 
     size_t s = stream_generic_workspace(2, M, in_f, out_f, b, rank);
     return s > tiled ? s : tiled;
   }
-  const size_t rows = monarch_rows_bytes(M, in_f, b, rank, dtype);
-  return rows > tiled ? rows : tiled;
+  return tiled;
 }
 
 int blr_monarch_fwd(const void* x, int64_t ldx, const void* w1, const void* w2,
@@ -605,17 +617,6 @@ int blr_monarch_fwd(const void* x, int64_t ldx, const void* w1, const void* w2,
     return stream_generic_launch(s, st);
   }
   if (a != BLR_ALGO_TILED) { set_error("monarch: algorithm %d not available", a); return BLR_ERR_UNSUPPORTED; }
-  if (!out1 && ws && monarch_rows_bytes(M, in_f, b, rank, dtype) && ws_bytes >= monarch_rows_bytes(M, in_f, b, rank, dtype)) {
-    StreamBlastArgs bl = {};
-    bl.x = x; bl.ldx = ldx; bl.U = w2; bl.V = w1; bl.S = nullptr; bl.out = out; bl.ldo = ldo;
-    bl.M = M; bl.in_f = in_f; bl.out_f = out_f; bl.b = b; bl.bo = b; bl.r = rank;
-    bl.dtype = dtype; bl.u_layout = w2_layout == BLR_W2_SR ? BLR_U_QR : BLR_U_RQ; bl.s_layout = BLR_S_IJR; bl.wbits = 16;
-    bl.perm_per = per;
-    if (out_order == BLR_OUT_INTERLEAVED) { bl.out_bs = 1; bl.out_ns = b; }
-    else { bl.out_bs = S; bl.out_ns = 1; }
-    const int rc = decode_rows_launch(bl, ws, ws_bytes, st);
-    if (rc != 1) return rc;
-  }
   const size_t need = out1 ? 0 : align_up((size_t)b * M * rank * elt_size(dtype), 256);
   if (need && (!ws || ws_bytes < need)) { set_error("monarch: workspace %zu < %zu", ws_bytes, need); return BLR_ERR_WORKSPACE; }
   void* O1 = out1 ? out1 : ws;
@@ -643,19 +644,6 @@ int blr_monarch_fwd(const void* x, int64_t ldx, const void* w1, const void* w2,
 }
 
 // ---- low rank -------------------------------------------------------------------------------------
-// Low rank at 17..128 rows through the few-row kernels: BLAST with the input cut into 16 (or 8, 4, 2) slices, one output block
-// and S = 1.  Bytes of its intermediates (0 when the shape is not for it); the launch returns 1 when it does not apply.
-static int low_rank_slices(int in_f) {
-  for (int c = 16; c >= 2; c >>= 1)
-    if (in_f % c == 0 && (in_f / c) % 8 == 0) return c;
-  return 0;
-}
-static size_t low_rank_rows_bytes(int M, int in_f, int r, int dtype) {
-  const int bi = low_rank_slices(in_f);
-  if (M <= 16 || M > 128 || dtype == BLR_F32 || !bi) return 0;
-  return align_up((size_t)bi * M * r * 4, 256) + align_up((size_t)M * r * 2, 256);   // fp32 partial sums of the slices, then z
-}
-
 size_t blr_low_rank_workspace_bytes(int M, int in_f, int out_f, int r, int dtype, int algo) {
   if (M <= 0 || r <= 0) return 0;
   int a = resolve_algo(algo, M, dtype, false);
@@ -664,9 +652,7 @@ size_t blr_low_rank_workspace_bytes(int M, int in_f, int out_f, int r, int dtype
     size_t s = stream_generic_workspace(1, M, in_f, out_f, 1, r);
     return s > tiled ? s : tiled;
   }
-  size_t need = tiled + gemm_splitk_bytes(M, r, in_f, dtype);   // x.A has few output tiles and a long reduction: room to cut it along K
-  const size_t rows = low_rank_rows_bytes(M, in_f, r, dtype);   // 17..128 rows: the few-row path (x A in up to 16 slices of the input)
-  return rows > need ? rows : need;
+  return tiled + gemm_splitk_bytes(M, r, in_f, dtype);   // x.A has few output tiles and a long reduction: room to cut it along K
 }
 
 int blr_low_rank_fwd(const void* x, int64_t ldx, const void* A, const void* B,
@@ -688,14 +674,6 @@ int blr_low_rank_fwd(const void* x, int64_t ldx, const void* A, const void* B,
     return stream_generic_launch(s, st);
   }
   if (a != BLR_ALGO_TILED) { set_error("low_rank: algorithm %d not available", a); return BLR_ERR_UNSUPPORTED; }
-  if (!z_out && ws && low_rank_rows_bytes(M, in_f, r, dtype) && ws_bytes >= low_rank_rows_bytes(M, in_f, r, dtype)) {
-    StreamBlastArgs bl = {};
-    bl.x = x; bl.ldx = ldx; bl.U = B; bl.V = A; bl.S = nullptr; bl.out = out; bl.ldo = ldo;
-    bl.M = M; bl.in_f = in_f; bl.out_f = out_f; bl.b = low_rank_slices(in_f); bl.bo = 1; bl.r = r;
-    bl.dtype = dtype; bl.u_layout = BLR_U_RQ; bl.s_layout = BLR_S_IJR; bl.wbits = 16;
-    const int rc = decode_rows_launch(bl, ws, ws_bytes, st);
-    if (rc != 1) return rc;
-  }
   const size_t need = z_out ? 0 : align_up((size_t)M * r * elt_size(dtype), 256);
   if (need && (!ws || ws_bytes < need)) { set_error("low_rank: workspace %zu < %zu", ws_bytes, need); return BLR_ERR_WORKSPACE; }
   void* Z = z_out ? z_out : ws;
@@ -719,9 +697,7 @@ size_t blr_dense_workspace_bytes(int M, int in_f, int out_f, int dtype, int algo
   if (M <= 0) return 0;
   int a = resolve_algo(algo, M, dtype, false);
   if (a == BLR_ALGO_STREAM || a == BLR_ALGO_STREAM_SPLIT) return stream_generic_workspace(0, M, in_f, out_f, 1, 0);
-  const size_t rows = dense_rows_bytes(M, in_f, out_f, dtype);      // 17..128 rows: partial products of the slices of the reduction
-  const size_t splitk = gemm_splitk_bytes(M, out_f, in_f, dtype);    // more rows, few tiles: fp32 partial sums of the slices of K
-  return rows > splitk ? rows : splitk;
+  return gemm_splitk_bytes(M, out_f, in_f, dtype);    // few tiles: fp32 partial sums of the slices of K
 }
 
 int blr_dense_fwd(const void* x, int64_t ldx, const void* W, void* out, int64_t ldo,
@@ -742,12 +718,6 @@ int blr_dense_fwd(const void* x, int64_t ldx, const void* W, void* out, int64_t 
     return stream_generic_launch(s, st);
   }
   if (a != BLR_ALGO_TILED) { set_error("dense: algorithm %d not available", a); return BLR_ERR_UNSUPPORTED; }
-  {
-    // 17..128 rows: 256-row tiles would leave most compute units idle and give the others a long stream each (11008 -> 4096
-    // at 64 rows: 124 us); the few-row product kernel over tiles of 16 rows instead
-    const int rc = dense_rows_launch(x, ldx, W, out, ldo, M, in_f, out_f, dtype, ws, ws_bytes, st);
-    if (rc != 1) return rc;
-  }
   GemmArgs g = {};
   g.A = x; g.lda = ldx; g.B = W; g.ldb = out_f; g.b_kn = 1;
   g.C = out; g.ldc = ldo; g.cn = 1; g.M = M; g.N = out_f; g.K = in_f; g.batch = 1;

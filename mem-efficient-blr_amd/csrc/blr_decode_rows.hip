@@ -572,7 +572,8 @@ int rows_launch_m(RowsParams& p, int batch, hipStream_t st) {
 }
 template <typename T, int WB, bool NK = false>
 int rows_launch_t(RowsParams& p, int batch, hipStream_t st) {
-  return p.mtiles > 1 ? rows_launch_m<T, WB, NK, true>(p, batch, st) : rows_launch_m<T, WB, NK, false>(p, batch, st);
+  if constexpr (WB != 16) if (p.mtiles > 1) return rows_launch_m<T, WB, NK, true>(p, batch, st);
+  return rows_launch_m<T, WB, NK, false>(p, batch, st);
 }
 
 // Plans one batch of skinny products (chunk width, rounds, item order); returns 1 when the operands do not fit the kernel.
@@ -584,6 +585,7 @@ int rows_plan(RowsParams& p, int batch, int dtype, int wbits, bool nk) {
   if (wbits != 16 && dtype != BLR_F16 && dtype != BLR_BF16) return 1;
   p.rounds = (int)cdiv(p.K, DR_WAVES * DR_MAX_STEPS * 32);
   p.mtiles = (int)cdiv(p.M, 16);
+  if (p.mtiles > 1 && wbits == 16) return 1;           // floating weights above 16 rows: the small tiles of blr_gemm_mid.hip are faster
   if (p.mtiles > 1 && p.rounds > 1) return 1;          // more rows than one tile only with the whole factor slice in registers
   p.kw = (int)cdiv(cdiv(p.K, DR_WAVES * p.rounds), 32) * 32;
   const int cus = device_cus() > 0 ? device_cus() : 256;
@@ -645,7 +647,23 @@ RowsPrefetch rows_prefetch_plan(const RowsParams& p, int batch, int wbits, bool 
   return f;
 }
 
+int mix_launch(const void* Y, const void* S, void* Z, int M, int b, int R, int s_layout, int dtype, const RowsPrefetch& pf, hipStream_t st) {
+  int64_t si, sj, sr;
+  if (s_layout == BLR_S_JIR) { sj = (int64_t)b * R; si = R; sr = 1; }
+  else if (s_layout == BLR_S_RIJ) { sr = (int64_t)b * b; si = b; sj = 1; }
+  else { si = (int64_t)b * R; sj = R; sr = 1; }
+  if (sr == 1 && si % 4 == 0 && sj % 4 == 0 && R % 4 == 0 && aligned(S, 8) && (int64_t)M * b * (R / 4) * (R / 4) < ((int64_t)1 << 32) && b < 65536)   // the multiply-high division is exact below 2^32 / divisor
+    return dtype == BLR_F16 ? rows_mix_t<f16>(Y, S, Z, M, b, R, si, sj, pf, st) : rows_mix_t<bf16>(Y, S, Z, M, b, R, si, sj, pf, st);
+  if (s_layout == BLR_S_RIJ && b == 16 && R % 4 == 0 && aligned(S, 16) && (int64_t)M * (R / 4) * (R / 4) < ((int64_t)1 << 32))
+    return dtype == BLR_F16 ? rows_mix_rij_t<f16>(Y, S, Z, M, R, pf, st) : rows_mix_rij_t<bf16>(Y, S, Z, M, R, pf, st);
+  return blast_mix_launch(Y, S, Z, M, b, R, si, sj, sr, dtype, st, 0);
+}
+
 }  // namespace
+
+int rows_mix_launch(const void* Y, const void* S, void* Z, int M, int b, int R, int s_layout, int dtype, hipStream_t st) {
+  return mix_launch(Y, S, Z, M, b, R, s_layout, dtype, RowsPrefetch{}, st);
+}
 
 int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_bytes, hipStream_t st) {
   const int enabled = option_value(OPT_DECODE_ROWS, 1);
@@ -706,10 +724,6 @@ int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_byt
   const RowsPrefetch pf = ahead ? rows_prefetch_plan(s2, bo, a.wbits, u_nk) : RowsPrefetch{};
   rc = rows_launch(s1, b * mks, a.dtype, a.wbits, false, st);
   if (rc) return rc;
-  int64_t si, sj, sr;
-  if (a.s_layout == BLR_S_JIR) { sj = (int64_t)b * R; si = R; sr = 1; }
-  else if (a.s_layout == BLR_S_RIJ) { sr = (int64_t)b * b; si = b; sj = 1; }
-  else { si = (int64_t)b * R; sj = R; sr = 1; }
   if (monarch && mks > 1) {
     const int64_t items = (int64_t)bo * M * R / 4;
     const uint32_t nmix = (uint32_t)cdiv(items, 256);
@@ -724,65 +738,12 @@ int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_byt
     if (a.dtype == BLR_F16) hipLaunchKernelGGL(rows_sum_kernel<f16>, dim3(nmix + prefetch_blocks(pf)), dim3(256), 0, st, (const float*)Y, (f16*)Z, b, mr4, pf, nmix);
     else hipLaunchKernelGGL(rows_sum_kernel<bf16>, dim3(nmix + prefetch_blocks(pf)), dim3(256), 0, st, (const float*)Y, (bf16*)Z, b, mr4, pf, nmix);
     BLR_CHECK_LAUNCH("rows_sum");
-  } else if (sr == 1 && si % 4 == 0 && sj % 4 == 0 && R % 4 == 0 && aligned(a.S, 8) && (int64_t)M * b * (R / 4) * (R / 4) < ((int64_t)1 << 32) && b < 65536)   // the multiply-high division is exact below 2^32 / divisor
-    rc = a.dtype == BLR_F16 ? rows_mix_t<f16>(Y, a.S, Z, M, b, R, si, sj, pf, st) : rows_mix_t<bf16>(Y, a.S, Z, M, b, R, si, sj, pf, st);
-  else if (a.s_layout == BLR_S_RIJ && b == 16 && R % 4 == 0 && aligned(a.S, 16) && (int64_t)M * (R / 4) * (R / 4) < ((int64_t)1 << 32))
-    rc = a.dtype == BLR_F16 ? rows_mix_rij_t<f16>(Y, a.S, Z, M, R, pf, st) : rows_mix_rij_t<bf16>(Y, a.S, Z, M, R, pf, st);
-  else
-    rc = blast_mix_launch(Y, a.S, Z, M, b, R, si, sj, sr, a.dtype, st, 0);
+  } else
+    rc = mix_launch(Y, a.S, Z, M, b, R, a.s_layout, a.dtype, pf, st);
   if (rc) return rc;
   rc = rows_launch(s2, bo, a.dtype, a.wbits, u_nk, st);
   if (rc == BLR_OK && s2.ep) epilogue_taken();
   return rc == 1 ? BLR_ERR_UNSUPPORTED : rc;
-}
-
-// ---- dense at 17..128 rows ----------------------------------------------------------------------------------------------
-namespace {
-int dense_slices(int in_f) {
-  for (int c = 1; c <= 16; ++c)
-    if (in_f % c == 0 && (in_f / c) % 8 == 0 && in_f / c <= 1024) return c;
-  return 0;
-}
-}  // namespace
-
-// Measured against the 256-row tiles (us at 17 / 64 / 128 rows): 4096 -> 4096 13 / 17 / 23 against 47 / 49 / 56, 11008 -> 4096
-// 26 / 33 / 44 against 116 / 124 / 144, 4096 -> 22016 46 / 58 / 77 against 54 / 56 / 63 - a wide output has enough tiles of its own
-// and pays for the slices' partial products, so it comes here only up to 48 rows.
-static bool dense_rows_wanted(int M, int out_f) { return M > 16 && M <= DR_MAX_M && (out_f <= 8192 || M <= 48); }
-
-size_t dense_rows_bytes(int M, int in_f, int out_f, int dtype) {
-  const int bi = dense_slices(in_f);
-  if (!dense_rows_wanted(M, out_f) || (dtype != BLR_F16 && dtype != BLR_BF16) || !bi || out_f % 8) return 0;
-  return bi > 1 ? align_up((size_t)bi * M * out_f * 4, 256) : 0;    // fp32 partial sums of the slices
-}
-
-int dense_rows_launch(const void* x, int64_t ldx, const void* W, void* out, int64_t ldo, int M, int in_f, int out_f, int dtype,
-                      void* ws, size_t ws_bytes, hipStream_t st) {
-  const int enabled = option_value(OPT_DENSE_ROWS, 1);
-  const int bi = dense_slices(in_f);
-  if (!enabled || !dense_rows_wanted(M, out_f) || (dtype != BLR_F16 && dtype != BLR_BF16) || !bi || out_f % 8) return 1;
-  if (bi > 1 && (ldo != out_f || !ws || ws_bytes < dense_rows_bytes(M, in_f, out_f, dtype) || !aligned(out, 8))) return 1;
-  const int64_t x_elems = (int64_t)(M - 1) * ldx + in_f;
-  if (x_elems * 2 >= (int64_t)DR_OOB || ldx % 8 || !aligned(x, 16) || !aligned(W, 16)) return 1;
-  RowsParams s = {};
-  s.A = x; s.lda = ldx; s.a_bs = in_f / bi; s.a_bytes = (uint32_t)(x_elems * 2);
-  s.W = W; s.w_bs = (int64_t)(in_f / bi) * out_f;
-  s.out = bi > 1 ? ws : out; s.o_ms = bi > 1 ? out_f : ldo; s.o_bs = (int64_t)M * out_f; s.o_ns = 1;
-  s.M = M; s.K = in_f / bi; s.N = out_f; s.out_f32 = bi > 1 ? 1 : 0;
-  const void* ep_bias = nullptr; int ep_act = 0;
-  if (bi == 1 && epilogue_pending(&ep_bias, &ep_act)) { s.ep = 1; s.bias = ep_bias; s.act = ep_act; }
-  int rc = rows_plan(s, bi, dtype, 16, false);
-  if (rc) return rc;
-  rc = rows_launch(s, bi, dtype, 16, false, st);
-  if (rc) return rc == 1 ? BLR_ERR_UNSUPPORTED : rc;
-  if (bi == 1) { if (s.ep) epilogue_taken(); return BLR_OK; }
-  const int64_t mn4 = (int64_t)M * out_f / 4;
-  const uint32_t nsum = (uint32_t)cdiv(mn4, 256);
-  const RowsPrefetch none = {};
-  if (dtype == BLR_F16) hipLaunchKernelGGL(rows_sum_kernel<f16>, dim3(nsum), dim3(256), 0, st, (const float*)ws, (f16*)out, bi, mn4, none, nsum);
-  else hipLaunchKernelGGL(rows_sum_kernel<bf16>, dim3(nsum), dim3(256), 0, st, (const float*)ws, (bf16*)out, bi, mn4, none, nsum);
-  BLR_CHECK_LAUNCH("rows_sum");
-  return BLR_OK;
 }
 
 }  // namespace blr

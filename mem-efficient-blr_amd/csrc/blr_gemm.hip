@@ -1212,10 +1212,10 @@ size_t gemm_splitk_bytes(int M, int N, int K, int dtype) {
     const int s = K % 4 || N % 8 ? 1 : gemm_mid_f32_slices(M, N, K);
     return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
   }
-  if ((dtype != BLR_F16 && dtype != BLR_BF16) || M < 96 || N % 8 || K % 8 || K < 64) return 0;
+  if ((dtype != BLR_F16 && dtype != BLR_BF16) || M <= 16 || N % 8 || K % 8 || K < 64) return 0;
   const int cus = device_cus() > 0 ? device_cus() : 256;
-  if (cdiv(M, 128) * cdiv(N, 128) > cus) return 0;
-  const MidPlan pl = gemm_mid_plan(M, N, K, 1, true, true, true);
+  if (M > 128 && cdiv(M, 128) * cdiv(N, 128) > cus) return 0;
+  const MidPlan pl = gemm_mid_plan(M, N, K, 1, M >= 96, true, true);
   return pl.slices > 1 ? (size_t)pl.slices * M * N * sizeof(float) : 0;
 }
 
@@ -1232,15 +1232,15 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
   // BLR_GEMM_RING_WAVES = 4 or 8 the workgroup size of the two larger ones - options that tests switch with
   // blr_set_option).
   const int ring = option_value(OPT_GEMM_RING, 1);
-  // Products with at most one 128 x 128 tile per compute unit: smaller tiles, and slices of a long reduction, by the estimates of
+  // Products with at most one 128 x 128 tile per compute unit, or of at most 128 rows: smaller tiles, and slices of a long reduction, by the estimates of
   // blr_gemm_mid.hip.  BLR_GEMM_MID = 0 switches that off, 2 .. 6 asks for one of its five tiles wherever the operands allow it.
   const int mid = option_value(OPT_GEMM_MID, 1);
   if (mid > 1 && gemm_mid_ok(g, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16)) return gemm_mid_launch(g, mid - 2, false, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16, st);
   const int64_t r128_all = cdiv(g.M, 128) * cdiv(g.N, 128) * g.batch;
-  if (mid == 1 && ring == 1 && r128_all <= cus && option_value(OPT_GEMM_RING_TILE, 0) == 0) {
+  if (mid == 1 && ring == 1 && (r128_all <= cus || g.M <= 128) && option_value(OPT_GEMM_RING_TILE, 0) == 0) {
     constexpr int dt = std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16;
     const bool rk = g.cn == 1 && g.M >= 96 && g.K >= 64 && ring_ok(g), mk = gemm_mid_ok(g, dt);
-    bool cut = option_value(OPT_GEMM_SPLITK, 1) != 0 && rk && mk && g.epi == EPI_PLAIN && g.splitk_ws && aligned(g.splitk_ws, 16) && g.batch == 1 && !g.sat8 && !g.pair;
+    bool cut = option_value(OPT_GEMM_SPLITK, 1) != 0 && mk && g.cn == 1 && g.epi == EPI_PLAIN && g.splitk_ws && aligned(g.splitk_ws, 16) && g.batch == 1 && !g.sat8 && !g.pair;
     MidPlan pl = gemm_mid_plan(g.M, g.N, g.pair ? 2 * g.K : g.K, g.batch, rk, mk, cut);
     if (pl.slices > 1 && g.splitk_bytes < (size_t)pl.slices * g.M * g.N * sizeof(float)) pl = gemm_mid_plan(g.M, g.N, g.K, g.batch, rk, mk, false);
     if (pl.slices > 1) {                             // slices of K as the batch of a kernel that leaves partial sums

@@ -1,0 +1,81 @@
+"""BLAST from 17 rows on as two products on small tiles with the mix between them, and the kernels it takes the place of."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import assert_close, blast_inputs, dev, rounded, say
+from oracle import blr_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+# rows: the first, both sides of a tile of 32 and 64, the last of the rule for every rank, further by rows x rank; blocks: 16 (both mix
+# kernels), others; widths that are not whole tiles
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_bmm_fp16"])
+@pytest.mark.parametrize("b,p,q,r", [(16, 72, 72, 64), (16, 136, 200, 136), (16, 16, 8, 32), (3, 40, 88, 24), (2, 1096, 24, 8)])
+@pytest.mark.parametrize("M", [17, 32, 33, 65, 128, 129, 300])
+def test_blast(M, b, p, q, r, name, dtype):
+    from test_gpu_blast import _ref, _run_blast
+    x, U, Vt, S = blast_inputs(b, p, q, r, (M,), seed=M + b)
+    say(f"[case] few rows {name} b={b} p={p} q={q} r={r} M={M} {dtype}")
+    out = _run_blast(name, x, U, Vt, S, dtype, "auto")
+    assert_close(out, _ref(x, U, Vt, S, dtype)[0], dtype, f"{name} b={b} p={p} q={q} r={r} M={M}")
+
+
+@pytest.mark.parametrize("M", [40, 100])
+@pytest.mark.parametrize("b,p,q,r", [(16, 72, 72, 64), (16, 136, 72, 64), (16, 72, 200, 64)], ids=["one launch", "narrow out", "narrow in"])
+def test_fused_kernels_at_few_rows(b, p, q, r, M):
+    """BLR_DECODE_ROWS=0 leaves few rows to the kernels of many."""
+    from test_gpu_blast import _ref, _run_blast
+    from triton_funcs import _lib as L
+    x, U, Vt, S = blast_inputs(b, p, q, r, (M,), seed=M)
+    for name in ("triton_blast_full_fp16", "triton_blast_bmm_fp16"):
+        say(f"[case] fused at few rows {name} b={b} p={p} q={q} r={r} M={M}")
+        with L.options(BLR_DECODE_ROWS=0):
+            out = _run_blast(name, x, U, Vt, S, torch.float16, "auto")
+        assert_close(out, _ref(x, U, Vt, S, torch.float16)[0], torch.float16, f"{name} M={M}")
+
+
+@pytest.mark.parametrize("act", ["gelu_tanh", "silu_mul"])
+@pytest.mark.parametrize("M", [17, 100, 200])
+def test_output_stage(M, act):
+    """Bias, activation, gate and residual (or the gated halves) in the second product's output stage, rows of out wider than the result."""
+    from triton_funcs import blast_kernels as K, _lib as L
+    b, p, q, r, dtype = 4, 72, 80, 64, torch.float16
+    x, U, Vt, S = blast_inputs(b, p, q, r, (M,), seed=M)
+    Up, Vp, Sp = O.blast_to_partial_layout(U, Vt, S)
+    rng = np.random.default_rng(M)
+    bias = rng.standard_normal(b * q)
+    say(f"[case] few rows output stage {act} M={M}")
+    base = O.blast_forward(rounded(x, dtype), rounded(U, dtype), rounded(Vt, dtype), rounded(S, dtype))[0] + rounded(bias, dtype)
+    args = (dev(x, dtype), dev(Up, dtype), dev(Vp, dtype), dev(Sp, dtype))
+    if act == "silu_mul":
+        with L.fused_epilogue(dev(bias, dtype), act):
+            out = K.triton_blast_full_fp16(*args)
+        g, u = base[..., : b * q // 2], base[..., b * q // 2:]
+        assert_close(out, g / (1 + np.exp(-g)) * u, dtype, f"silu_mul M={M}", scale=2.0)
+        return
+    gate, resid = rng.standard_normal((2, b * q)), rng.standard_normal((M, b * q))
+    rows = (M + 1) // 2
+    with L.fused_epilogue(dev(bias, dtype), act, dev(gate, dtype), rows, dev(resid, dtype)):
+        out = K.triton_blast_full_fp16(*args)
+    v = 0.5 * base * (1.0 + np.tanh(np.sqrt(2.0 / np.pi) * (base + 0.044715 * base ** 3)))
+    assert_close(out, (rounded(resid, dtype) + rounded(gate, dtype)[np.arange(M) // rows] * v).reshape(out.shape), dtype, f"gate + residual M={M}", scale=2.0)
+
+
+# a few rows and a long reduction: slices on tiles of 32 rows; a wide output: more tiles than compute units
+@pytest.mark.parametrize("M,K,N", [(17, 4104, 136), (33, 11008, 72), (95, 2056, 1032), (17, 72, 33024), (64, 512, 65536)])
+def test_dense(M, K, N):
+    from triton_funcs import dense_kernels as D, _lib as L
+    dtype = torch.float16
+    g = torch.Generator("cuda").manual_seed(M)
+    x, w = torch.randn(M, K, device="cuda", generator=g).half(), (torch.randn(K, N, device="cuda", generator=g) / K ** 0.5).half()
+    say(f"[case] few rows dense {M} x {K} x {N}")
+    ref = (x.float() @ w.float()).double().cpu().numpy()              # (fp32 on the GPU: 1e-5 against the bound's 1e-2)
+    assert_close(D.triton_dense_fp16(x, w), ref, dtype, f"dense {M} x {K} x {N}")
+    bias = torch.randn(N, device="cuda", generator=g).half()
+    with L.fused_epilogue(bias, "silu"):
+        out = D.triton_dense_fp16(x, w)
+    v = ref + bias.double().cpu().numpy()
+    assert_close(out, v / (1 + np.exp(-v)), dtype, f"dense {M} x {K} x {N} + bias + silu")
