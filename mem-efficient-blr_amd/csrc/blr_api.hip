@@ -288,6 +288,9 @@ static int resolve_algo(int algo, int M, int dtype, bool want_intermediates) {
   return algo;
 }
 
+// The head of a streaming workspace, which calls that take other kernels leave as it is.
+static size_t stream_head_bytes() { return align_up(stream_ws_prefix_bytes(), 256); }
+
 // ---- BLAST ------------------------------------------------------------------------------------
 size_t blr_blast_workspace_bytes(int M, int in_f, int out_f, int b, int r, int dtype, int algo) {
   if (M <= 0 || b <= 0 || r <= 0) return 0;
@@ -644,12 +647,20 @@ int blr_monarch_fwd(const void* x, int64_t ldx, const void* w1, const void* w2,
 }
 
 // ---- low rank -------------------------------------------------------------------------------------
+// 2 .. 16 rows of a small layer: two products on small tiles instead of the three launches that stream larger factors better
+// (768 -> 3072, r = 128 at 2 / 16 rows 8.9 / 9.6 -> 7.3 / 7.5 us, 1152 -> 3456, r = 288 9.9 / 10.7 -> 8.7 / 9.2; but 1152 -> 4608,
+// r = 576 at 2 rows 10.7 against 11.0, and 3072 -> 768, r = 192, whose long reduction comes in slices, 9.3 against 9.9).
+static bool low_rank_by_tiles(int algo, int M, int in_f, int out_f, int r, int dtype) {
+  return algo == BLR_ALGO_AUTO && M >= 2 && M <= 16 && dtype != BLR_F32 && in_f <= 1536 && (int64_t)r * (in_f + out_f) <= 9 << 18;
+}
+
 size_t blr_low_rank_workspace_bytes(int M, int in_f, int out_f, int r, int dtype, int algo) {
   if (M <= 0 || r <= 0) return 0;
   int a = resolve_algo(algo, M, dtype, false);
   size_t tiled = align_up((size_t)M * r * elt_size(dtype), 256);
   if (a == BLR_ALGO_STREAM || a == BLR_ALGO_STREAM_SPLIT) {
     size_t s = stream_generic_workspace(1, M, in_f, out_f, 1, r);
+    if (low_rank_by_tiles(algo, M, in_f, out_f, r, dtype)) tiled += stream_head_bytes() + gemm_splitk_bytes(M, r, in_f, dtype);
     return s > tiled ? s : tiled;
   }
   return tiled + gemm_splitk_bytes(M, r, in_f, dtype);   // x.A has few output tiles and a long reduction: room to cut it along K
@@ -665,6 +676,19 @@ int blr_low_rank_fwd(const void* x, int64_t ldx, const void* A, const void* B,
   if (M <= 0 || in_f <= 0 || out_f <= 0 || r <= 0) { set_error("low_rank: non-positive size"); return BLR_ERR_BAD_ARG; }
   if (ldx < in_f || ldo < (silu_mul_armed() ? out_f / 2 : out_f)) { set_error("low_rank: leading dimension too small"); return BLR_ERR_BAD_ARG; }
   int a = resolve_algo(algo, M, dtype, z_out != nullptr);
+  const size_t tiled = align_up((size_t)M * r * elt_size(dtype), 256);
+  GemmArgs g1 = {}, g2 = {};
+  g1.A = x; g1.lda = ldx; g1.B = A; g1.ldb = r; g1.b_kn = 1;
+  g1.C = z_out ? z_out : ws; g1.ldc = r; g1.cn = 1; g1.M = M; g1.N = r; g1.K = in_f; g1.batch = 1;
+  g2.A = g1.C; g2.lda = r; g2.B = B; g2.ldb = out_f; g2.b_kn = 1;
+  g2.C = out; g2.ldc = ldo; g2.cn = 1; g2.M = M; g2.N = out_f; g2.K = r; g2.batch = 1;
+  size_t used = 0;                                   // a streaming workspace keeps its head
+  if (a == BLR_ALGO_STREAM && low_rank_by_tiles(algo, M, in_f, out_f, r, dtype) && ws && ws_bytes >= blr_low_rank_workspace_bytes(M, in_f, out_f, r, dtype, algo)) {
+    const size_t head = stream_head_bytes();
+    GemmArgs p1 = g1, p2 = g2;
+    p1.C = static_cast<char*>(ws) + head; p2.A = p1.C;
+    if (option_value(OPT_GEMM_MID, 1) && gemm_mid_ok(p1, dtype) && gemm_mid_ok(p2, dtype)) { g1 = p1; g2 = p2; used = head; a = BLR_ALGO_TILED; }
+  }
   if (a == BLR_ALGO_STREAM || a == BLR_ALGO_STREAM_SPLIT) {
     if (dtype == BLR_F32 || M > 16 || z_out) { set_error("low_rank: streaming algorithm needs f16/bf16, M <= 16, no intermediates"); return BLR_ERR_UNSUPPORTED; }
     StreamGenericArgs s = {};
@@ -674,19 +698,12 @@ int blr_low_rank_fwd(const void* x, int64_t ldx, const void* A, const void* B,
     return stream_generic_launch(s, st);
   }
   if (a != BLR_ALGO_TILED) { set_error("low_rank: algorithm %d not available", a); return BLR_ERR_UNSUPPORTED; }
-  const size_t need = z_out ? 0 : align_up((size_t)M * r * elt_size(dtype), 256);
+  const size_t need = z_out ? 0 : used + tiled;
   if (need && (!ws || ws_bytes < need)) { set_error("low_rank: workspace %zu < %zu", ws_bytes, need); return BLR_ERR_WORKSPACE; }
-  void* Z = z_out ? z_out : ws;
-  GemmArgs g1 = {};
-  g1.A = x; g1.lda = ldx; g1.B = A; g1.ldb = r; g1.b_kn = 1;
-  g1.C = Z; g1.ldc = r; g1.cn = 1; g1.M = M; g1.N = r; g1.K = in_f; g1.batch = 1;
-  const size_t tiled = align_up((size_t)M * r * elt_size(dtype), 256);
-  if (ws && ws_bytes > tiled) { g1.splitk_ws = static_cast<char*>(ws) + tiled; g1.splitk_bytes = ws_bytes - tiled; }
+  used += tiled;
+  if (ws && ws_bytes > used) { g1.splitk_ws = static_cast<char*>(ws) + used; g1.splitk_bytes = ws_bytes - used; }
   int rc = gemm_launch(g1, dtype, st);
   if (rc) return rc;
-  GemmArgs g2 = {};
-  g2.A = Z; g2.lda = r; g2.B = B; g2.ldb = out_f; g2.b_kn = 1;
-  g2.C = out; g2.ldc = ldo; g2.cn = 1; g2.M = M; g2.N = out_f; g2.K = r; g2.batch = 1;
   attach_epilogue(g2);
   if (g2.pair) { g2.N = out_f / 2; g2.pair_dA = 0; g2.pair_dB = out_f / 2; g2.pair_dbias = out_f / 2; }   // columns n and n + out_f / 2 of B
   return gemm_launch(g2, dtype, st);
@@ -696,7 +713,10 @@ int blr_low_rank_fwd(const void* x, int64_t ldx, const void* A, const void* B,
 size_t blr_dense_workspace_bytes(int M, int in_f, int out_f, int dtype, int algo) {
   if (M <= 0) return 0;
   int a = resolve_algo(algo, M, dtype, false);
-  if (a == BLR_ALGO_STREAM || a == BLR_ALGO_STREAM_SPLIT) return stream_generic_workspace(0, M, in_f, out_f, 1, 0);
+  if (a == BLR_ALGO_STREAM || a == BLR_ALGO_STREAM_SPLIT) {
+    const size_t s = stream_generic_workspace(0, M, in_f, out_f, 1, 0), tiles = stream_head_bytes() + gemm_splitk_bytes(M, out_f, in_f, dtype);
+    return algo == BLR_ALGO_AUTO && tiles > s ? tiles : s;
+  }
   return gemm_splitk_bytes(M, out_f, in_f, dtype);    // few tiles: fp32 partial sums of the slices of K
 }
 
@@ -709,6 +729,17 @@ int blr_dense_fwd(const void* x, int64_t ldx, const void* W, void* out, int64_t 
   if (M <= 0 || in_f <= 0 || out_f <= 0) { set_error("dense: non-positive size"); return BLR_ERR_BAD_ARG; }
   if (ldx < in_f || ldo < (silu_mul_armed() ? out_f / 2 : out_f)) { set_error("dense: leading dimension too small"); return BLR_ERR_BAD_ARG; }
   int a = resolve_algo(algo, M, dtype, false);
+  GemmArgs g = {};
+  g.A = x; g.lda = ldx; g.B = W; g.ldb = out_f; g.b_kn = 1;
+  g.C = out; g.ldc = ldo; g.cn = 1; g.M = M; g.N = out_f; g.K = in_f; g.batch = 1;
+  // Up to 16 rows too the small tiles, with slices of a long reduction (768 -> 3072 at 1 / 16 rows 8.0 / 8.4 us on the slab kernel and
+  // the launch that adds its slices, 4.8 / 5.0 here; 4096 -> 22016 33.8 / 38.1 against 31.5 / 31.5; 11008 -> 4096 equal at 1 row).
+  size_t head = 0;                                   // a streaming workspace keeps its head
+  if (a == BLR_ALGO_STREAM && algo == BLR_ALGO_AUTO && ws && ws_bytes >= blr_dense_workspace_bytes(M, in_f, out_f, dtype, algo) && option_value(OPT_GEMM_MID, 1) &&
+      gemm_mid_ok(g, dtype)) {
+    head = stream_head_bytes();
+    a = BLR_ALGO_TILED;
+  }
   if (a == BLR_ALGO_STREAM || a == BLR_ALGO_STREAM_SPLIT) {
     if (dtype == BLR_F32 || M > 16) { set_error("dense: streaming algorithm needs f16/bf16 and M <= 16"); return BLR_ERR_UNSUPPORTED; }
     StreamGenericArgs s = {};
@@ -718,11 +749,9 @@ int blr_dense_fwd(const void* x, int64_t ldx, const void* W, void* out, int64_t 
     return stream_generic_launch(s, st);
   }
   if (a != BLR_ALGO_TILED) { set_error("dense: algorithm %d not available", a); return BLR_ERR_UNSUPPORTED; }
-  GemmArgs g = {};
-  g.A = x; g.lda = ldx; g.B = W; g.ldb = out_f; g.b_kn = 1;
-  g.C = out; g.ldc = ldo; g.cn = 1; g.M = M; g.N = out_f; g.K = in_f; g.batch = 1;
   // few output tiles and a long reduction (11008 -> 4096 at 256 rows: 32 tiles): room to cut it along K
-  if (ws && gemm_splitk_bytes(M, out_f, in_f, dtype) && ws_bytes >= gemm_splitk_bytes(M, out_f, in_f, dtype)) { g.splitk_ws = ws; g.splitk_bytes = ws_bytes; }
+  const size_t splitk = gemm_splitk_bytes(M, out_f, in_f, dtype);
+  if (ws && splitk && ws_bytes >= head + splitk) { g.splitk_ws = static_cast<char*>(ws) + head; g.splitk_bytes = ws_bytes - head; }
   attach_epilogue(g);
   if (g.pair) { g.N = out_f / 2; g.pair_dA = 0; g.pair_dB = out_f / 2; g.pair_dbias = out_f / 2; g.splitk_ws = nullptr; g.splitk_bytes = 0; }
   return gemm_launch(g, dtype, st);

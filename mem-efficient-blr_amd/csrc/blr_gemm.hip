@@ -1212,7 +1212,7 @@ size_t gemm_splitk_bytes(int M, int N, int K, int dtype) {
     const int s = K % 4 || N % 8 ? 1 : gemm_mid_f32_slices(M, N, K);
     return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
   }
-  if ((dtype != BLR_F16 && dtype != BLR_BF16) || M <= 16 || N % 8 || K % 8 || K < 64) return 0;
+  if ((dtype != BLR_F16 && dtype != BLR_BF16) || M < 1 || N % 8 || K % 8 || K < 64) return 0;
   const int cus = device_cus() > 0 ? device_cus() : 256;
   if (M > 128 && cdiv(M, 128) * cdiv(N, 128) > cus) return 0;
   const MidPlan pl = gemm_mid_plan(M, N, K, 1, M >= 96, true, true);
@@ -1336,9 +1336,10 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
 
 int gemm_launch(const GemmArgs& g, int dtype, hipStream_t st) {
   if (g.M <= 0 || g.N <= 0 || g.K <= 0 || g.batch <= 0) { set_error("gemm: empty problem"); return BLR_ERR_BAD_ARG; }
-  // A handful of rows is a weight-streaming problem, not a tiling problem: plain products with (k, n)-ordered weights go to
-  // the slab kernel of the decode path (it declines what it cannot take, e.g. a reduction deeper than one slab here).
-  if (g.M <= 16 && g.b_kn && g.cn == 1 && g.epi == EPI_PLAIN && !g.sat8 && !g.bias && g.act == 0 && !g.gate && !g.resid && (dtype == BLR_F16 || dtype == BLR_BF16)) {
+  // A handful of rows with operands that the small tiles cannot take: plain products with (k, n)-ordered weights go to the slab
+  // kernel of the decode path (it declines what it cannot take, e.g. a reduction deeper than one slab here).
+  if (g.M <= 16 && g.b_kn && g.cn == 1 && g.epi == EPI_PLAIN && !g.sat8 && !g.bias && g.act == 0 && !g.gate && !g.resid && (dtype == BLR_F16 || dtype == BLR_BF16) &&
+      !gemm_mid_ok(g, dtype)) {
     int rc = slab_gemm_launch(g.A, g.lda, g.sA, g.B, g.ldb, g.sB, g.C, g.ldc, g.sC, g.M, g.N, g.K, g.batch, dtype, nullptr, 1, st);
     if (rc != 1) return rc;
   }

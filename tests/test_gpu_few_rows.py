@@ -65,7 +65,7 @@ def test_output_stage(M, act):
 
 
 # a few rows and a long reduction: slices on tiles of 32 rows; a wide output: more tiles than compute units
-@pytest.mark.parametrize("M,K,N", [(17, 4104, 136), (33, 11008, 72), (95, 2056, 1032), (17, 72, 33024), (64, 512, 65536)])
+@pytest.mark.parametrize("M,K,N", [(1, 8, 8), (1, 4104, 136), (5, 72, 1032), (16, 11008, 72), (16, 512, 33024), (17, 4104, 136), (33, 11008, 72), (95, 2056, 1032), (17, 72, 33024), (64, 512, 65536)])
 def test_dense(M, K, N):
     from triton_funcs import dense_kernels as D, _lib as L
     dtype = torch.float16
@@ -79,3 +79,19 @@ def test_dense(M, K, N):
         out = D.triton_dense_fp16(x, w)
     v = ref + bias.double().cpu().numpy()
     assert_close(out, v / (1 + np.exp(-v)), dtype, f"dense {M} x {K} x {N} + bias + silu")
+
+
+@pytest.mark.parametrize("M,in_f,r,out_f", [(2, 72, 8, 24), (7, 1536, 136, 200), (16, 768, 192, 2304), (16, 1544, 64, 72)])
+def test_low_rank_of_a_small_layer(M, in_f, r, out_f):
+    """Up to 16 rows, on either side of the rule; between a streaming call before and one after, whose workspace it shares."""
+    from triton_funcs import blast_kernels as B, low_rank_kernels as K
+    dtype = torch.float16
+    rng = np.random.default_rng(M)
+    x, a, bm = rng.standard_normal((M, in_f)), rng.standard_normal((in_f, r)) / np.sqrt(in_f), rng.standard_normal((r, out_f)) / np.sqrt(r)
+    xb, U, Vt, S = blast_inputs(4, 64, 96, 128, (1,), seed=M)
+    args = tuple(dev(t, dtype) for t in (xb,) + tuple(O.blast_to_partial_layout(U, Vt, S)))
+    say(f"[case] few rows low rank M={M} {in_f} -> {r} -> {out_f}")
+    before = B.triton_blast_full_fp16(*args)
+    out = K.triton_low_rank_fp16(dev(x, dtype), dev(a, dtype), dev(bm, dtype))
+    assert_close(out, rounded(rounded(x, dtype) @ rounded(a, dtype), dtype) @ rounded(bm, dtype), dtype, f"low rank M={M}", scale=2.0)
+    assert torch.equal(B.triton_blast_full_fp16(*args), before)
