@@ -55,7 +55,7 @@ class _StructuredLinear(nn.Module):
     def _stage(self):
         """The output stage to hand to the kernel (bias, act, gate, gate_rows, residual), or None; takes a gate / residual that the
         caller has armed."""
-        bias, act = self._parameters["bias"], self.fused_act
+        bias, act = self.bias, self.fused_act
         outer = getattr(L._ep_state, "outer", None)
         if bias is None and act is None and outer is None:
             return None
@@ -71,7 +71,11 @@ class _StructuredLinear(nn.Module):
         stage = self._stage() if self.fuses else None
         if stage is None:
             return self.func(*args), False
-        return self.func.with_epilogue(*args, stage), True
+        with_epilogue = getattr(self.func, "with_epilogue", None)
+        if with_epilogue is None:                      # a function put in the library's place, or one without an output stage of its own
+            with L.armed(stage):
+                return self.func(*args), True
+        return with_epilogue(*args, stage), True
 
     def _finish(self, out, fused=False):
         if isinstance(out, tuple):                     # torch baselines and the *_fp32 names: (out, intermediates...)
@@ -107,8 +111,7 @@ class BlastLinear(_StructuredLinear):
             self.S = self._param((b, b, rank), 1)
 
     def forward(self, x):
-        p = self._parameters
-        return self._finish(*self._call(x, p["U"], p["V"], p["S"]))
+        return self._finish(*self._call(x, self.U, self.V, self.S))
 
     def extra_repr(self):
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "
@@ -147,11 +150,11 @@ class QuantBlastLinear(BlastLinear):
 
     @property
     def Uq(self):
-        return QuantFactor(self._buffers["u_codes"], self._buffers["u_scales"], self.bits, self._u_shape)
+        return QuantFactor(self.u_codes, self.u_scales, self.bits, self._u_shape)
 
     @property
     def Vq(self):
-        return QuantFactor(self._buffers["v_codes"], self._buffers["v_scales"], self.bits, self._v_shape)
+        return QuantFactor(self.v_codes, self.v_scales, self.bits, self._v_shape)
 
     def get_extra_state(self):
         return {"format": self.PACK_FORMAT, "bits": self.bits, "u_shape": list(self._u_shape), "v_shape": list(self._v_shape)}
@@ -176,9 +179,9 @@ class QuantBlastLinear(BlastLinear):
         super()._load_from_state_dict(state_dict, prefix, local_metadata, strict, missing_keys, unexpected_keys, error_msgs)
 
     def forward(self, x):
-        args = (x, self.Uq, self.Vq, self._parameters["S"])
-        bias = self._parameters["bias"]
-        if (bias is not None or self.fused_act is not None) and not self.is_compiled and self.fused_act in L.ACTS:
+        args = (x, self.Uq, self.Vq, self.S)
+        bias = self.bias
+        if (bias is not None or self.fused_act is not None) and not self.is_compiled and hasattr(self.func, "with_epilogue") and self.fused_act in L.ACTS:
             out = self.func.with_epilogue(*args, (bias, L.ACTS[self.fused_act], None, 0, None))
             if out is not None:
                 return out
@@ -200,8 +203,7 @@ class MonarchLinear(_StructuredLinear):
             self.w2_bfly = self._param((b, s, rank), rank)
 
     def forward(self, x):
-        p = self._parameters
-        return self._finish(*self._call(x, p["w1_bfly"], p["w2_bfly"]))
+        return self._finish(*self._call(x, self.w1_bfly, self.w2_bfly))
 
     def extra_repr(self):
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "
@@ -220,8 +222,8 @@ class LowRankLinear(_StructuredLinear):
             self.U = self._param((out_features, rank), rank)
 
     def forward(self, x):
-        out, fused = self._call(x, self._parameters["V"], self._parameters["U"])
-        if not fused and self.kind == "triton" and not isinstance(out, tuple):   # the kernel returns (N, out_f): restore the leading dims
+        out, fused = self._call(x, self.V, self.U)
+        if self.kind == "triton" and not isinstance(out, tuple) and out.dim() != x.dim():   # the kernel returns (N, out_f): restore the leading dims
             out = out.reshape(*x.shape[:-1], out.shape[-1])
         return self._finish(out, fused)
 
@@ -236,8 +238,8 @@ class DenseLinear(_StructuredLinear):
         self.W = self._param(shape, in_features)
 
     def forward(self, x):
-        out, fused = self._call(x, self._parameters["W"])
-        if not fused and self.kind == "triton" and not isinstance(out, tuple):
+        out, fused = self._call(x, self.W)
+        if self.kind == "triton" and not isinstance(out, tuple) and out.dim() != x.dim():
             out = out.reshape(*x.shape[:-1], out.shape[-1])
         return self._finish(out, fused)
 

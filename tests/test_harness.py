@@ -81,6 +81,35 @@ def test_torch_wrappers_forward_match_oracle_with_bias():
     np.testing.assert_allclose(m(x).detach().numpy(), O.dense_forward(x.numpy(), m.W.detach().numpy()), atol=1e-10)
 
 
+def test_wrappers_take_pruned_weights_and_replaced_functions():
+    """A weight that pruning or parametrization has turned from a parameter into a plain attribute, and a function put in the place of
+    the library's, which gets bias and activation through the armed output stage."""
+    from torch.nn.utils import parametrize, prune
+    from models.wrappers import BlastLinear, DenseLinear, LowRankLinear, MonarchLinear
+    from triton_funcs import _lib as L
+    common = dict(device="cpu", dtype=torch.float32)
+    made = ((BlastLinear(32, 48, b=4, rank=8, func_path="torch_funcs.blast_funcs.torch_blast_baseline", **common), ("U", "V", "S")),
+            (MonarchLinear(32, 48, b=4, rank=8, func_path="torch_funcs.monarch_funcs.torch_monarch_baseline", **common), ("w1_bfly", "w2_bfly")),
+            (LowRankLinear(32, 48, rank=8, func_path="torch_funcs.low_rank_funcs.torch_low_rank_baseline", **common), ("U", "V")),
+            (DenseLinear(32, 48, func_path="torch_funcs.dense_funcs.torch_dense_baseline", **common), ("W",)))
+    x = torch.randn(2, 5, 32)
+    with torch.no_grad():
+        for m, names in made:
+            want = m(x)
+            for name in names + ("bias",):
+                prune.identity(m, name)
+            assert torch.equal(m(x), want)
+            for name in names + ("bias",):
+                prune.remove(m, name)
+                parametrize.register_parametrization(m, name, torch.nn.Identity())
+            assert torch.equal(m(x), want)
+        for cls, more, func in ((DenseLinear, {}, "dense_kernels.triton_dense_fp16"), (LowRankLinear, {"rank": 8}, "low_rank_kernels.triton_low_rank_fp16")):
+            m, seen = cls(32, 48, func_path="triton_funcs." + func, **more, **common), []
+            m.func = lambda x, *w: (seen.append(L.armed_epilogue()), torch.zeros(x.numel() // 32, 48))[1]
+            m.fused_act = "silu"
+            assert m(x).shape == (2, 5, 48) and seen[0][0] is m.bias and seen[0][1] == L.ACTS["silu"]
+
+
 def test_torch_funcs_match_oracle_including_bmm_and_intermediates():
     from torch_funcs.blast_funcs import torch_blast_baseline, torch_blast_bmm
     from torch_funcs.monarch_funcs import torch_monarch_baseline
