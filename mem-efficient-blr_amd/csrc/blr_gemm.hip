@@ -1240,7 +1240,9 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
   if (mid == 1 && ring == 1 && (r128_all <= cus || g.M <= 128) && option_value(OPT_GEMM_RING_TILE, 0) == 0) {
     constexpr int dt = std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16;
     const bool rk = g.cn == 1 && g.M >= 96 && g.K >= 64 && ring_ok(g), mk = gemm_mid_ok(g, dt);
-    bool cut = option_value(OPT_GEMM_SPLITK, 1) != 0 && mk && g.cn == 1 && g.epi == EPI_PLAIN && g.splitk_ws && aligned(g.splitk_ws, 16) && g.batch == 1 && !g.sat8 && !g.pair;
+    bool cut = option_value(OPT_GEMM_SPLITK, 1) != 0 && mk && g.cn == 1 && g.epi == EPI_PLAIN && g.splitk_ws && aligned(g.splitk_ws, 16) && g.batch == 1 && !g.sat8 && !g.pair &&
+               g.N % 8 == 0 && aligned(g.C, 16) && g.ldc % 8 == 0 && (!g.bias || aligned(g.bias, 16)) &&     // the sum of the slices moves eight columns at a time
+               (!g.gate || (aligned(g.gate, 16) && g.ld_gate % 8 == 0)) && (!g.resid || (aligned(g.resid, 16) && g.ld_resid % 8 == 0));
     MidPlan pl = gemm_mid_plan(g.M, g.N, g.pair ? 2 * g.K : g.K, g.batch, rk, mk, cut);
     if (pl.slices > 1 && g.splitk_bytes < (size_t)pl.slices * g.M * g.N * sizeof(float)) pl = gemm_mid_plan(g.M, g.N, g.K, g.batch, rk, mk, false);
     if (pl.slices > 1) {                             // slices of K as the batch of a kernel that leaves partial sums

@@ -110,3 +110,28 @@ def test_long_reductions_by_estimate(m, n, k, act, dtype):
     # the activation's exponential and reciprocal are good to a few units of fp32
     lim = 0.51 * torch.from_numpy(ulp(want.cpu().numpy(), dtype)).to(want.device) + slack + 1e-5 * want.abs()
     assert (err <= lim).all(), float((err / lim).max())
+
+
+@pytest.mark.parametrize("m,n,k", [(3, 768, 3072), (61, 136, 8672), (257, 144, 4104)])
+def test_output_operands_of_any_alignment(m, n, k):
+    """The same shapes with a bias, a gate and a residual that start two bytes past a 16-byte boundary: the sum of the slices reads eight
+    columns at a time and leaves such calls to the kernels that take any address."""
+    from triton_funcs import _lib as L, dense_kernels as D
+    dtype = torch.float16
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).to(dtype)
+    w = (torch.randn(k, n, device="cuda", generator=g) / k ** 0.5).to(dtype)
+    odd = lambda rows: torch.randn(rows * n + 1, device="cuda", generator=g).to(dtype)[1:].view(rows, n)
+    bias, gate, resid = odd(1).view(n), odd(1), odd(m)
+    say(f"[case] unaligned output stage m={m} n={n} k={k}")
+    with L.fused_epilogue(bias, None):
+        out = D.triton_dense_fp16(x, w)
+    ref, mag = x.double() @ w.double(), x.double().abs() @ w.double().abs()
+    step = lambda t: 0.51 * torch.from_numpy(ulp(t.cpu().numpy(), dtype)).to(t.device)
+    want, slack = ref + bias.double(), _bound(ref, mag, k, dtype)
+    assert ((out.double() - want).abs() <= step(want) + slack + 2.0 ** -23 * want.abs()).all()
+    with L.fused_epilogue(bias, None, gate, m, resid):
+        out = D.triton_dense_fp16(x, w)
+    full = want * gate.double() + resid.double()
+    lim = step(full) + (step(want) + slack) * gate.double().abs() + 2.0 ** -22 * (want * gate.double()).abs() + 2.0 ** -22 * resid.double().abs()
+    assert ((out.double() - full).abs() <= lim).all()
