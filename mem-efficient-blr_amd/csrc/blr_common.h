@@ -63,6 +63,17 @@ __device__ __forceinline__ float apply_act(float v, int act) {
   if (act == BLR_ACT_SILU) return v * __builtin_amdgcn_rcpf(1.0f + __expf(-v));
   return v;
 }
+// The same for N values, the choice made once: inside a loop every value would be a block of its own between two branches, and its
+// chain of an exponential and a reciprocal would run alone.
+template <int N> __device__ __forceinline__ void apply_act_n(float (&v)[N], int act) {
+  if (act == BLR_ACT_GELU_TANH) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) v[e] = apply_act(v[e], BLR_ACT_GELU_TANH);
+  } else if (act == BLR_ACT_SILU) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) v[e] = apply_act(v[e], BLR_ACT_SILU);
+  }
+}
 
 // 16-byte global load / store of 8 two-byte elements (pointer must be 16-byte aligned).
 template <typename V> __device__ __forceinline__ V ldg16(const void* p) {

@@ -28,43 +28,77 @@ __device__ __forceinline__ T ep_value(const GemmArgs& g, T r, int64_t in_row, in
   return TypeTraits<T>::from_f32(v);
 }
 
-// eight consecutive outputs; their offset inside the row is a multiple of 8, so the bias comes as one 16-byte load
+// U pieces of eight consecutive outputs; their offset inside the row is a multiple of 8, so bias, gate and residual come as 16-byte
+// loads.  What bounds a write-out with an output stage is not its bytes: with one piece at a time a thread waits for a trip to the L2
+// per piece (8 - 16 of them) and the values' exponentials follow one another.  So the operands of U pieces are asked for together,
+// and the activation is chosen outside the loop over their values.  Pieces that are not stored carry positions inside the operands.
+template <typename T, int U>
+__device__ __forceinline__ void ep_vectors(const GemmArgs& g, typename TypeTraits<T>::vec8 (&r)[U], const int64_t (&in_row)[U], const int (&row)[U]) {
+  using V8 = typename TypeTraits<T>::vec8;
+  V8 bv[U], gv[U], rv[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { bv[u][e] = (T)0.0f; gv[u][e] = (T)1.0f; rv[u][e] = (T)0.0f; }
+  if (g.bias) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) bv[u] = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.bias) + in_row[u]);
+  }
+  if (g.gate) {                                 // one row of gate per group of gate_rows rows of C
+#pragma unroll
+    for (int u = 0; u < U; ++u) gv[u] = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.gate) + (int64_t)(row[u] / g.gate_rows) * g.ld_gate + in_row[u]);
+  }
+  if (g.resid) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) rv[u] = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.resid) + (int64_t)row[u] * g.ld_resid + in_row[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = TypeTraits<T>::to_f32(r[u][e]) + TypeTraits<T>::to_f32(bv[u][e]);
+    apply_act_n(v, g.act);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[u][e] = TypeTraits<T>::from_f32(v[e]);
+  }
+  if (g.gate || g.resid) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) r[u][e] = TypeTraits<T>::from_f32(TypeTraits<T>::to_f32(r[u][e]) * TypeTraits<T>::to_f32(gv[u][e]) + TypeTraits<T>::to_f32(rv[u][e]));
+  }
+}
 template <typename T>
 __device__ __forceinline__ typename TypeTraits<T>::vec8 ep_vector(const GemmArgs& g, typename TypeTraits<T>::vec8 r, int64_t in_row, int row) {
-  using V8 = typename TypeTraits<T>::vec8;
-  V8 bv;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) bv[e] = (T)0.0f;
-  if (g.bias) bv = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.bias) + in_row);
-#pragma unroll
-  for (int e = 0; e < 8; ++e) r[e] = TypeTraits<T>::from_f32(apply_act(TypeTraits<T>::to_f32(r[e]) + TypeTraits<T>::to_f32(bv[e]), g.act));
-  if (g.gate || g.resid) {                      // one row of gate per group of gate_rows rows of C
-    V8 gv, rv;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { gv[e] = (T)1.0f; rv[e] = (T)0.0f; }
-    if (g.gate) gv = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.gate) + (int64_t)(row / g.gate_rows) * g.ld_gate + in_row);
-    if (g.resid) rv = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.resid) + (int64_t)row * g.ld_resid + in_row);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = TypeTraits<T>::from_f32(TypeTraits<T>::to_f32(r[e]) * TypeTraits<T>::to_f32(gv[e]) + TypeTraits<T>::to_f32(rv[e]));
-  }
-  return r;
+  typename TypeTraits<T>::vec8 v[1] = {r};
+  const int64_t at[1] = {in_row};
+  const int rows[1] = {row};
+  ep_vectors<T, 1>(g, v, at, rows);
+  return v[0];
 }
 
-// Second tile of a pair: (r + bias) rounded to T, times the first tile's result, which the same thread stored at `c` before.
-template <typename T>
-__device__ __forceinline__ typename TypeTraits<T>::vec8 ep_pair_up(const GemmArgs& g, typename TypeTraits<T>::vec8 r, int64_t in_row, const T* c) {
+// Second tile of a pair: (r + bias) rounded to T, times the first tile's result, which the same thread stored at c[u] before.
+template <typename T, int U>
+__device__ __forceinline__ void ep_pair_up(const GemmArgs& g, typename TypeTraits<T>::vec8 (&r)[U], const int64_t (&in_row)[U], const T* const (&c)[U]) {
   using V8 = typename TypeTraits<T>::vec8;
-  V8 bv;
+  V8 bv[U], gv[U];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) bv[e] = (T)0.0f;
-  if (g.bias) bv = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.bias) + in_row);
-  const V8 gv = *reinterpret_cast<const V8*>(c);
+  for (int u = 0; u < U; ++u)
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const T up = TypeTraits<T>::from_f32(TypeTraits<T>::to_f32(r[e]) + TypeTraits<T>::to_f32(bv[e]));
-    r[e] = TypeTraits<T>::from_f32(TypeTraits<T>::to_f32(gv[e]) * TypeTraits<T>::to_f32(up));
+    for (int e = 0; e < 8; ++e) bv[u][e] = (T)0.0f;
+  if (g.bias) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) bv[u] = *reinterpret_cast<const V8*>(reinterpret_cast<const T*>(g.bias) + in_row[u]);
   }
-  return r;
+#pragma unroll
+  for (int u = 0; u < U; ++u) gv[u] = *reinterpret_cast<const V8*>(c[u]);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const T up = TypeTraits<T>::from_f32(TypeTraits<T>::to_f32(r[u][e]) + TypeTraits<T>::to_f32(bv[u][e]));
+      r[u][e] = TypeTraits<T>::from_f32(TypeTraits<T>::to_f32(gv[u][e]) * TypeTraits<T>::to_f32(up));
+    }
 }
 
 }  // namespace blr

@@ -307,7 +307,13 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
         const int64_t in_row = (int64_t)bt * g.sC + gc;
         if constexpr (EP && ES == 2) {
           if (hf == 0) o = ep_vector<T>(g, o, in_row, gr);
-          else o = ep_pair_up<T>(g, o, in_row + g.pair_dbias, reinterpret_cast<const T*>(&first[n]));
+          else {
+            out8 up[1] = {o};
+            const int64_t at[1] = {in_row + g.pair_dbias};
+            const T* const c[1] = {reinterpret_cast<const T*>(&first[n])};
+            ep_pair_up<T, 1>(g, up, at, c);
+            o = up[0];
+          }
           if (hf + 1 < halves) { first[n] = o; continue; }
         }
         if (g.epi == EPI_MONARCH_SCATTER) {
