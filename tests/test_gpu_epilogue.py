@@ -244,3 +244,48 @@ def test_bad_activation_is_rejected():
     assert rc == -1 and b"activation" in lib.blr_last_error()
     with pytest.raises(L.BlrError):
         L.fused_epilogue(None, "relu")
+
+
+def _stage_case(call, out_f, M, dtype, act):
+    """call() under bias, act, a gate and a residual against the same call without them, finished in 64 bits.  Bound: one unit of the
+    plain result (the two may round a tie apart) and the roundings of h and of the result, through |act'| <= 1.13 and the gate."""
+    from triton_funcs import _lib as L
+    g = torch.Generator("cuda").manual_seed(M + out_f)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
+    rows = 257
+    bias, gate, resid = rand(out_f), rand(-(-M // rows), out_f), rand(M, out_f)
+    plain = call().reshape(M, out_f)
+    with L.fused_epilogue(bias, act, gate, rows, resid):
+        out = call().reshape(M, out_f).double()
+    unit = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    v = plain.double() + bias.double()
+    h = {None: lambda t: t, "silu": lambda t: t * torch.sigmoid(t), "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh")}[act](v)
+    grow = gate.double().repeat_interleave(rows, 0)[:M]
+    want = resid.double() + grow * h
+    lim = (1.13 * unit * plain.double().abs() + unit * h.abs() + 1e-5 * v.abs() + 2.0 ** -24) * grow.abs() + unit * want.abs() + 2.0 ** -24
+    assert ((out - want).abs() <= lim).all(), float(((out - want).abs() / lim).max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("act", [None, "gelu_tanh", "silu"])
+# ragged rows and columns of 128 x 128 and 256 x 128 tiles; 288-column batches on 96-column tiles are the next test's first shape
+@pytest.mark.parametrize("m,n,k", [(1000, 4616, 72), (2049, 4104, 200), (513, 9000, 1032)])
+def test_output_stage_over_ragged_tiles(m, n, k, act, dtype):
+    from triton_funcs import dense_kernels as D
+    x = torch.randn(m, k, device="cuda").to(dtype)
+    w = (torch.randn(k, n, device="cuda") / k ** 0.5).to(dtype)
+    say(f"[case] ragged tiles m={m} n={n} k={k} {act} {dtype}")
+    _stage_case(lambda: D.triton_dense_fp16(x, w), n, m, dtype, act)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+# (rows, columns of an input block, of an output block, rank): 96-column tiles; one launch; mix and product in one launch, whole and partial batches
+@pytest.mark.parametrize("m,p,q,r", [(2053, 72, 288, 576), (2053, 72, 72, 96), (2051, 96, 8, 128), (2053, 200, 80, 96), (2049, 288, 72, 160)])
+def test_output_stage_of_narrow_blocks(m, p, q, r, dtype):
+    from triton_funcs import blast_kernels as B
+    b = 16
+    x = torch.randn(1, m, b * p, device="cuda").to(dtype)
+    U, V = (torch.randn(b, q, r, device="cuda") / r ** 0.5).to(dtype), (torch.randn(b, p, r, device="cuda") / r ** 0.5).to(dtype)
+    S = torch.randn(r, b, b, device="cuda").to(dtype)
+    say(f"[case] narrow blocks m={m} p={p} q={q} r={r} {dtype}")
+    _stage_case(lambda: B.triton_blast_bmm_fp16(x, U, V, S), b * q, m, dtype, "silu" if q == 80 else None)
