@@ -651,22 +651,24 @@ __global__ __launch_bounds__(NWV * 64, (SHALLOW ? 2 : 1)) void gemm_ring_kernel(
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    // partial last tile: a lane's A fragment of slice kk covers k = (2 kk + half) * 8 .. + 7; those past ktail become zero
-    if (last_partial && half * 8 >= ktail) {
+    // partial last tile: a lane's fragments of slice kk cover k = (2 kk + half) * 8 .. + 7; those past ktail become zero, on both
+    // sides (one alone would make NaN of an infinity that was fetched again)
+    auto zero_tail = [&](int kk) {
+      if (last_partial && (2 * kk + half) * 8 >= ktail) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+        for (int e = 0; e < 8; ++e) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) af[0][i][e] = (T)0.0f;
-    }
+          for (int i = 0; i < TM; ++i) af[kk][i][e] = (T)0.0f;
+#pragma unroll
+          for (int j = 0; j < TN; ++j) bf[kk][j][e] = (T)0.0f;
+        }
+      }
+    };
+    zero_tail(0);
 #pragma unroll
     for (int m = 0; m < NMF; ++m) { mfma_one(0, m); slot(m); }
     __builtin_amdgcn_sched_barrier(0);
-    if (last_partial && (2 + half) * 8 >= ktail) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) af[1][i][e] = (T)0.0f;
-    }
+    zero_tail(1);
 #pragma unroll
     for (int m = 0; m < NMF / 2; ++m) { mfma_one(1, m); slot(NMF + m); }
     __builtin_amdgcn_sched_barrier(0);
@@ -899,12 +901,17 @@ __global__ __launch_bounds__(NWV * 64, (NWV / 4) * PER_CU) void gemm_ring64_kern
     const int i = idx / TN, j = idx % TN;
     acc[i][j] = TypeTraits<T>::mfma32(bf[set][j], af[set][i], acc[i][j]);
   };
-  auto zero_tail = [&](int set, int q) {               // a partial last stage: the A fragment of chunk 2 q + half is past ktail
-    if ((2 * q + half) * 8 >= ktail) {
+  // A partial last stage runs only the sub-steps that have something to add; where ktail ends in the middle of one, the lanes of its
+  // second chunk multiply zeros (on both sides: one alone would make NaN of an infinity that was fetched again).
+  auto zero_tail = [&](int set) {
+    if (half) {
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int e = 0; e < 8; ++e) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) af[set][i][e] = (T)0.0f;
+        for (int i = 0; i < TM; ++i) af[set][i][e] = (T)0.0f;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) bf[set][j][e] = (T)0.0f;
+      }
     }
   };
 
@@ -932,6 +939,7 @@ __global__ __launch_bounds__(NWV * 64, (NWV / 4) * PER_CU) void gemm_ring64_kern
     const bool pn = ktail && tn == KT - 1;
     const bool last_partial = ktail && t == KT - 1;
     const int nq = last_partial ? (ktail + 15) >> 4 : 4;             // sub-steps with anything to add
+    const int half_q = last_partial && (ktail & 8) ? nq - 1 : -1;    // the one of them that ends with its first chunk
     const int nx = cs + 1 == NST ? 0 : cs + 1;
     // With three stages the slot that the barrier of step t frees is needed only at the barrier of step t + 2, so its loads go out
     // over four sub-steps (part 0 in sub-step 3 of step t, parts 1..3 in sub-steps 0..2 of step t + 1) instead of queueing in the
@@ -964,11 +972,11 @@ __global__ __launch_bounds__(NWV * 64, (NWV / 4) * PER_CU) void gemm_ring64_kern
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    if (last_partial) zero_tail(0, 0);
+    if (half_q == 0) zero_tail(0);
     substep(0, true, cs, 1, 1);       // (in step 0 parts 1..3 repeat loads of the last stage the prologue asked for, into the same slot)
-    if (last_partial) zero_tail(1, 1);
+    if (half_q == 1) zero_tail(1);
     substep(1, nq > 1, cs, 2, 2);
-    if (last_partial) zero_tail(0, 2);
+    if (half_q == 2) zero_tail(0);
     substep(0, nq > 2, cs, 3, 3);
     // the step's barrier: stage t is in registers, stage t + 1 has landed
 #ifdef BLR_TRACE
@@ -985,7 +993,7 @@ __global__ __launch_bounds__(NWV * 64, (NWV / 4) * PER_CU) void gemm_ring64_kern
     trw_v += tw1 - tw0; trw_b += tw2 - tw1;
 #endif
     __builtin_amdgcn_sched_barrier(0);
-    if (last_partial) zero_tail(1, 3);
+    if (half_q == 3) zero_tail(1);
     substep(1, nq > 3, nx, 0, 0);
     cs = nx;
   }

@@ -182,15 +182,19 @@ __global__ __launch_bounds__((BM / 32 / TM) * (BN / 32 / TN) * KG * 64) void gem
         }
       }
     };
-    auto zero_tail = [&](int t, int set) {                           // a partial stage multiplies what it lacks with zeros
-      if (!(ktail && t * KG + kg == KT - 1)) return;
+    auto zero_tail = [&](int t, int set) {                           // what a partial stage lacks is zero on both sides (one alone would make
+      if (!(ktail && t * KG + kg == KT - 1)) return;                 // NaN of an infinity that was fetched again)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if ((2 * q + half) * CE >= ktail)
+        if ((2 * q + half) * CE >= ktail) {
 #pragma unroll
-          for (int i = 0; i < TM; ++i)
+          for (int e = 0; e < CE; ++e) {
 #pragma unroll
-            for (int e = 0; e < CE; ++e) af[set][q][i][e] = (T)0.0f;
+            for (int i = 0; i < TM; ++i) af[set][q][i][e] = (T)0.0f;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) bf[set][q][j][e] = (T)0.0f;
+          }
+        }
     };
     auto products = [&](int q, int set) {                            // (operands swapped: a lane gets runs of four columns of a row)
 #pragma unroll

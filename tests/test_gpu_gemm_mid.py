@@ -135,3 +135,36 @@ def test_output_operands_of_any_alignment(m, n, k):
     full = want * gate.double() + resid.double()
     lim = step(full) + (step(want) + slack) * gate.double().abs() + 2.0 ** -22 * (want * gate.double()).abs() + 2.0 ** -22 * resid.double().abs()
     assert ((out.double() - full).abs() <= lim).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m", [1, 16, 40, 100, 128, 200])
+@pytest.mark.parametrize("n,k", [(64, 72), (136, 1048), (264, 200), (2304, 776)])
+def test_infinite_weights(m, n, k, dtype):
+    """A weight of infinity anywhere in a reduction that ends in a partial stage gives infinities of the right sign, not NaN: what
+    stands in for the missing k of a stage meets zeros on both sides."""
+    from triton_funcs import _lib as L, dense_kernels as D, blast_kernels as B
+    g = torch.Generator("cuda").manual_seed(m + n + k)
+    x = (torch.rand(m, k, device="cuda", generator=g) + 0.5).to(dtype)
+    x[::2] *= -1
+    w = (torch.randn(k, n, device="cuda", generator=g) / k ** 0.5).to(dtype)
+    for col, row in enumerate((0, k - 1, k - 8, k - 5, k // 2)):
+        w[row, col] = float("inf")
+    say(f"[case] infinite weights {dtype} m={m} n={n} k={k}")
+    f = D.triton_dense_fp32 if dtype == torch.float32 else D.triton_dense_fp16
+    ref = x.double() @ w.double()
+    outs = [f(x, w)]
+    if dtype != torch.float32:
+        outs.append(f(x, w, {"algo": L.ALGO_TILED}))
+    if dtype != torch.float32 and m > 16:                            # (up to 16 rows BLAST streams its factors through other kernels)
+        # the same product with the weights' k contiguous: BLAST's second one, U (b, q, r), behind a first that hands x through
+        b = 2
+        V, S = torch.eye(k, device="cuda").to(dtype).expand(b, k, k).contiguous(), torch.zeros(k, b, b, device="cuda").to(dtype)
+        S[:, 0, 0] = S[:, 1, 1] = 1.0
+        out = B.triton_blast_bmm_fp16(torch.cat([x, x], 1)[None], w.t().contiguous().expand(b, n, k).contiguous(), V, S)
+        outs += [out[0, :, :n], out[0, :, n:]]
+    for i, out in enumerate(outs):
+        inf = torch.isinf(ref)
+        assert inf[:, :5].all() and not inf[:, 5:].any()
+        assert torch.equal(out[:, :5].double(), ref[:, :5]), i
+        assert torch.isfinite(out[:, 5:]).all(), i
