@@ -56,7 +56,7 @@ def build(verbose=True):
     out = _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", "-Wno-deprecated-declarations",
                 f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}",
                 os.path.join(HERE, "csrc", "blr_host.cpp"), "-o", host,
-                f"-L{root}/lib", "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10_hip", "-lc10"])
+                f"-L{root}/lib", "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10_hip", "-lc10", "-lamdhip64"])
     if verbose:
         print(out.strip() or f"built {host}")
     # the stand-alone probes (not part of the library): built next to their sources so that they compile as long as the tree does

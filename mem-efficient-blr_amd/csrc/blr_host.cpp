@@ -15,9 +15,11 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <algorithm>
 #include <cstdint>
 #include <map>
 #include <tuple>
+#include <vector>
 #include "../../include/blr.h"
 
 namespace {
@@ -48,13 +50,38 @@ PyObject* blr_error = nullptr;                     // triton_funcs._lib.BlrError
 
 // ---- workspaces: one per (device, stream, kind), kept until the process ends (the shims' contract; see _lib.workspace) -------
 // Only touched with the interpreter lock held, and never destroyed: the process may end after the device runtime did.
-auto& workspaces = *new std::map<std::tuple<int, void*, bool>, at::Tensor>;
+using WsKey = std::tuple<int, void*, bool>;
+auto& workspaces = *new std::map<WsKey, at::Tensor>;
+// Outgrown ones stay as they are: a graph captured while they were in use replays into their memory, the control words of a streaming
+// one among it.  Every growth doubles at least, so all of them together are smaller than the one in use.
+auto& outgrown = *new std::vector<at::Tensor>;
+// What a call under capture is given when none of them is large enough: memory of the graph, zeroed by every replay and by nothing
+// else, so only calls of the same capture use it.
+auto& captured = *new std::map<WsKey, std::pair<unsigned long long, at::Tensor>>;
+
+// the capture that `stream` is part of, 0 outside of one (the default stream cannot be)
+unsigned long long capture_of(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (!stream) return 0;
+  if (hipStreamGetCaptureInfo((hipStream_t)stream, &status, &id) != hipSuccess) { (void)hipGetLastError(); return 0; }
+  return status == hipStreamCaptureStatusActive ? id : 0;
+}
 
 const at::Tensor& workspace(const at::Device& dev, void* stream, size_t bytes, bool streaming) {
-  at::Tensor& ws = workspaces[{dev.index(), stream, streaming}];
-  if (!ws.defined() || (size_t)ws.numel() < bytes)
-    ws = at::zeros({(int64_t)std::max<size_t>(bytes, (size_t)1 << 20)}, at::TensorOptions().dtype(at::kByte).device(dev));
-  return ws;
+  const WsKey key{dev.index(), stream, streaming};
+  at::Tensor& ws = workspaces[key];
+  const size_t have = ws.defined() ? (size_t)ws.numel() : 0;
+  if (have >= bytes && have) return ws;
+  auto make = [&](size_t n) { return at::zeros({(int64_t)n}, at::TensorOptions().dtype(at::kByte).device(dev)); };
+  if (const unsigned long long id = capture_of(stream)) {
+    auto& c = captured[key];
+    if (c.first != id || (size_t)c.second.numel() < bytes) c = {id, make(bytes)};
+    return c.second;
+  }
+  at::Tensor grown = make(std::max({bytes, 2 * have, (size_t)1 << 20}));
+  if (have) outgrown.push_back(std::move(ws));
+  return ws = std::move(grown);
 }
 
 // ---- what a call looks at ---------------------------------------------------------------------------------------------------

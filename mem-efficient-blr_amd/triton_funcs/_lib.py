@@ -204,8 +204,11 @@ def rows(x):
 # Workspaces, one per (device, stream, kind).  kind "stream": the streaming kernels keep their
 # barrier and split counters in its head; it must start zeroed, they leave it zeroed, and nothing
 # else may scribble on it.  kind "scratch": plain scratch of the tiled kernels.  Work on one stream
-# is ordered, so sharing inside a stream is safe.
+# is ordered, so sharing inside a stream is safe.  One that is outgrown stays as it is, since a graph
+# captured with it replays into its memory; every growth doubles at least.  A call under capture that
+# finds none large enough gets memory of the graph, zeroed by every replay, which nothing else uses.
 _workspaces = {}
+_outgrown = []
 
 
 def workspace(device, nbytes, algo=ALGO_AUTO, M=None, dtype=None):
@@ -220,10 +223,14 @@ def workspace(device, nbytes, algo=ALGO_AUTO, M=None, dtype=None):
     key = (index, stream, "stream" if streaming else "scratch")
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
-        size = max(int(nbytes), 1 << 20)
-        ws = torch.zeros(size, dtype=torch.uint8, device=device)
+        capturing = torch.cuda.is_current_stream_capturing()
+        size = int(nbytes) if capturing else max(int(nbytes), 1 << 20, 0 if ws is None else 2 * ws.numel())
+        old, ws = ws, torch.zeros(size, dtype=torch.uint8, device=device)
         ws._blr_streaming = streaming
-        _workspaces[key] = ws
+        if not capturing:
+            if old is not None:
+                _outgrown.append(old)
+            _workspaces[key] = ws
     return ws
 
 
