@@ -29,12 +29,18 @@ def _bare(module, kind):
             and not m._global_forward_hooks and not m._global_forward_pre_hooks)
 
 
+def _library(x):
+    """The native call path, whose kernels stand in for torch's operators on x; something false where it is not there or those have to be
+    seen: torch.compile and torch.export trace operators and nothing else."""
+    return x.is_cuda and not torch.compiler.is_compiling() and L.call_path()
+
+
 def _norm_modulate(norm, x, shift, scale):
     """modulate(norm(x), shift, scale): one kernel where norm is a bare LayerNorm without an affine part and nothing but the result is
     wanted (inference on the GPU), torch's operators otherwise."""
-    if x.is_cuda and _bare(norm, nn.LayerNorm) and norm.weight is None and norm.bias is None and norm.normalized_shape == x.shape[-1:]:
-        host = L.call_path()
-        out = host.ln_modulate(x, shift, scale, norm.eps) if host else None
+    host = _library(x)
+    if host and _bare(norm, nn.LayerNorm) and norm.weight is None and norm.bias is None and norm.normalized_shape == x.shape[-1:]:
+        out = host.ln_modulate(x, shift, scale, norm.eps)
         if out is not None:
             return out
     return modulate(norm(x), shift, scale)
@@ -42,9 +48,9 @@ def _norm_modulate(norm, x, shift, scale):
 
 def _conditioned(proj, c):
     """proj(c) of an adaLN projection Sequential(SiLU, Linear): one kernel for the few rows of c at inference on the GPU."""
-    if c.is_cuda and _bare(proj, nn.Sequential) and len(proj) == 2 and _bare(proj[0], nn.SiLU) and not proj[0].inplace and _bare(proj[1], nn.Linear):
-        host = L.call_path()
-        out = host.silu_linear(c, proj[1].weight, proj[1].bias) if host else None
+    host = _library(c)
+    if host and _bare(proj, nn.Sequential) and len(proj) == 2 and _bare(proj[0], nn.SiLU) and not proj[0].inplace and _bare(proj[1], nn.Linear):
+        out = host.silu_linear(c, proj[1].weight, proj[1].bias)
         if out is not None:
             return out
     return proj(c)
@@ -89,9 +95,9 @@ class Attention(nn.Module):
 
     def _attend(self, qkv, B, N, C):
         """Attention over the packed qkv, (B, N, C): the library's kernel at inference with heads it has, torch's otherwise."""
-        if qkv.is_cuda and qkv.shape == (B, N, 3 * C):
-            host = L.call_path()
-            o = host.attention(qkv, self.heads) if host else None
+        host = _library(qkv)
+        if host and qkv.shape == (B, N, 3 * C):
+            o = host.attention(qkv, self.heads)
             if o is not None:
                 return o
         qkv = qkv.reshape(B, N, 3, self.heads, C // self.heads).permute(2, 0, 3, 1, 4)

@@ -161,3 +161,37 @@ def test_silu_linear_is_left_to_torch():
     assert h.silu_linear(c, lin.weight, lin.bias) is None                                    # the weight wants a gradient
     D._conditioned(proj, c).sum().backward()
     assert lin.weight.grad is not None
+
+
+def _layers():
+    """The parts of a DiT that the library's kernels stand in for, with torch's own linears, and a call of each."""
+    from models import dit_xl as D
+    torch.manual_seed(1)
+    x, c = torch.randn(2, 9, 128, device="cuda").half(), torch.randn(2, 128, device="cuda").half()
+    return [(m.cuda().half().eval(), x, c) for m in (D.DiTBlock(128, 2), D.FinalLayer(128, 2, 4))]
+
+
+def test_compiled_layers_are_left_to_torch():
+    """One graph, as torch's operators give it: the library's entries are nothing that a compiler can trace."""
+    for layer, x, c in _layers():
+        say(f"[case] compiled {type(layer).__name__}")
+        torch._dynamo.reset()
+        with torch.no_grad():
+            want = layer(x, c)
+            got = torch.compile(layer, fullgraph=True, backend="eager")(x, c)
+        assert torch.allclose(got.float(), want.float(), atol=2e-2, rtol=2e-2)
+
+
+def test_compiled_block_of_structured_linears():
+    from models import dit_xl as D
+    from models.wrappers import BlastLinear
+    layer, x, c = _layers()[0]
+    for at, name, n, m in ((layer.attn, "qkv", 128, 384), (layer.attn, "proj", 128, 128), (layer.mlp, "fc1", 128, 512), (layer.mlp, "fc2", 512, 128)):
+        setattr(at, name, BlastLinear(n, m, 4, 32, "triton_funcs.blast_kernels.triton_blast_bmm_fp16", "cuda", torch.float16))
+    layer.mlp.fc1.fused_act = "gelu_tanh"
+    torch._dynamo.reset()
+    with torch.no_grad():
+        want = layer(x, c)
+        got = torch.compile(layer, backend="eager")(x, c)
+    scale = want.float().abs().max().item()
+    assert torch.allclose(got.float(), want.float(), atol=2e-2 * scale)
