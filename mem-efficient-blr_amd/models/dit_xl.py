@@ -31,8 +31,8 @@ def _bare(module, kind):
 
 def _library(x):
     """The native call path, whose kernels stand in for torch's operators on x; something false where it is not there or those have to be
-    seen: torch.compile and torch.export trace operators and nothing else."""
-    return x.is_cuda and not torch.compiler.is_compiling() and L.call_path()
+    seen: torch.compile, torch.export and torch.fx (whose x is no tensor) trace operators and nothing else."""
+    return isinstance(x, torch.Tensor) and x.is_cuda and not torch.compiler.is_compiling() and L.call_path()
 
 
 def _norm_modulate(norm, x, shift, scale):
@@ -144,8 +144,13 @@ class FinalLayer(nn.Module):
         self.adaLN_modulation = nn.Sequential(nn.SiLU(), nn.Linear(hidden, 2 * hidden))
 
     def forward(self, x, c):
-        shift, scale = _conditioned(self.adaLN_modulation, c).chunk(2, dim=1)
-        return self.linear(_norm_modulate(self.norm_final, x, shift, scale))
+        if torch.jit.is_scripting():                         # (a script calls the modules themselves)
+            shift, scale = self.adaLN_modulation(c).chunk(2, dim=1)
+            h = modulate(self.norm_final(x), shift, scale)
+        else:
+            shift, scale = _conditioned(self.adaLN_modulation, c).chunk(2, dim=1)
+            h = _norm_modulate(self.norm_final, x, shift, scale)
+        return self.linear(h)
 
 
 def sincos_2d(dim, grid):

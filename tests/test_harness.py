@@ -286,3 +286,17 @@ def test_every_exported_operator_name_has_a_roofline_formula():
                 continue
             stem = name.rsplit("_", 1)[0]
             assert hasattr(R, f"{stem}_mem_flops"), f"{name}: no {stem}_mem_flops in roofline.py"
+
+
+def test_dit_layers_can_be_traced():
+    """The library's entries in a DiT's layers are out of the way of torch.fx, torch.jit and torch.export."""
+    from models.dit_xl import DiTBlock, FinalLayer
+    torch.manual_seed(0)
+    x, c = torch.randn(2, 9, 128), torch.randn(2, 128)
+    for layer in (DiTBlock(128, 2), FinalLayer(128, 2, 4)):
+        want = layer(x, c)
+        forms = [torch.fx.symbolic_trace(layer), torch.jit.trace(layer, (x, c)), torch.export.export(layer, (x, c)).module()]
+        if isinstance(layer, FinalLayer):
+            forms.append(torch.jit.script(layer))
+        for f in forms:
+            assert torch.allclose(f(x, c), want, atol=1e-5)
