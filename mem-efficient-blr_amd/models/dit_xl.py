@@ -12,6 +12,8 @@ import math
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from triton_funcs import _lib as L
 from utils import replace_linear_with_custom
@@ -31,8 +33,13 @@ def _bare(module, kind):
 
 def _library(x):
     """The native call path, whose kernels stand in for torch's operators on x; something false where it is not there or those have to be
-    seen: torch.compile, torch.export and torch.fx (whose x is no tensor) trace operators and nothing else."""
-    return isinstance(x, torch.Tensor) and x.is_cuda and not torch.compiler.is_compiling() and L.call_path()
+    seen: torch.compile, torch.export and torch.fx (whose x is no tensor) trace operators and nothing else, and a function mode sees each
+    of them (but for the one that sets the default device, which looks at factories only)."""
+    if not isinstance(x, torch.Tensor) or not x.is_cuda or torch.compiler.is_compiling():
+        return False
+    if torch._C._len_torch_function_stack() and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()):
+        return False
+    return L.call_path()
 
 
 def _norm_modulate(norm, x, shift, scale):

@@ -195,3 +195,21 @@ def test_compiled_block_of_structured_linears():
         got = torch.compile(layer, backend="eager")(x, c)
     scale = want.float().abs().max().item()
     assert torch.allclose(got.float(), want.float(), atol=2e-2 * scale)
+
+
+def test_function_modes_see_the_operators():
+    from torch.overrides import TorchFunctionMode
+
+    class Watch(TorchFunctionMode):
+        def __init__(self):
+            super().__init__()
+            self.seen = set()
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.seen.add(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    for layer, x, c in _layers():
+        with torch.no_grad(), Watch() as w:
+            layer(x, c)
+        assert {"layer_norm", "silu", "linear"} <= w.seen, w.seen
