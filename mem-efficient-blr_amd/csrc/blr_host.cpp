@@ -10,6 +10,7 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <ATen/ATen.h>
+#include <ATen/Context.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
@@ -441,6 +442,8 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const at::Tensor* x = tensor(args[0]);
   const int64_t H = PyLong_AsLong(args[1]);
   if (PyErr_Occurred() || !x || H < 1 || !torch_modes_off() || !plain(*x)) DECLINE;
+  // (a kernel of the flash kind: a caller that has those switched off, sdpa_kernel(MATH) for one, wants another one's arithmetic)
+  if (!at::globalContext().userEnabledFlashSDP()) DECLINE;
   const int dt = dtype_code(x->scalar_type());
   if ((dt != BLR_F16 && dt != BLR_BF16) || x->dim() != 3 || x->numel() == 0 || !x->is_contiguous() || !aligned16(*x) || x->size(2) % (3 * H)) DECLINE;
   const int64_t B = x->size(0), N = x->size(1), D = x->size(2) / (3 * H);

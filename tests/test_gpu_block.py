@@ -213,3 +213,15 @@ def test_function_modes_see_the_operators():
         with torch.no_grad(), Watch() as w:
             layer(x, c)
         assert {"layer_norm", "silu", "linear"} <= w.seen, w.seen
+
+
+def test_attention_backend_of_the_caller():
+    from torch.nn.attention import SDPBackend, sdpa_kernel
+    h, x = _host(), torch.randn(2, 8, 3 * 2 * 64, device="cuda").half()
+    with sdpa_kernel(SDPBackend.MATH):
+        assert h.attention(x, 2) is None
+    with sdpa_kernel(SDPBackend.EFFICIENT_ATTENTION):
+        assert h.attention(x, 2) is None
+    with sdpa_kernel([SDPBackend.MATH, SDPBackend.FLASH_ATTENTION]):
+        assert h.attention(x, 2) is not None
+    assert h.attention(x, 2) is not None
