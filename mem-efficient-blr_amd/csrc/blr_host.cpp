@@ -109,6 +109,13 @@ bool rows_of(const at::Tensor& x, int64_t in, Rows& r) {
   return true;
 }
 
+// no gradient or tangent, no transform and no lazy form
+bool plain(const at::Tensor& t) {
+  return t.is_cuda() && t.layout() == at::kStrided && !(at::GradMode::is_enabled() && t.requires_grad()) && !t._fw_grad(0).defined() &&
+         !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                                   c10::DispatchKey::Functionalize, c10::DispatchKey::Negative, c10::DispatchKey::Conjugate, c10::DispatchKey::ZeroTensor}));
+}
+
 struct Ep {
   bool on = false;
   const void* bias = nullptr; int act = 0;
@@ -260,6 +267,11 @@ PyObject* blast_q(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t b = vs->size(0), r = vs->size(1), q = us->size(1), p = vc->size(1), in = b * p, out_f = b * q;
   if (b < 2 || us->size(0) != b || uc->size(0) != b || vc->size(0) != b || uc->size(1) != r || uc->size(2) * 8 != q * bits || vc->size(2) * 8 != r * bits) DECLINE;
   if (uc->element_size() != 1 || vc->element_size() != 1 || S->size(0) != r || S->size(1) != b || S->size(2) != b) DECLINE;
+  // the module adds a bias that this one cannot take with torch, where it may be trained
+  if (args[7] != Py_None && PyTuple_Check(args[7]) && PyTuple_GET_SIZE(args[7]) == 5 && PyTuple_GET_ITEM(args[7], 0) != Py_None) {
+    const at::Tensor* bias = tensor(PyTuple_GET_ITEM(args[7], 0));
+    if (!bias || !plain(*bias)) DECLINE;
+  }
   Rows R;
   Ep e;
   if (!rows_of(*x, in, R) || !epilogue(args[7], *x, R.M, out_f, e)) DECLINE;
@@ -400,11 +412,6 @@ PyObject* dense(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 bool torch_modes_off() {
   const auto tls = c10::impl::tls_local_dispatch_key_set();
   return (tls.included_ - c10::default_included_set).empty() && !at::autocast::is_autocast_enabled(at::kCUDA);
-}
-bool plain(const at::Tensor& t) {
-  return t.is_cuda() && t.layout() == at::kStrided && !(at::GradMode::is_enabled() && t.requires_grad()) && !t._fw_grad(0).defined() &&
-         !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
-                                                   c10::DispatchKey::Functionalize, c10::DispatchKey::Negative, c10::DispatchKey::Conjugate, c10::DispatchKey::ZeroTensor}));
 }
 bool aligned16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
 

@@ -105,6 +105,27 @@ def test_quantized_module_bias_and_activation():
             assert (err <= slope + 4 * half * b[0].float().abs() + 1e-6).all(), (act, rows, float(err.max()))
 
 
+def test_quantized_module_bias_gradient():
+    """A bias that wants a gradient, or carries a tangent, is added by torch: the kernel's output stage has neither."""
+    from models.wrappers import QuantBlastLinear
+    torch.manual_seed(0)
+    m = QuantBlastLinear(128, 192, b=4, rank=64, func_path="triton_funcs.blast_sym_quant_kernels.triton_blast_bmm_int8_fp16", device="cuda", dtype=torch.float16)
+    for rows in (1, 9, 150):
+        x = torch.randn(1, rows, 128, device="cuda").half()
+        m.bias.grad = None
+        m(x).float().sum().backward()
+        assert torch.equal(m.bias.grad, torch.full_like(m.bias, rows))
+    m.fused_act, m.bias.grad = "silu", None
+    m(x).float().sum().backward()
+    assert m.bias.grad is not None and bool((m.bias.grad != 0).any())
+    m.fused_act = None
+    bias = m.bias.detach()
+    del m.bias
+    with torch.autograd.forward_ad.dual_level():
+        m.bias = torch.autograd.forward_ad.make_dual(bias, torch.ones_like(bias))
+        assert torch.autograd.forward_ad.unpack_dual(m(x)).tangent is not None
+
+
 def test_irregular_calls_raise_as_before():
     from triton_funcs import _lib as L, blast_kernels as B, dense_kernels as D
     (f, (U, V, S)), = _ops(torch.float16)[:1]
