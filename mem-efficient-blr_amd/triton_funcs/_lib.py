@@ -333,6 +333,14 @@ def ep_workspace_extra(ep, op, M, out_f, b, dt):
     return lib().blr_ep_workspace_bytes(op, M, out_f, b, dt, ep[1]) if ep is not None else 0
 
 
+def _rows_apart(t, out_f):
+    """t as rows of out_f values with a stride between them that the kernels take (an expanded row is copied out), and that stride."""
+    t = t.reshape(-1, out_f)
+    if t.stride(1) != 1 or (t.shape[0] > 1 and t.stride(0) < out_f):
+        t = t.clone(memory_format=torch.contiguous_format)
+    return t, t.stride(0) if t.shape[0] > 1 else out_f          # (torch leaves the stride of a single row open)
+
+
 def pending_epilogue(out_f, dtype, device):
     """(bias pointer or None, activation code, keep-alive, (gate pointer, gate_rows, ld_gate, residual pointer, ld_residual)) of the
     active context, or None."""
@@ -346,13 +354,9 @@ def pending_epilogue(out_f, dtype, device):
         bias = bias.detach().to(device=device, dtype=dtype).contiguous()
     extra = [None, 0, 0, None, 0]
     if gate is not None:
-        gate = gate.detach().to(device=device, dtype=dtype).reshape(-1, out_f)
-        if gate.stride(-1) != 1:
-            gate = gate.contiguous()
-        extra[0:3] = [gate.data_ptr(), gate_rows, gate.stride(0)]
+        gate, ld = _rows_apart(gate.detach().to(device=device, dtype=dtype), out_f)
+        extra[0:3] = [gate.data_ptr(), gate_rows, ld]
     if resid is not None:
-        resid = resid.detach().to(device=device, dtype=dtype).reshape(-1, out_f)
-        if resid.stride(-1) != 1:
-            resid = resid.contiguous()
-        extra[3:5] = [resid.data_ptr(), resid.stride(0)]
+        resid, ld = _rows_apart(resid.detach().to(device=device, dtype=dtype), out_f)
+        extra[3:5] = [resid.data_ptr(), ld]
     return (bias.data_ptr() if bias is not None else None), act, (bias, gate, resid), tuple(extra)

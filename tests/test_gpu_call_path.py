@@ -81,6 +81,32 @@ def test_same_output_stage(rows, dtype):
         _same(lambda: f.with_epilogue(x, *w, (None, 0, gate, rows, resid)))
 
 
+@pytest.mark.parametrize("rows", [1, 6, 40, 200])
+def test_expanded_gate_and_residual(rows):
+    """One row of modulation, or of the residual, for everything: a view without a stride between its rows."""
+    from triton_funcs import _lib as L
+    images = 3
+    for f, w in _ops(torch.float16):
+        if not hasattr(f, "with_epilogue") or "int8" in f.__name__:
+            continue
+        say(f"[case] expanded gate {f.__name__} {images} x {rows}")
+        x = torch.randn(images, rows, 128, device="cuda").half()
+        gate, resid = torch.randn(192, device="cuda").half(), torch.randn(192, device="cuda").half()
+        full = resid.expand(images * rows, 192)
+        want = f.with_epilogue(x, *w, (None, 0, gate.repeat(images, 1), rows, full.contiguous()))
+        for g, r in ((gate.expand(images, 192), full.contiguous()), (gate.expand(images, 192), full), (gate.repeat(images, 1), full)):
+            for got in _both(lambda: f.with_epilogue(x, *w, (None, 0, g, rows, r))):
+                assert torch.equal(got[0], want)
+            with L.fused_epilogue(None, None, g, rows, r):
+                assert torch.equal(f(x, *w).reshape(want.shape), want)
+        # a single row, whose stride torch is free to choose
+        one = torch.as_strided(gate, (1, 192), (0, 1))
+        x1 = x[:1].contiguous()
+        want = f.with_epilogue(x1, *w, (None, 0, gate.reshape(1, 192), rows, None))
+        for got in _both(lambda: f.with_epilogue(x1, *w, (None, 0, one, rows, None))):
+            assert torch.equal(got[0], want)
+
+
 def test_quantized_module_bias_and_activation():
     """QuantBlastLinear's bias and activation in the kernel's output stage: as the separate passes leave them."""
     from models.wrappers import QuantBlastLinear
