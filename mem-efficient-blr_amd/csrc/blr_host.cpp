@@ -144,7 +144,10 @@ bool epilogue(PyObject* ep, const at::Tensor& x, int64_t M, int64_t out_f, Ep& e
   int64_t ld_bias = 0;
   if (!operand(PyTuple_GET_ITEM(ep, 0), 1, &e.bias, &ld_bias) || !operand(PyTuple_GET_ITEM(ep, 2), 0, &e.gate, &e.ld_gate) ||
       !operand(PyTuple_GET_ITEM(ep, 4), M, &e.resid, &e.ld_resid)) return false;
-  if (e.gate) e.gate_rows = (int)PyLong_AsLong(PyTuple_GET_ITEM(ep, 3));
+  if (e.gate) {                                    // a row of it for every gate_rows rows of the result, the last ones too
+    e.gate_rows = (int)PyLong_AsLong(PyTuple_GET_ITEM(ep, 3));
+    if (e.gate_rows < 1 || tensor(PyTuple_GET_ITEM(ep, 2))->numel() / out_f * e.gate_rows < M) return false;
+  }
   return !PyErr_Occurred();
 }
 

@@ -341,8 +341,8 @@ def _rows_apart(t, out_f):
     return t, t.stride(0) if t.shape[0] > 1 else out_f          # (torch leaves the stride of a single row open)
 
 
-def pending_epilogue(out_f, dtype, device):
-    """(bias pointer or None, activation code, keep-alive, (gate pointer, gate_rows, ld_gate, residual pointer, ld_residual)) of the
+def pending_epilogue(rows, out_f, dtype, device):
+    """For `rows` rows of out_f values: (bias pointer or None, activation code, keep-alive, (gate pointer, gate_rows, ld_gate, residual pointer, ld_residual)) of the
     active context, or None."""
     ep = getattr(_ep_state, "ep", None)
     if ep is None:
@@ -355,8 +355,12 @@ def pending_epilogue(out_f, dtype, device):
     extra = [None, 0, 0, None, 0]
     if gate is not None:
         gate, ld = _rows_apart(gate.detach().to(device=device, dtype=dtype), out_f)
+        if gate.shape[0] * gate_rows < rows:
+            raise BlrError(f"a gate of {gate.shape[0]} rows, one for every {gate_rows} of the result, is too short for {rows}")
         extra[0:3] = [gate.data_ptr(), gate_rows, ld]
     if resid is not None:
         resid, ld = _rows_apart(resid.detach().to(device=device, dtype=dtype), out_f)
+        if resid.shape[0] < rows:
+            raise BlrError(f"a residual of {resid.shape[0]} rows is too short for {rows}")
         extra[3:5] = [resid.data_ptr(), ld]
     return (bias.data_ptr() if bias is not None else None), act, (bias, gate, resid), tuple(extra)

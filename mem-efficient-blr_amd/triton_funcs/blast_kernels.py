@@ -68,7 +68,7 @@ def _blast(name, x, U, V, S, u_layout, s_layout, algo, want_intermediates):
         y = torch.empty((b1, M, r), device=x.device, dtype=x.dtype)
         algo = L.ALGO_TILED
     lib = L.lib()
-    ep = None if want_intermediates else L.pending_epilogue(out_f, x.dtype, x.device)
+    ep = None if want_intermediates else L.pending_epilogue(M, out_f, x.dtype, x.device)
     out = torch.empty((M, L.ep_out_features(ep, out_f)), device=x.device, dtype=x.dtype)
     need = lib.blr_blast_workspace_bytes(M, in_f, out_f, b1, r, dt, algo) + L.ep_workspace_extra(ep, L.OP_BLAST, M, out_f, b1, dt)
     ws = L.workspace(x.device, need, algo, M, dt)

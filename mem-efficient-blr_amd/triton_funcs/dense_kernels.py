@@ -30,7 +30,7 @@ def _dense(name, x, w, algo):
     M, in_f = x2.shape
     out_f = w.shape[1]
     lib = L.lib()
-    ep = L.pending_epilogue(out_f, x.dtype, x.device)
+    ep = L.pending_epilogue(M, out_f, x.dtype, x.device)
     out = torch.empty((M, L.ep_out_features(ep, out_f)), device=x.device, dtype=x.dtype)
     ws = L.workspace(x.device, lib.blr_dense_workspace_bytes(M, in_f, out_f, dt, algo) + L.ep_workspace_extra(ep, L.OP_DENSE, M, out_f, 1, dt), algo, M, dt)
     if ep is not None:

@@ -32,7 +32,7 @@ def _low_rank(name, x, a, b, algo, want_z):
     r, out_f = b.shape
     z = torch.empty((M, r), device=x.device, dtype=x.dtype) if want_z else None
     lib = L.lib()
-    ep = None if want_z else L.pending_epilogue(out_f, x.dtype, x.device)
+    ep = None if want_z else L.pending_epilogue(M, out_f, x.dtype, x.device)
     out = torch.empty((M, L.ep_out_features(ep, out_f)), device=x.device, dtype=x.dtype)
     ws = L.workspace(x.device, lib.blr_low_rank_workspace_bytes(M, in_f, out_f, r, dt, algo) + L.ep_workspace_extra(ep, L.OP_LOW_RANK, M, out_f, 1, dt), algo, M, dt)
     if ep is not None:

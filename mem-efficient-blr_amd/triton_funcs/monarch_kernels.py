@@ -58,7 +58,7 @@ def _monarch(name, x, w1, w2, w2_layout, out_order, algo, want_out1):
     if want_out1:
         algo = L.ALGO_TILED
     lib = L.lib()
-    ep = None if want_out1 else L.pending_epilogue(out_f, x.dtype, x.device)
+    ep = None if want_out1 else L.pending_epilogue(M, out_f, x.dtype, x.device)
     out = torch.empty((M, L.ep_out_features(ep, out_f)), device=x.device, dtype=x.dtype)
     ws = L.workspace(x.device, lib.blr_monarch_workspace_bytes(M, in_f, out_f, k, q, dt, algo) + L.ep_workspace_extra(ep, L.OP_MONARCH, M, out_f, k, dt), algo, M, dt)
     if ep is not None:

@@ -7,20 +7,22 @@ from gpu_util import say
 pytestmark = pytest.mark.gpu
 
 
-def _both(f):
-    """f() on the native call path and on the Python path, as tuples of tensors."""
+def _on(native, f):
+    """f() on the native call path, or on the Python path."""
     from triton_funcs import _lib as L
     assert L.call_path(), "the native call path did not load"
-    outs = []
     host = L._host
-    for on in (True, False):
-        L._host = host if on else False
-        try:
-            o = f()
-        finally:
-            L._host = host
-        outs.append(o if isinstance(o, tuple) else (o,))
-    return outs
+    L._host = host if native else False
+    try:
+        return f()
+    finally:
+        L._host = host
+
+
+def _both(f):
+    """f() on the native call path and on the Python path, as tuples of tensors."""
+    outs = [_on(native, f) for native in (True, False)]
+    return [o if isinstance(o, tuple) else (o,) for o in outs]
 
 
 def _same(f):
@@ -168,3 +170,19 @@ def test_irregular_calls_raise_as_before():
     assert cfg["M"] == 4 and cfg["in_f"] == 128 and cfg["out_f"] == 192 and cfg["rank"] == 64 and cfg["dtype"] == "torch.float16"
     f(x[:, :3], U, V, S)
     assert B.get_triton_blast_full_fp16_config()["M"] == 3
+
+
+def test_gates_and_residuals_that_are_too_short_are_refused():
+    from triton_funcs import _lib as L
+    for f, w in _ops(torch.float16):
+        if not hasattr(f, "with_epilogue") or "int8" in f.__name__:
+            continue
+        for rows in (7, 100):
+            x = torch.randn(rows, 128, device="cuda").half()
+            t = lambda n: torch.randn(n, 192, device="cuda").half()
+            for gate, every, resid in ((t(2), 3, None), (t(1), rows - 1, None), (t(1), 0, None), (None, 0, t(rows - 1)), (t(1), rows, t(1))):
+                say(f"[case] too short {f.__name__} {rows} rows, one gate row for {every}")
+                for host in (True, False):
+                    with pytest.raises(L.BlrError):
+                        _on(host, lambda: f.with_epilogue(x, *w, (None, 0, gate, every, resid)))
+            f.with_epilogue(x, *w, (None, 0, t(2), -(-rows // 2), t(rows)))
