@@ -701,7 +701,9 @@ int blr_low_rank_fwd(const void* x, int64_t ldx, const void* A, const void* B,
   const size_t need = z_out ? 0 : used + tiled;
   if (need && (!ws || ws_bytes < need)) { set_error("low_rank: workspace %zu < %zu", ws_bytes, need); return BLR_ERR_WORKSPACE; }
   used += tiled;
-  if (ws && ws_bytes > used) { g1.splitk_ws = static_cast<char*>(ws) + used; g1.splitk_bytes = ws_bytes - used; }
+  // (never more than was asked for: what the workspace has beyond that is another call's, and must not decide on the slices)
+  const size_t splitk = gemm_splitk_bytes(M, r, in_f, dtype);
+  if (ws && splitk && ws_bytes >= used + splitk) { g1.splitk_ws = static_cast<char*>(ws) + used; g1.splitk_bytes = splitk; }
   int rc = gemm_launch(g1, dtype, st);
   if (rc) return rc;
   attach_epilogue(g2);
@@ -751,7 +753,7 @@ int blr_dense_fwd(const void* x, int64_t ldx, const void* W, void* out, int64_t 
   if (a != BLR_ALGO_TILED) { set_error("dense: algorithm %d not available", a); return BLR_ERR_UNSUPPORTED; }
   // few output tiles and a long reduction (11008 -> 4096 at 256 rows: 32 tiles): room to cut it along K
   const size_t splitk = gemm_splitk_bytes(M, out_f, in_f, dtype);
-  if (ws && splitk && ws_bytes >= head + splitk) { g.splitk_ws = static_cast<char*>(ws) + head; g.splitk_bytes = ws_bytes - head; }
+  if (ws && splitk && ws_bytes >= head + splitk) { g.splitk_ws = static_cast<char*>(ws) + head; g.splitk_bytes = splitk; }
   attach_epilogue(g);
   if (g.pair) { g.N = out_f / 2; g.pair_dA = 0; g.pair_dB = out_f / 2; g.pair_dbias = out_f / 2; g.splitk_ws = nullptr; g.splitk_bytes = 0; }
   return gemm_launch(g, dtype, st);

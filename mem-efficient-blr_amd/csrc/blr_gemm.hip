@@ -1245,16 +1245,18 @@ static int launch_ring64(const GemmArgs& g, hipStream_t st) {
   return BLR_OK;
 }
 
+// (in whole 256-byte pieces: an output stage carves its scratch off the end of the workspace on that, and a call must not find its
+// slices short of bytes that way)
 size_t gemm_splitk_bytes(int M, int N, int K, int dtype) {
   if (dtype == BLR_F32) {
     const int s = K % 4 || N % 8 ? 1 : gemm_mid_f32_slices(M, N, K);
-    return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+    return s > 1 ? align_up((size_t)s * M * N * sizeof(float), 256) : 0;
   }
   if ((dtype != BLR_F16 && dtype != BLR_BF16) || M < 1 || N % 8 || K % 8 || K < 64) return 0;
   const int cus = device_cus() > 0 ? device_cus() : 256;
   if (M > 128 && cdiv(M, 128) * cdiv(N, 128) > cus) return 0;
   const MidPlan pl = gemm_mid_plan(M, N, K, 1, M >= 96, true, true);
-  return pl.slices > 1 ? (size_t)pl.slices * M * N * sizeof(float) : 0;
+  return pl.slices > 1 ? align_up((size_t)pl.slices * M * N * sizeof(float), 256) : 0;
 }
 
 template <typename T>

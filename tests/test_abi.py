@@ -103,3 +103,22 @@ def test_run_time_options_are_named_and_range_checked():
                 assert name.encode() in lib.blr_last_error()
         assert lib.blr_set_option(name.encode(), 0, 1) == 0            # back to "not set"
     assert lib.blr_set_option(b"BLR_NO_SUCH_SWITCH", 1, 0) == -1
+
+
+def test_workspaces_come_in_whole_256_byte_pieces(handle):
+    """blr_ep_workspace_bytes() more bytes are carved off the end on 256: an operator's own figure has to survive that."""
+    import random
+    rng = random.Random(0)
+    size = ctypes.c_size_t
+    for n in ("blast", "blast_q", "monarch", "low_rank", "dense", "ep"):
+        getattr(handle, f"blr_{n}_workspace_bytes").restype = size
+    for _ in range(300):
+        M, b = rng.choice([1, 2, 7, 16, 17, 33, 61, 100, 128, 129, 200, 513]), rng.choice([2, 4, 16])
+        fi, fo, r = (8 * b * rng.randint(1, 400) for _ in range(3))
+        dt, algo, bits = rng.choice([0, 1, 2]), rng.choice([0, 1, 2]), rng.choice([4, 8])
+        r = min(r, 2048)
+        got = {"blast": handle.blr_blast_workspace_bytes(M, fi, fo, b, r, dt, algo), "blast_q": handle.blr_blast_q_workspace_bytes(M, fi, fo, b, r, bits),
+               "monarch": handle.blr_monarch_workspace_bytes(M, fi, fo, b, r, dt, algo), "low_rank": handle.blr_low_rank_workspace_bytes(M, fi, fo, r, dt, algo),
+               "dense": handle.blr_dense_workspace_bytes(M, fi, fo, dt, algo), "ep": handle.blr_ep_workspace_bytes(4, M, fo, b, dt, 3)}
+        for n, v in got.items():
+            assert v % 256 == 0, (n, M, fi, fo, b, r, dt, algo, v)

@@ -289,3 +289,32 @@ def test_output_stage_of_narrow_blocks(m, p, q, r, dtype):
     S = torch.randn(r, b, b, device="cuda").to(dtype)
     say(f"[case] narrow blocks m={m} p={p} q={q} r={r} {dtype}")
     _stage_case(lambda: B.triton_blast_bmm_fp16(x, U, V, S), b * q, m, dtype, "silu" if q == 80 else None)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+# up to 16 rows: the small tiles behind a streaming workspace's head; beyond: slices of a long reduction
+@pytest.mark.parametrize("op,m,k,n,r", [("dense", 9, 3064, 264, 0), ("dense", 33, 5184, 1032, 0), ("dense", 61, 11008, 520, 0),
+                                        ("low_rank", 9, 1032, 264, 136), ("low_rank", 33, 5184, 1032, 136), ("low_rank", 61, 11008, 520, 72)])
+def test_gated_halves_in_a_workspace_of_just_the_asked_size(op, m, k, n, r, dtype):
+    """silu(gate) * up with the bytes that were asked for and with more: the same kernels, the same bits."""
+    from triton_funcs import _lib as L
+    lib, dt = L.lib(), L.dtype_code(dtype)
+    x = torch.randn(m, k, device="cuda").to(dtype)
+    a, w = (torch.randn(k, r or n, device="cuda") / k ** 0.5).to(dtype), (torch.randn(r or 1, n, device="cuda") / (r or 1) ** 0.5).to(dtype)
+    need = lib.blr_dense_workspace_bytes(m, k, n, dt, L.ALGO_AUTO) if op == "dense" else lib.blr_low_rank_workspace_bytes(m, k, n, r, dt, L.ALGO_AUTO)
+    need += lib.blr_ep_workspace_bytes(L.OP_DENSE if op == "dense" else L.OP_LOW_RANK, m, n, 1, dt, L.ACT_SILU_MUL)
+    say(f"[case] gated {op} {m} x {k} -> {n} {dtype} in {need} bytes")
+    outs = []
+    for size in (need, 2 * need + 4096):
+        ws, out = torch.zeros(size, dtype=torch.uint8, device="cuda"), torch.empty(m, n // 2, device="cuda", dtype=dtype)
+        head = (x.data_ptr(), k, a.data_ptr()) + ((w.data_ptr(),) if r else ()) + (out.data_ptr(), n // 2, m, k, n) + ((r,) if r else ())
+        rc = (lib.blr_low_rank_fwd_ep if r else lib.blr_dense_fwd_ep)(*head, dt, L.ALGO_AUTO, ws.data_ptr(), size, L.stream_ptr(x.device), None, L.ACT_SILU_MUL)
+        L.check(rc, op)
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.equal(*outs)
+    v = x.double() @ a.double()
+    if r:
+        v = v @ w.double()
+    ref = torch.nn.functional.silu(v[:, :n // 2]) * v[:, n // 2:]
+    assert (outs[0].double() - ref).norm() <= (4e-3 if dtype == torch.float16 else 3e-2) * ref.norm()
