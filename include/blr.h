@@ -83,7 +83,8 @@ typedef enum { BLR_OP_BLAST = 0, BLR_OP_MONARCH = 1, BLR_OP_LOW_RANK = 2, BLR_OP
  *     next: every value a workgroup hands to another is stored together with the epoch of its call,
  *     and a call recognises its own values by that tag;
  *   - nothing else may write to it between calls, and it must not be shared by calls that can
- *     overlap: one workspace per stream, calls on it stream-ordered;
+ *     overlap: one workspace per stream, calls on it stream-ordered.  Threads may call on one stream
+ *     with one workspace: the launches of a call are enqueued without another call's between them;
  *   - the single-launch kernels wait for each other's values with every workgroup resident, so
  *     they expect the GPU to themselves while they run (a few microseconds); when another kernel
  *     occupies compute units at that moment a wait may run into its bound (about a second), the

@@ -196,7 +196,8 @@ PyObject* failed(PyObject* name, int rc) {
 
 bool streams(int algo, int64_t M, int dt) { return algo == BLR_ALGO_STREAM || algo == BLR_ALGO_STREAM_SPLIT || (algo == BLR_ALGO_AUTO && M <= 16 && dt != BLR_F32); }
 
-// (held over the launches, which run without the interpreter lock: another thread's call on the stream may replace the workspace)
+// (held over the launches, which run without the interpreter lock: another thread's call on the stream may replace the workspace; that
+// the launches of two calls do not interleave in one is the C entry points' part)
 struct Ws { void* p; size_t n; void* stream; at::Tensor held; };
 Ws find_ws(const at::Tensor& x, size_t need, bool streaming) {
   void* st = (void*)c10::hip::getCurrentHIPStream(x.device().index()).stream();

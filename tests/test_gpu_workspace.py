@@ -1,4 +1,7 @@
-"""The shims' workspaces under graphs: replays go on where the capture left them, whatever the stream's calls have needed since."""
+"""The shims' workspaces under graphs and threads: replays go on where the capture left them, whatever the stream's calls have needed
+since, and the launches of two threads' calls on one stream do not mix."""
+import threading
+
 import pytest
 import torch
 
@@ -94,3 +97,43 @@ def test_growth_under_capture(path, rows):
             assert all(torch.equal(o, want) for o in outs)
             assert torch.equal(larger(), want)
     torch.cuda.synchronize()
+
+
+# one row and a few: streaming workspaces; 40: three launches over scratch; 300: products in tiles; gated: the full-width result behind it
+@pytest.mark.parametrize("rows", [1, 4, 40, 300])
+def test_threads_on_one_stream(path, rows):
+    from triton_funcs import blast_kernels as B, dense_kernels as D
+    L = path
+    w = (torch.randn(1024, 512, device="cuda") / 32).half()
+    xs = [torch.randn(rows, 1024, device="cuda").half() for _ in range(2)]
+    args = [_problem(rows, 16, 64, 72, 128, seed) for seed in range(2)]
+
+    def calls(i):
+        def gated():
+            with L.fused_epilogue(None, "silu_mul"):
+                return D.triton_dense_fp16(xs[i], w)
+        return (lambda: B.triton_blast_full_fp16(*args[i])), gated
+
+    want = [[c() for c in calls(i)] for i in range(2)]
+    torch.cuda.synchronize()
+    say(f"[case] two threads on one stream, {rows} rows")
+    start, got, errors = threading.Barrier(2), [[], []], []
+
+    def work(i):
+        try:
+            cs = calls(i)
+            start.wait()
+            for n in range(100):
+                got[i].append((n % 2, cs[n % 2]()))
+        except Exception as e:                                      # noqa: BLE001 - shown by the test
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for i in range(2):
+        assert len(got[i]) == 100 and all(torch.equal(o, want[i][k]) for k, o in got[i])
