@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void quant_scale_kernel(const T* __restrict__ 
 // as 128 (int8) or 64 (int4) bytes each.  16 blocks of 1376 x 1024 in fp32: the transposed copy and the column kernel took 830 us,
 // the two launches 17 + 26 us (90 MB each, at 5.2 and 3.9 TB/s with the codes).
 template <typename T, int BITS>
-__global__ __launch_bounds__(256) void quant_turn_kernel(const T* __restrict__ w, int64_t reduce, int64_t inner, int vec_ok,
+__global__ __launch_bounds__(256) void quant_turn_kernel(const T* __restrict__ w, int64_t reduce, int64_t inner, int vec_ok, int words,
                                                          uint8_t* __restrict__ codes, const f16* __restrict__ scales) {
   __shared__ uint32_t s_codes[64][33];              // [value][channel / 4], padded: the 16 lanes of a channel meet 8 banks twice
   const int64_t o = blockIdx.z, q0 = (int64_t)blockIdx.x * 128, r0 = (int64_t)blockIdx.y * 64;
@@ -221,7 +221,6 @@ __global__ __launch_bounds__(256) void quant_turn_kernel(const T* __restrict__ w
   const int64_t row_bytes = inner * BITS / 8;       // (inner even for int4)
   uint8_t* co = codes + o * reduce * row_bytes;
   constexpr int DW = BITS == 8 ? 32 : 16;           // dwords of a tile row
-  const bool words = (row_bytes % 4) == 0;
   for (int i = threadIdx.x; i < 64 * DW; i += 256) {
     const int rr = i / DW, d = i % DW;
     const int64_t r = r0 + rr, byte = (BITS == 8 ? q0 : q0 / 2) + d * 4;
@@ -264,14 +263,15 @@ int quantize_any(const T* w, int64_t outer, int64_t reduce, int64_t inner, int b
 template <typename T>
 int quantize_turned(const T* w, int64_t outer, int64_t reduce, int64_t inner, int bits, uint8_t* codes, f16* scales, hipStream_t st) {
   const int64_t channels = outer * inner;
-  const bool vec = reduce % 4 == 0 && aligned(w, 4 * sizeof(T)) && aligned(codes, 4);
+  const bool vec = reduce % 4 == 0 && aligned(w, 4 * sizeof(T));                     // loads of four values
+  const bool words = (inner * bits / 8) % 4 == 0 && aligned(codes, 4);               // stores of four bytes of codes
   const float qmax = bits == 8 ? 127.0f : 7.0f;
   const dim3 g1((unsigned)cdiv(channels, 4));
   if (vec) hipLaunchKernelGGL((quant_scale_kernel<T, 4>), g1, dim3(256), 0, st, w, channels, reduce, qmax, scales);
   else hipLaunchKernelGGL((quant_scale_kernel<T, 1>), g1, dim3(256), 0, st, w, channels, reduce, qmax, scales);
   const dim3 g2((unsigned)cdiv(inner, 128), (unsigned)cdiv(reduce, 64), (unsigned)outer);
-  if (bits == 8) hipLaunchKernelGGL((quant_turn_kernel<T, 8>), g2, dim3(256), 0, st, w, reduce, inner, (int)vec, codes, (const f16*)scales);
-  else hipLaunchKernelGGL((quant_turn_kernel<T, 4>), g2, dim3(256), 0, st, w, reduce, inner, (int)vec, codes, (const f16*)scales);
+  if (bits == 8) hipLaunchKernelGGL((quant_turn_kernel<T, 8>), g2, dim3(256), 0, st, w, reduce, inner, (int)vec, (int)words, codes, (const f16*)scales);
+  else hipLaunchKernelGGL((quant_turn_kernel<T, 4>), g2, dim3(256), 0, st, w, reduce, inner, (int)vec, (int)words, codes, (const f16*)scales);
   BLR_CHECK_LAUNCH("quantize");
   return BLR_OK;
 }

@@ -49,6 +49,34 @@ def test_packed_factors_codes_bit_exact(b, p, q, r, bits, dtype):
         np.testing.assert_array_equal(got.scales.cpu().numpy(), scales)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("at", [0, 1, 2, 3])
+# (outer, reduce, inner): rows of codes of whole words, of halves of one, of odd bytes (int4: inner is even)
+@pytest.mark.parametrize("shape", [(2, 64, 128), (3, 33, 132), (2, 70, 130), (2, 9, 26)])
+def test_quantizer_codes_at_any_address(shape, at, bits, dtype):
+    """The C entries with a codes buffer that starts `at` bytes off: the same bytes, and none beside them."""
+    from triton_funcs import _lib as L
+    lib = L.lib()
+    outer, reduce, inner = shape
+    g = torch.Generator("cuda").manual_seed(reduce)
+    w = (torch.randn(outer, reduce, inner, device="cuda", generator=g) / 8).to(dtype)
+    turned = w.transpose(1, 2).contiguous()
+    n = outer * reduce * inner * bits // 8
+    say(f"[case] codes at byte {at} {shape} bits={bits} {dtype}")
+    rc, rs = O.quantize_sym(w.float().cpu().numpy(), 1, bits)
+    want = (rc if bits == 8 else O.pack_int4(rc)).view(np.uint8).reshape(-1)
+    for f, src in ((lib.blr_quantize_sym, w), (lib.blr_quantize_sym_t, turned)):
+        buf = torch.full((n + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+        scales = torch.empty(outer, inner, dtype=torch.float16, device="cuda")
+        L.check(f(src.data_ptr(), L.dtype_code(dtype), outer, reduce, inner, bits, buf.data_ptr() + 16 + at, scales.data_ptr(), L.stream_ptr(src.device)), "quantize")
+        torch.cuda.synchronize()
+        got = buf.cpu().numpy()
+        np.testing.assert_array_equal(got[16 + at:16 + at + n], want)
+        assert (got[:16 + at] == 0x5A).all() and (got[16 + at + n:] == 0x5A).all()
+        np.testing.assert_array_equal(scales.cpu().numpy(), rs)
+
+
 def test_quantizer_half_inputs_and_ties():
     from triton_funcs import blast_sym_quant_kernels as Q
     # values that land exactly on .5 after scaling: scale = 1/127*127 ... use amax = 127 -> scale 1
