@@ -71,7 +71,7 @@ class _StructuredLinear(nn.Module):
         stage = self._stage() if self.fuses else None
         if stage is None:
             return self.func(*args), False
-        with_epilogue = getattr(self.func, "with_epilogue", None)
+        with_epilogue = L.with_epilogue(self.func)
         if with_epilogue is None:                      # a function put in the library's place, or one without an output stage of its own
             with L.armed(stage):
                 return self.func(*args), True
@@ -181,8 +181,9 @@ class QuantBlastLinear(BlastLinear):
     def forward(self, x):
         args = (x, self.Uq, self.Vq, self.S)
         bias = self.bias
-        if (bias is not None or self.fused_act is not None) and not self.is_compiled and hasattr(self.func, "with_epilogue") and self.fused_act in L.ACTS:
-            out = self.func.with_epilogue(*args, (bias, L.ACTS[self.fused_act], None, 0, None))
+        with_epilogue = L.with_epilogue(self.func) if bias is not None or self.fused_act is not None else None
+        if with_epilogue is not None and self.fused_act in L.ACTS:
+            out = with_epilogue(*args, (bias, L.ACTS[self.fused_act], None, 0, None))
             if out is not None:
                 return out
         return self._finish(self.func(*args))

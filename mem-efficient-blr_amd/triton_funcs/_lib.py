@@ -318,6 +318,17 @@ class armed:
         return False
 
 
+def set_with_epilogue(func, call):
+    """func.with_epilogue(*args, ep) is func with its output stage as an argument."""
+    func.with_epilogue, func.with_epilogue_of = call, func
+
+
+def with_epilogue(func):
+    """func.with_epilogue, or None where func has none or took it over from another (functools.wraps, torch.compile): such a wrapper
+    has to be called itself."""
+    return func.with_epilogue if getattr(func, "with_epilogue_of", None) is func else None
+
+
 def armed_epilogue():
     """The output stage that the active context arms on this thread, as (bias, act, gate, gate_rows, residual), or None."""
     return getattr(_ep_state, "ep", None)

@@ -164,7 +164,7 @@ def _with_epilogue(func, u_layout, s_layout):
                 return out
         with L.armed(ep):
             return func(x, U, V, S)
-    func.with_epilogue = call
+    L.set_with_epilogue(func, call)
 
 
 for _f in (triton_blast_partial_fp16, triton_blast_partial_grouped_fp16, triton_blast_partial_grouped_persistent_fp16, triton_blast_full_fp16):

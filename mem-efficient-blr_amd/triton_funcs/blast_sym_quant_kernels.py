@@ -163,8 +163,8 @@ def _with_epilogue(x, U, V, S, ep):
     return host.blast_q("triton_blast_bmm_int8_fp16", _last_config, x, U, V, S, 0, ep) if host else None
 
 
-triton_blast_bmm_int8_fp16.with_epilogue = _with_epilogue
-triton_blast_bmm_int4_fp16.with_epilogue = _with_epilogue
+L.set_with_epilogue(triton_blast_bmm_int8_fp16, _with_epilogue)
+L.set_with_epilogue(triton_blast_bmm_int4_fp16, _with_epilogue)
 
 
 def get_triton_blast_bmm_xv_int8_fp16_config():

@@ -67,7 +67,7 @@ def _with_epilogue(x, w, ep):
     return out.reshape(*x.shape[:-1], out.shape[-1])
 
 
-triton_dense_fp16.with_epilogue = _with_epilogue
+L.set_with_epilogue(triton_dense_fp16, _with_epilogue)
 
 
 def _probe(x, w):

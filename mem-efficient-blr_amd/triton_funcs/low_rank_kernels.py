@@ -70,7 +70,7 @@ def _with_epilogue(x, a, b, ep):
     return out.reshape(*x.shape[:-1], out.shape[-1])
 
 
-triton_low_rank_fp16.with_epilogue = _with_epilogue
+L.set_with_epilogue(triton_low_rank_fp16, _with_epilogue)
 
 
 def _probe(x, a, b):

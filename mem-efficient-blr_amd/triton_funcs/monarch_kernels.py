@@ -137,7 +137,7 @@ def _with_epilogue(func, w2_layout, out_order):
                 return out
         with L.armed(ep):
             return func(x, w1, w2)
-    func.with_epilogue = call
+    L.set_with_epilogue(func, call)
 
 
 _with_epilogue(triton_monarch_right_fp16, L.W2_SR, L.OUT_INTERLEAVED)

@@ -110,6 +110,27 @@ def test_wrappers_take_pruned_weights_and_replaced_functions():
             assert m(x).shape == (2, 5, 48) and seen[0][0] is m.bias and seen[0][1] == L.ACTS["silu"]
 
 
+def test_functions_wrapped_around_the_librarys_are_called():
+    """functools.wraps (torch.compile too) copies a function's attributes to the wrapper: the module calls the wrapper all the same."""
+    import functools
+    from models.wrappers import BlastLinear, DenseLinear, LowRankLinear, MonarchLinear
+    from triton_funcs import _lib as L
+    x = torch.randn(2, 5, 32)
+    for cls, more, path in ((BlastLinear, {"b": 4, "rank": 8}, "blast_kernels.triton_blast_full_fp16"), (BlastLinear, {"b": 4, "rank": 8}, "blast_kernels.triton_blast_bmm_fp16"),
+                            (MonarchLinear, {"b": 4, "rank": 8}, "monarch_kernels.triton_monarch_right_fp16"), (LowRankLinear, {"rank": 8}, "low_rank_kernels.triton_low_rank_fp16"),
+                            (DenseLinear, {}, "dense_kernels.triton_dense_fp16")):
+        m, seen = cls(32, 48, func_path="triton_funcs." + path, device="cpu", dtype=torch.float32, **more), []
+        assert hasattr(m.func, "with_epilogue")
+
+        @functools.wraps(m.func)
+        def watched(x, *w):
+            seen.append(L.armed_epilogue())
+            return torch.zeros(2, 5, 48)
+
+        m.func = watched
+        assert m(x).shape == (2, 5, 48) and len(seen) == 1 and seen[0][0] is m.bias
+
+
 def test_torch_funcs_match_oracle_including_bmm_and_intermediates():
     from torch_funcs.blast_funcs import torch_blast_baseline, torch_blast_bmm
     from torch_funcs.monarch_funcs import torch_monarch_baseline
