@@ -98,6 +98,7 @@ void epilogue_taken();
 // Every run-time switch of the library (blr_set_option): each starts from the environment variable of its name, read once, and
 // is range-checked where it is set.  The first six pick the GEMM variant, the rest switch a kernel family off (0) so that the
 // call falls through to the next one that serves it - for A/B measurements and as a way out should a kernel misbehave.
+// (OPT_DENSE_ROWS has no reader: the name is still taken from programs that set it.)
 enum { OPT_GEMM_RING = 0, OPT_GEMM_RING_TILE, OPT_GEMM_RING_PER_CU, OPT_GEMM_RING_WAVES, OPT_GEMM_RING_BK, OPT_GEMM_SPLITK, OPT_GEMM_MID,
        OPT_DECODE2, OPT_DECODE3, OPT_DECODE_PAIR, OPT_DECODE_ROWS, OPT_DENSE_SLAB, OPT_DENSE_ROWS, OPT_BLAST_MIXU, OPT_BLAST_ONE, OPT_BLAST_YMIXW, OPT_COUNT };
 int option_value(int id, int dflt);             // the option's value, or dflt when it is unset

@@ -69,17 +69,25 @@ def test_same_output_stage(rows, dtype):
     for f, w in _ops(dtype):
         if not hasattr(f, "with_epilogue") or "int8" in f.__name__:
             continue
-        x = torch.randn(1, rows, 128, device="cuda").to(dtype)
+        images = 3
+        x = torch.randn(images, rows, 128, device="cuda").to(dtype)
         bias = torch.randn(192, device="cuda").to(dtype)
-        mod = torch.randn(1, 5 * 192, device="cuda").to(dtype)
-        resid = torch.randn(1, rows, 192, device="cuda").to(dtype)
+        mod = torch.randn(images, 5 * 192, device="cuda").to(dtype)
+        resid = torch.randn(images * rows, 2 * 192, device="cuda").to(dtype)[:, 192:]
         for act in (None, "gelu_tanh", "silu_mul"):
             say(f"[case] output stage {f.__name__} {dtype} rows={rows} {act}")
             _same(lambda: f.with_epilogue(x, *w, (bias, L.ACTS[act], None, 0, None)))
-        gate = mod[:, 192:384]                                     # rows of a wider matrix
-        got = f.with_epilogue(x, *w, (bias, 0, gate, rows, resid))
-        want = f.with_epilogue(x, *w, (bias, 0, gate.contiguous(), rows, resid))
-        assert torch.equal(got, want)
+        gate = mod[:, 192:384]                                     # a row for each image, both operands rows of a wider matrix
+        assert not gate.is_contiguous() and not resid.is_contiguous()
+        want = f.with_epilogue(x, *w, (bias, 0, gate.contiguous(), rows, resid.contiguous()))
+        rest = f(x, *w).reshape(-1, 192).double() + bias.double()
+        ref = resid.double() + gate.double().repeat_interleave(rows, 0) * rest
+        # (op + bias and the result are each rounded; the factor 8 leaves room for the operator's own rounding points)
+        unit = 2.0 ** (-11 if dtype == torch.float16 else -8)
+        assert (want.reshape(-1, 192).double() - ref).abs().max() <= 8 * unit * (ref.abs().max() + gate.abs().max().double() * rest.abs().max())
+        for g, r in ((gate, resid), (gate, resid.contiguous()), (gate.contiguous(), resid)):
+            for got in _both(lambda: f.with_epilogue(x, *w, (bias, 0, g, rows, r))):
+                assert torch.equal(got[0], want)
         _same(lambda: f.with_epilogue(x, *w, (None, 0, gate, rows, resid)))
 
 

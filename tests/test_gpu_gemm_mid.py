@@ -33,7 +33,7 @@ def test_mid_tiles(m, n, k, tile, dtype):
     x = torch.randn(m, k, device="cuda", generator=g).to(dtype)
     w = (torch.randn(k, n, device="cuda", generator=g) / k ** 0.5).to(dtype)
     say(f"[case] mid tile {tile} {dtype} m={m} n={n} k={k}")
-    with L.options(BLR_GEMM_MID=tile, BLR_DENSE_ROWS=0):
+    with L.options(BLR_GEMM_MID=tile):
         _check(D.triton_dense_fp16(x, w, {"algo": L.ALGO_TILED}), x, w, dtype, "dense (k, n)")
         # batched, both weight orders: BLAST's two products through the names that return the intermediates' arithmetic unfused
         b = 2
