@@ -86,8 +86,15 @@ const at::Tensor& workspace(const at::Device& dev, void* stream, size_t bytes, b
 }
 
 // ---- what a call looks at ---------------------------------------------------------------------------------------------------
-// (plain tensors and parameters: a subclass may mean something else by its data)
-const at::Tensor* tensor(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+// (plain tensors and parameters with memory of their own: a subclass may mean something else by its data, and what vmap, grad and their
+// like hand out has none.  Asking those for their address throws, which must not happen once the interpreter lock is given up.)
+const at::Tensor* tensor(PyObject* o) {
+  if (!THPVariable_CheckExact(o)) return nullptr;
+  const at::Tensor& t = THPVariable_Unpack(o);
+  constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                         c10::DispatchKey::Functionalize});
+  return t.has_storage() && !t.key_set().has_any(wrapped) ? &t : nullptr;
+}
 
 int dtype_code(at::ScalarType t) { return t == at::kHalf ? BLR_F16 : t == at::kBFloat16 ? BLR_BF16 : t == at::kFloat ? BLR_F32 : -1; }
 

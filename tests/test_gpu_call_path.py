@@ -194,3 +194,18 @@ def test_gates_and_residuals_that_are_too_short_are_refused():
                     with pytest.raises(L.BlrError):
                         _on(host, lambda: f.with_epilogue(x, *w, (None, 0, gate, every, resid)))
             f.with_epilogue(x, *w, (None, 0, t(2), -(-rows // 2), t(rows)))
+
+
+def test_transformed_tensors_raise():
+    """Tensors of vmap, grad and jvp have no memory: an error, as on the Python path, and the next call is as good as the one before."""
+    for f, w in _ops(torch.float16):
+        say(f"[case] transforms of {f.__name__}")
+        x = torch.randn(2, 5, 128, device="cuda").half()
+        want = f(x[0], *w)
+        for call in (lambda: torch.func.vmap(lambda t: f(t, *w))(x),
+                     lambda: torch.func.grad(lambda t: f(t, *w).float().sum())(x[0]),
+                     lambda: torch.func.jvp(lambda t: f(t, *w), (x[0],), (x[1],))):
+            for native in (True, False):
+                with pytest.raises(RuntimeError):
+                    _on(native, call)
+        assert torch.equal(f(x[0], *w), want)
