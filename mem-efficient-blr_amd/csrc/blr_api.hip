@@ -673,11 +673,13 @@ int blr_monarch_fwd(const void* x, int64_t ldx, const void* w1, const void* w2,
 }
 
 // ---- low rank -------------------------------------------------------------------------------------
-// 2 .. 16 rows of a small layer: two products on small tiles instead of the three launches that stream larger factors better
-// (768 -> 3072, r = 128 at 2 / 16 rows 8.9 / 9.6 -> 7.3 / 7.5 us, 1152 -> 3456, r = 288 9.9 / 10.7 -> 8.7 / 9.2; but 1152 -> 4608,
-// r = 576 at 2 rows 10.7 against 11.0, and 3072 -> 768, r = 192, whose long reduction comes in slices, 9.3 against 9.9).
+// 2 .. 16 rows of a small layer: two products on small tiles instead of the three launches that stream larger factors better.  What
+// decides is factors that come from HBM, as they do in a network that does not fit the 256 MB Infinity Cache: 768 -> 3072, r = 128 at
+// 2 / 16 rows 9.0 / 9.7 us streamed and 8.9 / 8.9 here (in the cache 8.1 / 9.0 and 7.3 / 7.3), 768 -> 2304, r = 192 9.2 / 10.3 and
+// 9.0 / 9.1; but 1280 -> 1280, r = 128 8.8 / 9.8 and 9.8 / 10.4, 1024 -> 2048, r = 160 9.2 / 10.0 and 10.1 / 10.3, 1152 -> 6912, r = 256
+// 9.8 / 10.3 and 13.7 / 13.9: x A is a handful of workgroups that each wait for a long column of A.
 static bool low_rank_by_tiles(int algo, int M, int in_f, int out_f, int r, int dtype) {
-  return algo == BLR_ALGO_AUTO && M >= 2 && M <= 16 && dtype != BLR_F32 && in_f <= 1536 && (int64_t)r * (in_f + out_f) <= 9 << 18;
+  return algo == BLR_ALGO_AUTO && M >= 2 && M <= 16 && dtype != BLR_F32 && in_f <= 768 && (int64_t)r * (in_f + out_f) <= 5 << 17;
 }
 
 size_t blr_low_rank_workspace_bytes(int M, int in_f, int out_f, int r, int dtype, int algo) {
@@ -739,13 +741,22 @@ int blr_low_rank_fwd(const void* x, int64_t ldx, const void* A, const void* B,
 }
 
 // ---- dense ----------------------------------------------------------------------------------------
+// Up to 16 rows of a short reduction on the small tiles: one launch instead of the slab kernel and the one that adds its slices (768 -> 768
+// at 1 / 16 rows 7.2 / 8.0 -> 5.4 / 5.4 us, 768 -> 3072 8.0 / 8.6 -> 7.8 / 8.0, 1152 -> 3456 8.2 / 9.3 -> 7.4 / 7.8 with weights from HBM; in
+// the 256 MB Infinity Cache 6.8 / 7.2 -> 4.2, 7.0 / 7.9 -> 4.2 / 4.3, 7.3 / 8.1 -> 5.6).  Longer ones stream better through the slab kernel:
+// few tiles keep too little in flight, and slices need the second launch as well.  Weights from HBM, slab and tiles, 1 / 16 rows:
+// 3072 -> 768 8.6 / 9.5 and 9.3 / 10.0, 4096 -> 4096 11.8 / 13.4 and 13.9 / 14.5, 8192 -> 8192 27.3 / 29.1 and 33.8 / 34.5, 4096 -> 22016
+// 35.6 / 39.8 and 38.0 / 39.7 (in the cache, where networks of such layers do not fit, the tiles are 0 .. 25 % faster on all but
+// 8192 -> 8192).  Near the line 1024 -> 2048 loses 7.6 / 8.1 -> 8.5 / 8.8 from HBM and gains 7.0 / 7.8 -> 4.9 / 5.1 in the cache,
+// 1536 -> 8192 10.1 -> 10.4 and 9.3 -> 6.6.
+static bool dense_by_tiles(int algo, int M, int in_f, int out_f, int dtype) {
+  return algo == BLR_ALGO_AUTO && M <= 16 && dtype != BLR_F32 && in_f <= 1536 && gemm_splitk_bytes(M, out_f, in_f, dtype) == 0;
+}
+
 size_t blr_dense_workspace_bytes(int M, int in_f, int out_f, int dtype, int algo) {
   if (M <= 0) return 0;
   int a = resolve_algo(algo, M, dtype, false);
-  if (a == BLR_ALGO_STREAM || a == BLR_ALGO_STREAM_SPLIT) {
-    const size_t s = stream_generic_workspace(0, M, in_f, out_f, 1, 0), tiles = stream_head_bytes() + gemm_splitk_bytes(M, out_f, in_f, dtype);
-    return algo == BLR_ALGO_AUTO && tiles > s ? tiles : s;
-  }
+  if (a == BLR_ALGO_STREAM || a == BLR_ALGO_STREAM_SPLIT) return stream_generic_workspace(0, M, in_f, out_f, 1, 0);
   return gemm_splitk_bytes(M, out_f, in_f, dtype);    // few tiles: fp32 partial sums of the slices of K
 }
 
@@ -762,14 +773,7 @@ int blr_dense_fwd(const void* x, int64_t ldx, const void* W, void* out, int64_t 
   GemmArgs g = {};
   g.A = x; g.lda = ldx; g.B = W; g.ldb = out_f; g.b_kn = 1;
   g.C = out; g.ldc = ldo; g.cn = 1; g.M = M; g.N = out_f; g.K = in_f; g.batch = 1;
-  // Up to 16 rows too the small tiles, with slices of a long reduction (768 -> 3072 at 1 / 16 rows 8.0 / 8.4 us on the slab kernel and
-  // the launch that adds its slices, 4.8 / 5.0 here; 4096 -> 22016 33.8 / 38.1 against 31.5 / 31.5; 11008 -> 4096 equal at 1 row).
-  size_t head = 0;                                   // a streaming workspace keeps its head
-  if (a == BLR_ALGO_STREAM && algo == BLR_ALGO_AUTO && ws && ws_bytes >= blr_dense_workspace_bytes(M, in_f, out_f, dtype, algo) && option_value(OPT_GEMM_MID, 1) &&
-      gemm_mid_ok(g, dtype)) {
-    head = stream_head_bytes();
-    a = BLR_ALGO_TILED;
-  }
+  if (a == BLR_ALGO_STREAM && dense_by_tiles(algo, M, in_f, out_f, dtype) && option_value(OPT_GEMM_MID, 1) && gemm_mid_ok(g, dtype)) a = BLR_ALGO_TILED;
   if (a == BLR_ALGO_STREAM || a == BLR_ALGO_STREAM_SPLIT) {
     if (dtype == BLR_F32 || M > 16) { set_error("dense: streaming algorithm needs f16/bf16 and M <= 16"); return BLR_ERR_UNSUPPORTED; }
     StreamGenericArgs s = {};
@@ -781,7 +785,7 @@ int blr_dense_fwd(const void* x, int64_t ldx, const void* W, void* out, int64_t 
   if (a != BLR_ALGO_TILED) { set_error("dense: algorithm %d not available", a); return BLR_ERR_UNSUPPORTED; }
   // few output tiles and a long reduction (11008 -> 4096 at 256 rows: 32 tiles): room to cut it along K
   const size_t splitk = gemm_splitk_bytes(M, out_f, in_f, dtype);
-  if (ws && splitk && ws_bytes >= head + splitk) { g.splitk_ws = static_cast<char*>(ws) + head; g.splitk_bytes = splitk; }
+  if (ws && splitk && ws_bytes >= splitk) { g.splitk_ws = ws; g.splitk_bytes = splitk; }
   attach_epilogue(g);
   if (g.pair) { g.N = out_f / 2; g.pair_dA = 0; g.pair_dB = out_f / 2; g.pair_dbias = out_f / 2; g.splitk_ws = nullptr; g.splitk_bytes = 0; }
   return gemm_launch(g, dtype, st);

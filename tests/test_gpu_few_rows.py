@@ -95,3 +95,19 @@ def test_low_rank_of_a_small_layer(M, in_f, r, out_f):
     out = K.triton_low_rank_fp16(dev(x, dtype), dev(a, dtype), dev(bm, dtype))
     assert_close(out, rounded(rounded(x, dtype) @ rounded(a, dtype), dtype) @ rounded(bm, dtype), dtype, f"low rank M={M}", scale=2.0)
     assert torch.equal(B.triton_blast_full_fp16(*args), before)
+
+
+@pytest.mark.parametrize("M", [1, 2, 16])
+def test_long_reductions_stream(M):
+    """Up to 16 rows, layers that the small tiles would cut into slices or feed too slowly from HBM: by default the bits of the streaming kernels."""
+    from triton_funcs import dense_kernels as D, low_rank_kernels as K, _lib as L
+    g = torch.Generator("cuda").manual_seed(M)
+    t = lambda *s: (torch.randn(*s, device="cuda", generator=g) / s[0] ** 0.5).half()
+    for i, o in ((1544, 768), (3072, 768), (2048, 2048), (4096, 4096)):
+        say(f"[case] few rows dense {M} x {i} x {o} streams")
+        x, w = t(M, i), t(i, o)
+        assert torch.equal(D._dense("test", x, w, L.ALGO_AUTO)[0], D._dense("test", x, w, L.ALGO_STREAM)[0])
+    for i, r, o in ((776, 128, 768), (1152, 256, 6912), (768, 256, 2304)):
+        say(f"[case] few rows low rank {M} x {i} x {r} x {o} streams")
+        x, a, b = t(M, i), t(i, r), t(r, o)
+        assert torch.equal(K._low_rank("test", x, a, b, L.ALGO_AUTO, False)[0], K._low_rank("test", x, a, b, L.ALGO_STREAM, False)[0])
