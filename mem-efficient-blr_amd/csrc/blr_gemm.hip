@@ -1277,7 +1277,13 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
   const int mid = option_value(OPT_GEMM_MID, 1);
   if (mid > 1 && gemm_mid_ok(g, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16)) return gemm_mid_launch(g, mid - 2, false, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16, st);
   const int64_t r128_all = cdiv(g.M, 128) * cdiv(g.N, 128) * g.batch;
-  if (mid == 1 && ring == 1 && (r128_all <= cus || g.M <= 128) && option_value(OPT_GEMM_RING_TILE, 0) == 0) {
+  // Interleaved columns with work for more than half of the compute units, whole row tiles and a reduction of some length: the rules
+  // below, whose tiles of 128 x 128 store two bytes at a time at a better rate than 64 x 64 ones (second product of Monarch, whole calls:
+  // 2048 -> 2048 in 16 blocks, r = 256 at 1300 / 1500 / 2000 rows 28.5 / 29.4 / 35.2 -> 26.3 / 26.6 / 31.6 us, 1536 -> 1536 28.5 / 29.6 / 34.8
+  // -> 24.2 / 24.8 / 29.1, 4096 -> 4096 in 4 blocks, r = 1024 at 1000 rows 43.9 -> 36.7; but 768 -> 2304, r = 128 at 1300 rows 14.1 against 15.1,
+  // 1152 -> 1152, r = 288 at 1500 rows 17.1 against 21.4 with 105 tiles' worth of results, 2048 -> 8192 in 16 blocks at 260 rows 25.5 against 28.0).
+  const bool interleaved = g.cn != 1 && g.K >= 256 && (int64_t)g.M * g.N * g.batch * 2 > (int64_t)cus * 128 * 128 && (int64_t)g.M * 8 >= cdiv(g.M, 128) * 128 * 7;
+  if (mid == 1 && ring == 1 && (r128_all <= cus || g.M <= 128) && !interleaved && option_value(OPT_GEMM_RING_TILE, 0) == 0) {
     constexpr int dt = std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16;
     const bool rk = g.cn == 1 && g.M >= 96 && g.K >= 64 && ring_ok(g), mk = gemm_mid_ok(g, dt);
     bool cut = option_value(OPT_GEMM_SPLITK, 1) != 0 && mk && g.cn == 1 && g.epi == EPI_PLAIN && g.splitk_ws && aligned(g.splitk_ws, 16) && g.batch == 1 && !g.sat8 && !g.pair &&

@@ -111,3 +111,18 @@ def test_long_reductions_stream(M):
         say(f"[case] few rows low rank {M} x {i} x {r} x {o} streams")
         x, a, b = t(M, i), t(i, r), t(r, o)
         assert torch.equal(K._low_rank("test", x, a, b, L.ALGO_AUTO, False)[0], K._low_rank("test", x, a, b, L.ALGO_STREAM, False)[0])
+
+
+@pytest.mark.parametrize("b,p,r,q,M", [(16, 32, 256, 128, 1100), (16, 32, 256, 96, 1500), (12, 32, 384, 128, 1409), (4, 32, 264, 1000, 1000)])
+def test_monarch_interleaved_columns(b, p, r, q, M):
+    """Interleaved columns with work for half of the chip: the bits of the kernels that BLR_GEMM_MID=0 leaves."""
+    from triton_funcs import monarch_kernels as K, _lib as L
+    g = torch.Generator("cuda").manual_seed(M)
+    t = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    x, w1, w2 = t(M, b * p).half(), (t(b, p, r) / p ** 0.5).half(), (t(b, r, q) / r ** 0.5).half()
+    say(f"[case] monarch interleaved b={b} p={p} r={r} q={q} M={M}")
+    out = K.triton_monarch_right_left_fp16(x, w1, w2)
+    with L.options(BLR_GEMM_MID=0):
+        assert torch.equal(K.triton_monarch_right_left_fp16(x, w1, w2), out)
+    want = K.triton_monarch_right_left_fp32(x.float(), w1.float(), w2.float())[0]       # (fp32 throughout: only Z is not rounded on the way)
+    assert_close(out, want.double().cpu().numpy(), torch.float16, f"monarch interleaved b={b} M={M}", scale=2.0)
