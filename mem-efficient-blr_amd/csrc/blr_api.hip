@@ -354,7 +354,7 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
   else { si = (int64_t)b * r; sj = r; sr = 1; }
   int rc = 1;
   int mixu_prepared = 0;
-  // Few rows and small ranks (blast_by_three): both products on the kernels for problems that do not fill the chip, which give a
+  // Few rows and small ranks: both products on the kernels for problems that do not fill the chip, which give a
   // 16-block layer of a thousand columns one to several hundred small workgroups where the fused kernels below have 4 .. 32, and
   // the mix as a launch of its own in between.  The cost of that launch goes with M r; up to where it lies below what the fused
   // kernel of the shape gains by not having it, measured over the layers of the configurations at 17 .. 1024 rows:
@@ -363,10 +363,13 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
   //   S with the rank contiguous: to M r = 2^18 (2048 -> 8192, r = 512 at 512 rows 34.9 against 31.1 us, at 768 rows 39.4 against 42.4),
   //   3/4 of that where output blocks are narrow (1152 -> 1152, r = 288 at 512 rows 27.3 against 23.4, at 768 rows 27.1 against 28.0);
   //   S (r, i, j): the same, but with input blocks that the fused first half takes as they are 80 x 1024 (1152 -> 3456, r = 288 at
-  //   256 rows 18.3 against 17.0, at 384 rows 19.6 against 21.3; 2048 -> 8192, r = 768 at 144 rows 23.6 against 24.7).
+  //   256 rows 18.3 against 17.0, at 384 rows 19.6 against 21.3; 2048 -> 8192, r = 768 at 144 rows 23.6 against 24.7), and not with 9 .. 15
+  //   blocks, whose mix has no fast kernel for that order (1536 -> 1536, b = 12, r = 256 at 260 rows 26.5 against 16.5 fused); as many blocks
+  //   of that width with the rank contiguous: 5 x 2^15 (1152 -> 2304, b = 12, r = 128 at 1500 / 2000 rows 28.3 / 32.5 against 25.2 / 27.1).
   // Longer calls of tiny ranks are left to the fused kernels, which were fitted there.
   const bool narrow_out = b == 16 && Q % 8 == 0 && Q <= 80 && r % 32 == 0 && !silu_mul_armed();
-  const int64_t by_three = narrow_out ? 3 << 16 : sr != 1 && P <= 128 ? 80 << 10 : 1 << 18;
+  const bool odd_blocks = b > 8 && b != 16;
+  const int64_t by_three = narrow_out ? 3 << 16 : P > 128 ? 1 << 18 : sr != 1 ? (odd_blocks ? 0 : 80 << 10) : odd_blocks ? 5 << 15 : 1 << 18;
   const bool few = M <= 128 || (M <= 2048 && (int64_t)M * r <= by_three);
   if (few && !y_out && !z_out && !sat8 && fused <= 0 && dtype != BLR_F32 && option_value(OPT_DECODE_ROWS, 1)) {
     if (M > 16) {

@@ -113,6 +113,22 @@ def test_long_reductions_stream(M):
         assert torch.equal(K._low_rank("test", x, a, b, L.ALGO_AUTO, False)[0], K._low_rank("test", x, a, b, L.ALGO_STREAM, False)[0])
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("name,b,p,q,r,M", [("triton_blast_bmm_fp16", 12, 96, 104, 64, 129), ("triton_blast_bmm_fp16", 9, 128, 64, 32, 300),
+                                            ("triton_blast_full_fp16", 12, 96, 104, 128, 1300)])
+def test_nine_to_fifteen_blocks(name, b, p, q, r, M, dtype):
+    """Above 128 rows, and with the rank contiguous beyond 5 * 2^15 rows x rank, narrow blocks without a fast mix of their own keep the
+    kernels of many rows, bit for bit."""
+    from test_gpu_blast import _ref, _run_blast
+    from triton_funcs import _lib as L
+    x, U, Vt, S = blast_inputs(b, p, q, r, (M,), seed=M + b)
+    say(f"[case] {name} b={b} p={p} q={q} r={r} M={M} {dtype}")
+    out = _run_blast(name, x, U, Vt, S, dtype, "auto")
+    assert_close(out, _ref(x, U, Vt, S, dtype)[0], dtype, f"{name} b={b} M={M}")
+    with L.options(BLR_DECODE_ROWS=0):
+        assert torch.equal(_run_blast(name, x, U, Vt, S, dtype, "auto"), out)
+
+
 @pytest.mark.parametrize("b,p,r,q,M", [(16, 32, 256, 128, 1100), (16, 32, 256, 96, 1500), (12, 32, 384, 128, 1409), (4, 32, 264, 1000, 1000)])
 def test_monarch_interleaved_columns(b, p, r, q, M):
     """Interleaved columns with work for half of the chip: the bits of the kernels that BLR_GEMM_MID=0 leaves."""
