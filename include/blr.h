@@ -52,8 +52,8 @@ typedef enum {
   BLR_ALGO_AUTO = 0,
   BLR_ALGO_STREAM = 1,        /* the few-row kernels, M <= 16, f16/bf16: one to three launches chosen by row count and shape (one or two
                                  at M = 1, three on the matrix cores at 2..16 rows; a single persistent launch for what those decline) */
-  BLR_ALGO_TILED = 2,         /* up to 128 rows: the three-launch few-row kernels over tiles of 16 rows; above: MFMA tiled GEMMs with the
-                                 rank-space intermediates in the workspace (narrow blocks: fused launches that keep Y and / or Z on chip) */
+  BLR_ALGO_TILED = 2,         /* MFMA tiled GEMMs with the rank-space intermediates in the workspace, small tiles where large ones would not
+                                 fill the chip (narrow blocks: fused launches that keep Y and / or Z on chip; codes to 128 rows: streamed) */
   BLR_ALGO_FUSED = 3,         /* BLAST: x V and the mix in one launch, Y = x V only ever in LDS; then the batched GEMM with U.
                                  Needs f16/bf16, 4 | b <= 16, 8 | in_f / b, 8 | r, y_out == NULL; else BLR_ERR_UNSUPPORTED */
   BLR_ALGO_STREAM_SPLIT = 4   /* the STREAM phases as separate launches (no grid barrier)   */
