@@ -1379,17 +1379,23 @@ int stream_generic_launch(const StreamGenericArgs& a, hipStream_t st) {
   // Monarch: out1 = scatter(x_k w1_k); out = out1_l w2_l
   const int P = a.in_f / a.b, S = a.out_f / a.b, per = a.r / a.b;
   WsLayout w = ws_carve(a.ws, (size_t)a.b * a.M * a.r);
-  if (!a.split && a.w2_layout == BLR_W2_RS && a.b >= 2 && a.r % a.b == 0) {
-    // Two-stage decode kernel: a BLAST-shaped call whose mix is the Monarch permutation.
+  if (!a.split && a.b >= 2 && a.r % a.b == 0) {
+    // A BLAST-shaped call whose mix is the Monarch permutation.
+    const bool sr = a.w2_layout == BLR_W2_SR;
     StreamBlastArgs bl = {};
     bl.x = a.x; bl.ldx = a.ldx; bl.U = a.W2; bl.V = a.W1; bl.S = nullptr; bl.out = a.out; bl.ldo = a.ldo;
     bl.M = a.M; bl.in_f = a.in_f; bl.out_f = a.out_f; bl.b = a.b; bl.bo = a.b; bl.r = a.r;
-    bl.dtype = a.dtype; bl.u_layout = BLR_U_RQ; bl.s_layout = BLR_S_IJR; bl.wbits = 16;
+    bl.dtype = a.dtype; bl.u_layout = sr ? BLR_U_QR : BLR_U_RQ; bl.s_layout = BLR_S_IJR; bl.wbits = 16;
     bl.perm_per = per;
     if (a.out_order == BLR_OUT_INTERLEAVED) { bl.out_bs = 1; bl.out_ns = a.b; }
     else { bl.out_bs = S; bl.out_ns = 1; }
     if (decode2_applicable(bl)) {
-      int rc = decode2_blast_launch(bl, w.d2, w.plain, w.ctrl + D2_EPOCH, w.ctrl + D2_ARRIVE, w.ctrl + BAR_ERR, st);
+      // w2 (l, s, r), at one row too: the two skinny products of blr_decode_rows.hip.  The phase engine below took these calls before:
+      // 4096 -> 22016, rank 1024 at 1 / 3 / 16 rows 28.7 / 51.6 / 96.7 -> 17.7 / 17.9 / 19.0 us, 768 -> 2304, rank 128 15.1 / 24.3 / 54.3
+      // -> 7.7 .. 8.9 at all of them (eager calls; two launches of an eager stream), 1408 -> 3584 in 16 blocks, rank 304 17.5 / 26.2 /
+      // 30.6 -> 7.9 .. 8.8.  w2 (l, r, s): the single-row kernels have a say at one row.
+      int rc = sr ? decode_rows_launch(bl, w.plain, decode2_plain_bytes(), st)
+                  : decode2_blast_launch(bl, w.d2, w.plain, w.ctrl + D2_EPOCH, w.ctrl + D2_ARRIVE, w.ctrl + BAR_ERR, st);
       if (rc <= 0) return rc;
     }
   }

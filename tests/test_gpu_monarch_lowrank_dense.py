@@ -88,6 +88,20 @@ def test_monarch_small_all_algorithms(name, shape, algo, dtype):
     assert_close(out, ref, dtype, f"{name}/{algo}")
 
 
+# every name at few rows on the skinny products: whole 16-byte pieces and periods (rank / b) that cut through four columns, input
+# blocks deeper than a round of the first product (sliced, then permuted), column counts that are no whole chunk
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("name", ["triton_monarch_right_fp16", "triton_monarch_right_ideal_fp16", "triton_monarch_right_left_fp16"])
+@pytest.mark.parametrize("b,p,rank,s", [(16, 88, 304, 224), (3, 40, 72, 24), (4, 64, 128, 8), (2, 1104, 176, 136), (2, 1104, 16, 24), (16, 8, 16, 8), (16, 1040, 48, 40)])
+@pytest.mark.parametrize("M", [1, 2, 15, 16])
+def test_monarch_few_rows(M, b, p, rank, s, name, dtype):
+    say(f"[case] {name} few rows M={M} b={b} p={p} rank={rank} s={s} {dtype}")
+    x, w1_t, w2_t = monarch_inputs(b, p, rank, s, (M,), seed=M + rank)
+    out = _run_monarch(name, x, w1_t, w2_t, dtype)
+    ref = _ref_monarch(x, w1_t, w2_t, dtype)[0]
+    assert_close(out, _blocked(ref, b) if "ideal" in name else ref, dtype, f"{name} M={M} b={b} rank={rank}")
+
+
 LLAMA_IO = {"qkvo": (4096, 4096), "gate_up": (4096, 22016), "down": (11008, 4096)}
 
 
