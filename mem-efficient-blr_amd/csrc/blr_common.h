@@ -215,6 +215,7 @@ int blast_ymixw_launch(const void* x, int64_t ldx, const void* V, const void* S,
                       hipStream_t st);
 // The mix at few rows (blr_decode_rows.hip), two-byte types: same result, Y re-read from the L2 by one thread per four or eight ranks.
 int rows_mix_launch(const void* Y, const void* S, void* Z, int M, int b, int R, int s_layout, int dtype, hipStream_t st);
+int rows_mix_try(const void* Y, const void* S, void* Z, int M, int b, int R, int64_t si, int64_t sj, int64_t sr, int dtype, hipStream_t st);   // 1: not taken
 // Second half for output blocks of at most 80 columns: out_i = mix(S, Y)_i U_i with U (b, Q, R) (u_rq: (b, R, Q)), in one launch and without Z;
 // the fused output stage (bias, act, gate, resid) is taken from `ep`.  Same return convention; scratch as above.
 int blast_mixu_launch(const void* Y, const void* S, const void* U, void* out, int64_t ldo, const GemmArgs& ep, int M, int b, int R, int Q,

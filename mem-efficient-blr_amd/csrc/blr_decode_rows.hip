@@ -20,6 +20,7 @@
 // does).  The number of column pieces per chunk is planned so that the chunks spread evenly over the compute units
 // (a compute unit draws about 35 GB/s, so the bytes of the busiest one bound the launch).
 #include <type_traits>
+#include <utility>
 #include "blr_common.h"
 #include "blr_decode.h"
 #include "blr_decode_dev.h"
@@ -30,6 +31,7 @@ namespace {
 constexpr int DR_NT = 512;
 constexpr int DR_WAVES = 8;
 constexpr int DR_MAX_STEPS = 4;           // 32-row steps of a wave: 8 loads per lane each
+constexpr int64_t MIX_ANY_MAX = 1 << 20;  // b M R up to which rows_mix_any_kernel takes a call (beyond, every element of Y is loaded once for all blocks instead: blast_mix_launch)
 constexpr int DR_MAX_M = 128;             // token rows: tiles of 16 over the same registers of weights
 constexpr uint32_t DR_OOB = 0x80000000u;
 }  // namespace
@@ -525,6 +527,41 @@ __global__ __launch_bounds__(256) void rows_mix_rij_kernel(const T* __restrict__
   *reinterpret_cast<V4*>(Z + ((int64_t)i * M + m) * R + r4 * 4) = o;
 }
 
+// The same order of S with any other number of blocks (2 .. 15): thread = (rank, output block), the output block fastest, so that a wave
+// reads one contiguous run of S; the thread's row of S stays in registers and meets MB token rows of Y at a time, whose loads (B per row, one
+// element each - the lanes of a rank share them) are all in flight at once.  fp32 sums in input-block order.  Bound by one trip to
+// memory and the launch.  It took the place of a kernel that kept a chunk of 16 ranks and all of its token rows in one workgroup (R / 16
+// workgroups whatever M: 5.6 .. 7.5 us where the launches beside it take 3 .. 4) and, beyond 16 rows, of 64 ranks x 64 rows per workgroup.  Whole
+// calls: the three int4 linears of a GPT-2 block (4 and 6 blocks) at 14 rows 48.9 -> 34.5 us, 1152 -> 6912 in 9 blocks, rank 256 at
+// 93 rows 20.4 -> 11.4, 1536 -> 1536 in 12 blocks at 100 rows 26.1 -> 13.3, 768 -> 2304 in 6 blocks, int4 at 81 rows 29.4 -> 24.5.
+template <typename T, int B, int MB>
+__global__ __launch_bounds__(256) void rows_mix_any_kernel(const T* __restrict__ Y, const T* __restrict__ S, T* __restrict__ Z, int M, int R) {
+  constexpr int BYTES = B * (int)sizeof(T), AL = (BYTES & -BYTES) < 16 ? (BYTES & -BYTES) : 16, PE = AL / (int)sizeof(T);   // (S is aligned to 16 bytes)
+  struct alignas(AL) Piece { T v[PE]; };
+  const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
+  if (idx >= (uint32_t)B * (uint32_t)R) return;
+  const uint32_t r = idx / B, i = idx - r * B;
+  const int m0 = (int)blockIdx.y * MB;
+  const int64_t y_sj = (int64_t)M * R;
+  Piece sv[B / PE];
+#pragma unroll
+  for (int k = 0; k < B / PE; ++k) sv[k] = *reinterpret_cast<const Piece*>(S + (int64_t)idx * B + k * PE);
+  T yv[MB][B];
+#pragma unroll
+  for (int u = 0; u < MB; ++u) {
+    const T* yp = Y + (int64_t)min(m0 + u, M - 1) * R + r;               // (rows past the end: the last one again, not stored)
+#pragma unroll
+    for (int j = 0; j < B; ++j) yv[u][j] = yp[j * y_sj];
+  }
+#pragma unroll
+  for (int u = 0; u < MB; ++u) {
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < B; ++j) acc += TypeTraits<T>::to_f32(sv[j / PE].v[j % PE]) * TypeTraits<T>::to_f32(yv[u][j]);
+    if (m0 + u < M) Z[((int64_t)i * M + m0 + u) * R + r] = TypeTraits<T>::from_f32(acc);
+  }
+}
+
 namespace {
 
 inline unsigned prefetch_blocks(const RowsPrefetch& pf) { return pf.nblocks2 ? (pf.nblocks2 + 7u) & ~7u : 0u; }
@@ -551,9 +588,20 @@ int rows_mix_t(const void* Y, const void* S, void* Z, int M, int b, int R, int64
   const uint32_t nmix = (uint32_t)cdiv(total, nt);
   const dim3 grid(nmix + prefetch_blocks(pf)), block(nt);
   const FastDiv r4div = fd_make((uint32_t)(R / vw)), bdiv = fd_make((uint32_t)b);
-  if (wide) hipLaunchKernelGGL((rows_mix_kernel<T, 16, 8>), grid, block, 0, st, (const T*)Y, (const T*)S, (T*)Z, M, b, R, s_si, s_sj, r4div, bdiv, total, pf, nmix);
-  else if (b == 16) hipLaunchKernelGGL((rows_mix_kernel<T, 16, 4>), grid, block, 0, st, (const T*)Y, (const T*)S, (T*)Z, M, b, R, s_si, s_sj, r4div, bdiv, total, pf, nmix);
-  else hipLaunchKernelGGL((rows_mix_kernel<T, 0, 4>), grid, block, 0, st, (const T*)Y, (const T*)S, (T*)Z, M, b, R, s_si, s_sj, r4div, bdiv, total, pf, nmix);
+#define BLR_ROWS_MIX(B, VW) hipLaunchKernelGGL((rows_mix_kernel<T, B, VW>), grid, block, 0, st, (const T*)Y, (const T*)S, (T*)Z, M, b, R, s_si, s_sj, r4div, bdiv, total, pf, nmix)
+  if (wide) BLR_ROWS_MIX(16, 8);
+  else switch (b) {                                        // a fixed number of blocks: all loads of a thread in flight at once
+    case 2: BLR_ROWS_MIX(2, 4); break;
+    case 3: BLR_ROWS_MIX(3, 4); break;
+    case 4: BLR_ROWS_MIX(4, 4); break;
+    case 6: BLR_ROWS_MIX(6, 4); break;
+    case 8: BLR_ROWS_MIX(8, 4); break;
+    case 9: BLR_ROWS_MIX(9, 4); break;
+    case 12: BLR_ROWS_MIX(12, 4); break;
+    case 16: BLR_ROWS_MIX(16, 4); break;
+    default: BLR_ROWS_MIX(0, 4);
+  }
+#undef BLR_ROWS_MIX
   BLR_CHECK_LAUNCH("rows_mix");
   return BLR_OK;
 }
@@ -665,22 +713,52 @@ RowsPrefetch rows_prefetch_plan(const RowsParams& p, int batch, int wbits, bool 
   return f;
 }
 
+template <typename T, int B>
+void rows_mix_any_b(const void* Y, const void* S, void* Z, int M, int R, hipStream_t st) {
+  // one token row per thread while that gives at most two waves per SIMD, four beyond (a quarter of the loads of S)
+  const unsigned gx = (unsigned)cdiv((int64_t)B * R, 256);
+  if ((int64_t)gx * M <= 512) hipLaunchKernelGGL((rows_mix_any_kernel<T, B, 1>), dim3(gx, (unsigned)M), dim3(256), 0, st, (const T*)Y, (const T*)S, (T*)Z, M, R);
+  else hipLaunchKernelGGL((rows_mix_any_kernel<T, B, 4>), dim3(gx, (unsigned)cdiv(M, 4)), dim3(256), 0, st, (const T*)Y, (const T*)S, (T*)Z, M, R);
+}
+template <typename T, int... B>
+bool rows_mix_any_t(std::integer_sequence<int, B...>, int b, const void* Y, const void* S, void* Z, int M, int R, hipStream_t st) {
+  return ((b == B + 2 ? (rows_mix_any_b<T, B + 2>(Y, S, Z, M, R, st), true) : false) || ...);
+}
+
+// The mix on one of the kernels above; 1 if none of them takes it.
+int mix_launch(const void* Y, const void* S, void* Z, int M, int b, int R, int64_t si, int64_t sj, int64_t sr, int dtype, const RowsPrefetch& pf, hipStream_t st) {
+  if (dtype != BLR_F16 && dtype != BLR_BF16) return 1;
+  if (sr == 1 && si % 4 == 0 && sj % 4 == 0 && R % 4 == 0 && aligned(S, 8) && aligned(Y, 8) && aligned(Z, 8) &&
+      (int64_t)M * b * (R / 4) * (R / 4) < ((int64_t)1 << 32) && b < 65536)   // the multiply-high division is exact below 2^32 / divisor
+    return dtype == BLR_F16 ? rows_mix_t<f16>(Y, S, Z, M, b, R, si, sj, pf, st) : rows_mix_t<bf16>(Y, S, Z, M, b, R, si, sj, pf, st);
+  const bool rij = sj == 1 && si == b && sr == (int64_t)b * b && aligned(S, 16);
+  if (rij && b == 16 && R % 4 == 0 && aligned(Y, 8) && aligned(Z, 8) && (int64_t)M * (R / 4) * (R / 4) < ((int64_t)1 << 32))
+    return dtype == BLR_F16 ? rows_mix_rij_t<f16>(Y, S, Z, M, R, pf, st) : rows_mix_rij_t<bf16>(Y, S, Z, M, R, pf, st);
+  if (rij && b >= 2 && b <= 16 && (int64_t)M * b * R <= MIX_ANY_MAX && M <= 65535) {
+    using Blocks = std::make_integer_sequence<int, 15>;
+    if (dtype == BLR_F16) rows_mix_any_t<f16>(Blocks{}, b, Y, S, Z, M, R, st); else rows_mix_any_t<bf16>(Blocks{}, b, Y, S, Z, M, R, st);
+    BLR_CHECK_LAUNCH("rows_mix_any");
+    return BLR_OK;
+  }
+  return 1;
+}
+
 int mix_launch(const void* Y, const void* S, void* Z, int M, int b, int R, int s_layout, int dtype, const RowsPrefetch& pf, hipStream_t st) {
   int64_t si, sj, sr;
   if (s_layout == BLR_S_JIR) { sj = (int64_t)b * R; si = R; sr = 1; }
   else if (s_layout == BLR_S_RIJ) { sr = (int64_t)b * b; si = b; sj = 1; }
   else { si = (int64_t)b * R; sj = R; sr = 1; }
-  if (sr == 1 && si % 4 == 0 && sj % 4 == 0 && R % 4 == 0 && aligned(S, 8) && (int64_t)M * b * (R / 4) * (R / 4) < ((int64_t)1 << 32) && b < 65536)   // the multiply-high division is exact below 2^32 / divisor
-    return dtype == BLR_F16 ? rows_mix_t<f16>(Y, S, Z, M, b, R, si, sj, pf, st) : rows_mix_t<bf16>(Y, S, Z, M, b, R, si, sj, pf, st);
-  if (s_layout == BLR_S_RIJ && b == 16 && R % 4 == 0 && aligned(S, 16) && (int64_t)M * (R / 4) * (R / 4) < ((int64_t)1 << 32))
-    return dtype == BLR_F16 ? rows_mix_rij_t<f16>(Y, S, Z, M, R, pf, st) : rows_mix_rij_t<bf16>(Y, S, Z, M, R, pf, st);
-  return blast_mix_launch(Y, S, Z, M, b, R, si, sj, sr, dtype, st, 0);
+  const int rc = mix_launch(Y, S, Z, M, b, R, si, sj, sr, dtype, pf, st);
+  return rc != 1 ? rc : blast_mix_launch(Y, S, Z, M, b, R, si, sj, sr, dtype, st, 0);
 }
 
 }  // namespace
 
 int rows_mix_launch(const void* Y, const void* S, void* Z, int M, int b, int R, int s_layout, int dtype, hipStream_t st) {
   return mix_launch(Y, S, Z, M, b, R, s_layout, dtype, RowsPrefetch{}, st);
+}
+int rows_mix_try(const void* Y, const void* S, void* Z, int M, int b, int R, int64_t si, int64_t sj, int64_t sr, int dtype, hipStream_t st) {
+  return mix_launch(Y, S, Z, M, b, R, si, sj, sr, dtype, RowsPrefetch{}, st);
 }
 
 int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_bytes, hipStream_t st) {

@@ -1472,66 +1472,72 @@ static void mix_dispatch(dim3 grid, size_t lds, hipStream_t st, const void* Y, c
     hipLaunchKernelGGL((blast_mix_kernel<T, 0>), grid, dim3(256), lds, st, (const T*)Y, (const T*)S, (T*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, sat8);
 }
 
-// S slab of a workgroup of the mix kernels: s_t[(j * b + i) * MIX_LDR + r] = S(i, j, r0 + r) for 64 ranks, zero past R.  Rows
-// of 72 elements, not 64: staging S stored (r, i, j) writes one (j, i) row per lane, and with rows of 128 bytes every lane of a
-// wave would hit the same bank (the mix of a 4608 -> 1152, rank 576 layer at 4096 rows took 54 us with S in that order and
-// 40 us with S (j, i, r); 16-byte reads of a row stay aligned with 144-byte rows).
-constexpr int MIX_LDR = 72;
-// 16-byte pieces along whichever of r or j is contiguous in memory; element-wise otherwise.
+// S slab of a workgroup of the mix kernels: s_t[(j * b + i) * mix_ldr + r] = S(i, j, r0 + r) for the 8 x 16 bytes of ranks of a chunk
+// (64 of two-byte types, 32 of float), zero past R.  Rows of 72 two-byte elements, not 64: staging S stored (r, i, j) writes one (j, i) row per
+// lane, and with rows of 128 bytes every lane of a wave would hit the same bank (the mix of a 4608 -> 1152, rank 576 layer at 4096
+// rows took 54 us with S in that order and 40 us with S (j, i, r); 16-byte reads of a row stay aligned with 144-byte rows).
+template <typename T> constexpr int mix_vw = 16 / (int)sizeof(T);      // ranks per 16-byte piece
+template <typename T> constexpr int mix_ch = 8 * mix_vw<T>;            // ranks of a chunk
+template <typename T> constexpr int mix_ldr = 9 * mix_vw<T>;
+enum { MIX_S_ANY = 0, MIX_S_R = 1, MIX_S_RIJ = 2 };                    // element by element; 16-byte pieces along r; pieces of the run of (r, i, j)
+// MIX_S_RIJ reads the chunk as the one contiguous run that it is and lets each element find its place (element by element, a wave's
+// lanes lay 2 b^2 bytes apart; the three linears of a GPT-2 block, 4 and 6 blocks, at 1158 rows 60.7 -> 56.6 us).
 template <typename T>
 __device__ __forceinline__ void mix_stage_s(const T* __restrict__ S, T* s_t, int b, int R, int r0,
-                                            int64_t s_si, int64_t s_sj, int64_t s_sr, int vec_ok) {
-  using V8 = typename TypeTraits<T>::vec8;
+                                            int64_t s_si, int64_t s_sj, int64_t s_sr, int s_order) {
+  constexpr int VW = mix_vw<T>, CH = mix_ch<T>, LDR = mix_ldr<T>;
+  struct alignas(16) V8 { T v[VW]; };
   const int tid = threadIdx.x;
-  if (vec_ok && s_sr == 1) {                                   // (j, i, r) or (i, j, r): r contiguous
+  if (s_order == MIX_S_R) {                                    // (j, i, r) or (i, j, r): r contiguous
     for (int idx = tid; idx < b * b * 8; idx += 256) {
-      const int r8 = (idx & 7) * 8, ji = idx >> 3;
+      const int r8 = (idx & 7) * VW, ji = idx >> 3;
       const int j = ji / b, i = ji - j * b;
-      V8 v;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = (T)0.0f;
+      V8 v = {};
       if (r0 + r8 < R) v = *reinterpret_cast<const V8*>(&S[(int64_t)i * s_si + (int64_t)j * s_sj + r0 + r8]);
-      *reinterpret_cast<V8*>(&s_t[ji * MIX_LDR + r8]) = v;
+      *reinterpret_cast<V8*>(&s_t[ji * LDR + r8]) = v;
     }
-  } else if (vec_ok && s_sj == 1 && (b & 7) == 0) {            // (r, i, j): j contiguous
-    const int jv = b >> 3;
-    for (int idx = tid; idx < 64 * b * jv; idx += 256) {
-      const int j8 = (idx % jv) * 8, t = idx / jv;
-      const int i = t % b, r = t / b;
-      V8 v;
+  } else if (s_order == MIX_S_RIJ) {                           // (r, i, j): whole pieces, R being a multiple of VW
+    const int bb = b * b, valid = min(CH, R - r0) * bb;
+    for (int idx = tid; idx < 8 * bb; idx += 256) {
+      const int e0 = idx * VW;
+      V8 v = {};
+      if (e0 < valid) v = *reinterpret_cast<const V8*>(&S[(int64_t)r0 * bb + e0]);
+      int r = e0 / bb, ij = e0 - r * bb, i = ij / b, j = ij - i * b;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = (T)0.0f;
-      if (r0 + r < R) v = *reinterpret_cast<const V8*>(&S[(int64_t)(r0 + r) * s_sr + (int64_t)i * s_si + j8]);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s_t[((j8 + e) * b + i) * MIX_LDR + r] = v[e];
+      for (int e = 0; e < VW; ++e) {
+        s_t[(j * b + i) * LDR + r] = v.v[e];
+        if (++j == b) { j = 0; if (++i == b) { i = 0; ++r; } }
+      }
     }
   } else {
-    for (int idx = tid; idx < b * b * 64; idx += 256) {
-      const int r = idx & 63, ji = idx >> 6;
+    for (int idx = tid; idx < b * b * CH; idx += 256) {
+      const int r = idx % CH, ji = idx / CH;
       const int j = ji / b, i = ji - j * b;
       T v = (T)0.0f;
       if (r0 + r < R) v = S[(int64_t)i * s_si + (int64_t)j * s_sj + (int64_t)(r0 + r) * s_sr];
-      s_t[ji * MIX_LDR + r] = v;
+      s_t[ji * LDR + r] = v;
     }
   }
 }
 
-// Vector variant for two-byte types, b <= 16, R % 8 == 0: thread = (8 consecutive r, one m); all
-// b vectors Y_j[m, r..r+7] are loaded (16 bytes each) before the b x b x 8 multiply-adds, S comes
-// from an LDS slab [j][i][64] staged once per workgroup and reused for 128 rows of m.
+// Vector variant for b <= 16 and ranks in whole 16-byte pieces: thread = (one piece of consecutive r, one m); all b vectors Y_j[m, r..] are loaded
+// (16 bytes each) before the b x b x VW multiply-adds, S comes from an LDS slab [j][i][chunk] staged once per workgroup.
+// float took blast_mix_kernel before, whose workgroups staged 64 KB of S element by element for 8 rows each: that mix was 132 of the 250 us
+// of a 2048 -> 8192 call of rank 768 at 724 rows with its intermediates, the call now 148; 4608 -> 1152, rank 576 at 756 rows 185 -> 92.
 template <typename T>
 __global__ __launch_bounds__(256) void blast_mix_vec_kernel(const T* __restrict__ Y, const T* __restrict__ S,
                                                             T* __restrict__ Z, int M, int b, int R,
-                                                            int64_t s_si, int64_t s_sj, int64_t s_sr, int m_per_wg, int s_vec, int sat8) {
-  using V8 = typename TypeTraits<T>::vec8;
+                                                            int64_t s_si, int64_t s_sj, int64_t s_sr, int m_per_wg, int s_order, int sat8) {
+  constexpr int VW = mix_vw<T>, LDR = mix_ldr<T>;
+  struct alignas(16) V8 { T v[VW]; };
   extern __shared__ float s_lds[];
-  T* s_t = reinterpret_cast<T*>(s_lds);      // [b][b][64]  (j, i, r)
+  T* s_t = reinterpret_cast<T*>(s_lds);      // [b][b][chunk]  (j, i, r)
   const int tid = threadIdx.x;
-  const int r0 = blockIdx.x * 64;
-  mix_stage_s<T>(S, s_t, b, R, r0, s_si, s_sj, s_sr, s_vec);
+  const int r0 = blockIdx.x * mix_ch<T>;
+  mix_stage_s<T>(S, s_t, b, R, r0, s_si, s_sj, s_sr, s_order);
   __syncthreads();
   const int rl = tid & 7, ms = tid >> 3;     // 8 r-vectors x 32 m slots
-  const int r = r0 + rl * 8;
+  const int r = r0 + rl * VW;
   if (r >= R) return;
   const int m_begin = blockIdx.y * m_per_wg;
   const int m_end = min(M, m_begin + m_per_wg);
@@ -1541,20 +1547,20 @@ __global__ __launch_bounds__(256) void blast_mix_vec_kernel(const T* __restrict_
     for (int j = 0; j < 16; ++j)                     // unconditional: planes past b re-read the last one and are not used
       yv[j] = ldg16<V8>(&Y[((int64_t)min(j, b - 1) * M + m) * R + r]);
     for (int i = 0; i < b; ++i) {
-      float acc[8];
+      float acc[VW];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
+      for (int e = 0; e < VW; ++e) acc[e] = 0.0f;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         if (j < b) {
-          V8 sv = *reinterpret_cast<const V8*>(&s_t[(j * b + i) * MIX_LDR + rl * 8]);
+          const V8 sv = *reinterpret_cast<const V8*>(&s_t[(j * b + i) * LDR + rl * VW]);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) acc[e] = fmaf(TypeTraits<T>::to_f32(sv[e]), TypeTraits<T>::to_f32(yv[j][e]), acc[e]);
+          for (int e = 0; e < VW; ++e) acc[e] = fmaf(TypeTraits<T>::to_f32(sv.v[e]), TypeTraits<T>::to_f32(yv[j].v[e]), acc[e]);
         }
       }
       V8 o;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = TypeTraits<T>::from_f32(sat8 ? sat8_rne(acc[e]) : acc[e]);
+      for (int e = 0; e < VW; ++e) o.v[e] = TypeTraits<T>::from_f32(sat8 ? sat8_rne(acc[e]) : acc[e]);
       *reinterpret_cast<V8*>(&Z[((int64_t)i * M + m) * R + r]) = o;
     }
   }
@@ -1566,14 +1572,14 @@ __global__ __launch_bounds__(256) void blast_mix_vec_kernel(const T* __restrict_
 template <bool FULL16, int MB>                   // FULL16: b == 16, so no load sits under a condition; MB rows of m per thread
 __global__ __launch_bounds__(256) void blast_mix_h2_kernel(const f16* __restrict__ Y, const f16* __restrict__ S,
                                                            f16* __restrict__ Z, int M, int b, int R,
-                                                           int64_t s_si, int64_t s_sj, int64_t s_sr, int m_per_wg, int s_vec) {
+                                                           int64_t s_si, int64_t s_sj, int64_t s_sr, int m_per_wg, int s_order) {
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
   struct H8 { h2 v[4]; };
   extern __shared__ float s_lds[];
   f16* s_t = reinterpret_cast<f16*>(s_lds);      // [b][b][64]  (j, i, r)
   const int tid = threadIdx.x;
   const int r0 = blockIdx.x * 64;
-  mix_stage_s<f16>(S, s_t, b, R, r0, s_si, s_sj, s_sr, s_vec);
+  mix_stage_s<f16>(S, s_t, b, R, r0, s_si, s_sj, s_sr, s_order);
   __syncthreads();
   const int rl = tid & 7, ms = tid >> 3;     // 8 r-vectors x 32 m slots
   const int r = r0 + rl * 8;
@@ -1599,7 +1605,7 @@ __global__ __launch_bounds__(256) void blast_mix_h2_kernel(const f16* __restrict
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         if (FULL16 || j < b) {
-          const H8 sv = *reinterpret_cast<const H8*>(&s_t[(j * b + i) * MIX_LDR + rl * 8]);
+          const H8 sv = *reinterpret_cast<const H8*>(&s_t[(j * b + i) * mix_ldr<f16> + rl * 8]);
 #pragma unroll
           for (int u = 0; u < MB; ++u)
 #pragma unroll
@@ -1613,66 +1619,38 @@ __global__ __launch_bounds__(256) void blast_mix_h2_kernel(const f16* __restrict
   }
 }
 
-// The mix for a handful of rows (M <= 16, b <= 16): workgroup = 16 ranks x all output blocks, thread = (block i, rank).
-// The Y values of the chunk (b x M x 16) are staged in LDS once; every thread keeps its b values of S in registers.
-template <typename T>
-__global__ __launch_bounds__(256) void blast_mix_small_kernel(const T* __restrict__ Y, const T* __restrict__ S, T* __restrict__ Z,
-                                                              int M, int b, int R, int64_t s_si, int64_t s_sj, int64_t s_sr) {
-  __shared__ float ys[16 * 16 * 16];                  // [j][m][rank in chunk]
-  const int tid = threadIdx.x, g = tid >> 4, rr = tid & 15;
-  const int r0 = blockIdx.x * 16, r = r0 + rr;
-  float sv[16];
-#pragma unroll
-  for (int j = 0; j < 16; ++j)
-    sv[j] = (g < b && j < b && r < R) ? TypeTraits<T>::to_f32(S[(int64_t)g * s_si + (int64_t)j * s_sj + (int64_t)r * s_sr]) : 0.0f;
-  const int total = b * M * 16;
-  for (int idx = tid; idx < total; idx += 256) {
-    const int c = idx & 15, jm = idx >> 4;            // jm = j * M + m
-    ys[idx] = (r0 + c < R) ? TypeTraits<T>::to_f32(Y[(int64_t)jm * R + r0 + c]) : 0.0f;
-  }
-  __syncthreads();
-  if (g < b && r < R) {
-    for (int m = 0; m < M; ++m) {
-      float z = 0.0f;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) z = fmaf(sv[j], j < b ? ys[(j * M + m) * 16 + rr] : 0.0f, z);
-      Z[((int64_t)g * M + m) * R + r] = TypeTraits<T>::from_f32(z);
-    }
-  }
-}
-
 int blast_mix_launch(const void* Y, const void* S, void* Z, int M, int b, int R,
                      int64_t s_si, int64_t s_sj, int64_t s_sr, int dtype, hipStream_t st, int sat8) {
-  if (M <= 16 && b <= 16 && !sat8 && (dtype == BLR_F16 || dtype == BLR_BF16)) {
-    const dim3 grid((unsigned)cdiv(R, 16));
-    if (dtype == BLR_F16) hipLaunchKernelGGL(blast_mix_small_kernel<f16>, grid, dim3(256), 0, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr);
-    else hipLaunchKernelGGL(blast_mix_small_kernel<bf16>, grid, dim3(256), 0, st, (const bf16*)Y, (const bf16*)S, (bf16*)Z, M, b, R, s_si, s_sj, s_sr);
-    BLR_CHECK_LAUNCH("blast_mix_small");
-    return BLR_OK;
+  if (M <= 16 && b <= 16 && !sat8) {               // a handful of rows
+    const int rc = rows_mix_try(Y, S, Z, M, b, R, s_si, s_sj, s_sr, dtype, st);
+    if (rc != 1) return rc;
   }
-  int r_chunks = (int)cdiv(R, 64);
-  if (dtype != BLR_F32 && b <= 16 && R % 8 == 0 && aligned(Y, 16) && aligned(Z, 16)) {
-    size_t lds = (size_t)b * b * MIX_LDR * 2;
-    // S may be fetched in 16-byte pieces if every piece starts on a 16-byte boundary
-    const int s_vec = aligned(S, 16) && ((s_sr == 1 && s_si % 8 == 0 && s_sj % 8 == 0) ||
-                                         (s_sj == 1 && s_si % 8 == 0 && s_sr % 8 == 0));
-    const bool use_h2 = dtype == BLR_F16 && !sat8;
+  const int vw = dtype == BLR_F32 ? 4 : 8;
+  if (b <= 16 && R % vw == 0 && aligned(Y, 16) && aligned(Z, 16)) {
+    const int r_chunks = (int)cdiv(R, 8 * vw);
+    const size_t lds = (size_t)b * b * 144;
+    const int s_order = !aligned(S, 16) ? MIX_S_ANY : s_sr == 1 && s_si % vw == 0 && s_sj % vw == 0 ? MIX_S_R
+                        : s_sj == 1 && s_si == b && s_sr == (int64_t)b * b ? MIX_S_RIJ : MIX_S_ANY;
+    const bool use_h2 = dtype == BLR_F16 && !sat8 && M > 16;
     const int mb = use_h2 && M >= 64 ? 2 : 1;
-    int m_per_wg = 32 * mb;                        // one pass of the 32 row slots: more, smaller workgroups measured fastest
+    const int m_per_wg = 32 * mb;                  // one pass of the 32 row slots: more, smaller workgroups measured fastest
     dim3 grid(r_chunks, (unsigned)cdiv(M, m_per_wg));
     if (use_h2 && mb == 2)
-      if (b == 16) hipLaunchKernelGGL((blast_mix_h2_kernel<true, 2>), grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_vec);
-      else hipLaunchKernelGGL((blast_mix_h2_kernel<false, 2>), grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_vec);
+      if (b == 16) hipLaunchKernelGGL((blast_mix_h2_kernel<true, 2>), grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_order);
+      else hipLaunchKernelGGL((blast_mix_h2_kernel<false, 2>), grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_order);
     else if (use_h2)
-      if (b == 16) hipLaunchKernelGGL((blast_mix_h2_kernel<true, 1>), grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_vec);
-      else hipLaunchKernelGGL((blast_mix_h2_kernel<false, 1>), grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_vec);
+      if (b == 16) hipLaunchKernelGGL((blast_mix_h2_kernel<true, 1>), grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_order);
+      else hipLaunchKernelGGL((blast_mix_h2_kernel<false, 1>), grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_order);
     else if (dtype == BLR_F16)
-      hipLaunchKernelGGL(blast_mix_vec_kernel<f16>, grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_vec, sat8);
+      hipLaunchKernelGGL(blast_mix_vec_kernel<f16>, grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_order, sat8);
+    else if (dtype == BLR_BF16)
+      hipLaunchKernelGGL(blast_mix_vec_kernel<bf16>, grid, dim3(256), lds, st, (const bf16*)Y, (const bf16*)S, (bf16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_order, sat8);
     else
-      hipLaunchKernelGGL(blast_mix_vec_kernel<bf16>, grid, dim3(256), lds, st, (const bf16*)Y, (const bf16*)S, (bf16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_vec, sat8);
+      hipLaunchKernelGGL(blast_mix_vec_kernel<float>, grid, dim3(256), lds, st, (const float*)Y, (const float*)S, (float*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_order, sat8);
     BLR_CHECK_LAUNCH("blast_mix_vec");
     return BLR_OK;
   }
+  const int r_chunks = (int)cdiv(R, 64);
   size_t lds = (size_t)b * b * 64 * sizeof(float);
   if (lds > 64 * 1024) { set_error("blast mix: b=%d too large for the LDS slab", b); return BLR_ERR_UNSUPPORTED; }
   int m_per_wg = 64;

@@ -29,6 +29,37 @@ def test_blast(name, M, dtype):
     assert_close(out, _ref(x, U, Vt, S, dtype)[0], dtype, f"{name} M={M}")
 
 
+# the mix with any number of blocks and S (r, i, j): one token row per thread, four of them (a last group of one to three), more rows than
+# its thread per (rank, block) is used for; ranks that leave a chunk of 64 part empty; S off a 16-byte boundary (element by element)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,r", [(1, 8), (3, 72), (16, 200), (130, 264), (257, 1032)])
+@pytest.mark.parametrize("b", list(range(2, 17)))
+def test_mix_any_blocks(b, M, r, dtype):
+    from triton_funcs import blast_kernels as K
+    p, q = 8, 16
+    x, U, Vt, S = blast_inputs(b, p, q, r, (M,), seed=M + b)
+    Ub, Vb, Sb = O.blast_to_bmm_layout(U, Vt, S)
+    say(f"[case] mix b={b} M={M} r={r} {dtype}")
+    ref = O.blast_forward(rounded(x, dtype), rounded(U, dtype), rounded(Vt, dtype), rounded(S, dtype))[0]
+    args = dev(x, dtype), dev(Ub, dtype), dev(Vb, dtype)
+    assert_close(K.triton_blast_bmm_fp16(*args, dev(Sb, dtype)), ref, dtype, f"mix b={b} M={M} r={r}")
+    room = torch.zeros(Sb.size + 8, device="cuda", dtype=dtype)
+    off = room[1:1 + Sb.size].view(r, b, b)
+    off.copy_(dev(Sb, dtype))
+    assert_close(K.triton_blast_bmm_fp16(*args, off), ref, dtype, f"mix b={b} M={M} r={r}, S one element off")
+
+
+# fp32: chunks of 32 ranks, whole and not, ranks in whole pieces of four and not, both orders of S
+@pytest.mark.parametrize("name", ["triton_blast_full_fp32", "triton_blast_bmm_fp32"])
+@pytest.mark.parametrize("b,M,r", [(2, 1, 4), (3, 33, 36), (6, 70, 200), (16, 31, 64), (16, 65, 100), (5, 40, 30)])
+def test_mix_fp32(b, M, r, name):
+    from test_gpu_blast import _ref, _run_blast
+    x, U, Vt, S = blast_inputs(b, 8, 16, r, (M,), seed=M + b)
+    say(f"[case] fp32 mix {name} b={b} M={M} r={r}")
+    out = _run_blast(name, x, U, Vt, S, torch.float32, "auto")
+    assert_close(out[0] if isinstance(out, tuple) else out, _ref(x, U, Vt, S, torch.float32)[0], torch.float32, f"{name} b={b} M={M} r={r}")
+
+
 @pytest.mark.parametrize("layer", ["qkvo", "gate_up", "down"])
 def test_blast_llama7b_64_rows_with_bias_and_activation(layer):
     from triton_funcs import blast_kernels as K, _lib as L
