@@ -173,6 +173,11 @@ int blr_quantize_sym(const void* w, int dtype, int64_t outer, int64_t reduce, in
  * without a transposed copy of it.  bits = 4 needs an even `inner`.                                              */
 int blr_quantize_sym_t(const void* w, int dtype, int64_t outer, int64_t reduce, int64_t inner,
                        int bits, void* codes, void* scales, void* stream);
+/* Both factors of a layer at once: U (b, q, r) as blr_quantize_sym_t(U, b, r, q), V (b, p, r) as blr_quantize_sym(V, b, p, r),
+ * with the same bytes as a result.  One launch that reads every weight once where the shapes allow it.  bits = 4 needs
+ * even q and r.                                                                                                  */
+int blr_quantize_blast(const void* U, const void* V, int dtype, int64_t b, int64_t q, int64_t p, int64_t r, int bits,
+                       void* u_codes, void* u_scales, void* v_codes, void* v_scales, void* stream);
 
 /* ---- Monarch ------------------------------------------------------------------------------
  * w1 (b, in_f/b, rank) with pre-permuted columns (reference layer.py:221-224), w2 per

@@ -614,6 +614,14 @@ int blr_quantize_sym_t(const void* w, int dtype, int64_t outer, int64_t reduce, 
   return quantize_t_launch(w, dtype, outer, reduce, inner, bits, codes, scales, (hipStream_t)stream);
 }
 
+int blr_quantize_blast(const void* U, const void* V, int dtype, int64_t b, int64_t q, int64_t p, int64_t r, int bits,
+                       void* u_codes, void* u_scales, void* v_codes, void* v_scales, void* stream) {
+  if (!U || !V || !u_codes || !u_scales || !v_codes || !v_scales) { set_error("quantize: null pointer"); return BLR_ERR_BAD_ARG; }
+  if (b <= 0 || q <= 0 || p <= 0 || r <= 0 || (bits != 8 && bits != 4) || !dtype_ok(dtype)) { set_error("quantize: bad argument"); return BLR_ERR_BAD_ARG; }
+  if (bits == 4 && (q % 2 || r % 2)) { set_error("quantize: int4 needs an even contiguous axis"); return BLR_ERR_BAD_SHAPE; }
+  return quantize_pair_launch(U, V, dtype, b, q, p, r, bits, u_codes, u_scales, v_codes, v_scales, (hipStream_t)stream);
+}
+
 // ---- Monarch --------------------------------------------------------------------------------------
 size_t blr_monarch_workspace_bytes(int M, int in_f, int out_f, int b, int rank, int dtype, int algo) {
   if (M <= 0 || b <= 0 || rank <= 0) return 0;

@@ -43,6 +43,7 @@ _SIGNATURES = {
     "blr_blast_q_workspace_bytes": (_sz, [_i] * 6),
     "blr_blast_q_fwd": (_i, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64] + [_i] * 8 + [_vp, _sz, _vp]),
     "blr_quantize_sym": (_i, [_vp, _i, _i64, _i64, _i64, _i, _vp, _vp, _vp]),
+    "blr_quantize_blast": (_i, [_vp, _vp, _i, _i64, _i64, _i64, _i64, _i, _vp, _vp, _vp, _vp, _vp]),
     "blr_quantize_sym_t": (_i, [_vp, _i, _i64, _i64, _i64, _i, _vp, _vp, _vp]),
     "blr_monarch_workspace_bytes": (_sz, [_i] * 7),
     "blr_monarch_fwd": (_i, [_vp, _i64, _vp, _vp, _vp, _i64, _vp] + [_i] * 9 + [_vp, _sz, _vp]),

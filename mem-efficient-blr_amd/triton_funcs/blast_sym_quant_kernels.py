@@ -82,6 +82,19 @@ def quantize_blast_factors(U, V, bits=8):
         assert q % 2 == 0, "int4 packing needs an even last axis"
         uc = torch.empty((b, r, q // 2), dtype=torch.uint8, device=U.device)
     us = torch.empty((b, q), dtype=torch.float16, device=U.device)
+    if V.dtype == U.dtype and V.dim() == 3 and V.shape[0] == b and V.shape[2] == r and V.device == U.device:
+        V = V.contiguous()
+        p = V.shape[1]
+        if bits == 8:
+            vc = torch.empty((b, p, r), dtype=torch.int8, device=U.device)
+        else:
+            assert r % 2 == 0, "int4 packing needs an even last axis"
+            vc = torch.empty((b, p, r // 2), dtype=torch.uint8, device=U.device)
+        vs = torch.empty((b, r), dtype=torch.float16, device=U.device)
+        rc = L.lib().blr_quantize_blast(U.data_ptr(), V.data_ptr(), L.dtype_code(U.dtype), b, q, p, r, bits, uc.data_ptr(), us.data_ptr(),
+                                        vc.data_ptr(), vs.data_ptr(), L.stream_ptr(U.device))
+        L.check(rc, "blr_quantize_blast")
+        return QuantFactor(uc, us, bits, tuple(U.shape)), QuantFactor(vc, vs, bits, tuple(V.shape))
     rc = L.lib().blr_quantize_sym_t(U.data_ptr(), L.dtype_code(U.dtype), b, r, q, bits, uc.data_ptr(), us.data_ptr(), L.stream_ptr(U.device))
     L.check(rc, "blr_quantize_sym_t")
     vc, vs = quantize_sym(V, 1, bits)

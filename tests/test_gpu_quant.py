@@ -49,6 +49,17 @@ def test_packed_factors_codes_bit_exact(b, p, q, r, bits, dtype):
         np.testing.assert_array_equal(got.scales.cpu().numpy(), scales)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("bits", [8, 4])
+# the launch for both factors: r at 256, 512 and 1024 and on either side (1028: back to a launch per factor), p at the rows that 128, 64 and
+# 32 row groups hold in 4, 8 and 16 registers, the last of them and one more; channel groups of 32 that are part empty; rows of codes in
+# stores of 16, 4 and 1 bytes
+@pytest.mark.parametrize("b,p,q,r", [(2, 128, 32, 256), (16, 256, 68, 128), (2, 129, 34, 260), (3, 513, 100, 516), (2, 1024, 40, 512), (2, 2048, 8, 1024),
+                                     (2, 2049, 36, 64), (3, 70, 72, 1028), (2, 5, 2, 4)])
+def test_packed_in_one_launch_bit_exact(b, p, q, r, bits, dtype):
+    test_packed_factors_codes_bit_exact(b, p, q, r, bits, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("bits", [8, 4])
 @pytest.mark.parametrize("at", [0, 1, 2, 3])
