@@ -367,7 +367,7 @@ __device__ unsigned long long g_trace_gemm[4096 * 8];
 // The tile's way out of a ring kernel: accumulators -> LDS (as T, the stages are done with) -> whole rows to memory, through the
 // output stage where there is one.  acc[i][j][4 q + e] is row (lane & 31), column 8 q + 4 (lane >> 5) + e of the 32 x 32 block
 // (i, j) of the wave's WM x WN part (the products were formed transposed).  hf: which tile of a pair this is.
-template <typename T, int BM, int BN, int BNC, int NWV, int WM, int WN, int TM, int TN, bool EP, bool PAIRS>
+template <typename T, int BM, int BN, int BNC, int NWV, int WM, int WN, int TM, int TN, bool EP, bool PAIRS, bool SCAT = false>
 __device__ __forceinline__ void ring_write_out(const GemmArgs& g, f32x16 (&acc)[TM][TN], unsigned char* smem, T* C, int m0, int n0, int wm, int wn,
                                                int bt, int hf) {
   using V8 = typename TypeTraits<T>::vec8;
@@ -395,6 +395,36 @@ __device__ __forceinline__ void ring_write_out(const GemmArgs& g, f32x16 (&acc)[
   if (g.cn != 1) {
     // interleaved columns (column n of batch bt is element n * cn + bt of the row): two-byte stores, lanes along n, so
     // that an instruction touches cn * 128 contiguous bytes; the other batches fill the gaps
+    if constexpr (EP && NWV * 64 % BNC == 0) {
+      // (a thread stays in its column: one value of the bias; eight rows at a time, their activations next to each other;
+      // 2048 -> 8192 in 16 blocks, rank 512 at 3000 rows with a bias 142.9 -> 112.2 us against gemm_mfma_kernel)
+      constexpr int RPP = NWV * 64 / BNC;
+      static_assert(BM % (RPP * 8) == 0, "whole batches of rows");
+      const int col = tid % BNC, gc = n0 + col;
+      if (gc >= g.N) return;
+      const int64_t in_row = (int64_t)bt * g.sC + (int64_t)gc * g.cn;
+      const float bias = g.bias ? TypeTraits<T>::to_f32(reinterpret_cast<const T*>(g.bias)[in_row]) : 0.0f;
+      for (int row0 = tid / BNC; row0 < BM; row0 += RPP * 8) {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = TypeTraits<T>::to_f32(cs[(row0 + RPP * e) * CLD + col]) + bias;
+        apply_act_n(v, g.act);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int gr = m0 + row0 + RPP * e;
+          if (gr >= g.M) continue;
+          T o = TypeTraits<T>::from_f32(v[e]);
+          if (g.gate || g.resid) {
+            float w = TypeTraits<T>::to_f32(o);
+            if (g.gate) w *= TypeTraits<T>::to_f32(reinterpret_cast<const T*>(g.gate)[(int64_t)(gr / g.gate_rows) * g.ld_gate + in_row]);
+            if (g.resid) w += TypeTraits<T>::to_f32(reinterpret_cast<const T*>(g.resid)[(int64_t)gr * g.ld_resid + in_row]);
+            o = TypeTraits<T>::from_f32(w);
+          }
+          C[in_row + (int64_t)gr * g.ldc] = o;
+        }
+      }
+      return;
+    }
     for (int v = tid; v < BM * BNC; v += NWV * 64) {
       const int row = v / BNC, col = v - row * BNC;
       const int gr = m0 + row, gc = n0 + col;
@@ -439,6 +469,29 @@ __device__ __forceinline__ void ring_write_out(const GemmArgs& g, f32x16 (&acc)[
     }
     return;
   }
+  if constexpr (SCAT) {                                // (a kernel of its own: the code below costs the others 2 %)
+    // a period that cuts through pieces of eight columns: as many together as stay together (four, two or one), lanes along the columns.
+    // gemm_mfma_kernel took these products before: 6528 -> 1536 in 8 blocks, rank 800 (period 100) at 550 rows 40.4 -> 26.7 us, 5504 -> 3200
+    // in 16 blocks, rank 400 (period 25) at 1189 rows 75.7 -> 57.9.  Where the small tiles of blr_gemm_mid.hip take a product they stay ahead.
+    auto scatter = [&](auto w) {
+      constexpr int E = decltype(w)::value, VPE = BNC / E;
+      typedef T VE __attribute__((ext_vector_type(E > 1 ? E : 2)));
+      for (int v = tid; v < BM * VPE; v += NWV * 64) {
+        const int row = v / VPE, c = (v - row * VPE) * E;
+        const int gr = m0 + row, gc = n0 + c;
+        if (gr >= g.M || gc >= g.N) continue;
+        const int d = gc / g.per;
+        T* o = &C[(int64_t)d * g.sL + (int64_t)gr * g.ldc + (int64_t)bt * g.per + (gc - d * g.per)];
+        if constexpr (E > 1) *reinterpret_cast<VE*>(o) = *reinterpret_cast<const VE*>(&cs[row * CLD + c]);
+        else *o = cs[row * CLD + c];
+      }
+    };
+    const int64_t all = g.per | g.sL | g.ldc;
+    if (all % 4 == 0) scatter(std::integral_constant<int, 4>{});
+    else if (all % 2 == 0) scatter(std::integral_constant<int, 2>{});
+    else scatter(std::integral_constant<int, 1>{});
+    return;
+  }
   for (int v = tid; v < BM * VPR; v += NWV * 64) {
     const int row = v / VPR, cvec = (v - row * VPR) * 8;
     const int gr = m0 + row, gc = n0 + cvec;
@@ -457,7 +510,7 @@ __device__ __forceinline__ void ring_write_out(const GemmArgs& g, f32x16 (&acc)[
 // BNC: the columns of a tile that are computed and written.  Below BN (96 of 128) the stages keep their 128-column layout and the
 // four waves sit above each other, 64 rows x 96 columns each: for output widths like 288 that 128-column tiles cover with a
 // quarter of their matrix instructions wasted.
-template <typename T, bool B_KN, int BM, int BN, bool EP = false, bool SHALLOW = false, int NWV = 4, bool PARTIAL = false, int BNC = BN>
+template <typename T, bool B_KN, int BM, int BN, bool EP = false, bool SHALLOW = false, int NWV = 4, bool PARTIAL = false, int BNC = BN, bool SCAT = false>
 __global__ __launch_bounds__(NWV * 64, (SHALLOW ? 2 : 1)) void gemm_ring_kernel(GemmArgs g, int tiles_m, int tiles_n, int per_xcd, int group_m, int side_wgs) {
   constexpr int NA = ring_na<SHALLOW>(), NB = ring_nb<SHALLOW>();
   constexpr int ASTG = BM * 64, BSTG = BN * 64, BRING = NA * ASTG;   // stage sizes, start of the B ring
@@ -702,7 +755,7 @@ __global__ __launch_bounds__(NWV * 64, (SHALLOW ? 2 : 1)) void gemm_ring_kernel(
       }
     return;
   }
-  ring_write_out<T, BM, BN, BNC, NWV, WM, WN, TM, TN, EP, PAIRS>(g, acc, smem, C, m0, n0, wm, wn, bt, hf);
+  ring_write_out<T, BM, BN, BNC, NWV, WM, WN, TM, TN, EP, PAIRS, SCAT>(g, acc, smem, C, m0, n0, wm, wn, bt, hf);
   if (hf + 1 < halves) __syncthreads();              // the staged tile has been read: the rings may be filled again
   }  // tiles of a pair
   TRG(4);
@@ -1150,16 +1203,17 @@ static int splitk_reduce_launch(const GemmArgs& g, int splits, hipStream_t st) {
   return BLR_OK;
 }
 
+// Monarch's scatter with a period that cuts through pieces of eight columns
+static bool ring_scatter_odd(const GemmArgs& g) { return g.epi == EPI_MONARCH_SCATTER && (g.per % 8 || g.sL % 8); }
+
 static bool ring_ok(const GemmArgs& g) {
   if (g.cn < 1 || g.N < 8 || g.N % 8 || g.K % 8) return false;
-  // Monarch's scatter of the first product: an 8-column vector stays inside one destination block when the period is a multiple of 8
-  if (g.epi == EPI_MONARCH_SCATTER && (g.per % 8 || g.sL % 8 || g.cn != 1 || g.sat8 || g.bias || g.act || g.gate || g.resid)) return false;
+  // Monarch's scatter of the first product
+  if (g.epi == EPI_MONARCH_SCATTER && (g.cn != 1 || (ring_scatter_odd(g) && !g.b_kn) || g.sat8 || g.bias || g.act || g.gate || g.resid)) return false;
   if (g.epi != EPI_PLAIN && g.epi != EPI_MONARCH_SCATTER) return false;
   if (!aligned(g.A, 16) || !aligned(g.B, 16) || g.lda % 8 || g.sA % 8 || g.ldb % 8 || g.sB % 8) return false;
   if (g.cn == 1) {                                   // 16-byte stores, the fused output stage reads its vector the same way
     if (!aligned(g.C, 16) || (g.bias && !aligned(g.bias, 16)) || (g.gate && (!aligned(g.gate, 16) || g.ld_gate % 8)) || (g.resid && (!aligned(g.resid, 16) || g.ld_resid % 8)) || g.ldc % 8 || g.sC % 8) return false;
-  } else if (g.bias || g.act || g.gate || g.resid) {
-    return false;                                    // interleaved columns are stored one by one, without an output stage
   }
   const int64_t lim = (int64_t)1 << 32;
   if ((int64_t)(g.M - 1) * g.lda * 2 + 64 >= lim) return false;
@@ -1177,6 +1231,7 @@ static int launch_ring(const GemmArgs& g, hipStream_t st) {
     fn = g.b_kn ? (void*)gemm_ring_kernel<T, true, BM, BN, false, SHALLOW, NWV, true> : (void*)gemm_ring_kernel<T, false, BM, BN, false, SHALLOW, NWV, true>;
   else
     fn = ep ? (g.b_kn ? (void*)gemm_ring_kernel<T, true, BM, BN, true, SHALLOW, NWV, false, BNC> : (void*)gemm_ring_kernel<T, false, BM, BN, true, SHALLOW, NWV, false, BNC>)
+            : ring_scatter_odd(g) ? (void*)gemm_ring_kernel<T, true, BM, BN, false, SHALLOW, NWV, false, BNC, true>
             : (g.b_kn ? (void*)gemm_ring_kernel<T, true, BM, BN, false, SHALLOW, NWV, false, BNC> : (void*)gemm_ring_kernel<T, false, BM, BN, false, SHALLOW, NWV, false, BNC>);
   static std::mutex mu;
   static std::set<void*> raised;
@@ -1285,7 +1340,7 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
   const bool interleaved = g.cn != 1 && g.K >= 256 && (int64_t)g.M * g.N * g.batch * 2 > (int64_t)cus * 128 * 128 && (int64_t)g.M * 8 >= cdiv(g.M, 128) * 128 * 7;
   if (mid == 1 && ring == 1 && (r128_all <= cus || g.M <= 128) && !interleaved && option_value(OPT_GEMM_RING_TILE, 0) == 0) {
     constexpr int dt = std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16;
-    const bool rk = g.cn == 1 && g.M >= 96 && g.K >= 64 && ring_ok(g), mk = gemm_mid_ok(g, dt);
+    const bool rk = g.cn == 1 && g.M >= 96 && g.K >= 64 && !ring_scatter_odd(g) && ring_ok(g), mk = gemm_mid_ok(g, dt);
     bool cut = option_value(OPT_GEMM_SPLITK, 1) != 0 && mk && g.cn == 1 && g.epi == EPI_PLAIN && g.splitk_ws && aligned(g.splitk_ws, 16) && g.batch == 1 && !g.sat8 && !g.pair &&
                g.N % 8 == 0 && aligned(g.C, 16) && g.ldc % 8 == 0 && (!g.bias || aligned(g.bias, 16)) &&     // the sum of the slices moves eight columns at a time
                (!g.gate || (aligned(g.gate, 16) && g.ld_gate % 8 == 0)) && (!g.resid || (aligned(g.resid, 16) && g.ld_resid % 8 == 0));
@@ -1355,7 +1410,7 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
       // 11008 -> 4096, whose Z U has 256 tiles, gains: 139.3 -> 134.8 us; Monarch 4096 -> 4096 / 11008 -> 4096
       // 64.9 -> 61.8 / 96.3 -> 88.8 us, side by side on one box; DiT-XL/2 with dense layers 11.67 -> 11.04 ms, with BLAST layers 11.76 -> 12.25 ms when
       // forced).  BLR_GEMM_RING_BK = 32 / 64 decides for every problem.
-      if (option_value(OPT_GEMM_RING_BK, wide64 || (g.K >= 1024 && (g.batch == 1 || t128 <= 2 * (int64_t)cus)) ? 64 : 32) == 64 && g.cn == 1) {
+      if (option_value(OPT_GEMM_RING_BK, wide64 || (g.K >= 1024 && (g.batch == 1 || t128 <= 2 * (int64_t)cus)) ? 64 : 32) == 64 && g.cn == 1 && !ring_scatter_odd(g)) {
         const bool w8 = option_value(OPT_GEMM_RING_WAVES, 8) == 8;
         if (rt == 256256) return !w8 && !g.pair ? launch_ring64<T, 256, 256, 4, 2, 1>(g, st) : launch_ring64<T, 256, 256, 8, 2, 1>(g, st);
         if (rt == 256128) return w8 ? launch_ring64<T, 256, 128, 8, 3, 1>(g, st) : launch_ring64<T, 256, 128, 4, 3, 1>(g, st);

@@ -169,6 +169,24 @@ def test_low_rank_and_monarch_through_ring_kernel(dtype, ring_forced):
     assert_close(out, ref, dtype, "monarch", scale=2.0)
 
 
+# periods (rank / b) that hold whole pieces of four columns, of two, of one, in every tile of the ring kernel; interleaved columns with bias
+# and activation; rows and columns past the last whole tile
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,p,rank,s,M", [(4, 72, 144 + 16, 96, 300), (2, 136, 20 * 8, 72, 130), (4, 64, 8 * 27, 40, 257), (8, 40, 8 * 33, 24, 140), (16, 72, 16 * 5 + 160, 200, 97)])
+def test_monarch_odd_periods_and_interleaved_output_stage(b, p, rank, s, M, dtype, ring_forced):
+    from test_gpu_monarch_lowrank_dense import _ref_monarch, _run_monarch, monarch_inputs
+    from triton_funcs import _lib as L
+    x, w1_t, w2_t = monarch_inputs(b, p, rank, s, (M,), seed=rank)
+    bias = np.random.default_rng(rank).standard_normal(b * s)
+    say(f"[case] ring monarch b={b} rank={rank} M={M} {dtype} tile {ring_forced}")
+    ref = _ref_monarch(x, w1_t, w2_t, dtype)[0]
+    assert_close(_run_monarch("triton_monarch_right_fp16", x, w1_t, w2_t, dtype, "tiled"), ref, dtype, f"monarch period {rank // b}", scale=2.0)
+    with L.fused_epilogue(dev(bias, dtype), "silu"):
+        out = _run_monarch("triton_monarch_right_fp16", x, w1_t, w2_t, dtype, "tiled")
+    v = ref + rounded(bias, dtype)
+    assert_close(out, v / (1.0 + np.exp(-v)), dtype, f"monarch period {rank // b}, bias and SiLU", scale=2.0)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,in_f,r,out_f", [(300, 2056, 136, 264), (2048, 4096, 1024, 512), (130, 1024, 64, 128), (97, 6000, 8, 72)])
 def test_low_rank_with_the_reduction_cut_into_slices(M, in_f, r, out_f, dtype):
