@@ -61,6 +61,7 @@ struct RowsParams {
                                           // weights then stay in registers and every further tile costs products and a reduction
   int per; int64_t o_ls; FastDiv perdiv;  // per > 0: Monarch scatter - column c of entry bt goes to out[(c / per) * o_ls + m * o_ms + bt * per + c % per]
                                           // (any period; the columns of one that is a multiple of 4 are stored four at a time)
+  int k_total;                            // > 0: the batch entries are slices of a reduction of this many rows, the last one shorter than K
   int npc;                                // 16-byte column pieces of a chunk (1..16)
   FastDiv nch;                            // chunks per batch entry
   uint32_t xcd_span;                      // items per XCD when the grid is a multiple of 8, else 0 (plain order)
@@ -164,7 +165,7 @@ __global__ __launch_bounds__(DR_NT) void rows_product_kernel(RowsParams p) {
   // number of lines) go to one XCD, i.e. one L2
   const uint32_t item = p.xcd_span ? (blockIdx.x & 7u) * p.xcd_span + (blockIdx.x >> 3) : blockIdx.x;
   const uint32_t bt = fd_div(item, p.nch), ch = item - bt * p.nch.d;
-  const int N = p.N, K = p.K;
+  const int N = p.N, K = p.k_total ? min(p.K, p.k_total - (int)bt * p.K) : p.K;
   const int cw = p.npc * (NK ? 16 : 8);                  // columns of a chunk
   const int col0 = (int)ch * cw;                         // first column of the chunk
   const int colp = col0 + (NK ? n : n * 8);              // first column of this lane's pieces
@@ -765,7 +766,7 @@ int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_byt
   const int enabled = option_value(OPT_DECODE_ROWS, 1);
   if (!enabled) return 1;
   const int bo = a.bo > 0 ? a.bo : a.b;
-  const int b = a.b, M = a.M, R = a.r, P = a.in_f / a.b, Q = a.out_f / bo;
+  const int b = a.b, M = a.M, R = a.r, P = a.slice > 0 ? a.slice : a.in_f / a.b, Q = a.out_f / bo;
   const bool u_nk = a.u_layout == BLR_U_QR;
   const bool monarch = a.perm_per > 0;                  // the mix is a permutation, folded into the store of the first product
   const bool lowrank = !monarch && !a.S && bo == 1;     // one output block, S = 1: the mix is the sum over the input slices
@@ -798,6 +799,7 @@ int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_byt
   s1.A = a.x; s1.lda = a.ldx; s1.a_bs = P; s1.a_bytes = (uint32_t)(x_elems * 2);
   s1.W = a.V; s1.w_bs = (int64_t)P * R;
   s1.out = Y; s1.o_ms = R; s1.o_bs = (int64_t)M * R; s1.o_ns = 1;
+  s1.k_total = a.slice > 0 ? a.in_f : 0;
   s1.M = M; s1.K = P; s1.N = R; s1.scales = a.wbits != 16 ? (const f16*)a.v_scales : nullptr;
   if (monarch && mks == 1) { s1.out = Z; s1.o_bs = 0; s1.per = a.perm_per; s1.o_ls = (int64_t)M * R; s1.perdiv = fd_make((uint32_t)a.perm_per); }
   if (mks > 1) { s1.a_bs = P / mks; s1.w_bs = (int64_t)(P / mks) * R; s1.K = P / mks; }

@@ -1313,18 +1313,21 @@ int stream_generic_launch(const StreamGenericArgs& a, hipStream_t st) {
   }
   if (a.op == 1) {                             // low rank: z = x A (in, r); out = z B (r, out)
     WsLayout w = ws_carve(a.ws, (size_t)a.M * a.r);
-    constexpr int rows_min_m = 2;
-    if (!a.split && a.M >= rows_min_m) {
-      // From two rows up: the three-launch matrix-core path, low rank being BLAST with the input cut into 16 (or 8, 4, 2) slices of
-      // rows of A, one output block and S = 1 (the mix is the sum over the slices).
-      int bi = 0;
-      for (int c = 16; c >= 2 && !bi; c >>= 1)
-        if (a.in_f % c == 0 && (a.in_f / c) % 8 == 0) bi = c;
+    int equal = 0;                           // equal slices of whole 16-byte pieces, as many as there are
+    for (int c = 16; c >= 2 && !equal; c >>= 1)
+      if (a.in_f % c == 0 && (a.in_f / c) % 8 == 0) equal = c;
+    if (!a.split && (a.M >= 2 || !equal)) {
+      // From two rows up: the three-launch matrix-core path, low rank being BLAST with the input cut into 16 (or 8) slices of
+      // rows of A, one output block and S = 1 (the mix is the sum over the slices).  Where there are fewer equal slices, or none, 16 with
+      // a shorter last one, at one row too: 3736 -> 1712, r = 376 at 1 / 4 / 16 rows 21.9 / 48.6 / 17.6
+      // us on what follows, 9.9 / 10.3 / 11.0 here; 3728 inputs (two slices) at 4 rows 15.3 -> 10.5; 920 -> 8000, r = 136 at 2 rows 25.1 -> 9.6.
+      int bi = equal >= 8 ? equal : 0, slice = 0;
+      if (!bi && a.in_f % 8 == 0) { slice = (int)cdiv(cdiv(a.in_f, 16), 8) * 8; bi = (int)cdiv(a.in_f, slice); }
       if (bi) {
         StreamBlastArgs bl = {};
         bl.x = a.x; bl.ldx = a.ldx; bl.U = a.W2; bl.V = a.W1; bl.S = nullptr; bl.out = a.out; bl.ldo = a.ldo;
         bl.M = a.M; bl.in_f = a.in_f; bl.out_f = a.out_f; bl.b = bi; bl.bo = 1; bl.r = a.r;
-        bl.dtype = a.dtype; bl.u_layout = BLR_U_RQ; bl.s_layout = BLR_S_IJR; bl.wbits = 16;
+        bl.dtype = a.dtype; bl.u_layout = BLR_U_RQ; bl.s_layout = BLR_S_IJR; bl.wbits = 16; bl.slice = slice;
         const int rc = decode_rows_launch(bl, w.plain, decode2_plain_bytes(), st);
         if (rc != 1) return rc;
       }
@@ -1345,9 +1348,7 @@ int stream_generic_launch(const StreamGenericArgs& a, hipStream_t st) {
     if (!a.split) {
       // The two-stage decode kernel sees a low-rank layer as a BLAST layer with the input cut into
       // blocks of rows of A, a single output block and S = 1.
-      int bi = 0;
-      for (int c = 16; c >= 2 && !bi; c >>= 1)
-        if (a.in_f % c == 0 && (a.in_f / c) % 8 == 0) bi = c;
+      const int bi = equal;
       if (bi) {
         StreamBlastArgs bl = {};
         bl.x = a.x; bl.ldx = a.ldx; bl.U = a.W2; bl.V = a.W1; bl.S = nullptr; bl.out = a.out; bl.ldo = a.ldo;

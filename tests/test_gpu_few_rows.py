@@ -64,6 +64,20 @@ def test_output_stage(M, act):
     assert_close(out, (rounded(resid, dtype) + rounded(gate, dtype)[np.arange(M) // rows] * v).reshape(out.shape), dtype, f"gate + residual M={M}", scale=2.0)
 
 
+# low rank whose input has no equal slices of whole pieces (odd multiples of 8), two or four of them; the last slice from 8 rows up
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M", [1, 2, 5, 16])
+@pytest.mark.parametrize("in_f,r,out_f", [(3736, 376, 1712), (3728, 72, 264), (8, 8, 8), (72, 16, 40), (1032, 200, 136), (776, 128, 3072), (4104, 1032, 520), (11000, 8, 72)])
+def test_low_rank_unequal_slices(M, in_f, r, out_f, dtype):
+    from triton_funcs import low_rank_kernels as LR
+    g = torch.Generator("cuda").manual_seed(M + in_f)
+    x = torch.randn(M, in_f, device="cuda", generator=g).to(dtype)
+    a, b = (torch.randn(in_f, r, device="cuda", generator=g) / in_f ** 0.5).to(dtype), (torch.randn(r, out_f, device="cuda", generator=g) / r ** 0.5).to(dtype)
+    say(f"[case] low rank {in_f} -> {out_f} r={r} M={M} {dtype}")
+    ref = x.double().cpu() @ a.double().cpu() @ b.double().cpu()
+    assert_close(LR.triton_low_rank_fp16(x, a, b), ref.numpy(), dtype, f"low rank {in_f} -> {out_f} M={M}", scale=2.0)
+
+
 # a few rows and a long reduction: slices on tiles of 32 rows; a wide output: more tiles than compute units
 @pytest.mark.parametrize("M,K,N", [(1, 8, 8), (1, 4104, 136), (5, 72, 1032), (16, 11008, 72), (16, 512, 33024), (17, 4104, 136), (33, 11008, 72), (95, 2056, 1032), (17, 72, 33024), (64, 512, 65536)])
 def test_dense(M, K, N):
