@@ -1541,13 +1541,13 @@ template <typename T>
 __device__ __forceinline__ void mix_stage_s(const T* __restrict__ S, T* s_t, int b, int R, int r0,
                                             int64_t s_si, int64_t s_sj, int64_t s_sr, int s_order) {
   constexpr int VW = mix_vw<T>, CH = mix_ch<T>, LDR = mix_ldr<T>;
-  struct alignas(16) V8 { T v[VW]; };
+  typedef T V8 __attribute__((ext_vector_type(VW)));
   const int tid = threadIdx.x;
   if (s_order == MIX_S_R) {                                    // (j, i, r) or (i, j, r): r contiguous
     for (int idx = tid; idx < b * b * 8; idx += 256) {
       const int r8 = (idx & 7) * VW, ji = idx >> 3;
       const int j = ji / b, i = ji - j * b;
-      V8 v = {};
+      V8 v = (T)0.0f;
       if (r0 + r8 < R) v = *reinterpret_cast<const V8*>(&S[(int64_t)i * s_si + (int64_t)j * s_sj + r0 + r8]);
       *reinterpret_cast<V8*>(&s_t[ji * LDR + r8]) = v;
     }
@@ -1555,12 +1555,12 @@ __device__ __forceinline__ void mix_stage_s(const T* __restrict__ S, T* s_t, int
     const int bb = b * b, valid = min(CH, R - r0) * bb;
     for (int idx = tid; idx < 8 * bb; idx += 256) {
       const int e0 = idx * VW;
-      V8 v = {};
+      V8 v = (T)0.0f;
       if (e0 < valid) v = *reinterpret_cast<const V8*>(&S[(int64_t)r0 * bb + e0]);
       int r = e0 / bb, ij = e0 - r * bb, i = ij / b, j = ij - i * b;
 #pragma unroll
       for (int e = 0; e < VW; ++e) {
-        s_t[(j * b + i) * LDR + r] = v.v[e];
+        s_t[(j * b + i) * LDR + r] = v[e];
         if (++j == b) { j = 0; if (++i == b) { i = 0; ++r; } }
       }
     }
@@ -1584,7 +1584,7 @@ __global__ __launch_bounds__(256) void blast_mix_vec_kernel(const T* __restrict_
                                                             T* __restrict__ Z, int M, int b, int R,
                                                             int64_t s_si, int64_t s_sj, int64_t s_sr, int m_per_wg, int s_order, int sat8) {
   constexpr int VW = mix_vw<T>, LDR = mix_ldr<T>;
-  struct alignas(16) V8 { T v[VW]; };
+  typedef T V8 __attribute__((ext_vector_type(VW)));
   extern __shared__ float s_lds[];
   T* s_t = reinterpret_cast<T*>(s_lds);      // [b][b][chunk]  (j, i, r)
   const int tid = threadIdx.x;
@@ -1610,12 +1610,12 @@ __global__ __launch_bounds__(256) void blast_mix_vec_kernel(const T* __restrict_
         if (j < b) {
           const V8 sv = *reinterpret_cast<const V8*>(&s_t[(j * b + i) * LDR + rl * VW]);
 #pragma unroll
-          for (int e = 0; e < VW; ++e) acc[e] = fmaf(TypeTraits<T>::to_f32(sv.v[e]), TypeTraits<T>::to_f32(yv[j].v[e]), acc[e]);
+          for (int e = 0; e < VW; ++e) acc[e] = fmaf(TypeTraits<T>::to_f32(sv[e]), TypeTraits<T>::to_f32(yv[j][e]), acc[e]);
         }
       }
       V8 o;
 #pragma unroll
-      for (int e = 0; e < VW; ++e) o.v[e] = TypeTraits<T>::from_f32(sat8 ? sat8_rne(acc[e]) : acc[e]);
+      for (int e = 0; e < VW; ++e) o[e] = TypeTraits<T>::from_f32(sat8 ? sat8_rne(acc[e]) : acc[e]);
       *reinterpret_cast<V8*>(&Z[((int64_t)i * M + m) * R + r]) = o;
     }
   }
