@@ -16,6 +16,12 @@
 //            the layout of the bmm names; any other layout is transposed once per call into scratch by a small kernel.
 //            A wave takes 16 ranks of the tile, keeps the products of eight ranks in registers and stores 16 bytes of
 //            Z per (i, m).  Z leaves as T.
+// Phase 1 is bound by the address path (60 loads a wave at 72 columns per block), phase 2 by LDS and by the rate at which the chip
+// takes Z, and Y leaves no LDS for a second workgroup.  So with more tiles than compute units a workgroup walks several (WALK): the next
+// tile's first step is asked for before this one is mixed, the stores of Z drain under the next phase 1, and S is loaded once per
+// rank tile.  4096 rows, fp16, 16 blocks of 72, r = 576 and 288, mean of the two: 41.5 -> 37.5 us; whole calls 1152 -> 4608 79.9 -> 76.6,
+// 1152 -> 3456 47.8 -> 45.7, 1024 -> 8192 with r = 512 99.4 -> 83, 512 -> 4096 in 8 blocks with r = 1024 at 2000 rows 42.2 -> 40.
+// With one tile each there is nothing to walk, and the addresses kept for it cost 2 %: a kernel of its own.
 // What follows is an ordinary batched GEMM out_i = Z_i U_i.
 #include <hip/hip_runtime.h>
 #include <cmath>
@@ -46,6 +52,7 @@ struct YmixParams {
   int npc;                      // 16-byte rank pieces of a tile (1..16): the tile spans BR = 8 npc ranks
   int ksteps;                   // 32-row k-steps that cover P
   FastDiv nmt;                  // row tiles
+  int items;                    // rank tiles x row tiles
   const void* St;               // S as (r, i, j), the input block contiguous
 };
 
@@ -75,19 +82,27 @@ __device__ __forceinline__ uint32_t ym_pack(float lo, float hi) {
   return __builtin_bit_cast(u32x2, v)[0];
 }
 
-template <typename T, bool STAGE>
+// a barrier that orders LDS and leaves loads and stores of memory in flight
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <typename T, bool STAGE, bool WALK>
 __global__ __launch_bounds__(YM_NT) void blast_ymix_kernel(YmixParams p) {
   extern __shared__ __attribute__((aligned(16))) uint32_t ym_lds[];
-  const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, n = l & 15, g = l >> 4;
+  int tid = threadIdx.x;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int n = tid & 15, g = (tid >> 4) & 3;
   const int b = p.b, P = p.P, R = p.R, M = p.M, BR = p.npc * 8, JP = b >> 1;
   // Y pairs (Y_2jp, Y_2jp+1) as [jp][m][r]: rows padded by 4 dwords and input-block planes by 16, so that the 16-byte
   // writes of phase 1 stay aligned and the reads of phase 2 (16 rows x 4 planes of one rank) spread over the banks
   const int RS = BR + 4, JS = YM_BM * RS + 16;
   uint32_t* y_s = ym_lds;
-  // workgroups of one rank tile follow each other within an XCD: its slice of V stays in that L2 while the rows stream
-  const uint32_t item = xcd_item(blockIdx.x, gridDim.x);
-  const uint32_t rt = fd_div(item, p.nmt), mt = item - rt * p.nmt.d;
-  const int m0 = (int)mt * YM_BM, r0 = (int)rt * BR;
+  // A workgroup walks a run of tiles.  Tiles of one rank tile follow each other, within a run and within an XCD: its slice of V stays in
+  // that L2 while the rows stream, and S in the registers.
+  const uint32_t wg = xcd_item(blockIdx.x, gridDim.x), G = gridDim.x;
+  uint32_t item = (uint32_t)((uint64_t)wg * (uint32_t)p.items / G);
+  const uint32_t item_end = (uint32_t)((uint64_t)(wg + 1) * (uint32_t)p.items / G);
+  uint32_t rt = fd_div(item, p.nmt);
+  int m0 = (int)(item - rt * p.nmt.d) * YM_BM, r0 = (int)rt * BR;
   TR6(0);
   // the mix's S operands depend on nothing and are used after phase 1: asked for behind the first loads of phase 1 (the
   // memory pipeline takes an instruction every 16 cycles, and the products can only start on those first loads).  Lane (n, g)
@@ -110,164 +125,179 @@ __global__ __launch_bounds__(YM_NT) void blast_ymix_kernel(YmixParams p) {
   // ---------------------------------------------- phase 1: Y pairs into LDS ----------------------------------------------
   // One pipeline over the k-steps of the wave's two input blocks (no drain between them): step q < KS belongs to block
   // 2 wv, step q >= KS to block 2 wv + 1; the accumulators of the first block are packed away at the boundary.
-  if (wv < JP) {
-    const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, p.x_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t vbuf = wbuf(reinterpret_cast<const T*>(p.V) + (int64_t)(2 * wv) * P * R, (uint32_t)((int64_t)2 * P * R * 2));
-    const bool live = n < p.npc && r0 + n * 8 < R;
-    const int KS = p.ksteps;                                // 32-row steps per input block
-    uint32_t h0[2][4][4];                                   // Y of the wave's first input block, packed two ranks to a dword
-    f32x4 acc[2][8];
+  // step s of a block covers k = 32 s .. 32 s + 31; this lane holds k = 32 s + 8 g .. + 7 of row 16 mg + n (x) and of its
+  // rank piece (V).  No branch around the loads (the compiler then waits for exactly the step it needs): what lies
+  // outside - rows past M, k past P, lanes without a rank piece - asks for an offset out of bounds and reads zeros.
+  const int KS = p.ksteps;                                   // 32-row steps per input block
+  const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, p.x_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t vbuf = wbuf(reinterpret_cast<const T*>(p.V) + (int64_t)(2 * (wv < JP ? wv : 0)) * P * R, (uint32_t)((int64_t)2 * P * R * 2));
+  u32x4 a0[2], a1[2], b0[8], b1[8];
+  auto load_ab = [&](u32x4 (&a)[2], u32x4 (&bb)[8], int q) {
+    const int jj = q >= KS ? 1 : 0, sst = q - jj * KS;
+    const int k = 32 * sst + 8 * g;
+    const bool kin = k < P, live = n < p.npc && r0 + n * 8 < R;
 #pragma unroll
-    for (int mg = 0; mg < 2; ++mg)
+    for (int mg = 0; mg < 2; ++mg) {
+      const int m = m0 + 16 * mg + n;
+      const uint32_t off = (m < M && kin) ? (uint32_t)((int64_t)m * p.ldx + (int64_t)(2 * wv + jj) * P + k) * 2u : YM_OOB;
+      a[mg] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, off, 0, 0));
+    }
+    const uint32_t base = (live && kin) ? (uint32_t)((jj * P + k) * R + r0 + n * 8) * 2u : YM_OOB;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[mg][e] = f32x4{0.f, 0.f, 0.f, 0.f};
-    u32x4 a0[2], a1[2], b0[8], b1[8];
-    // step s of a block covers k = 32 s .. 32 s + 31; this lane holds k = 32 s + 8 g .. + 7 of row 16 mg + n (x) and of its
-    // rank piece (V).  No branch around the loads (the compiler then waits for exactly the step it needs): what lies
-    // outside - rows past M, k past P, lanes without a rank piece, steps past the second block - asks for an offset out
-    // of bounds and reads zeros.
-    auto load_ab = [&](u32x4 (&a)[2], u32x4 (&bb)[8], int q) {
-      const int jj = q >= KS ? 1 : 0, sst = q - jj * KS;
-      const int k = 32 * sst + 8 * g;
-      const bool kin = k < P && q < 2 * KS;
-#pragma unroll
-      for (int mg = 0; mg < 2; ++mg) {
-        const int m = m0 + 16 * mg + n;
-        const uint32_t off = (m < M && kin) ? (uint32_t)((int64_t)m * p.ldx + (int64_t)(2 * wv + jj) * P + k) * 2u : YM_OOB;
-        a[mg] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, off, 0, 0));
-      }
-      const uint32_t base = (live && kin) ? (uint32_t)((jj * P + k) * R + r0 + n * 8) * 2u : YM_OOB;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) bb[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vbuf, base + (uint32_t)(t * R) * 2u, 0, 0));
-    };
-    auto step = [&](const u32x4 (&a)[2], const u32x4 (&bb)[8]) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
-        u32x4 bv;
-#pragma unroll
-        for (int h = 0; h < 4; ++h) bv[h] = __builtin_amdgcn_perm(bb[2 * h + 1][e >> 1], bb[2 * h][e >> 1], sel);
-#pragma unroll
-        for (int mg = 0; mg < 2; ++mg) acc[mg][e] = YmDot<T>::mfma(a[mg], bv, acc[mg][e]);
-      }
-    };
-    auto next_block = [&]() {                                // pack away the first block's Y, start the second from zero
-#pragma unroll
-      for (int mg = 0; mg < 2; ++mg)
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) h0[mg][t][q] = ym_pack<T>(acc[mg][2 * q][t], acc[mg][2 * q + 1][t]);
+    for (int t = 0; t < 8; ++t) bb[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vbuf, base + (uint32_t)(t * R) * 2u, 0, 0));
+  };
+  if (wv < JP) load_ab(a0, b0, 0);
+  load_sa();
+  TR6(1);
+  for (;;) {
+    if (WALK) asm volatile("" : "+v"(tid), "+v"(n), "+v"(g));         // addresses are formed again for each tile: kept, they would not fit beside the operands
+    if (wv < JP) {
+      uint32_t h0[2][4][4];                                   // Y of the wave's first input block, packed two ranks to a dword
+      f32x4 acc[2][8];
 #pragma unroll
       for (int mg = 0; mg < 2; ++mg)
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[mg][e] = f32x4{0.f, 0.f, 0.f, 0.f};
-    };
-    load_ab(a0, b0, 0);
-    load_sa();
-    TR6(1);
-    int q = 0;
-    for (; q + 2 < 2 * KS; q += 2) {                         // two steps per trip (the two register sets take turns)
+      auto step = [&](const u32x4 (&a)[2], const u32x4 (&bb)[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+          u32x4 bv;
+#pragma unroll
+          for (int h = 0; h < 4; ++h) bv[h] = __builtin_amdgcn_perm(bb[2 * h + 1][e >> 1], bb[2 * h][e >> 1], sel);
+#pragma unroll
+          for (int mg = 0; mg < 2; ++mg) acc[mg][e] = YmDot<T>::mfma(a[mg], bv, acc[mg][e]);
+        }
+      };
+      auto next_block = [&]() {                                // pack away the first block's Y, start the second from zero
+#pragma unroll
+        for (int mg = 0; mg < 2; ++mg)
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) h0[mg][t][q] = ym_pack<T>(acc[mg][2 * q][t], acc[mg][2 * q + 1][t]);
+#pragma unroll
+        for (int mg = 0; mg < 2; ++mg)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[mg][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+      };
+      int q = 0;
+      for (; q + 2 < 2 * KS; q += 2) {                         // two steps per trip (the two register sets take turns)
+        if (q == KS) next_block();
+        load_ab(a1, b1, q + 1);
+        step(a0, b0);
+        if (q + 1 == KS) next_block();
+        load_ab(a0, b0, q + 2);
+        step(a1, b1);
+      }
+      // the last trip on its own: nothing is left to ask for behind it (ten loads that would all be out of bounds still cost
+      // their turns in the memory pipeline)
       if (q == KS) next_block();
       load_ab(a1, b1, q + 1);
       step(a0, b0);
       if (q + 1 == KS) next_block();
-      load_ab(a0, b0, q + 2);
       step(a1, b1);
-    }
-    // the last trip on its own: nothing is left to ask for behind it (ten loads that would all be out of bounds still cost
-    // their turns in the memory pipeline)
-    if (q == KS) next_block();
-    load_ab(a1, b1, q + 1);
-    step(a0, b0);
-    if (q + 1 == KS) next_block();
-    step(a1, b1);
-    TR6(2);
-    // acc[mg][e][t] is Y of block 2 wv + 1 at [m0 + 16 mg + 4 g + t][r0 + 8 n + e]; h0 holds block 2 wv
-    if (n < p.npc) {
+      TR6(2);
+      // acc[mg][e][t] is Y of block 2 wv + 1 at [m0 + 16 mg + 4 g + t][r0 + 8 n + e]; h0 holds block 2 wv
+      if (n < p.npc) {
 #pragma unroll
-      for (int mg = 0; mg < 2; ++mg)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          uint32_t pr[8];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const uint32_t h1 = ym_pack<T>(acc[mg][2 * q][t], acc[mg][2 * q + 1][t]);
-            pr[2 * q] = __builtin_amdgcn_perm(h1, h0[mg][t][q], 0x05040100u);          // rank 8 n + 2 q:     (Y_2w, Y_2w+1)
-            pr[2 * q + 1] = __builtin_amdgcn_perm(h1, h0[mg][t][q], 0x07060302u);      // rank 8 n + 2 q + 1
-          }
-          uint32_t* dst = &y_s[wv * JS + (16 * mg + 4 * g + t) * RS + n * 8];
-          *reinterpret_cast<u32x4*>(dst) = u32x4{pr[0], pr[1], pr[2], pr[3]};
-          *reinterpret_cast<u32x4*>(dst + 4) = u32x4{pr[4], pr[5], pr[6], pr[7]};
-        }
-    }
-  } else {
-    load_sa();
-  }
-  TR6(3);
-  __syncthreads();
-  TR6(4);
-
-  // ---------------------------------------------- phase 2: the mix ----------------------------------------------------------
-  // lane (n, g): operand A = S_r(i = n, j = 4 g .. 4 g + 3), operand B = Y_r(j = 4 g .. 4 g + 3, m = 16 mg + n); the
-  // product's lane holds Z_r(i = 4 g + t, m = 16 mg + n), t = 0..3
-  // A lane's 16 bytes of Z belong to a row (i, m) of their own: stored from here, an instruction touches 64 cache lines and
-  // holds the memory pipeline eight times as long as one that writes whole rows (5.3 of a workgroup's 15 us were these
-  // stores).  STAGE: the 16 rows of a product group go through LDS behind Y ([i][m][rank], 16 lanes per row) and leave as
-  // runs of BR ranks; without (the tile's Y leaves no room for that) the lanes store their pieces themselves.
-  const bool b_ok = 2 * g < JP;
-  const int ZRS = BR / 2 + 4;                                // dwords per staged row
-  uint32_t* const z_st = ym_lds + JP * JS;
-#pragma unroll
-  for (int mg = 0; mg < 2; ++mg) {
-    if (STAGE && mg == 1) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // the first group's rows have been read
-    if (rw < BR) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {                          // eight ranks at a time
-        if (rw + 8 * h < BR) {
-          f32x4 d[8];
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            const int rr = rw + 8 * h + q;
-            u32x2 yb = {0u, 0u};
-            if (b_ok) {
-              const uint32_t* src = &y_s[(2 * g) * JS + (16 * mg + n) * RS + rr];
-              yb[0] = src[0]; yb[1] = src[JS];
-            }
-            d[q] = YmDot<T>::mfma16(sa[8 * h + q], yb, f32x4{0.f, 0.f, 0.f, 0.f});
-          }
-          const int m = m0 + 16 * mg + n, r = r0 + rw + 8 * h;
+        for (int mg = 0; mg < 2; ++mg)
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
-            const int i = 4 * g + t;
-            u32x4 o;
+            uint32_t pr[8];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) o[q] = ym_pack<T>(d[2 * q][t], d[2 * q + 1][t]);
-            if (STAGE) {
-              if (i < b) *reinterpret_cast<u32x4*>(&z_st[(i * 16 + n) * ZRS + (rw + 8 * h) / 2]) = o;
-            } else if (m < M && r < R && i < b) {
-              *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.Z) + ((int64_t)i * M + m) * R + r) = o;
+            for (int q = 0; q < 4; ++q) {
+              const uint32_t h1 = ym_pack<T>(acc[mg][2 * q][t], acc[mg][2 * q + 1][t]);
+              pr[2 * q] = __builtin_amdgcn_perm(h1, h0[mg][t][q], 0x05040100u);          // rank 8 n + 2 q:     (Y_2w, Y_2w+1)
+              pr[2 * q + 1] = __builtin_amdgcn_perm(h1, h0[mg][t][q], 0x07060302u);      // rank 8 n + 2 q + 1
+            }
+            uint32_t* dst = &y_s[wv * JS + (16 * mg + 4 * g + t) * RS + n * 8];
+            *reinterpret_cast<u32x4*>(dst) = u32x4{pr[0], pr[1], pr[2], pr[3]};
+            *reinterpret_cast<u32x4*>(dst + 4) = u32x4{pr[4], pr[5], pr[6], pr[7]};
+          }
+      }
+    }
+    TR6(3);
+    // the next tile's first step flies while this one is mixed and stored: phase 1 is bound by the address path, phase 2 by LDS and by
+    // the chip's write rate, and one workgroup's LDS leaves no room for a second one whose phases would fill the gaps
+    const int mt0 = m0, rt0 = r0;                              // this tile's origin
+    const bool more = WALK && ++item < item_end;
+    const uint32_t rt_next = more ? fd_div(item, p.nmt) : rt;
+#pragma unroll
+    for (int q = 0; WALK && q < 16; ++q) asm volatile("" : "+v"(sa[q]));    // S has arrived by now: said here, or the products of phase 2 wait for the next tile's loads with it
+    if (more) {
+      m0 = (int)(item - rt_next * p.nmt.d) * YM_BM;
+      r0 = (int)rt_next * BR;
+      if (wv < JP) load_ab(a0, b0, 0);
+    }
+    lds_barrier();
+    TR6(4);
+
+    // ---------------------------------------------- phase 2: the mix ----------------------------------------------------------
+    // lane (n, g): operand A = S_r(i = n, j = 4 g .. 4 g + 3), operand B = Y_r(j = 4 g .. 4 g + 3, m = 16 mg + n); the
+    // product's lane holds Z_r(i = 4 g + t, m = 16 mg + n), t = 0..3
+    // A lane's 16 bytes of Z belong to a row (i, m) of their own: stored from here, an instruction touches 64 cache lines and
+    // holds the memory pipeline eight times as long as one that writes whole rows (5.3 of a workgroup's 15 us were these
+    // stores).  STAGE: the 16 rows of a product group go through LDS behind Y ([i][m][rank], 16 lanes per row) and leave as
+    // runs of BR ranks; without (the tile's Y leaves no room for that) the lanes store their pieces themselves.
+    const bool b_ok = 2 * g < JP;
+    const int ZRS = BR / 2 + 4;                                // dwords per staged row
+    uint32_t* const z_st = ym_lds + JP * JS;
+#pragma unroll
+    for (int mg = 0; mg < 2; ++mg) {
+      if (STAGE && mg == 1) lds_barrier();     // the first group's rows have been read
+      if (rw < BR) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {                          // eight ranks at a time
+          if (rw + 8 * h < BR) {
+            f32x4 d[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+              const int rr = rw + 8 * h + q;
+              u32x2 yb = {0u, 0u};
+              if (b_ok) {
+                const uint32_t* src = &y_s[(2 * g) * JS + (16 * mg + n) * RS + rr];
+                yb[0] = src[0]; yb[1] = src[JS];
+              }
+              d[q] = YmDot<T>::mfma16(sa[8 * h + q], yb, f32x4{0.f, 0.f, 0.f, 0.f});
+            }
+            const int m = mt0 + 16 * mg + n, r = rt0 + rw + 8 * h;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              const int i = 4 * g + t;
+              u32x4 o;
+#pragma unroll
+              for (int q = 0; q < 4; ++q) o[q] = ym_pack<T>(d[2 * q][t], d[2 * q + 1][t]);
+              if (STAGE) {
+                if (i < b) *reinterpret_cast<u32x4*>(&z_st[(i * 16 + n) * ZRS + (rw + 8 * h) / 2]) = o;
+              } else if (m < M && r < R && i < b) {
+                *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.Z) + ((int64_t)i * M + m) * R + r) = o;
+              }
             }
           }
         }
       }
-    }
-    if (STAGE) {
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      const int pc = tid & 15, r = r0 + pc * 8;
-      if (pc < p.npc && r < R) {                           // 32 rows per pass: output blocks 2 it, 2 it + 1
-        const int rr = tid >> 4, m = m0 + 16 * mg + (rr & 15);
-        u32x4 v[8];
-#pragma unroll
-        for (int it = 0; it < 8; ++it)
-          if (2 * it < b) v[it] = *reinterpret_cast<const u32x4*>(&z_st[(rr + 32 * it) * ZRS + pc * 4]);
-        if (m < M) {
+      if (STAGE) {
+        lds_barrier();
+        const int pc = tid & 15, r = rt0 + pc * 8;
+        if (pc < p.npc && r < R) {                           // 32 rows per pass: output blocks 2 it, 2 it + 1
+          const int rr = tid >> 4, m = mt0 + 16 * mg + (rr & 15);
+          u32x4 v[8];
 #pragma unroll
           for (int it = 0; it < 8; ++it)
-            if (2 * it + (rr >> 4) < b) *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.Z) + ((int64_t)(2 * it + (rr >> 4)) * M + m) * R + r) = v[it];
+            if (2 * it < b) v[it] = *reinterpret_cast<const u32x4*>(&z_st[(rr + 32 * it) * ZRS + pc * 4]);
+          if (m < M) {
+#pragma unroll
+            for (int it = 0; it < 8; ++it)
+              if (2 * it + (rr >> 4) < b) *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.Z) + ((int64_t)(2 * it + (rr >> 4)) * M + m) * R + r) = v[it];
+          }
         }
       }
     }
+    if (!more) break;
+    // Y is free for the next tile: its last reads lie before the barrier in front of the last stores (STAGE), or before this one
+    if (!STAGE) lds_barrier();
+    if (rt_next != rt) { rt = rt_next; load_sa(); }
   }
   TR6(14);
 }
@@ -297,22 +327,27 @@ int blast_ymix_launch(const void* x, int64_t ldx, const void* V, const void* S, 
   YmixParams p = {};
   p.x = x; p.ldx = ldx; p.x_bytes = (uint32_t)(x_elems * 2); p.V = V; p.S = S; p.Z = Z;
   p.M = M; p.b = b; p.P = P; p.R = R;
-  // Rank pieces per tile.  One workgroup per compute unit at a time; a workgroup takes about 10 + 0.85 npc us at 72-column input
-  // blocks, i.e. 12 + npc units, and a last round that is not full costs about half of what it leaves empty.  Measured at 4096
-  // rows, r = 576: 15 pieces = 640 workgroups (2.5 rounds) 68 us, 12 = 768 (3 rounds) 60 us, 9 = 1024 (4 rounds) 72 us; r = 288:
-  // 12 pieces = 384 (1.5 rounds) 34.8 us, 9 = 512 (2 rounds) 36.2 us.
+  // Rank pieces per tile.  One workgroup per compute unit at a time.  A tile costs about 27 + npc units of 0.33 us, a third more where Z's rows
+  // do not fit LDS behind Y and 4 % more where its runs of Z end inside 64 bytes; a last round that is not full costs about half of what it
+  // leaves empty, the first one all of it.  Measured over 6 to 16 pieces, whole calls, at 4096 rows: 1152 -> 4608, r = 576: 6 / 8 / 9 / 11 / 12 / 13 / 16
+  // pieces (6 / 4.5 / 4 / 3.5 / 3 / 3 / 2.5 rounds) 104 / 90 / 88 / 90 / 78 / 93 / 86 us; 1152 -> 3456, r = 288: 6 / 9 / 12 / 13 / 16
+  // (3 / 2 / 1.5 / 1.5 / 1.5) 56 / 49 / 46 / 52 / 53; 768 -> 3072, r = 1000: 8 / 12 / 14 / 16 pieces 116 / 112 / 121 / 118.
   const int pieces = R / 8;
   const int cus = device_cus() > 0 ? device_cus() : 256;
+  const auto lds_y_of = [&](int npc) { return (size_t)(b / 2) * (YM_BM * (npc * 8 + 4) + 16) * 4; };
+  const auto lds_z_of = [&](int npc) { return (size_t)b * 16 * (npc * 4 + 4) * 4; };      // the rows of one product group on their way out
+  const auto staged = [&](int npc) { return lds_y_of(npc) + lds_z_of(npc) <= 160 * 1024; };
   int best_npc = 16; double best_cost = -1.0;
   for (int npc = 16; npc >= 4; --npc) {
     const double x = (double)(cdiv(pieces, npc) * cdiv(M, YM_BM)) / cus;
-    const double cost = 0.5 * (std::ceil(x) + x) * (12 + npc);
+    const double cost = (x <= 1.0 ? 1.0 : 0.5 * (std::ceil(x) + x)) * (27 + npc) * (staged(npc) ? 1.0 : 1.35) * (npc % 4 ? 1.04 : 1.0);
     if (best_cost < 0 || cost < best_cost - 1e-9) { best_cost = cost; best_npc = npc; }
   }
   p.npc = best_npc;
   const int nrt = (int)cdiv(pieces, p.npc), nmt = (int)cdiv(M, YM_BM);
   if ((int64_t)nrt * nmt >= 65536 || nmt >= 65536) return 1;
   p.nmt = fd_make((uint32_t)nmt);
+  p.items = nrt * nmt;
   p.ksteps = (int)cdiv(P, 32);
   if (s_layout == BLR_S_RIJ && aligned(S, 8)) {
     p.St = S;
@@ -324,22 +359,22 @@ int blast_ymix_launch(const void* x, int64_t ldx, const void* V, const void* S, 
     BLR_CHECK_LAUNCH("ym_s_transpose");
     p.St = scratch;
   }
-  const int BR = p.npc * 8;
-  const size_t lds_y = (size_t)(b / 2) * (YM_BM * (BR + 4) + 16) * 4;
-  const size_t lds_z = (size_t)b * 16 * (BR / 2 + 4) * 4;                 // the rows of one product group on their way out
-  const bool stage = lds_y + lds_z <= 160 * 1024;
-  const size_t lds = lds_y + (stage ? lds_z : 0);
-  const int fi = (dtype == BLR_F16 ? 0 : 2) + (stage ? 1 : 0);
-  void* const fns[4] = {(void*)blast_ymix_kernel<f16, false>, (void*)blast_ymix_kernel<f16, true>,
-                        (void*)blast_ymix_kernel<bf16, false>, (void*)blast_ymix_kernel<bf16, true>};
-  static bool attr_set[4] = {false, false, false, false};
+  const bool stage = staged(p.npc);
+  const size_t lds = lds_y_of(p.npc) + (stage ? lds_z_of(p.npc) : 0);
+  const bool walk = p.items > cus;
+  const int fi = (dtype == BLR_F16 ? 0 : 4) + (stage ? 2 : 0) + (walk ? 1 : 0);
+  void* const fns[8] = {(void*)blast_ymix_kernel<f16, false, false>, (void*)blast_ymix_kernel<f16, false, true>,
+                        (void*)blast_ymix_kernel<f16, true, false>, (void*)blast_ymix_kernel<f16, true, true>,
+                        (void*)blast_ymix_kernel<bf16, false, false>, (void*)blast_ymix_kernel<bf16, false, true>,
+                        (void*)blast_ymix_kernel<bf16, true, false>, (void*)blast_ymix_kernel<bf16, true, true>};
+  static bool attr_set[8] = {};
   if (!attr_set[fi]) {
     hipError_t e = hipFuncSetAttribute(fns[fi], hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (e != hipSuccess) { set_error("blast_ymix: cannot raise the LDS limit: %s", hipGetErrorString(e)); return BLR_ERR_LAUNCH; }
     attr_set[fi] = true;
   }
   void* args[] = {&p};
-  hipError_t e = hipLaunchKernel(fns[fi], dim3((unsigned)(nrt * nmt)), dim3(YM_NT), args, lds, st);
+  hipError_t e = hipLaunchKernel(fns[fi], dim3((unsigned)(walk ? cus : p.items)), dim3(YM_NT), args, lds, st);
   if (e != hipSuccess) { set_error("blast_ymix: launch failed: %s", hipGetErrorString(e)); return BLR_ERR_LAUNCH; }
   return BLR_OK;
 }

@@ -115,6 +115,24 @@ def test_blast_fused_algorithm(name, shape, dtype):
     assert_close(out, back(tiled), dtype, f"fused against tiled {name}")
 
 
+# more tiles of the fused first half than compute units, so that a workgroup walks several: runs that go from one rank tile to the next, a last
+# tile with few rows and few ranks, one to four 32-column steps, four to sixteen blocks; 128 ranks at 16 blocks (Z's rows do not fit LDS behind Y)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,p,r,M", [(16, 72, 576, 4101), (16, 72, 296, 2990), (16, 8, 128, 12001), (4, 40, 136, 9001), (12, 32, 200, 5000), (8, 128, 1024, 1500)])
+def test_blast_fused_first_half_walks(b, p, r, M, dtype):
+    from triton_funcs import blast_kernels as K
+    q = 96
+    say(f"[case] fused walk b={b} p={p} r={r} M={M} {dtype}")
+    g = torch.Generator("cuda").manual_seed(M)
+    x, U, V, S = (torch.randn(s, device="cuda", generator=g).mul_(f).to(dtype) for s, f in
+                  (((M, b * p), 1.0), ((b, q, r), r ** -0.5), ((b, p, r), r ** -0.5), ((r, b, b), 1.0)))
+    Y = torch.bmm(x.double().view(M, b, p).transpose(0, 1).contiguous(), V.double())
+    out = K.triton_blast_bmm_fp16(x, U, V, S, {"algo": ALGO["fused"]})
+    for i in range(b):
+        ref = (Y * S[:, i].double().t()[:, None]).sum(0) @ U[i].double().t().contiguous()
+        assert_close(out.view(M, b, q)[:, i].contiguous(), ref.cpu().numpy(), dtype, f"fused walk, output block {i}")
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_bmm_fp16"])
 @pytest.mark.parametrize("shape", [(16, 256, 256, 512, (1100,)), (16, 192, 88, 256, (8, 130))])
