@@ -58,8 +58,11 @@ __device__ __forceinline__ float sat8_rne(float v) { return fminf(fmaxf(rintf(v)
 // Activation of the fused output stage (blr_act): GELU with the tanh approximation (what the reference's DiT uses,
 // DiT/models.py:111: approx_gelu = nn.GELU(approximate="tanh")) or SiLU (Llama's gate).
 __device__ __forceinline__ float apply_act(float v, int act) {
-  // 0.5 v (1 + tanh u) = v / (1 + exp(-2u)), u = sqrt(2/pi) (v + 0.044715 v^3): one exponential and one reciprocal
-  if (act == BLR_ACT_GELU_TANH) return v * __builtin_amdgcn_rcpf(1.0f + __expf(-1.5957691216057308f * (v + 0.044715f * v * v * v)));
+  // 0.5 v (1 + tanh u) = v / (1 + 2^(-2 log2(e) u)), u = sqrt(2/pi) (v + 0.044715 v^3): one exponential and one reciprocal, and the
+  // constants folded so that its argument takes three instructions (v v, one multiply-add, v times that) instead of five: 1576 x 3072 x 768 in
+  // 3 blocks with bias and GELU 20.4 -> 20.0 us; largest relative error against 64 bits 1.3e-5 -> 0.9e-5
+  constexpr double k = -1.5957691216057308 * 1.4426950408889634;
+  if (act == BLR_ACT_GELU_TANH) return v * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(v * fmaf(v * v, (float)(0.044715 * k), (float)k)));
   if (act == BLR_ACT_SILU) return v * __builtin_amdgcn_rcpf(1.0f + __expf(-v));
   return v;
 }
