@@ -246,6 +246,7 @@ struct StreamBlastArgs {
   int M, in_f, out_f, b, r;
   int bo;                                       // output blocks when they differ from b (0: same); S may then be null (all ones)
   int slice;                                    // > 0: low rank - input blocks of this many rows, the last one what is left of in_f (which b need not divide)
+  int z_f32;                                    // low rank and Monarch at up to four rows: the intermediate stays in fp32 on the skinny products too
   int perm_per;                                 // > 0: Monarch - the mix is the permutation with this period, S is unused
   int64_t out_bs, out_ns;                       // output strides of (block, column); out_ns == 0: blocked (bs = q, ns = 1)
   int dtype, u_layout, s_layout;

@@ -26,7 +26,7 @@ int decode3_blast_launch(const StreamBlastArgs& a, void* region, unsigned* epoch
 int decode_pair_launch(const StreamBlastArgs& a, void* region, size_t region_bytes, hipStream_t st);
 
 // The same call as three launches - y = x V and out = z U on the matrix cores with the rank-space mix between them
-// (blr_decode_rows.hip; up to 16 token rows, with codes up to 128 in tiles of 16).  region: scratch for y and z as T.  Same
+// (blr_decode_rows.hip; up to 16 token rows, with codes up to 128 in tiles of 16).  region: scratch for y and z (as T; z in fp32 where z_f32 asks for it).  Same
 // return convention.
 int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_bytes, hipStream_t st);
 

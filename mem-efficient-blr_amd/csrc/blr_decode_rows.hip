@@ -51,8 +51,8 @@ struct RowsParams {
   const void* bias; int act;              // fused output stage (bias of T indexed like a row of out, or null; blr_act), applied to
                                           // the result rounded to T - what a separate elementwise kernel would see
   int ep;
-  int out_f32;                            // the product is one slice of a reduction: out holds fp32 partial sums (plain row-major
-                                          // store, no scales, no output stage) that the next launch adds in slice order
+  int out_f32;                            // out is fp32 (no scales, no output stage): slices of a reduction that the next launch adds in slice
+                                          // order, or the intermediate of a call that keeps it in fp32 (rows_product_f32_kernel)
   const f16* scales;                      // codes: the product's column n of entry bt is multiplied by scales[bt * N + n]; else null
   int M, K, N;
   int kw;                                 // rows of a wave's share per round (a multiple of 32)
@@ -149,6 +149,60 @@ template <typename T> struct RowsPiece<T, 4> {
     }
   }
 };
+
+// Four neighbouring columns of a product, sums over all rows of the weights, on their way out: scales of codes, output stage, store
+// (N is a multiple of 8 and col of 4: the four columns are all inside or all outside).
+template <typename OT>
+__device__ __forceinline__ void rows_store(const RowsParams& p, const f32x4& tot, int bt, int row, int col) {
+  typedef OT vec4 __attribute__((ext_vector_type(4)));
+  OT* o = reinterpret_cast<OT*>(p.out) + (int64_t)row * p.o_ms + (int64_t)bt * p.o_bs;
+  int ocol = col;
+  if (p.per & 3) {                                       // a period that cuts through the four columns: each goes to its own place
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t l = fd_div((uint32_t)(col + e), p.perdiv);
+      reinterpret_cast<OT*>(p.out)[(int64_t)l * p.o_ls + (int64_t)row * p.o_ms + (int64_t)bt * p.per + (col + e - (int)l * p.per)] = TypeTraits<OT>::from_f32(tot[e]);
+    }
+    return;
+  }
+  if (p.per > 0) {
+    const uint32_t l = fd_div((uint32_t)col, p.perdiv);
+    o = reinterpret_cast<OT*>(p.out) + (int64_t)l * p.o_ls + (int64_t)row * p.o_ms + (int64_t)bt * p.per;
+    ocol = col - (int)l * p.per;
+  }
+  if (p.o_ns == 1 && col + 3 < p.N && ((reinterpret_cast<uintptr_t>(o + ocol) & (4 * sizeof(OT) - 1)) == 0)) {
+    vec4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = TypeTraits<OT>::from_f32(tot[e]);
+    *reinterpret_cast<vec4*>(o + ocol) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (col + e < p.N) o[(int64_t)(ocol + e) * p.o_ns] = TypeTraits<OT>::from_f32(tot[e]);
+  }
+}
+template <typename T>
+__device__ __forceinline__ void rows_finish(const RowsParams& p, f32x4 tot, int bt, int row, int col, bool in) {
+  if (p.scales && in) {
+    const f16* sc = p.scales + (int64_t)bt * p.N + col;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (col + e < p.N) tot[e] *= (float)sc[e];
+  }
+  if (p.ep && in) {
+    const T* bias = reinterpret_cast<const T*>(p.bias);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (col + e < p.N) {
+        float v = TypeTraits<T>::to_f32(TypeTraits<T>::from_f32(tot[e]));
+        if (bias) v += TypeTraits<T>::to_f32(bias[(int64_t)bt * p.o_bs + (int64_t)(col + e) * p.o_ns]);
+        tot[e] = apply_act(v, p.act);
+      }
+  }
+  if (!in) return;
+  if (p.out_f32) rows_store<float>(p, tot, bt, row, col);
+  else rows_store<T>(p, tot, bt, row, col);
+}
 
 // NK: the factor is stored transposed, W[bt][n][k] with k contiguous (U of the bmm names, (b, q, r)).  A 16-byte load then is
 // a lane's matrix-core operand as it stands: the lane of slot n and k-group g loads k .. k + 7 of column 16 cg + n for each of
@@ -288,53 +342,7 @@ __global__ __launch_bounds__(DR_NT) void rows_product_kernel(RowsParams p) {
 #pragma unroll
   for (int w = 1; w < DR_WAVES; ++w) tot += *reinterpret_cast<const f32x4*>(&red[(w * 16 + m) * 128 + c4]);
   const int col = col0 + c4;
-  if (p.scales && mrow0 + m < p.M && c4 < cw && col < N) {
-    const f16* sc = p.scales + (int64_t)bt * N + col;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (col + e < N) tot[e] *= (float)sc[e];
-  }
-  if (p.ep && mrow0 + m < p.M && c4 < cw && col < N) {
-    const T* bias = reinterpret_cast<const T*>(p.bias);
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (col + e < N) {
-        float v = TypeTraits<T>::to_f32(TypeTraits<T>::from_f32(tot[e]));
-        if (bias) v += TypeTraits<T>::to_f32(bias[(int64_t)bt * p.o_bs + (int64_t)(col + e) * p.o_ns]);
-        tot[e] = apply_act(v, p.act);
-      }
-  }
-  if (p.out_f32) {
-    // (N is a multiple of 8 and col of 4: the four columns are all inside)
-    if (mrow0 + m < p.M && c4 < cw && col < N)
-      *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.out) + (int64_t)(mrow0 + m) * p.o_ms + (int64_t)bt * p.o_bs + col) = tot;
-  } else if (mrow0 + m < p.M && c4 < cw && col < N) {
-    T* o = reinterpret_cast<T*>(p.out) + (int64_t)(mrow0 + m) * p.o_ms + (int64_t)bt * p.o_bs;
-    int ocol = col;
-    if (p.per & 3) {                                     // a period that cuts through the four columns: each goes to its own place
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t l = fd_div((uint32_t)(col + e), p.perdiv);
-        reinterpret_cast<T*>(p.out)[(int64_t)l * p.o_ls + (int64_t)(mrow0 + m) * p.o_ms + (int64_t)bt * p.per + (col + e - (int)l * p.per)] = TypeTraits<T>::from_f32(tot[e]);
-      }
-    } else {
-    if (p.per > 0) {
-      const uint32_t l = fd_div((uint32_t)col, p.perdiv);
-      o = reinterpret_cast<T*>(p.out) + (int64_t)l * p.o_ls + (int64_t)(mrow0 + m) * p.o_ms + (int64_t)bt * p.per;
-      ocol = col - (int)l * p.per;
-    }
-    if (p.o_ns == 1 && col + 3 < N && ((reinterpret_cast<uintptr_t>(o + ocol) & 7) == 0)) {
-      typename TypeTraits<T>::vec4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = TypeTraits<T>::from_f32(tot[e]);
-      *reinterpret_cast<typename TypeTraits<T>::vec4*>(o + ocol) = v;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (col + e < N) o[(int64_t)(ocol + e) * p.o_ns] = TypeTraits<T>::from_f32(tot[e]);
-    }
-    }
-  }
+  rows_finish<T>(p, tot, (int)bt, mrow0 + m, col, mrow0 + m < p.M && c4 < cw && col < N);
   if (!MULTI || !more) break;
   __syncthreads();                                       // red is free again
 #pragma unroll
@@ -345,6 +353,127 @@ __global__ __launch_bounds__(DR_NT) void rows_product_kernel(RowsParams p) {
                                                          // moved in front of the loop by the compiler and done once)
   }  // tiles of 16 rows
   TR5(4);
+}
+
+// The same product with activations in fp32, at one row (MR = 1) or up to four (MR = 4): the second product of calls whose intermediate is not
+// rounded on the way (StreamBlastArgs::z_f32).  No split into two-byte parts for the matrix cores: fp16 parts do not have fp32's range.  The
+// weights are widened and multiplied in fp32: one row by multiply-adds, up to four by 4 x 4 x 1 matrix instructions, sixteen blocks at a
+// time, whose four columns are those of four neighbouring lanes (half the cycles of four multiply-adds: 4096 -> 22016, rank 1024 at four rows 21.2 -> 20.6 us,
+// 11008 -> 4096 19.0 -> 16.1).  Weights, chunks and rounds as above; each wave stages its share of the activations in LDS by itself (asked for
+// ahead of the weights), lane (n, g) sums its eight k of every step.  Bound by the latency of one trip to memory and, from two rows up, 12 cycles per
+// weight and lane that follow it.  Whole calls against the kernel above, which rounds: w2 (l, s, r), 4096 -> 22016, rank 1024 at 1 / 2 / 4 rows 18.2 / 18.3
+// / 18.5 -> 18.6 / 20.2 / 20.3 us (the phase engine: 29.4 / 38.0 / 58.3); low rank 3736 -> 1712, r = 376 10.8 / 10.9 / 11.1 -> 10.9 / 12.6 / 13.0 (24.0 / 32.6 /
+// 50.2).  Relative error against 64 bits, fp16 / bf16: 2.94e-4 / 2.35e-3 -> 2.07e-4 / 1.65e-3, what rounding the result alone gives.
+template <typename T, int STEPS, bool NK, int MR>
+__global__ __launch_bounds__(DR_NT) void rows_product_f32_kernel(RowsParams p) {
+  using Piece = RowsPiece<T, 16>;
+  using V8 = typename TypeTraits<T>::vec8;
+  constexpr int KW = 32 * STEPS, NA = MR * KW / 4, AP = (NA + 63) / 64;      // a wave's activations of a round: 16-byte pieces, and per lane
+  __shared__ __attribute__((aligned(16))) float a_s[DR_WAVES][MR][KW];
+  __shared__ __attribute__((aligned(16))) float red[DR_WAVES][MR][128];
+  const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, n = l & 15, g = l >> 4;
+  const uint32_t item = p.xcd_span ? (blockIdx.x & 7u) * p.xcd_span + (blockIdx.x >> 3) : blockIdx.x;
+  const uint32_t bt = fd_div(item, p.nch), ch = item - bt * p.nch.d;
+  const int N = p.N, K = p.K;
+  const int cw = p.npc * (NK ? 16 : 8), col0 = (int)ch * cw, colp = col0 + (NK ? n : n * 8);
+  const bool live = NK ? true : (n < p.npc && colp < N);
+  const __amdgpu_buffer_rsrc_t abuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.A), 0, p.a_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t wb = wbuf(reinterpret_cast<const T*>(p.W) + (int64_t)bt * p.w_bs, (uint32_t)((int64_t)K * N * 2));
+  typedef float frow __attribute__((ext_vector_type(MR)));
+  frow acc[8];                                           // [column or column group][row]
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  const auto madd = [](float a, float w, frow c) -> frow {
+    if constexpr (MR == 4) return __builtin_amdgcn_mfma_f32_4x4x1f32(a, w, c, 0, 0, 0);
+    else return fmaf(a, w, c[0]);
+  };
+  for (int ro = 0; ro < p.rounds; ++ro) {
+    const int k0 = (ro * DR_WAVES + wv) * KW;            // first of the wave's rows (rows past K: activations and weights read as zero)
+    u32x4 ap[AP], wr[STEPS][8];
+#pragma unroll
+    for (int u = 0; u < AP; ++u) {
+      const int i = u * 64 + l, m = i / (KW / 4), k = k0 + (i - m * (KW / 4)) * 4;
+      const uint32_t off = m < p.M && k < K ? (uint32_t)((int64_t)m * p.lda + (int64_t)bt * p.a_bs + k) * 4u : DR_OOB;
+      ap[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(abuf, off, 0, 0));
+    }
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+      for (int t = 0; t < 8; ++t) asm volatile("" : "=v"(wr[s][t]));         // (as above: what is not asked for stays undefined and reaches no stored column)
+    if constexpr (NK) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        if (t < p.npc) {
+#pragma unroll
+          for (int s = 0; s < STEPS; ++s) {
+            const int c = colp + 16 * t, k = k0 + 32 * s + 8 * g;
+            wr[s][t] = Piece::load(wb, (c < N && k < K) ? (uint32_t)(c * K + k) * 2u : DR_OOB);
+          }
+        }
+      }
+    } else if (live) {
+      const uint32_t wbase = (uint32_t)((k0 + 8 * g) * N + colp) * 2u, rowb = (uint32_t)N * 2u;
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int t = 0; t < 8; ++t) wr[s][t] = Piece::load(wb, wbase + (uint32_t)(32 * s + t) * rowb);
+    }
+#pragma unroll
+    for (int u = 0; u < AP; ++u)
+      if (u * 64 + l < NA) *reinterpret_cast<u32x4*>(&a_s[wv][0][(u * 64 + l) * 4]) = ap[u];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");                   // (the wave's own LDS: its accesses are carried out in order)
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      const float* ar = &a_s[wv][l & (MR - 1)][32 * s + 8 * g];              // four rows: lane 4 i + m holds row m for its block of four columns
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(ar), hi = *reinterpret_cast<const f32x4*>(ar + 4);
+      const float a[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        if (NK && t >= p.npc) break;
+        const V8 w = __builtin_bit_cast(V8, wr[s][t]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if constexpr (NK) acc[t] = madd(a[e], TypeTraits<T>::to_f32(w[e]), acc[t]);     // eight k of column group t
+          else acc[e] = madd(a[t], TypeTraits<T>::to_f32(w[e]), acc[e]);                  // k = 8 g + t of eight columns
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  // the four lanes of a column add up their k; of four rows lane g keeps row g (each swap moves half of what a shuffle would, in one instruction for two rows)
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    if constexpr (MR == 4) {
+      const auto swap_add = [](float x, float y, auto f) {
+        const auto r = f(__float_as_uint(x), __float_as_uint(y));
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      };
+      const auto by32 = [](uint32_t x, uint32_t y) { return __builtin_amdgcn_permlane32_swap(x, y, false, false); };
+      const auto by16 = [](uint32_t x, uint32_t y) { return __builtin_amdgcn_permlane16_swap(x, y, false, false); };
+      v[e] = swap_add(swap_add(acc[e][0], acc[e][2], by32), swap_add(acc[e][1], acc[e][3], by32), by16);
+    } else {
+      v[e] = acc[e][0];
+      v[e] += __shfl_xor(v[e], 16, 64);
+      v[e] += __shfl_xor(v[e], 32, 64);
+    }
+  }
+  if (g < MR) {
+    if constexpr (NK) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) red[wv][g][16 * e + n] = v[e];
+    } else {
+      *reinterpret_cast<f32x4*>(&red[wv][g][n * 8]) = f32x4{v[0], v[1], v[2], v[3]};
+      *reinterpret_cast<f32x4*>(&red[wv][g][n * 8 + 4]) = f32x4{v[4], v[5], v[6], v[7]};
+    }
+  }
+  __syncthreads();
+  const int m = tid >> 5, c4 = (tid & 31) * 4, col = col0 + c4;
+  if (m >= MR) return;
+  f32x4 tot = *reinterpret_cast<const f32x4*>(&red[0][m][c4]);
+#pragma unroll
+  for (int w = 1; w < DR_WAVES; ++w) tot += *reinterpret_cast<const f32x4*>(&red[w][m][c4]);
+  rows_finish<T>(p, tot, (int)bt, m, col, m < p.M && c4 < cw && col < N);
 }
 
 // ---- warming the L2 for the second product ---------------------------------------------------------------------------------
@@ -439,7 +568,7 @@ __global__ __launch_bounds__(256) void rows_sum_kernel(const float* __restrict__
   if (blockIdx.x >= nmix) { rows_prefetch(pf, nmix); return; }
   const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (item >= MR4) return;
-  using V4 = typename TypeTraits<T>::vec4;
+  typedef T V4 __attribute__((ext_vector_type(4)));
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   for (int j0 = 0; j0 < b; j0 += 8) {
     f32x4 v[8];
@@ -466,7 +595,7 @@ __global__ __launch_bounds__(256) void rows_perm_sum_kernel(const float* __restr
   if (blockIdx.x >= nmix) { rows_prefetch(pf, nmix); return; }
   const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (item >= items) return;
-  using V4 = typename TypeTraits<T>::vec4;
+  typedef T V4 __attribute__((ext_vector_type(4)));
   const int r4n = R >> 2;
   const int r = (int)(item % r4n) * 4;
   const int64_t lm = item / r4n;
@@ -681,6 +810,27 @@ int rows_launch(RowsParams p, int batch, int dtype, int wbits, bool nk, hipStrea
   return dtype == BLR_F16 ? rows_launch_t<f16, 4>(p, batch, st) : rows_launch_t<bf16, 4>(p, batch, st);
 }
 
+template <typename T, bool NK, int MR>
+int rows_f32_launch_t(const RowsParams& p, int batch, hipStream_t st) {
+  const dim3 grid((unsigned)(batch * p.nch.d)), block(DR_NT);
+  switch (p.kw / 32) {
+    case 1: hipLaunchKernelGGL((rows_product_f32_kernel<T, 1, NK, MR>), grid, block, 0, st, p); break;
+    case 2: hipLaunchKernelGGL((rows_product_f32_kernel<T, 2, NK, MR>), grid, block, 0, st, p); break;
+    case 3: hipLaunchKernelGGL((rows_product_f32_kernel<T, 3, NK, MR>), grid, block, 0, st, p); break;
+    default: hipLaunchKernelGGL((rows_product_f32_kernel<T, 4, NK, MR>), grid, block, 0, st, p); break;
+  }
+  BLR_CHECK_LAUNCH("rows_product_f32");
+  return BLR_OK;
+}
+template <typename T, bool NK>
+int rows_f32_launch_m(const RowsParams& p, int batch, hipStream_t st) {
+  return p.M == 1 ? rows_f32_launch_t<T, NK, 1>(p, batch, st) : rows_f32_launch_t<T, NK, 4>(p, batch, st);
+}
+int rows_f32_launch(const RowsParams& p, int batch, int dtype, bool nk, hipStream_t st) {
+  if (dtype == BLR_F16) return nk ? rows_f32_launch_m<f16, true>(p, batch, st) : rows_f32_launch_m<f16, false>(p, batch, st);
+  return nk ? rows_f32_launch_m<bf16, true>(p, batch, st) : rows_f32_launch_m<bf16, false>(p, batch, st);
+}
+
 // What the launch before a planned product can fetch ahead for it; nblocks2 = 0 when the chunks are not whole 16-byte pieces
 // or the factor is too small to matter.
 RowsPrefetch rows_prefetch_plan(const RowsParams& p, int batch, int wbits, bool nk) {
@@ -772,8 +922,8 @@ int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_byt
   const bool lowrank = !monarch && !a.S && bo == 1;     // one output block, S = 1: the mix is the sum over the input slices
   if (M < 1 || M > DR_MAX_M || (!monarch && !lowrank && !a.S) || (bo != b && !lowrank) || (u_nk && a.wbits != 16)) return 1;
   if (lowrank && a.wbits != 16) return 1;
-  // (a period that is no multiple of 4, w2 (l, r, s): 1408 -> 3584 in 16 blocks, rank 304 at 2 / 16 rows 11.9 / 23.6 us on the hand-over
-  // kernel, 7.9 / 8.0 here; up to four blocks, where ranks that real layers have give whole fours, such a call is left to that kernel:
+  // (a period that is no multiple of 4, w2 (l, r, s): 1408 -> 3584 in 16 blocks, rank 304 at 2 / 4 / 16 rows 12.4 / 18.5 / 23.6 us on the hand-over
+  // kernels, 10.2 / 10.4 / 8.0 here; up to four blocks, where ranks that real layers have give whole fours, such a call is left to that kernel:
   // it is what the tests of its bounded waits run)
   if (monarch && a.perm_per % 4 && b <= 4 && !u_nk) return 1;
   if (monarch && (a.wbits != 16 || R % a.perm_per || R / a.perm_per != b || a.perm_per >= 65536)) return 1;
@@ -788,7 +938,9 @@ int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_byt
       if (P % ks == 0 && (P / ks) % 8 == 0) { mks = ks; break; }
   }
   const bool y_f32 = lowrank || mks > 1;                // y holds slices of one reduction: fp32 partial sums, rounded once after their sum
-  const size_t ybytes = align_up((size_t)b * mks * M * R * (y_f32 ? 4 : 2), 256), zbytes = align_up((size_t)bo * M * R * 2, 256);
+  const bool z_f32 = a.z_f32 && M <= 4;                 // (rows_product_f32_kernel)
+  const size_t zel = z_f32 ? 4 : 2;
+  const size_t ybytes = align_up((size_t)b * mks * M * R * (y_f32 ? 4 : 2), 256), zbytes = align_up((size_t)bo * M * R * zel, 256);
   if (ybytes + zbytes > region_bytes) return 1;
   void* Y = region;
   void* Z = reinterpret_cast<char*>(region) + ybytes;
@@ -803,9 +955,9 @@ int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_byt
   s1.M = M; s1.K = P; s1.N = R; s1.scales = a.wbits != 16 ? (const f16*)a.v_scales : nullptr;
   if (monarch && mks == 1) { s1.out = Z; s1.o_bs = 0; s1.per = a.perm_per; s1.o_ls = (int64_t)M * R; s1.perdiv = fd_make((uint32_t)a.perm_per); }
   if (mks > 1) { s1.a_bs = P / mks; s1.w_bs = (int64_t)(P / mks) * R; s1.K = P / mks; }
-  s1.out_f32 = y_f32 ? 1 : 0;
+  s1.out_f32 = y_f32 || (monarch && z_f32) ? 1 : 0;
   RowsParams s2 = {};
-  s2.A = Z; s2.lda = R; s2.a_bs = (int64_t)M * R; s2.a_bytes = (uint32_t)((size_t)bo * M * R * 2);
+  s2.A = Z; s2.lda = R; s2.a_bs = (int64_t)M * R; s2.a_bytes = (uint32_t)((size_t)bo * M * R * zel);
   s2.W = a.U; s2.w_bs = (int64_t)R * Q;
   s2.out = a.out; s2.o_ms = a.ldo;
   s2.o_bs = a.out_ns ? a.out_bs : Q; s2.o_ns = a.out_ns ? a.out_ns : 1;
@@ -829,21 +981,23 @@ int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_byt
   if (monarch && mks > 1) {
     const int64_t items = (int64_t)bo * M * R / 4;
     const uint32_t nmix = (uint32_t)cdiv(items, 256);
-    if (a.dtype == BLR_F16) hipLaunchKernelGGL(rows_perm_sum_kernel<f16>, dim3(nmix + prefetch_blocks(pf)), dim3(256), 0, st, (const float*)Y, (f16*)Z, mks, M, R, a.perm_per, items, pf, nmix);
-    else hipLaunchKernelGGL(rows_perm_sum_kernel<bf16>, dim3(nmix + prefetch_blocks(pf)), dim3(256), 0, st, (const float*)Y, (bf16*)Z, mks, M, R, a.perm_per, items, pf, nmix);
+#define BLR_PERM_SUM(T) hipLaunchKernelGGL(rows_perm_sum_kernel<T>, dim3(nmix + prefetch_blocks(pf)), dim3(256), 0, st, (const float*)Y, (T*)Z, mks, M, R, a.perm_per, items, pf, nmix)
+    if (z_f32) BLR_PERM_SUM(float); else if (a.dtype == BLR_F16) BLR_PERM_SUM(f16); else BLR_PERM_SUM(bf16);
+#undef BLR_PERM_SUM
     BLR_CHECK_LAUNCH("rows_perm_sum");
   } else if (monarch)
     rc = BLR_OK;
   else if (lowrank) {
     const int64_t mr4 = (int64_t)M * R / 4;
     const uint32_t nmix = (uint32_t)cdiv(mr4, 256);
-    if (a.dtype == BLR_F16) hipLaunchKernelGGL(rows_sum_kernel<f16>, dim3(nmix + prefetch_blocks(pf)), dim3(256), 0, st, (const float*)Y, (f16*)Z, b, mr4, pf, nmix);
-    else hipLaunchKernelGGL(rows_sum_kernel<bf16>, dim3(nmix + prefetch_blocks(pf)), dim3(256), 0, st, (const float*)Y, (bf16*)Z, b, mr4, pf, nmix);
+#define BLR_ROWS_SUM(T) hipLaunchKernelGGL(rows_sum_kernel<T>, dim3(nmix + prefetch_blocks(pf)), dim3(256), 0, st, (const float*)Y, (T*)Z, b, mr4, pf, nmix)
+    if (z_f32) BLR_ROWS_SUM(float); else if (a.dtype == BLR_F16) BLR_ROWS_SUM(f16); else BLR_ROWS_SUM(bf16);
+#undef BLR_ROWS_SUM
     BLR_CHECK_LAUNCH("rows_sum");
   } else
     rc = mix_launch(Y, a.S, Z, M, b, R, a.s_layout, a.dtype, pf, st);
   if (rc) return rc;
-  rc = rows_launch(s2, bo, a.dtype, a.wbits, u_nk, st);
+  rc = z_f32 ? rows_f32_launch(s2, bo, a.dtype, u_nk, st) : rows_launch(s2, bo, a.dtype, a.wbits, u_nk, st);
   if (rc == BLR_OK && s2.ep) epilogue_taken();
   return rc == 1 ? BLR_ERR_UNSUPPORTED : rc;
 }

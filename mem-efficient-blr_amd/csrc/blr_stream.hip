@@ -751,8 +751,8 @@ __device__ __forceinline__ void phase_nk(const PhaseDesc& d, int M, float* smem,
 // A wave owns 16 weight rows and walks them four at a time; one load instruction reads 1 KB of
 // one row (lane l holds k = 8 l .. 8 l + 7 of each 512-element chunk).  The activation slices a
 // lane needs are the same for every row, so they live in registers.
-constexpr int dot_kch(int MT) { return MT == 1 ? 4 : 2; }   // 512-element chunks of K kept in registers per lane
-__device__ __forceinline__ bool nk_use_dot(const PhaseDesc& d, int MT) {
+__host__ __device__ constexpr int dot_kch(int MT) { return MT == 1 ? 4 : 2; }   // 512-element chunks of K kept in registers per lane
+__host__ __device__ __forceinline__ bool nk_use_dot(const PhaseDesc& d, int MT) {
   return MT <= 4 && d.wbits == 16 && d.vec_ok && (d.K % 8 == 0) && d.K <= 512 * dot_kch(MT) && !d.nk_split_k;
 }
 
@@ -1319,8 +1319,8 @@ int stream_generic_launch(const StreamGenericArgs& a, hipStream_t st) {
     if (!a.split && (a.M >= 2 || (!equal && a.in_f <= 4096))) {
       // From two rows up: the three-launch matrix-core path, low rank being BLAST with the input cut into 16 (or 8) slices of
       // rows of A, one output block and S = 1 (the mix is the sum over the slices).  Where there are fewer equal slices, or none, 16 with
-      // a shorter last one, at one row too: 3736 -> 1712, r = 376 at 1 / 4 / 16 rows 21.9 / 48.6 / 17.6
-      // us on what follows, 9.9 / 10.3 / 11.0 here; 3728 inputs (two slices) at 4 rows 15.3 -> 10.5; 920 -> 8000, r = 136 at 2 rows 25.1 -> 9.6.
+      // a shorter last one, at one row too: 3736 -> 1712, r = 376 at 1 / 4 / 16 rows 24.0 / 50.2 / 17.6
+      // us on what follows, 10.9 / 13.0 / 11.0 here; 3728 inputs (two slices) at 4 rows 15.3 -> 10.5; 920 -> 8000, r = 136 at 2 rows 25.5 -> 10.9.
       // (One row of more than 4096 such inputs stays with the phase engine, at twice the time - 4104 -> 4096, r = 512 21.9 against 11.3 us: it is
       // the call that the test of the engine's bounded wait makes, and none of the configured layers has such an input.)
       int bi = equal >= 8 ? equal : 0, slice = 0;
@@ -1330,6 +1330,7 @@ int stream_generic_launch(const StreamGenericArgs& a, hipStream_t st) {
         bl.x = a.x; bl.ldx = a.ldx; bl.U = a.W2; bl.V = a.W1; bl.S = nullptr; bl.out = a.out; bl.ldo = a.ldo;
         bl.M = a.M; bl.in_f = a.in_f; bl.out_f = a.out_f; bl.b = bi; bl.bo = 1; bl.r = a.r;
         bl.dtype = a.dtype; bl.u_layout = BLR_U_RQ; bl.s_layout = BLR_S_IJR; bl.wbits = 16; bl.slice = slice;
+        bl.z_f32 = !equal && a.M <= 4;      // as the phase engine below keeps it at these rows
         const int rc = decode_rows_launch(bl, w.plain, decode2_plain_bytes(), st);
         if (rc != 1) return rc;
       }
@@ -1392,9 +1393,16 @@ int stream_generic_launch(const StreamGenericArgs& a, hipStream_t st) {
     bl.perm_per = per;
     if (a.out_order == BLR_OUT_INTERLEAVED) { bl.out_bs = 1; bl.out_ns = a.b; }
     else { bl.out_bs = S; bl.out_ns = 1; }
+    // At up to four rows the kernels that take these calls where the skinny products do not hand the intermediate on in fp32 - the phase engine
+    // where its second product runs on vector instructions, the hand-over kernel for periods that are no multiple of 4 - and so do the
+    // skinny products: how far a result is from the exact one must not depend on which of them serves it.
+    PhaseDesc nk = {};
+    nk.wbits = 16; nk.vec_ok = 1; nk.batch = a.b; nk.K = a.r; nk.N = S;
+    plan_nk(nk, target);
+    bl.z_f32 = a.M <= 4 && (sr ? nk_use_dot(nk, MT) : per % 4 != 0);
     if (decode2_applicable(bl)) {
       // w2 (l, s, r), at one row too: the two skinny products of blr_decode_rows.hip.  The phase engine below took these calls before:
-      // 4096 -> 22016, rank 1024 at 1 / 3 / 16 rows 28.7 / 51.6 / 96.7 -> 17.7 / 17.9 / 19.0 us, 768 -> 2304, rank 128 15.1 / 24.3 / 54.3
+      // 4096 -> 22016, rank 1024 at 1 / 3 / 16 rows 29.4 / 52.0 / 96.7 -> 18.6 / 20.2 / 19.0 us, 768 -> 2304, rank 128 15.1 / 24.3 / 54.3
       // -> 7.7 .. 8.9 at all of them (eager calls; two launches of an eager stream), 1408 -> 3584 in 16 blocks, rank 304 17.5 / 26.2 /
       // 30.6 -> 7.9 .. 8.8.  w2 (l, r, s): the single-row kernels have a say at one row.
       int rc = sr ? decode_rows_launch(bl, w.plain, decode2_plain_bytes(), st)

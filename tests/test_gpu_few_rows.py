@@ -157,3 +157,50 @@ def test_monarch_interleaved_columns(b, p, r, q, M):
         assert torch.equal(K.triton_monarch_right_left_fp16(x, w1, w2), out)
     want = K.triton_monarch_right_left_fp32(x.float(), w1.float(), w2.float())[0]       # (fp32 throughout: only Z is not rounded on the way)
     assert_close(out, want.double().cpu().numpy(), torch.float16, f"monarch interleaved b={b} M={M}", scale=2.0)
+
+
+def _small_integers(rng, *shape, top):
+    return rng.integers(-top, top + 1, shape).astype(np.float64)
+
+
+# w2 (l, s, r) with more than 256 groups of 64 output columns and ranks up to 1024 (one row: 2048): whole 16-byte pieces of the period and not, one to four
+# steps of a round, two rounds, sliced input blocks (1104, 1040 and 2048 rows); w2 (l, r, s) with a period that is no multiple of 4; low rank without equal slices
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("name,b,p,rank,s", [("triton_monarch_right_fp16", *c) for c in [(4, 512, 1024, 4200), (16, 88, 304, 1032), (16, 8, 16, 1040), (16, 1040, 48, 1032),
+                                                                                         (12, 40, 744, 1416), (2, 1104, 176, 8200), (4, 8, 2048, 4104)]]
+                         + [("triton_monarch_right_ideal_fp16", 4, 2048, 512, 4104)]
+                         + [("triton_monarch_right_left_fp16", *c) for c in [(16, 88, 304, 224), (16, 8, 16, 8), (16, 1040, 48, 40), (8, 136, 1032, 72), (12, 40, 744, 136)]]
+                         + [("low_rank", 1, *c) for c in [(3736, 376, 1712), (8, 8, 8), (72, 16, 40), (4088, 1032, 136), (11000, 2056, 72)]])
+def test_intermediate_stays_in_fp32_up_to_four_rows(name, b, p, rank, s, M, dtype):
+    """Whole numbers and halves of them down to 2^-k whose sums fp32 holds exactly in any order, the intermediate among them, which takes up to 14 bits:
+    the result is the exact one, rounded once."""
+    if M == 1 and "right_left" in name:
+        pytest.skip("served by the single-row kernels")
+    if M > 1 and rank == 2048:
+        pytest.skip("the intermediate is rounded to the operand type")
+    from triton_funcs import low_rank_kernels as LR, _lib as L
+    from test_gpu_monarch_lowrank_dense import _blocked, _run_monarch
+    rng = np.random.default_rng(rank + M)
+    say(f"[case] exact intermediate {name} b={b} p={p} rank={rank} s={s} M={M} {dtype}")
+    top = max(2, int((9000 / p ** 0.5) ** 0.5))                      # z of 3000 in the mean square, at most top^2 p
+    x, w1 = _small_integers(rng, M, b * p, top=top), _small_integers(rng, b, rank, p, top=top)
+    scale = 2.0 ** -round(np.log2(6 * (2 * rank / 3) ** 0.5))       # results of about 500
+    w2 = _small_integers(rng, b, s, rank, top=1) * scale
+    if name == "low_rank":
+        z = x @ w1[0].T
+        ref, size = z @ w2[0].T, np.abs(z) @ np.abs(w2[0].T)            # (size: no partial sum is larger)
+        run = lambda: LR.triton_low_rank_fp16(*(torch.from_numpy(np.ascontiguousarray(t)).cuda().to(dtype) for t in (x, w1[0].T, w2[0].T)), {"algo": L.ALGO_STREAM})
+    else:
+        ref, _, z, _ = O.monarch_forward(x, w1, w2)
+        size = np.abs(z) @ np.abs(w2).transpose(0, 2, 1)
+        if "ideal" in name:
+            ref = _blocked(ref, b)
+        run = lambda: _run_monarch(name, x, w1, w2, dtype)
+    assert p * top * top < 2 ** 24 and size.max() / scale < 2 ** 24
+    want = torch.from_numpy(ref).float().to(dtype)
+    assert torch.equal(run().cpu().reshape(want.shape), want)
+    bias = torch.from_numpy(_small_integers(rng, b * s, top=200)).to(dtype)
+    with L.fused_epilogue(bias.cuda(), None):
+        out = run().cpu().reshape(want.shape)
+    assert torch.equal(out, (want.float() + bias.float()).to(dtype))
