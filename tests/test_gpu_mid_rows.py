@@ -49,6 +49,24 @@ def test_mix_any_blocks(b, M, r, dtype):
     assert_close(K.triton_blast_bmm_fp16(*args, off), ref, dtype, f"mix b={b} M={M} r={r}, S one element off")
 
 
+# a handful of rows with ranks that no vector kernel takes (chunks of 16 ranks, whole and not) and S off every boundary, both orders of S
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_bmm_fp16"])
+@pytest.mark.parametrize("b,M,r", [(2, 1, 3), (6, 8, 33), (6, 9, 34), (6, 16, 50), (7, 9, 16), (7, 16, 63), (16, 2, 510), (16, 16, 17)])
+def test_mix_few_rows_any_ranks(b, M, r, name, dtype):
+    from triton_funcs import blast_kernels as K
+    x, Ut, Vt, St = blast_inputs(b, 8, 16, r, (M,), seed=M + b)
+    U, V, S = (O.blast_to_bmm_layout if "bmm" in name else O.blast_to_partial_layout)(Ut, Vt, St)
+    say(f"[case] mix at few rows {name} b={b} M={M} r={r} {dtype}")
+    room = torch.zeros(S.size + 8, device="cuda", dtype=dtype)
+    off = room[1:1 + S.size].view(S.shape)
+    off.copy_(dev(S, dtype))
+    args = dev(x, dtype), dev(U, dtype), dev(V, dtype)
+    ref = O.blast_forward(rounded(x, dtype), rounded(Ut, dtype), rounded(Vt, dtype), rounded(St, dtype))[0]
+    for s in (dev(S, dtype), off):
+        assert_close(getattr(K, name)(*args, s, {"algo": 2}), ref, dtype, f"{name} b={b} M={M} r={r}")
+
+
 # fp32: chunks of 32 ranks, whole and not, ranks in whole pieces of four and not, both orders of S
 @pytest.mark.parametrize("name", ["triton_blast_full_fp32", "triton_blast_bmm_fp32"])
 @pytest.mark.parametrize("b,M,r", [(2, 1, 4), (3, 33, 36), (6, 70, 200), (16, 31, 64), (16, 65, 100), (5, 40, 30)])
