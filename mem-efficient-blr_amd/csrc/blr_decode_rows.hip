@@ -706,6 +706,15 @@ int rows_mix_rij_t(const void* Y, const void* S, void* Z, int M, int R, const Ro
   return BLR_OK;
 }
 
+// Every number of blocks up to 16 has a kernel of its own, whose loop over them is unrolled: all loads of a thread in flight at once
+// (128 columns a block both ways, r = 256, whole calls against the kernel with a loop, at 16 / 128 rows: 5 blocks 11.0 / 11.7 -> 10.4 / 10.9 us, 7 blocks
+// 11.5 / 12.5 -> 10.7 / 10.9, 10 blocks 12.2 / 13.6 -> 10.9 / 11.8, 15 blocks 13.7 / 15.5 -> 10.9 / 12.9)
+template <typename T, int... I>
+auto rows_mix_fn(std::integer_sequence<int, I...>, int b) {
+  auto fn = rows_mix_kernel<T, 0, 4>;
+  ((b == I + 2 ? void(fn = rows_mix_kernel<T, I + 2, 4>) : void()), ...);
+  return fn;
+}
 template <typename T>
 int rows_mix_t(const void* Y, const void* S, void* Z, int M, int b, int R, int64_t s_si, int64_t s_sj, const RowsPrefetch& pf, hipStream_t st) {
   // eight ranks per thread once four would make more than two workgroups of 256 threads per compute unit (side by side at 64 rows:
@@ -718,20 +727,8 @@ int rows_mix_t(const void* Y, const void* S, void* Z, int M, int b, int R, int64
   const uint32_t nmix = (uint32_t)cdiv(total, nt);
   const dim3 grid(nmix + prefetch_blocks(pf)), block(nt);
   const FastDiv r4div = fd_make((uint32_t)(R / vw)), bdiv = fd_make((uint32_t)b);
-#define BLR_ROWS_MIX(B, VW) hipLaunchKernelGGL((rows_mix_kernel<T, B, VW>), grid, block, 0, st, (const T*)Y, (const T*)S, (T*)Z, M, b, R, s_si, s_sj, r4div, bdiv, total, pf, nmix)
-  if (wide) BLR_ROWS_MIX(16, 8);
-  else switch (b) {                                        // a fixed number of blocks: all loads of a thread in flight at once
-    case 2: BLR_ROWS_MIX(2, 4); break;
-    case 3: BLR_ROWS_MIX(3, 4); break;
-    case 4: BLR_ROWS_MIX(4, 4); break;
-    case 6: BLR_ROWS_MIX(6, 4); break;
-    case 8: BLR_ROWS_MIX(8, 4); break;
-    case 9: BLR_ROWS_MIX(9, 4); break;
-    case 12: BLR_ROWS_MIX(12, 4); break;
-    case 16: BLR_ROWS_MIX(16, 4); break;
-    default: BLR_ROWS_MIX(0, 4);
-  }
-#undef BLR_ROWS_MIX
+  const auto fn = wide ? rows_mix_kernel<T, 16, 8> : rows_mix_fn<T>(std::make_integer_sequence<int, 15>{}, b);
+  hipLaunchKernelGGL(fn, grid, block, 0, st, (const T*)Y, (const T*)S, (T*)Z, M, b, R, s_si, s_sj, r4div, bdiv, total, pf, nmix);
   BLR_CHECK_LAUNCH("rows_mix");
   return BLR_OK;
 }

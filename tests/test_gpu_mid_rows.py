@@ -49,6 +49,18 @@ def test_mix_any_blocks(b, M, r, dtype):
     assert_close(K.triton_blast_bmm_fp16(*args, off), ref, dtype, f"mix b={b} M={M} r={r}, S one element off")
 
 
+# the same mix with the rank contiguous in S: every number of blocks that has a kernel of its own, and one more; threads in one workgroup and in several
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,r", [(2, 8), (3, 72), (16, 136)])
+@pytest.mark.parametrize("b", list(range(2, 18)))
+def test_mix_any_blocks_rank_contiguous(b, M, r, dtype):
+    from test_gpu_blast import _ref, _run_blast
+    x, U, Vt, S = blast_inputs(b, 8, 16, r, (M,), seed=M + b)
+    say(f"[case] mix, rank contiguous b={b} M={M} r={r} {dtype}")
+    out = _run_blast("triton_blast_full_fp16", x, U, Vt, S, dtype, "auto")
+    assert_close(out, _ref(x, U, Vt, S, dtype)[0], dtype, f"mix, rank contiguous b={b} M={M} r={r}")
+
+
 # a handful of rows with ranks that no vector kernel takes (chunks of 16 ranks, whole and not) and S off every boundary, both orders of S
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_bmm_fp16"])
