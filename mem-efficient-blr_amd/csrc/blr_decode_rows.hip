@@ -31,7 +31,11 @@ namespace {
 constexpr int DR_NT = 512;
 constexpr int DR_WAVES = 8;
 constexpr int DR_MAX_STEPS = 4;           // 32-row steps of a wave: 8 loads per lane each
-constexpr int64_t MIX_ANY_MAX = 1 << 20;  // b M R up to which rows_mix_any_kernel takes a call (beyond, every element of Y is loaded once for all blocks instead: blast_mix_launch)
+// b M R up to which rows_mix_any_kernel takes a call; beyond, every element of Y is loaded once for all blocks instead (blast_mix_launch).  Whole calls with the
+// kernel here / there, S (r, i, j): at 2^20 15 blocks, r = 512 20.5 / 32.6 us, 9 blocks, r = 256 19.8 / 24.2, 6 blocks, r = 512 16.8 / 19.7; at 2^20.5 24.2 / 34.4,
+// 25.4 / 28.2 and 18.9 / 20.8; at 2^21 30.9 / 36.7 and 29.8 / 31.3, 10 blocks, r = 1024 26.3 / 29.7; at 2^21.5 15 blocks 35.8 / 39.9, 12 blocks, r = 512 31.0 / 33.0
+// (larger ones were not measured: the line is drawn where the gain is down to a few per cent).
+constexpr int64_t MIX_ANY_MAX = 1 << 21;
 constexpr int DR_MAX_M = 128;             // token rows: tiles of 16 over the same registers of weights
 constexpr uint32_t DR_OOB = 0x80000000u;
 }  // namespace
