@@ -1316,13 +1316,12 @@ int stream_generic_launch(const StreamGenericArgs& a, hipStream_t st) {
     int equal = 0;                           // equal slices of whole 16-byte pieces, as many as there are
     for (int c = 16; c >= 2 && !equal; c >>= 1)
       if (a.in_f % c == 0 && (a.in_f / c) % 8 == 0) equal = c;
-    if (!a.split && (a.M >= 2 || (!equal && a.in_f <= 4096))) {
+    if (!a.split && (a.M >= 2 || !equal)) {
       // From two rows up: the three-launch matrix-core path, low rank being BLAST with the input cut into 16 (or 8) slices of
-      // rows of A, one output block and S = 1 (the mix is the sum over the slices).  Where there are fewer equal slices, or none, 16 with
-      // a shorter last one, at one row too: 3736 -> 1712, r = 376 at 1 / 4 / 16 rows 24.0 / 50.2 / 17.6
-      // us on what follows, 10.9 / 13.0 / 11.0 here; 3728 inputs (two slices) at 4 rows 15.3 -> 10.5; 920 -> 8000, r = 136 at 2 rows 25.5 -> 10.9.
-      // (One row of more than 4096 such inputs stays with the phase engine, at twice the time - 4104 -> 4096, r = 512 21.9 against 11.3 us: it is
-      // the call that the test of the engine's bounded wait makes, and none of the configured layers has such an input.)
+      // rows of A, one output block and S = 1 (the mix is the sum over the slices).  Where there are fewer equal slices, 16 with a shorter last
+      // one; where there are none, at one row too (one row with equal slices is the two-stage kernel's, below): 3736 -> 1712, r = 376 at 1 / 4 / 16
+      // rows 24.0 / 50.2 / 17.6 us on what follows, 10.9 / 13.0 / 11.0 here, 4104 -> 4096, r = 512 at one row 22.9 -> 11.5; 3728 inputs (two slices) at 4
+      // rows 15.3 -> 10.5; 920 -> 8000, r = 136 at 2 rows 25.5 -> 10.9.
       int bi = equal >= 8 ? equal : 0, slice = 0;
       if (!bi && a.in_f % 8 == 0) { slice = (int)cdiv(cdiv(a.in_f, 16), 8) * 8; bi = (int)cdiv(a.in_f, slice); }
       if (bi) {

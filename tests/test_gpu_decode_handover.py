@@ -133,8 +133,8 @@ def _spinning_cases(dtype):
         "monarch_m8": _monarch_case(4, 1024, 1016, 1024, 8, dtype, 60),
         # U as (b, q, r) with a rank that is not a power of two: the single-launch kernel (its workgroups hand y and z over)
         "blast_bmm_m1": _blast_case(16, 256, 256, 480, 1, "triton_blast_bmm_fp16", dtype, 61),
-        # 4104 input features cannot be cut into equal blocks of whole 16-byte pieces: the phase engine serves the call
-        # (one launch, a barrier of the whole grid between the two products)
+        # 4104 input features cannot be cut into equal blocks of whole 16-byte pieces: without the skinny products (BLR_DECODE_ROWS=0) the
+        # phase engine serves the call (one launch, a barrier of the whole grid between the two products)
         "low_rank_phases_m1": _low_rank_case(4104, 4096, 512, 1, dtype, 62),
     }
 
@@ -144,7 +144,11 @@ def test_wait_that_gives_up_is_reported_and_leaves_the_workspace_usable(case):
     """With the poll limit forced to 1 from the host every wait gives up at once: the kernel still ends, the status query
     returns BLR_ERR_TIMEOUT exactly once, and the next call at the normal limit is correct and reports a clean status."""
     from triton_funcs import _lib as L
-    fn, ref = _spinning_cases(torch.float16)[case]
+    call, ref = _spinning_cases(torch.float16)[case]
+
+    def fn():
+        with L.options(BLR_DECODE_ROWS=0):
+            return call()
     say(f"[case] forced give-up {case}")
     good = fn().clone()
     assert_close(good, ref.reshape(tuple(good.shape)), torch.float16, case)
@@ -169,6 +173,25 @@ def test_wait_that_gives_up_is_reported_and_leaves_the_workspace_usable(case):
         out = fn()
         assert torch.equal(out, good), f"call {rep} after the give-up differs from the result before it"
     assert L.workspace_status(ws) == 0
+
+
+@pytest.mark.parametrize("case", ["low_rank_phases_m1"])
+def test_the_same_calls_wait_for_nothing_by_default(case):
+    """The skinny products take them: separate launches, so that a poll limit of 1 gives up nowhere and changes nothing."""
+    from triton_funcs import _lib as L
+    fn, ref = _spinning_cases(torch.float16)[case]
+    say(f"[case] no wait {case}")
+    good = fn().clone()
+    assert_close(good, ref.reshape(tuple(good.shape)), torch.float16, case)
+    ws = L.workspace(good.device, 1, L.ALGO_STREAM)
+    L.lib().blr_set_spin_limit(1)
+    try:
+        out = fn()
+        torch.cuda.synchronize()
+        assert L.workspace_status(ws) == 0
+    finally:
+        L.lib().blr_set_spin_limit(0)
+    assert torch.equal(out, good)
 
 
 def test_single_launch_and_multi_launch_calls_alternate_on_one_workspace():
