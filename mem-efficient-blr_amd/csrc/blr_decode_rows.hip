@@ -923,10 +923,11 @@ int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_byt
   const bool lowrank = !monarch && !a.S && bo == 1;     // one output block, S = 1: the mix is the sum over the input slices
   if (M < 1 || M > DR_MAX_M || (!monarch && !lowrank && !a.S) || (bo != b && !lowrank) || (u_nk && a.wbits != 16)) return 1;
   if (lowrank && a.wbits != 16) return 1;
-  // (a period that is no multiple of 4, w2 (l, r, s): 1408 -> 3584 in 16 blocks, rank 304 at 2 / 4 / 16 rows 12.4 / 18.5 / 23.6 us on the hand-over
-  // kernels, 10.2 / 10.4 / 8.0 here; up to four blocks, where ranks that real layers have give whole fours, such a call is left to that kernel:
-  // it is what the tests of its bounded waits run)
-  if (monarch && a.perm_per % 4 && b <= 4 && !u_nk) return 1;
+  // A period that is no multiple of 4, w2 (l, r, s): 1408 -> 3584 in 16 blocks, rank 304 at 2 / 4 / 16 rows 12.4 / 18.5 / 23.6 us on the hand-over
+  // kernels, 10.2 / 10.4 / 8.0 here; 4096 -> 4096 in 4 blocks, rank 1016 at 3 / 4 / 5 / 16 rows 21.2 / 23.3 / 27.0 / 32.9 against 17.2 / 17.3 / 14.1 / 15.1.  At two rows
+  // the vector hand-over kernel is ahead with long periods, whose narrow column chunks leave most lanes of the fp32 product below idle: periods of 250 and
+  // more (4096 -> 4096 in 4 blocks, rank 1016 / 1512 / 2024 15.6 / 17.7 / 21.6 against 16.9 / 22.0 / 23.1; rank 760, a period of 190, 15.2 against 15.0).
+  if (monarch && a.perm_per % 4 && !u_nk && M == 2 && a.perm_per >= 250) return 1;
   if (monarch && (a.wbits != 16 || R % a.perm_per || R / a.perm_per != b || a.perm_per >= 65536)) return 1;
   if (a.wbits != 16 && (!a.u_scales || !a.v_scales)) return 1;
   if (a.dtype != BLR_F16 && a.dtype != BLR_BF16) return 1;

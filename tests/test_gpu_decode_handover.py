@@ -129,7 +129,7 @@ def _monarch_case(b, p, rank, s_out, M, dtype, seed):
 def _spinning_cases(dtype):
     """Calls served by kernels whose workgroups wait for each other (shapes at which the wait lasts microseconds)."""
     return {
-        # a permutation period of 254 (not a multiple of 4) keeps this call on the single-launch kernels
+        # without the skinny products (BLR_DECODE_ROWS=0) the matrix-core single-launch kernel serves this call
         "monarch_m8": _monarch_case(4, 1024, 1016, 1024, 8, dtype, 60),
         # U as (b, q, r) with a rank that is not a power of two: the single-launch kernel (its workgroups hand y and z over)
         "blast_bmm_m1": _blast_case(16, 256, 256, 480, 1, "triton_blast_bmm_fp16", dtype, 61),
@@ -175,7 +175,7 @@ def test_wait_that_gives_up_is_reported_and_leaves_the_workspace_usable(case):
     assert L.workspace_status(ws) == 0
 
 
-@pytest.mark.parametrize("case", ["low_rank_phases_m1"])
+@pytest.mark.parametrize("case", ["monarch_m8", "low_rank_phases_m1"])
 def test_the_same_calls_wait_for_nothing_by_default(case):
     """The skinny products take them: separate launches, so that a poll limit of 1 gives up nowhere and changes nothing."""
     from triton_funcs import _lib as L

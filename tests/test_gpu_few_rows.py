@@ -170,7 +170,8 @@ def _small_integers(rng, *shape, top):
 @pytest.mark.parametrize("name,b,p,rank,s", [("triton_monarch_right_fp16", *c) for c in [(4, 512, 1024, 4200), (16, 88, 304, 1032), (16, 8, 16, 1040), (16, 1040, 48, 1032),
                                                                                          (12, 40, 744, 1416), (2, 1104, 176, 8200), (4, 8, 2048, 4104)]]
                          + [("triton_monarch_right_ideal_fp16", 4, 2048, 512, 4104)]
-                         + [("triton_monarch_right_left_fp16", *c) for c in [(16, 88, 304, 224), (16, 8, 16, 8), (16, 1040, 48, 40), (8, 136, 1032, 72), (12, 40, 744, 136)]]
+                         + [("triton_monarch_right_left_fp16", *c) for c in [(16, 88, 304, 224), (16, 8, 16, 8), (16, 1040, 48, 40), (8, 136, 1032, 72), (12, 40, 744, 136),
+                                                                         (4, 1024, 1016, 72), (4, 64, 1032, 40), (4, 2752, 8, 8)]]
                          + [("low_rank", 1, *c) for c in [(3736, 376, 1712), (8, 8, 8), (72, 16, 40), (4088, 1032, 136), (11000, 2056, 72)]])
 def test_intermediate_stays_in_fp32_up_to_four_rows(name, b, p, rank, s, M, dtype):
     """Whole numbers and halves of them down to 2^-k whose sums fp32 holds exactly in any order, the intermediate among them, which takes up to 14 bits:
@@ -200,6 +201,8 @@ def test_intermediate_stays_in_fp32_up_to_four_rows(name, b, p, rank, s, M, dtyp
     assert p * top * top < 2 ** 24 and size.max() / scale < 2 ** 24
     want = torch.from_numpy(ref).float().to(dtype)
     assert torch.equal(run().cpu().reshape(want.shape), want)
+    with L.options(BLR_DECODE_ROWS=0):                               # the kernels that take the call where the skinny products do not
+        assert torch.equal(run().cpu().reshape(want.shape), want)
     bias = torch.from_numpy(_small_integers(rng, b * s, top=200)).to(dtype)
     with L.fused_epilogue(bias.cuda(), None):
         out = run().cpu().reshape(want.shape)
