@@ -169,10 +169,15 @@ def test_low_rank_and_monarch_through_ring_kernel(dtype, ring_forced):
     assert_close(out, ref, dtype, "monarch", scale=2.0)
 
 
-# periods (rank / b) that hold whole pieces of four columns, of two, of one, in every tile of the ring kernel; interleaved columns with bias
-# and activation; rows and columns past the last whole tile
+ODD_PERIODS = [(4, 72, 144 + 16, 96, 300), (2, 136, 20 * 8, 72, 130), (4, 64, 8 * 27, 40, 257), (8, 40, 8 * 33, 24, 140), (16, 72, 16 * 5 + 160, 200, 97),
+               (4, 64, 144, 96, 300), (2, 136, 136, 72, 130), (8, 72, 800, 40, 259)]
+assert {next(e for e in (8, 4, 2, 1) if rank // b % e == 0) for b, _, rank, _, _ in ODD_PERIODS} == {8, 4, 2, 1}
+
+
+# periods (rank / b) that hold whole pieces of eight columns (the store of the others), of four, of two, of one, in every tile of the ring kernel; interleaved columns
+# with bias and activation, with bias, gate and residual (rows of the gate shared by three); rows and columns past the last whole tile
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("b,p,rank,s,M", [(4, 72, 144 + 16, 96, 300), (2, 136, 20 * 8, 72, 130), (4, 64, 8 * 27, 40, 257), (8, 40, 8 * 33, 24, 140), (16, 72, 16 * 5 + 160, 200, 97)])
+@pytest.mark.parametrize("b,p,rank,s,M", ODD_PERIODS)
 def test_monarch_odd_periods_and_interleaved_output_stage(b, p, rank, s, M, dtype, ring_forced):
     from test_gpu_monarch_lowrank_dense import _ref_monarch, _run_monarch, monarch_inputs
     from triton_funcs import _lib as L
@@ -185,6 +190,11 @@ def test_monarch_odd_periods_and_interleaved_output_stage(b, p, rank, s, M, dtyp
         out = _run_monarch("triton_monarch_right_fp16", x, w1_t, w2_t, dtype, "tiled")
     v = ref + rounded(bias, dtype)
     assert_close(out, v / (1.0 + np.exp(-v)), dtype, f"monarch period {rank // b}, bias and SiLU", scale=2.0)
+    gate, resid = np.random.default_rng(M).standard_normal((-(-M // 3), b * s)), np.random.default_rng(M + 1).standard_normal((M, b * s))
+    with L.fused_epilogue(dev(bias, dtype), None, gate=dev(gate, dtype), gate_rows=3, residual=dev(resid, dtype)):
+        out = _run_monarch("triton_monarch_right_fp16", x, w1_t, w2_t, dtype, "tiled")
+    want = rounded(resid, dtype) + np.repeat(rounded(gate, dtype), 3, axis=0)[:M] * v
+    assert_close(out, want, dtype, f"monarch period {rank // b}, bias, gate and residual", scale=2.0)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
