@@ -51,11 +51,14 @@ def test_packed_factors_codes_bit_exact(b, p, q, r, bits, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("bits", [8, 4])
-# the launch for both factors: r at 256, 512 and 1024 and on either side (1028: back to a launch per factor), p at the rows that 128, 64 and
-# 32 row groups hold in 4, 8 and 16 registers, the last of them and one more; channel groups of 32 that are part empty; rows of codes in
-# stores of 16, 4 and 1 bytes
+# the launch for both factors: r at 256, 512 and 1024 and on either side (1028: back to a launch per factor); p at the last row that 128 row groups of V
+# hold (few columns), and with column chunks for every compute unit what 32 row groups hold in 4, 8 and 16 registers and one more (64 row
+# groups), what 64 hold and one more, columns that leave the last chunk part empty at 32 and at 64 row groups; channel groups of 32 that are
+# part empty; rows of codes in stores of 16, 4 and 1 bytes
 @pytest.mark.parametrize("b,p,q,r", [(2, 128, 32, 256), (16, 256, 68, 128), (2, 129, 34, 260), (3, 513, 100, 516), (2, 1024, 40, 512), (2, 2048, 8, 1024),
-                                     (2, 2049, 36, 64), (3, 70, 72, 1028), (2, 5, 2, 4)])
+                                     (2, 2049, 36, 64), (3, 70, 72, 1028), (2, 5, 2, 4),
+                                     (64, 128, 8, 256), (64, 129, 8, 256), (32, 256, 8, 512), (32, 257, 8, 512), (16, 512, 8, 1024), (16, 513, 8, 1024),
+                                     (16, 1024, 8, 1024), (16, 1025, 8, 1024), (16, 512, 8, 1000), (16, 512, 8, 488)])
 def test_packed_in_one_launch_bit_exact(b, p, q, r, bits, dtype):
     test_packed_factors_codes_bit_exact(b, p, q, r, bits, dtype)
 
@@ -155,6 +158,7 @@ def test_blast_q_llama7b(layer, bits, M, dtype):
     uc, us = O.quantize_sym(U, 2, bits); vc, vs = O.quantize_sym(V, 1, bits)
     got_uc = Uq.codes.cpu().numpy() if bits == 8 else O.unpack_int4(Uq.codes.cpu().numpy())
     np.testing.assert_array_equal(got_uc.transpose(0, 2, 1), uc)      # U codes are stored (b, r, q)
+    np.testing.assert_array_equal(Vq.codes.cpu().numpy() if bits == 8 else O.unpack_int4(Vq.codes.cpu().numpy()), vc)
     np.testing.assert_array_equal(Uq.scales.cpu().numpy(), us)
     np.testing.assert_array_equal(Vq.scales.cpu().numpy(), vs)
     out = Q.triton_blast_bmm_int8_fp16(dev(x, dtype), Uq, Vq, dev(S, dtype))
