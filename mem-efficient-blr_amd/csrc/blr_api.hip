@@ -364,7 +364,10 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
   //   3/4 of that where output blocks are narrow (1152 -> 1152, r = 288 at 512 rows 27.3 against 23.4, at 768 rows 27.1 against 28.0);
   //   S (r, i, j): the same, but with input blocks that the fused first half takes as they are 80 x 1024 (1152 -> 3456, r = 288 at
   //   256 rows 18.3 against 17.0, at 384 rows 19.6 against 21.3; 2048 -> 8192, r = 768 at 144 rows 23.6 against 24.7), and not with 9 .. 15
-  //   blocks, whose mix has no fast kernel for that order (1536 -> 1536, b = 12, r = 256 at 260 rows 26.5 against 16.5 fused); as many blocks
+  //   blocks: that line is older than the mix kernel that such calls have now and lies too low for most of them (fused, or for an odd number of blocks
+  //   GEMM and mix, against three launches: 1536 -> 1536, b = 12, r = 256 at 129 / 260 / 400 / 600 rows 16.1 / 16.4 / 17.2 / 18.0 against 13.8 / 15.6 / 18.3 / 21.1;
+  //   1152 -> 6912, b = 9, r = 256 at 129 / 600 / 1000 rows 19.9 / 27.0 / 31.1 against 13.1 / 24.2 / 30.4; 1040 -> 1040, b = 10, r = 192 at 129 / 1000 rows 19.9 / 25.0
+  //   against 11.1 / 21.6; but 768 -> 3072, b = 12, r = 384 at 129 / 260 rows 14.1 / 15.5 against 14.9 / 18.9); as many blocks
   //   of that width with the rank contiguous: 5 x 2^15 (1152 -> 2304, b = 12, r = 128 at 1500 / 2000 rows 28.3 / 32.5 against 25.2 / 27.1).
   // Longer calls of tiny ranks are left to the fused kernels, which were fitted there.
   const bool narrow_out = b == 16 && Q % 8 == 0 && Q <= 80 && r % 32 == 0 && !silu_mul_armed();

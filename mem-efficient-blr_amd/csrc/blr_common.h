@@ -158,9 +158,10 @@ __device__ __forceinline__ void side_prep_item(const SidePrep& s, int64_t idx) {
 // w (outer, reduce, inner) contiguous; codes in the same order, scales (outer, inner).
 int quantize_launch(const void* w, int dtype, int64_t outer, int64_t reduce, int64_t inner, int bits, void* codes, void* scales, hipStream_t st);
 // w (outer, inner, reduce) contiguous; the same codes and scales, i.e. transposed on the way: codes (outer, reduce, inner).
+int quantize_t_launch(const void* w, int dtype, int64_t outer, int64_t reduce, int64_t inner, int bits, void* codes, void* scales, hipStream_t st);
+// Both factors of a BLAST layer, U (b, q, r) as quantize_t_launch(U, b, r, q) and V (b, p, r) as quantize_launch(V, b, p, r).
 int quantize_pair_launch(const void* U, const void* V, int dtype, int64_t b, int64_t q, int64_t p, int64_t r, int bits,
                          void* u_codes, void* u_scales, void* v_codes, void* v_scales, hipStream_t st);
-int quantize_t_launch(const void* w, int dtype, int64_t outer, int64_t reduce, int64_t inner, int bits, void* codes, void* scales, hipStream_t st);
 
 // ---- tiled GEMM (blr_gemm.hip) ----------------------------------------------------------
 enum { EPI_PLAIN = 0, EPI_MONARCH_SCATTER = 1 };

@@ -19,8 +19,9 @@
 // Phase 1 is bound by the address path (60 loads a wave at 72 columns per block), phase 2 by LDS and by the rate at which the chip
 // takes Z, and Y leaves no LDS for a second workgroup.  So with more tiles than compute units a workgroup walks several (WALK): the next
 // tile's first step is asked for before this one is mixed, the stores of Z drain under the next phase 1, and S is loaded once per
-// rank tile.  4096 rows, fp16, 16 blocks of 72, r = 576 and 288, mean of the two: 41.5 -> 37.5 us; whole calls 1152 -> 4608 79.9 -> 76.6,
-// 1152 -> 3456 47.8 -> 45.7, 1024 -> 8192 with r = 512 99.4 -> 83, 512 -> 4096 in 8 blocks with r = 1024 at 2000 rows 42.2 -> 40.
+// rank tile.  4096 rows, fp16, 16 blocks of 72, r = 576 and 288, mean of the two: 41.5 -> 37.5 us; whole calls, together with
+// what the choice of ranks per tile gave, 1152 -> 4608 87.9 -> 84.7, 1152 -> 3456 54.3 -> 51.9, 1024 -> 8192 with r = 512 109.6 -> 94.7, 768 -> 3072 with r = 1000
+// 131.6 -> 115.6, 512 -> 4096 in 8 blocks with r = 1024 at 2000 rows 46.8 -> 45.0 (factors from memory, one run; cards differ by a few per cent).
 // With one tile each there is nothing to walk, and the addresses kept for it cost 2 %: a kernel of its own.
 // What follows is an ordinary batched GEMM out_i = Z_i U_i.
 #include <hip/hip_runtime.h>
