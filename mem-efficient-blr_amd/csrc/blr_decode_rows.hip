@@ -364,18 +364,23 @@ __global__ __launch_bounds__(DR_NT) void rows_product_kernel(RowsParams p) {
 // weights are widened and multiplied in fp32: one row by multiply-adds, up to four by 4 x 4 x 1 matrix instructions, sixteen blocks at a
 // time, whose four columns are those of four neighbouring lanes (half the cycles of four multiply-adds: 4096 -> 22016, rank 1024 at four rows 21.2 -> 20.6 us,
 // 11008 -> 4096 19.0 -> 16.1).  Weights, chunks and rounds as above; each wave stages its share of the activations in LDS by itself (asked for
-// ahead of the weights), lane (n, g) sums its eight k of every step.  Bound by the latency of one trip to memory and, from two rows up, 12 cycles per
+// ahead of the weights), lane (n, g) sums its eight k of every step.  FOLD = 4, (k, n) weights in chunks of at most four pieces: only a quarter of the
+// lanes would have a piece, so four lanes share one and take a step each (low rank 3736 -> 1712, r = 376 at 2 / 4 rows 12.6 / 13.0 -> 11.3 / 11.4 us, Monarch 4096 ->
+// 4096, rank 1016 17.0 / 17.3 -> 13.7 / 13.9).  Bound by the latency of one trip to memory and, from two rows up, 12 cycles per
 // weight and lane that follow it.  Whole calls against the kernel above, which rounds: w2 (l, s, r), 4096 -> 22016, rank 1024 at 1 / 2 / 4 rows 18.2 / 18.3
-// / 18.5 -> 18.6 / 20.2 / 20.3 us (the phase engine: 29.4 / 38.0 / 58.3); low rank 3736 -> 1712, r = 376 10.8 / 10.9 / 11.1 -> 10.9 / 12.6 / 13.0 (24.0 / 32.6 /
+// / 18.5 -> 18.6 / 20.1 / 20.3 us (the phase engine: 29.4 / 38.0 / 58.3); low rank 3736 -> 1712, r = 376 10.8 / 10.8 / 10.9 -> 10.8 / 11.3 / 11.4 (24.0 / 32.6 /
 // 50.2).  Relative error against 64 bits, fp16 / bf16: 2.94e-4 / 2.35e-3 -> 2.07e-4 / 1.65e-3, what rounding the result alone gives.
-template <typename T, int STEPS, bool NK, int MR>
+template <typename T, int STEPS, bool NK, int MR, int FOLD>
 __global__ __launch_bounds__(DR_NT) void rows_product_f32_kernel(RowsParams p) {
   using Piece = RowsPiece<T, 16>;
   using V8 = typename TypeTraits<T>::vec8;
   constexpr int KW = 32 * STEPS, NA = MR * KW / 4, AP = (NA + 63) / 64;      // a wave's activations of a round: 16-byte pieces, and per lane
+  constexpr int ST = FOLD > 1 ? 1 : STEPS;                                   // steps of a lane
+  static_assert(FOLD == 1 || (FOLD == 4 && !NK), "four lanes per column piece and lane group share the (up to four) steps");
   __shared__ __attribute__((aligned(16))) float a_s[DR_WAVES][MR][KW];
   __shared__ __attribute__((aligned(16))) float red[DR_WAVES][MR][128];
-  const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, n = l & 15, g = l >> 4;
+  const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, n = l & (16 / FOLD - 1), g = l >> 4;
+  const int sl = FOLD > 1 ? (l >> 2) & 3 : 0;            // first step of this lane
   const uint32_t item = p.xcd_span ? (blockIdx.x & 7u) * p.xcd_span + (blockIdx.x >> 3) : blockIdx.x;
   const uint32_t bt = fd_div(item, p.nch), ch = item - bt * p.nch.d;
   const int N = p.N, K = p.K;
@@ -393,7 +398,7 @@ __global__ __launch_bounds__(DR_NT) void rows_product_f32_kernel(RowsParams p) {
   };
   for (int ro = 0; ro < p.rounds; ++ro) {
     const int k0 = (ro * DR_WAVES + wv) * KW;            // first of the wave's rows (rows past K: activations and weights read as zero)
-    u32x4 ap[AP], wr[STEPS][8];
+    u32x4 ap[AP], wr[ST][8];
 #pragma unroll
     for (int u = 0; u < AP; ++u) {
       const int i = u * 64 + l, m = i / (KW / 4), k = k0 + (i - m * (KW / 4)) * 4;
@@ -401,7 +406,7 @@ __global__ __launch_bounds__(DR_NT) void rows_product_f32_kernel(RowsParams p) {
       ap[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(abuf, off, 0, 0));
     }
 #pragma unroll
-    for (int s = 0; s < STEPS; ++s)
+    for (int s = 0; s < ST; ++s)
 #pragma unroll
       for (int t = 0; t < 8; ++t) asm volatile("" : "=v"(wr[s][t]));         // (as above: what is not asked for stays undefined and reaches no stored column)
     if constexpr (NK) {
@@ -409,16 +414,17 @@ __global__ __launch_bounds__(DR_NT) void rows_product_f32_kernel(RowsParams p) {
       for (int t = 0; t < 8; ++t) {
         if (t < p.npc) {
 #pragma unroll
-          for (int s = 0; s < STEPS; ++s) {
+          for (int s = 0; s < ST; ++s) {
             const int c = colp + 16 * t, k = k0 + 32 * s + 8 * g;
             wr[s][t] = Piece::load(wb, (c < N && k < K) ? (uint32_t)(c * K + k) * 2u : DR_OOB);
           }
         }
       }
     } else if (live) {
-      const uint32_t wbase = (uint32_t)((k0 + 8 * g) * N + colp) * 2u, rowb = (uint32_t)N * 2u;
+      const uint32_t rowb = (uint32_t)N * 2u;            // (a step past the wave's share reads as zero)
+      const uint32_t wbase = sl < STEPS ? (uint32_t)((k0 + 32 * sl + 8 * g) * N + colp) * 2u : DR_OOB;
 #pragma unroll
-      for (int s = 0; s < STEPS; ++s)
+      for (int s = 0; s < ST; ++s)
 #pragma unroll
         for (int t = 0; t < 8; ++t) wr[s][t] = Piece::load(wb, wbase + (uint32_t)(32 * s + t) * rowb);
     }
@@ -427,10 +433,13 @@ __global__ __launch_bounds__(DR_NT) void rows_product_f32_kernel(RowsParams p) {
       if (u * 64 + l < NA) *reinterpret_cast<u32x4*>(&a_s[wv][0][(u * 64 + l) * 4]) = ap[u];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");                   // (the wave's own LDS: its accesses are carried out in order)
 #pragma unroll
-    for (int s = 0; s < STEPS; ++s) {
-      const float* ar = &a_s[wv][l & (MR - 1)][32 * s + 8 * g];              // four rows: lane 4 i + m holds row m for its block of four columns
+    for (int s = 0; s < ST; ++s) {
+      const float* ar = &a_s[wv][l & (MR - 1)][32 * (FOLD > 1 ? min(sl, STEPS - 1) : s) + 8 * g];   // four rows: lane 4 i + m holds row m for its block of four columns
       const f32x4 lo = *reinterpret_cast<const f32x4*>(ar), hi = *reinterpret_cast<const f32x4*>(ar + 4);
-      const float a[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      float a[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      if (FOLD > STEPS && sl >= STEPS)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a[e] = 0.f;
 #pragma unroll
       for (int t = 0; t < 8; ++t) {
         if (NK && t >= p.npc) break;
@@ -461,8 +470,12 @@ __global__ __launch_bounds__(DR_NT) void rows_product_f32_kernel(RowsParams p) {
       v[e] += __shfl_xor(v[e], 16, 64);
       v[e] += __shfl_xor(v[e], 32, 64);
     }
+    if (FOLD > 1) {
+      v[e] += __shfl_xor(v[e], 4, 64);
+      v[e] += __shfl_xor(v[e], 8, 64);
+    }
   }
-  if (g < MR) {
+  if (g < MR && sl == 0) {
     if constexpr (NK) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) red[wv][g][16 * e + n] = v[e];
@@ -811,21 +824,23 @@ int rows_launch(RowsParams p, int batch, int dtype, int wbits, bool nk, hipStrea
   return dtype == BLR_F16 ? rows_launch_t<f16, 4>(p, batch, st) : rows_launch_t<bf16, 4>(p, batch, st);
 }
 
-template <typename T, bool NK, int MR>
+template <typename T, bool NK, int MR, int FOLD>
 int rows_f32_launch_t(const RowsParams& p, int batch, hipStream_t st) {
   const dim3 grid((unsigned)(batch * p.nch.d)), block(DR_NT);
   switch (p.kw / 32) {
-    case 1: hipLaunchKernelGGL((rows_product_f32_kernel<T, 1, NK, MR>), grid, block, 0, st, p); break;
-    case 2: hipLaunchKernelGGL((rows_product_f32_kernel<T, 2, NK, MR>), grid, block, 0, st, p); break;
-    case 3: hipLaunchKernelGGL((rows_product_f32_kernel<T, 3, NK, MR>), grid, block, 0, st, p); break;
-    default: hipLaunchKernelGGL((rows_product_f32_kernel<T, 4, NK, MR>), grid, block, 0, st, p); break;
+    case 1: hipLaunchKernelGGL((rows_product_f32_kernel<T, 1, NK, MR, FOLD>), grid, block, 0, st, p); break;
+    case 2: hipLaunchKernelGGL((rows_product_f32_kernel<T, 2, NK, MR, FOLD>), grid, block, 0, st, p); break;
+    case 3: hipLaunchKernelGGL((rows_product_f32_kernel<T, 3, NK, MR, FOLD>), grid, block, 0, st, p); break;
+    default: hipLaunchKernelGGL((rows_product_f32_kernel<T, 4, NK, MR, FOLD>), grid, block, 0, st, p); break;
   }
   BLR_CHECK_LAUNCH("rows_product_f32");
   return BLR_OK;
 }
 template <typename T, bool NK>
 int rows_f32_launch_m(const RowsParams& p, int batch, hipStream_t st) {
-  return p.M == 1 ? rows_f32_launch_t<T, NK, 1>(p, batch, st) : rows_f32_launch_t<T, NK, 4>(p, batch, st);
+  if constexpr (!NK)
+    if (p.npc <= 4) return p.M == 1 ? rows_f32_launch_t<T, NK, 1, 4>(p, batch, st) : rows_f32_launch_t<T, NK, 4, 4>(p, batch, st);
+  return p.M == 1 ? rows_f32_launch_t<T, NK, 1, 1>(p, batch, st) : rows_f32_launch_t<T, NK, 4, 1>(p, batch, st);
 }
 int rows_f32_launch(const RowsParams& p, int batch, int dtype, bool nk, hipStream_t st) {
   if (dtype == BLR_F16) return nk ? rows_f32_launch_m<f16, true>(p, batch, st) : rows_f32_launch_m<f16, false>(p, batch, st);
@@ -924,10 +939,10 @@ int decode_rows_launch(const StreamBlastArgs& a, void* region, size_t region_byt
   if (M < 1 || M > DR_MAX_M || (!monarch && !lowrank && !a.S) || (bo != b && !lowrank) || (u_nk && a.wbits != 16)) return 1;
   if (lowrank && a.wbits != 16) return 1;
   // A period that is no multiple of 4, w2 (l, r, s): 1408 -> 3584 in 16 blocks, rank 304 at 2 / 4 / 16 rows 12.4 / 18.5 / 23.6 us on the hand-over
-  // kernels, 10.2 / 10.4 / 8.0 here; 4096 -> 4096 in 4 blocks, rank 1016 at 3 / 4 / 5 / 16 rows 21.2 / 23.3 / 27.0 / 32.9 against 17.2 / 17.3 / 14.1 / 15.1.  At two rows
-  // the vector hand-over kernel is ahead with long periods, whose narrow column chunks leave most lanes of the fp32 product below idle: periods of 250 and
-  // more (4096 -> 4096 in 4 blocks, rank 1016 / 1512 / 2024 15.6 / 17.7 / 21.6 against 16.9 / 22.0 / 23.1; rank 760, a period of 190, 15.2 against 15.0).
-  if (monarch && a.perm_per % 4 && !u_nk && M == 2 && a.perm_per >= 250) return 1;
+  // kernels, 8.7 / 8.8 / 8.0 here; 4096 -> 4096 in 4 blocks, rank 1016 at 2 / 3 / 4 / 5 / 16 rows 15.6 / 21.2 / 23.3 / 27.0 / 32.9 against 13.7 / 13.8 / 13.9 / 14.1 / 15.1.
+  // At two rows the vector hand-over kernel is ahead where long periods meet output blocks whose column chunks do not fold (below): 4 blocks, rank 1016, of 2752 and 5504
+  // columns 14.4 against 15.3 and 15.7 against 17.0, but rank 760, a period of 190, 14.3 against 13.4 and 15.1 against 14.4.
+  if (monarch && a.perm_per % 4 && !u_nk && M == 2 && a.perm_per >= 250 && Q > 2048) return 1;
   if (monarch && (a.wbits != 16 || R % a.perm_per || R / a.perm_per != b || a.perm_per >= 65536)) return 1;
   if (a.wbits != 16 && (!a.u_scales || !a.v_scales)) return 1;
   if (a.dtype != BLR_F16 && a.dtype != BLR_BF16) return 1;

@@ -1320,7 +1320,7 @@ int stream_generic_launch(const StreamGenericArgs& a, hipStream_t st) {
       // From two rows up: the three-launch matrix-core path, low rank being BLAST with the input cut into 16 (or 8) slices of
       // rows of A, one output block and S = 1 (the mix is the sum over the slices).  Where there are fewer equal slices, 16 with a shorter last
       // one; where there are none, at one row too (one row with equal slices is the two-stage kernel's, below): 3736 -> 1712, r = 376 at 1 / 4 / 16
-      // rows 24.0 / 50.2 / 17.6 us on what follows, 10.9 / 13.0 / 11.0 here, 4104 -> 4096, r = 512 at one row 22.9 -> 11.5; 3728 inputs (two slices) at 4
+      // rows 24.0 / 50.2 / 17.6 us on what follows, 10.8 / 11.4 / 11.0 here, 4104 -> 4096, r = 512 at one row 22.9 -> 11.3; 3728 inputs (two slices) at 4
       // rows 15.3 -> 10.5; 920 -> 8000, r = 136 at 2 rows 25.5 -> 10.9.
       int bi = equal >= 8 ? equal : 0, slice = 0;
       if (!bi && a.in_f % 8 == 0) { slice = (int)cdiv(cdiv(a.in_f, 16), 8) * 8; bi = (int)cdiv(a.in_f, slice); }

@@ -164,14 +164,15 @@ def _small_integers(rng, *shape, top):
 
 
 # w2 (l, s, r) with more than 256 groups of 64 output columns and ranks up to 1024 (one row: 2048): whole 16-byte pieces of the period and not, one to four
-# steps of a round, two rounds, sliced input blocks (1104, 1040 and 2048 rows); w2 (l, r, s) with a period that is no multiple of 4; low rank without equal slices
+# steps of a round, two rounds, sliced input blocks (1104, 1040 and 2048 rows); w2 (l, r, s) with a period that is no multiple of 4, in column
+# chunks of up to four pieces, whose lanes share the steps, and wider; low rank without equal slices
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
 @pytest.mark.parametrize("name,b,p,rank,s", [("triton_monarch_right_fp16", *c) for c in [(4, 512, 1024, 4200), (16, 88, 304, 1032), (16, 8, 16, 1040), (16, 1040, 48, 1032),
                                                                                          (12, 40, 744, 1416), (2, 1104, 176, 8200), (4, 8, 2048, 4104)]]
                          + [("triton_monarch_right_ideal_fp16", 4, 2048, 512, 4104)]
                          + [("triton_monarch_right_left_fp16", *c) for c in [(16, 88, 304, 224), (16, 8, 16, 8), (16, 1040, 48, 40), (8, 136, 1032, 72), (12, 40, 744, 136),
-                                                                         (4, 1024, 1016, 72), (4, 64, 1032, 40), (4, 2752, 8, 8)]]
+                                                                         (4, 1024, 1016, 72), (4, 64, 1032, 40), (4, 2752, 8, 8), (4, 64, 760, 1376), (4, 64, 1016, 2056), (4, 64, 232, 1032)]]
                          + [("low_rank", 1, *c) for c in [(3736, 376, 1712), (8, 8, 8), (72, 16, 40), (4088, 1032, 136), (11000, 2056, 72)]])
 def test_intermediate_stays_in_fp32_up_to_four_rows(name, b, p, rank, s, M, dtype):
     """Whole numbers and halves of them down to 2^-k whose sums fp32 holds exactly in any order, the intermediate among them, which takes up to 14 bits:
