@@ -104,7 +104,8 @@ void blr_set_spin_limit(unsigned polls);
 /* The run-time switches of the library (no counterpart in the reference), all of them: the GEMM variant - BLR_GEMM_RING
  * (0..2), BLR_GEMM_RING_TILE (0, 256256, 256128, 256096, 128128), BLR_GEMM_RING_PER_CU (0..2), BLR_GEMM_RING_WAVES (4, 8),
  * BLR_GEMM_RING_BK (32, 64: k per operand stage), BLR_GEMM_SPLITK (0, 1), BLR_GEMM_MID (0..6: small tiles for products that do
- * not fill the chip - 0 never, 1 by estimate, 2..6 always 32x64, 32x64 deep, 64x64, 64x64 deep, 64x128) - and kernel families on / off - BLR_DECODE2, BLR_DECODE3, BLR_DECODE_ROWS, BLR_DENSE_SLAB,
+ * not fill the chip - 0 never, 1 by estimate, 2..6 always 32x64, 32x64 deep, 64x64, 64x64 deep, 64x128), BLR_GEMM_WIDE (0, 1, 3..11: tiles
+ * of 256 x 96 .. 352 for products of more tiles than compute units - 0 never, 1 by estimate, 3..11 always that many times 32 columns) - and kernel families on / off - BLR_DECODE2, BLR_DECODE3, BLR_DECODE_ROWS, BLR_DENSE_SLAB,
  * BLR_BLAST_ONE, BLR_BLAST_YMIXW (0, 1), BLR_DECODE_PAIR, BLR_BLAST_MIXU (0..2); a family that is off hands its calls to the
  * next one that serves them.  BLR_DENSE_ROWS (0, 1) is accepted and has no effect: its kernels are gone.  Each starts from the environment variable of its name (read once; a value out of range is
  * ignored); unset != 0 returns it to "not set".  Returns BLR_ERR_BAD_ARG for an unknown name or a value out of range.  */

@@ -99,10 +99,10 @@ unsigned spin_limit_now();
 bool epilogue_pending(const void** bias, int* act);   // (false when a gate or a residual is armed: only the tiled path fuses those)
 void epilogue_taken();
 // Every run-time switch of the library (blr_set_option): each starts from the environment variable of its name, read once, and
-// is range-checked where it is set.  The first six pick the GEMM variant, the rest switch a kernel family off (0) so that the
+// is range-checked where it is set.  The first eight pick the GEMM variant, the rest switch a kernel family off (0) so that the
 // call falls through to the next one that serves it - for A/B measurements and as a way out should a kernel misbehave.
 // (OPT_DENSE_ROWS has no reader: the name is still taken from programs that set it.)
-enum { OPT_GEMM_RING = 0, OPT_GEMM_RING_TILE, OPT_GEMM_RING_PER_CU, OPT_GEMM_RING_WAVES, OPT_GEMM_RING_BK, OPT_GEMM_SPLITK, OPT_GEMM_MID,
+enum { OPT_GEMM_RING = 0, OPT_GEMM_RING_TILE, OPT_GEMM_RING_PER_CU, OPT_GEMM_RING_WAVES, OPT_GEMM_RING_BK, OPT_GEMM_SPLITK, OPT_GEMM_MID, OPT_GEMM_WIDE,
        OPT_DECODE2, OPT_DECODE3, OPT_DECODE_PAIR, OPT_DECODE_ROWS, OPT_DENSE_SLAB, OPT_DENSE_ROWS, OPT_BLAST_MIXU, OPT_BLAST_ONE, OPT_BLAST_YMIXW, OPT_COUNT };
 int option_value(int id, int dflt);             // the option's value, or dflt when it is unset
 // true when p is aligned to `bytes`.
@@ -200,6 +200,11 @@ bool gemm_mid_ok(const GemmArgs& a, int dtype); // whether the operands suit kin
 int gemm_mid_launch(const GemmArgs& a, int kind, bool partial, int dtype, hipStream_t st);
 int gemm_mid_f32_slices(int M, int N, int K);   // slices that the reduction of a single fp32 product is worth cutting into
 int gemm_mid_f32_launch(const GemmArgs& a, bool partial, hipStream_t st);
+// Kernels for products of more tiles than compute units, on tiles of 256 x 32 tn (blr_gemm_wide.hip): whether they take the operands, the tn
+// (3 .. 11) for the shape - or, where ring64, 0 .. 2 for a ring kernel that is faster -, and the launch.
+bool gemm_wide_ok(const GemmArgs& a);
+int gemm_wide_plan(const GemmArgs& a, bool ring64);
+int gemm_wide_launch(const GemmArgs& a, int tn, int dtype, hipStream_t st);
 // Scratch a plain single GEMM M x N x K of dtype wants in GemmArgs::splitk_ws so that a problem with few output tiles and
 // a long reduction can be cut along K to fill the chip (fp32 partial results, summed in a fixed order).  0: no split.
 size_t gemm_splitk_bytes(int M, int N, int K, int dtype);

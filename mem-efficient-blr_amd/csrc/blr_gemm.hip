@@ -1330,6 +1330,7 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
   // Products with at most one 128 x 128 tile per compute unit, or of at most 128 rows: smaller tiles, and slices of a long reduction, by the estimates of
   // blr_gemm_mid.hip.  BLR_GEMM_MID = 0 switches that off, 2 .. 6 asks for one of its five tiles wherever the operands allow it.
   const int mid = option_value(OPT_GEMM_MID, 1);
+  const bool forced_wide = option_value(OPT_GEMM_WIDE, 1) > 1 && gemm_wide_ok(g);
   if (mid > 1 && gemm_mid_ok(g, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16)) return gemm_mid_launch(g, mid - 2, false, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16, st);
   const int64_t r128_all = cdiv(g.M, 128) * cdiv(g.N, 128) * g.batch;
   // Interleaved columns with work for more than half of the compute units, whole row tiles and a reduction of some length: the rules
@@ -1338,7 +1339,7 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
   // -> 24.2 / 24.8 / 29.1, 4096 -> 4096 in 4 blocks, r = 1024 at 1000 rows 43.9 -> 36.7; but 768 -> 2304, r = 128 at 1300 rows 14.1 against 15.1,
   // 1152 -> 1152, r = 288 at 1500 rows 17.1 against 21.4 with 105 tiles' worth of results, 2048 -> 8192 in 16 blocks at 260 rows 25.5 against 28.0).
   const bool interleaved = g.cn != 1 && g.K >= 256 && (int64_t)g.M * g.N * g.batch * 2 > (int64_t)cus * 128 * 128 && (int64_t)g.M * 8 >= cdiv(g.M, 128) * 128 * 7;
-  if (mid == 1 && ring == 1 && (r128_all <= cus || g.M <= 128) && !interleaved && option_value(OPT_GEMM_RING_TILE, 0) == 0) {
+  if (mid == 1 && ring == 1 && !forced_wide && (r128_all <= cus || g.M <= 128) && !interleaved && option_value(OPT_GEMM_RING_TILE, 0) == 0) {
     constexpr int dt = std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16;
     const bool rk = g.cn == 1 && g.M >= 96 && g.K >= 64 && !ring_scatter_odd(g) && ring_ok(g), mk = gemm_mid_ok(g, dt);
     bool cut = option_value(OPT_GEMM_SPLITK, 1) != 0 && mk && g.cn == 1 && g.epi == EPI_PLAIN && g.splitk_ws && aligned(g.splitk_ws, 16) && g.batch == 1 && !g.sat8 && !g.pair &&
@@ -1358,6 +1359,15 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
     if (pl.kind == MID_RING_128) return launch_ring64<T, 128, 128, 4, 3, 1>(g, st);
     if (pl.kind == MID_RING_128_TWO) return launch_ring64<T, 128, 128, 4, 2, 2>(g, st);
     if (pl.kind >= 0) return gemm_mid_launch(g, pl.kind, false, dt, st);
+  }
+  // More tiles than compute units: the width of the tile, or one of the ring kernels with stages of 64 k, by the estimates of blr_gemm_wide.hip
+  // (BLR_GEMM_WIDE: 0 never, 1 by this rule, 3 .. 11 tiles of that many times 32 columns for every product that the kernels take).
+  const int wide = option_value(OPT_GEMM_WIDE, 1);
+  const bool ring_asked = ring != 1 || option_value(OPT_GEMM_RING_TILE, 0) || option_value(OPT_GEMM_RING_PER_CU, 0) || option_value(OPT_GEMM_RING_WAVES, 0) || option_value(OPT_GEMM_RING_BK, 0);
+  if (wide && (wide > 1 || !ring_asked) && gemm_wide_ok(g)) {
+    const int w = wide > 1 ? wide : gemm_wide_plan(g, ring_ok(g) && g.epi == EPI_PLAIN);
+    if (w >= 3) return gemm_wide_launch(g, w, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16, st);
+    return w == 0 ? launch_ring64<T, 128, 128, 4, 2, 2>(g, st) : w == 1 ? launch_ring64<T, 256, 128, 8, 3, 1>(g, st) : launch_ring64<T, 256, 256, 8, 2, 1>(g, st);
   }
   if (g.pair && (!ring_ok(g) || g.epi != EPI_PLAIN || g.cn != 1 || g.sat8 || g.gate || g.resid || g.pair_dA % 8 || g.pair_dB % 8 || g.pair_dbias % 8 || !aligned(g.C, 16))) {
     set_error("gemm: a pair of tiles (SiLU-gated halves) needs 16-byte aligned operands, K and the half width multiples of 8, a plain row-major output");

@@ -1,0 +1,124 @@
+"""GPU parity of the GEMM on tiles of 256 rows x 96 .. 352 columns (csrc/blr_gemm_wide.hip) against the oracle.
+
+BLR_GEMM_WIDE = 3 .. 11 asks for tiles of that many times 32 columns for every product that the kernels take, so the edges of every width are met
+on small problems: one row or column more or less than a tile, reductions that end inside a stage of 64 k (with 8 .. 56 k left over),
+more tiles than compute units (a workgroup walks several), the output stage, gated halves and Monarch's scatter.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import blr_oracle as O
+from gpu_util import assert_close, blast_inputs, dev, rounded, say, ulp
+
+pytestmark = pytest.mark.gpu
+
+TILED = {"algo": 2}
+WIDTHS = list(range(3, 12))
+
+
+def _product_close(out, x, w, dtype, what):
+    """One rounding of a sum in fp32: half a unit of dtype, and K roundings of fp32 of the terms' absolute sum."""
+    ref, mag = x @ w, np.abs(x) @ np.abs(w)
+    err = np.abs(out.double().cpu().numpy() - ref)
+    bound = 0.5 * ulp(ref, dtype) * (1 + 2.0 ** -9) + x.shape[1] * 2.0 ** -24 * mag
+    assert (err <= bound).all(), f"{what}: {np.max(err / bound):.3f} of the bound"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tn", WIDTHS)
+def test_dense_ragged_tiles(tn, dtype):
+    from triton_funcs import dense_kernels as K, _lib as L
+    w32 = 32 * tn
+    for m, k, n in ((256, 128, w32), (257, 72, w32 + 8), (255, 136, w32 - 8), (31, 1000, 2 * w32 - 24), (513, 192, 8), (300, 120, 3 * w32 + 16), (40, 352, w32)):
+        rng = np.random.default_rng(m + k + tn)
+        x, w = rounded(rng.standard_normal((m, k)), dtype), rounded(rng.standard_normal((k, n)) / np.sqrt(k), dtype)
+        say(f"[case] wide dense tn={tn} {m}x{n}x{k} {dtype}")
+        with L.options(BLR_GEMM_WIDE=tn):
+            out = K.triton_dense_fp16(dev(x, dtype), dev(w, dtype), TILED)
+        _product_close(out, x, w, dtype, f"{m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("tn", WIDTHS)
+def test_workgroups_that_walk_several_tiles(tn):
+    """More than two tiles for most of 256 compute units, the last ones ragged in rows and columns; every kind of last stage."""
+    from triton_funcs import dense_kernels as K, _lib as L
+    dtype = torch.float16
+    for k in (72, 128, 168):
+        m, n = 256 * 8 + 19, 32 * tn * 66 + 24
+        g = torch.Generator("cuda").manual_seed(tn + k)
+        x = torch.randn(m, k, device="cuda", generator=g).to(dtype)
+        w = (torch.randn(k, n, device="cuda", generator=g) / k ** 0.5).to(dtype)
+        say(f"[case] wide dense tn={tn} {m}x{n}x{k}, several tiles a workgroup")
+        with L.options(BLR_GEMM_WIDE=tn):
+            out = K.triton_dense_fp16(x, w, TILED)
+        ref, mag = x.float() @ w.float(), x.float().abs() @ w.float().abs()        # (fp32 itself adds k roundings on this side)
+        err = (out.float() - ref).abs()
+        assert (err <= 2.0 ** -11 * 1.01 * ref.abs() + 2 * k * 2.0 ** -24 * mag + 2.0 ** -24).all(), f"tn={tn} k={k}: {float(err.max())}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tn", WIDTHS)
+def test_blast_and_low_rank_through_wide_tiles(tn, dtype):
+    """Batches, both orders of the second operand, and a side job of the first product (16 blocks, narrow outputs)."""
+    from triton_funcs import blast_kernels as K, low_rank_kernels as LR, _lib as L
+    for b, p, q, r, m in ((4, 80, 40, 72, 300), (2, 176, 264, 136, 257), (16, 136, 72, 96, 130)):
+        x, U, Vt, S = blast_inputs(b, p, q, r, (m,), seed=b + m)
+        ref = O.blast_forward(rounded(x, dtype), rounded(U, dtype), rounded(Vt, dtype), rounded(S, dtype))[0]
+        for name, lay in (("triton_blast_full_fp16", O.blast_to_partial_layout), ("triton_blast_bmm_fp16", O.blast_to_bmm_layout)):
+            Uk, Vk, Sk = lay(U, Vt, S)
+            say(f"[case] wide {name} tn={tn} b={b} p={p} q={q} r={r} m={m} {dtype}")
+            with L.options(BLR_GEMM_WIDE=tn):
+                out = getattr(K, name)(dev(x, dtype), dev(Uk, dtype), dev(Vk, dtype), dev(Sk, dtype), TILED)
+            assert_close(out, ref, dtype, name)
+
+
+@pytest.mark.parametrize("tn", WIDTHS)
+def test_output_stage_and_gated_halves(tn):
+    from triton_funcs import dense_kernels as D, _lib as L
+    dtype = torch.float16
+    for m, k, n in ((300, 136, 32 * tn + 40), (256 * 5 + 3, 72, 32 * tn * 60 + 8)):
+        g = torch.Generator("cuda").manual_seed(m + tn)
+        rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
+        x, w, bias, resid = rnd(m, k), rnd(k, 2 * n), rnd(2 * n), rnd(m, n)
+        w = (w.float() / k ** 0.5).to(dtype)
+        gate = rnd(-(-m // 7), n)
+        say(f"[case] wide output stage tn={tn} {m}x{n}x{k}")
+        y = (x.double() @ w.double()).half().double() + bias.double()               # the result is rounded before the bias is added
+        h = torch.nn.functional.gelu(y[:, :n], approximate="tanh").half().double()
+        ref = resid.double() + gate.double().repeat_interleave(7, 0)[:m] * h
+        with L.options(BLR_GEMM_WIDE=tn), L.fused_epilogue(bias[:n].contiguous(), "gelu_tanh", gate=gate, gate_rows=7, residual=resid):
+            out = D.triton_dense_fp16(x, w[:, :n].contiguous(), TILED)
+        assert_close(out, ref.cpu().numpy(), dtype, "gate and residual")
+        with L.options(BLR_GEMM_WIDE=tn), L.fused_epilogue(bias, "silu_mul"):
+            out = D.triton_dense_fp16(x, w, TILED)
+        ref = torch.nn.functional.silu(y[:, :n]).half().double() * y[:, n:].half().double()
+        assert_close(out, ref.cpu().numpy(), dtype, "gated halves")
+
+
+@pytest.mark.parametrize("tn", WIDTHS)
+def test_monarch_scatter(tn):
+    """A permutation writes every value where the other kernels write it."""
+    from triton_funcs import monarch_kernels as K, _lib as L
+    dtype = torch.float16
+    for b, p, rank, s, m in ((4, 96, 160, 72, 300), (2, 80, 32 * tn, 40, 257), (16, 128, 384, 24, 270)):
+        g = torch.Generator("cuda").manual_seed(b + tn)
+        rnd = lambda *sh: torch.randn(*sh, device="cuda", generator=g).to(dtype)
+        x, w1, w2 = rnd(1, m, b * p), (rnd(b, p, rank).float() / p ** 0.5).to(dtype), (rnd(b, rank, s).float() / rank ** 0.5).to(dtype)
+        say(f"[case] wide monarch tn={tn} b={b} p={p} rank={rank} s={s} m={m}")
+        with L.options(BLR_GEMM_WIDE=tn):
+            out = K.triton_monarch_right_left_fp16(x, w1, w2, TILED)
+        with L.options(BLR_GEMM_WIDE=0):
+            ref = K.triton_monarch_right_left_fp16(x, w1, w2, TILED)
+        assert_close(out, ref.double().cpu().numpy(), dtype, "monarch", scale=0.5)
+
+
+@pytest.mark.parametrize("k", [72, 88, 120, 184])
+def test_infinite_weights_stay_infinite(k):
+    """The last stage of a reduction is read again from before its start: what it shares with the stage before counts once, infinities too."""
+    from triton_funcs import dense_kernels as K, _lib as L
+    x, w = np.ones((40, k)), np.ones((k, 96))
+    w[k - 64, 3] = w[k - 1, 5] = w[0, 7] = w[63, 9] = np.inf
+    with L.options(BLR_GEMM_WIDE=3):
+        out = K.triton_dense_fp16(dev(x, torch.float16), dev(w, torch.float16), TILED).double().cpu().numpy()
+    assert (out == x @ w).all()
