@@ -423,14 +423,11 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
     rc = 1;
   }
   const bool mixu = mixu_shape && (mixu_mode >= 2 || (mixu_mode == 1 && (P > fuse_max_p || fused < 0)));
-  // Wide input blocks (16 of them, a multiple of 64 columns each, rank a multiple of 64): x V as one GEMM whose 64 x 64 tile keeps Y
-  // of all 16 blocks in registers, then the mix, in one launch (blast_ymixw_kernel) - by itself from half a round of tiles on
-  // (whole calls, before -> after: 4096 -> 4096, r = 512 at 1024 / 2048 / 4096 rows 47.1 -> 46.1 / 65.7 -> 56.3 / 101.9 -> 96.2 us,
-  // at 512 rows 40.1 -> 44.3; 4096 -> 22016, r = 1024 at 512 / 1024 / 2048 / 4096 rows 78.6 -> 77.7 / 114.4 -> 104.3 / 179.5 -> 174.0 /
-  // 350.6 -> 344.2 us, at 256 rows 55.2 -> 59.3).  BLR_BLAST_YMIXW=0 switches it off; BLR_ALGO_FUSED asks for it at any row count.
-  const int cus_now = device_cus() > 0 ? device_cus() : 256;
-  const bool ymixw_fill = cdiv(M, 64) * (int64_t)(r / 64) * 2 >= cus_now;
-  if (!mixu && !y_out && !sat8 && fused >= 0 && P > fuse_max_p && option_value(OPT_BLAST_YMIXW, 1) && (fused == 1 || ymixw_fill))
+  // Wide input blocks (16 of them, a multiple of 64 columns each, rank a multiple of 64): x V as one GEMM whose 64 x 64 tile keeps Y of all
+  // 16 blocks in registers, then the mix, in one launch (blast_ymixw_kernel).  Only where the caller asks for the fused algorithm: the
+  // product on wide tiles and the mix on the matrix cores take no longer (the six linears of a Llama-7B block at 2048 rows 481 us with it, 450 without; 5120 -> 5120,
+  // r = 640 at 2048 rows 69 and 53, 8192 -> 2048, r = 768 85 and 59, 4096 -> 4096, r = 512 at 3000 rows 68 and 59, at 1000 rows and below level).
+  if (!mixu && !y_out && !sat8 && fused == 1 && P > fuse_max_p && option_value(OPT_BLAST_YMIXW, 1))
     rc = blast_ymixw_launch(x, ldx, V, S, Z, M, in_f, b, r, si, sj, sr, s_layout, dtype, Y, ybytes, st);
   if (rc < 0) return rc;
   if (rc == 1 && !mixu && !y_out && !sat8 && fused >= 0 && (fused == 1 || P <= fuse_max_p))

@@ -224,6 +224,8 @@ int blast_ymix_launch(const void* x, int64_t ldx, const void* V, const void* S, 
 int blast_ymixw_launch(const void* x, int64_t ldx, const void* V, const void* S, void* Z, int M, int in_f, int b, int R,
                       int64_t s_si, int64_t s_sj, int64_t s_sr, int s_layout, int dtype, void* scratch, size_t scratch_bytes,
                       hipStream_t st);
+// The mix alone on the matrix cores (blr_prefill.hip).  Same return convention.
+int blast_mixm_launch(const void* Y, const void* S, void* Z, int M, int b, int R, int64_t s_si, int64_t s_sj, int64_t s_sr, int dtype, hipStream_t st);
 // The mix at few rows (blr_decode_rows.hip), two-byte types: same result, Y re-read from the L2 by one thread per four or eight ranks.
 int rows_mix_launch(const void* Y, const void* S, void* Z, int M, int b, int R, int s_layout, int dtype, hipStream_t st);
 int rows_mix_try(const void* Y, const void* S, void* Z, int M, int b, int R, int64_t si, int64_t sj, int64_t sr, int dtype, hipStream_t st);   // 1: not taken

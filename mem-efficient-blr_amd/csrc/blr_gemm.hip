@@ -1742,6 +1742,10 @@ int blast_mix_launch(const void* Y, const void* S, void* Z, int M, int b, int R,
       return BLR_OK;
     }
   }
+  if (M > 16 && !sat8) {
+    const int rc = blast_mixm_launch(Y, S, Z, M, b, R, s_si, s_sj, s_sr, dtype, st);
+    if (rc != 1) return rc;
+  }
   const int vw = dtype == BLR_F32 ? 4 : 8;
   if (b <= 16 && R % vw == 0 && aligned(Y, 16) && aligned(Z, 16)) {
     const int r_chunks = (int)cdiv(R, 8 * vw);

@@ -303,6 +303,137 @@ __global__ __launch_bounds__(YM_NT) void blast_ymix_kernel(YmixParams p) {
   TR6(14);
 }
 
+// ---- the mix on its own: Z_i = sum_j S(i, j, r) Y_j for two-byte types, 4 / 8 / 12 / 16 blocks, ranks in pieces of eight -------------------------
+// For one rank the mix is a b x b product with the rows: one 16 x 16 x 16 matrix instruction per rank and 16 rows, as in the kernels around it, which
+// leaves the kernel to the memory: Y once in, Z once out.  (The kernels in blr_gemm.hip do it on the vector units, b x 8 multiply-adds per
+// 16 bytes: with the arithmetic of bf16 in fp32 that was what bound them.)  A workgroup of eight waves takes 32 rows x 64 ranks of all blocks:
+// whole 128-byte lines straight into LDS, 64 KB for 16 blocks, so two workgroups share a compute unit and one's loads run under the other's
+// stores.  Wave w owns ranks 8 w .. 8 w + 7.  Lane (n, g) reads Y_j, j = 4 g .. 4 g + 3, of row n - 16 bytes are its eight ranks -, turns them
+// into one operand per rank (byte permutes), and its products are Z_i, i = 4 g .. 4 g + 3, of the same row and ranks: they go back where
+// the lane read Y.  Nothing crosses waves but the loads and the stores of whole rows on either side.  S is kept in registers along the row tiles
+// that a workgroup walks; with the rank contiguous it comes through the same LDS, as (r, i, j) straight in operand order.
+// 16 blocks, r = 1024 at 2048 rows (134 MB in and out): 32.9 -> 24.4 us = 5.5 TB/s, the rate of a device copy; bf16 24.6.
+struct MixmParams {
+  const void* Y; const void* S; void* Z;
+  int M, b, R;
+  int64_t s_si, s_sj;           // strides of S where the rank is contiguous (RIJ: not used)
+  FastDiv nmt;                  // row tiles
+  int items;                    // rank tiles x row tiles
+};
+// eight ranks x four blocks: v[t] = 8 ranks of block t -> one operand (four blocks) per rank
+__device__ __forceinline__ void mixm_turn(const u32x4 (&v)[4], u32x2 (&o)[8]) {
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const uint32_t sel = (q & 1) ? 0x07060302u : 0x05040100u;
+    o[q][0] = __builtin_amdgcn_perm(v[1][q >> 1], v[0][q >> 1], sel);
+    o[q][1] = __builtin_amdgcn_perm(v[3][q >> 1], v[2][q >> 1], sel);
+  }
+}
+template <typename T, bool RIJ>
+__global__ __launch_bounds__(512, 4) void blast_mixm_kernel(MixmParams p) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char mx_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g = lane >> 4, b = p.b, M = p.M, R = p.R;
+  const uint32_t wg = xcd_item(blockIdx.x, gridDim.x), G = gridDim.x;
+  uint32_t item = (uint32_t)((uint64_t)wg * (uint32_t)p.items / G);
+  const uint32_t item_end = (uint32_t)((uint64_t)(wg + 1) * (uint32_t)p.items / G);
+  const uint32_t lds0 = ring_lds_addr(mx_lds);
+  // piece c of row r (128 bytes) of a plane lies at c ^ ((r >> 1) & 7): 16 rows' pieces of one number then lie in different banks
+  const int r8 = lane >> 3;                            // a load or store instruction of a wave: eight rows, eight lanes each
+  const bool live = 4 * g < b;                         // (4 g + 3 < b as well: b is a multiple of four)
+  u32x2 sa[8];
+  uint32_t rt_have = ~0u;
+  for (; item < item_end; ++item) {
+    const uint32_t rt = fd_div(item, p.nmt);
+    const int m0 = (int)(item - rt * p.nmt.d) * 32, r0 = (int)rt * 64;
+    const int piece = r0 + wave * 8;
+    if (rt != rt_have) {
+      rt_have = rt;
+      if constexpr (RIJ) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          sa[q] = u32x2{0u, 0u};
+          if (live && n < b && piece < R) sa[q] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const T*>(p.S) + ((int64_t)(piece + q) * b + n) * b + 4 * g);
+        }
+      } else {                                         // rows (i, j) of the tile's 64 ranks, i b + j; b b is a multiple of 16
+        for (int k = wave; k * 8 < b * b; k += 8) {
+          const int row = k * 8 + r8, i = row / b, j = row - i * b, c = (lane & 7) ^ ((row >> 1) & 7);
+          ring_load_lds(p.S, (uint32_t)((i * p.s_si + j * p.s_sj + min(r0 + c * 8, R - 8)) * 2), lds0 + k * 1024);
+        }
+        __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));
+        lds_barrier();
+        u32x4 v[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int row = n * b + 4 * g + t;
+          v[t] = u32x4{0u, 0u, 0u, 0u};
+          if (live && n < b) v[t] = *reinterpret_cast<const u32x4*>(mx_lds + row * 128 + ((wave ^ ((row >> 1) & 7)) << 4));
+        }
+        mixm_turn(v, sa);
+        lds_barrier();                                 // read by every wave
+      }
+    }
+    // in: plane j, rows 8 k .. 8 k + 7 (four instructions a plane)
+    for (int k = wave; k < 4 * b; k += 8) {
+      const int row = (k & 3) * 8 + r8, c = (lane & 7) ^ ((row >> 1) & 7);
+      ring_load_lds(p.Y, (uint32_t)(((int64_t)(k >> 2) * M + min(m0 + row, M - 1)) * R + min(r0 + c * 8, R - 8)) * 2u, lds0 + k * 1024);
+    }
+    __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));         // (S of this tile as well)
+    lds_barrier();
+#pragma unroll
+    for (int mg = 0; mg < 2; ++mg) {
+      unsigned char* const at = mx_lds + 4 * g * 4096 + (mg * 16 + n) * 128 + ((wave ^ ((n >> 1) & 7)) << 4);
+      u32x4 v[4];
+      u32x2 yb[8];
+      f32x4 d[8];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        v[t] = u32x4{0u, 0u, 0u, 0u};
+        if (live) v[t] = *reinterpret_cast<const u32x4*>(at + t * 4096);
+      }
+      mixm_turn(v, yb);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) d[q] = YmDot<T>::mfma16(sa[q], yb[q], f32x4{0.f, 0.f, 0.f, 0.f});
+      if (live) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          *reinterpret_cast<u32x4*>(at + t * 4096) = u32x4{ym_pack<T>(d[0][t], d[1][t]), ym_pack<T>(d[2][t], d[3][t]), ym_pack<T>(d[4][t], d[5][t]), ym_pack<T>(d[6][t], d[7][t])};
+      }
+    }
+    lds_barrier();
+    for (int k = wave; k < 4 * b; k += 8) {
+      const int row = (k & 3) * 8 + r8, c = (lane & 7) ^ ((row >> 1) & 7);
+      const u32x4 z = *reinterpret_cast<const u32x4*>(mx_lds + k * 1024 + lane * 16);
+      if (m0 + row < M && r0 + c * 8 < R) *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.Z) + ((int64_t)(k >> 2) * M + m0 + row) * R + r0 + c * 8) = z;
+    }
+    lds_barrier();                                     // the rows have been read: the next tile may land
+  }
+}
+
+// Returns BLR_OK, a negative blr_status, or 1 when the kernel does not take the operands.
+int blast_mixm_launch(const void* Y, const void* S, void* Z, int M, int b, int R, int64_t s_si, int64_t s_sj, int64_t s_sr, int dtype, hipStream_t st) {
+  if ((dtype != BLR_F16 && dtype != BLR_BF16) || b < 4 || b > 16 || b % 4 || R % 8 || !aligned(Y, 16) || !aligned(Z, 16)) return 1;
+  const int64_t lim = (int64_t)1 << 31;
+  if ((int64_t)b * M * R * 2 >= lim) return 1;
+  const bool rij = s_sj == 1 && s_si == b && s_sr == (int64_t)b * b && aligned(S, 8);
+  const bool run = s_sr == 1 && s_si % 8 == 0 && s_sj % 8 == 0 && s_si >= 0 && s_sj >= 0 && aligned(S, 16) && ((b - 1) * (s_si + s_sj) + R) * 2 < lim;
+  if (!rij && !run) return 1;
+  MixmParams p = {};
+  p.Y = Y; p.S = S; p.Z = Z; p.M = M; p.b = b; p.R = R; p.s_si = s_si; p.s_sj = s_sj;
+  const int nrt = (int)cdiv(R, 64), nmt = (int)cdiv(M, 32);
+  if ((int64_t)nrt * nmt >= 65536 || nmt >= 65536) return 1;
+  p.nmt = fd_make((uint32_t)nmt);
+  p.items = nrt * nmt;
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  const unsigned grid = (unsigned)(p.items < 2 * cus ? p.items : 2 * cus);
+  void* const fn = dtype == BLR_F16 ? (rij ? (void*)blast_mixm_kernel<f16, true> : (void*)blast_mixm_kernel<f16, false>)
+                                    : (rij ? (void*)blast_mixm_kernel<bf16, true> : (void*)blast_mixm_kernel<bf16, false>);
+  void* args[] = {&p};
+  const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(512), args, (size_t)b * 4096, st);
+  if (e != hipSuccess) { set_error("blast_mixm: launch failed: %s", hipGetErrorString(e)); return BLR_ERR_LAUNCH; }
+  return BLR_OK;
+}
+
 // S(i, j, r) with any strides -> St[(r b + i) b + j]: one thread per (i, r), neighbouring threads on neighbouring ranks.
 template <typename T>
 __global__ __launch_bounds__(256) void ym_s_transpose_kernel(const T* __restrict__ S, T* __restrict__ St, int b, int R,
