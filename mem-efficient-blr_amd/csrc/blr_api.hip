@@ -400,10 +400,12 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
     rc = 1;
   }
   // Nobody asked for Y: x V and the mix can run as one launch with Y kept inside the compute units (BLR_ALGO_FUSED).  Chosen
-  // by itself only for narrow input blocks: the fused kernel re-reads V once per 32 rows, and from about 128 columns per
-  // block on that costs more than the round trip of Y it saves (measured at 4096 rows: 1152 -> 1152, r = 288: 64 against
-  // 68 us; 4608 -> 1152, r = 576: 154 against 122 us; Llama-7B gate_up at 2048 rows: 201 against 186 us).
-  constexpr int fuse_max_p = 128;
+  // by itself only for narrow input blocks: the fused kernel re-reads V once per 32 rows, and that must cost less than the round trip of Y that
+  // it saves.  Whole calls, fused against the product on wide tiles and the mix alone: 2048 -> 8192 in 16 blocks of 128, r = 768 at 2000 / 4096 rows
+  // 60.6 / 113.9 and 60.9 / 120.7 us, 1152 -> 4608 in 16 of 72, r = 576 38.4 / 63.4 and 43.5 / 73.7; but 3072 -> 3072 in 16 of 192, r = 768 61.1 / 105.2
+  // and 53.3 / 101.0.  With fewer blocks Y is smaller beside V's rows: 1536 -> 3072 in 8 of 192, r = 256 23.2 / 31.7 and 27.9 / 34.1, 640 -> 2560 in 4 of 160,
+  // r = 256 17.4 / 24.5 and 20.4 / 28.6, 1024 -> 4096 in 4 of 256, r = 512 27.5 / 44.8 and 31.5 / 42.2.
+  const int fuse_max_p = b <= 8 ? 192 : 128;
   // Narrow output blocks (either layout of U: it is re-laid for the kernel anyway): the mix and the product with U run as one launch that reads Y once and
   // never writes Z (blast_mixu_kernel); the first half is then the plain GEMM, which leaves Y.  Measured at 4096 rows against the
   // mix kernel + batched GEMM: 4608 -> 1152, r = 576: 90 against 122 us; against the fused first half + batched GEMM: 1152 -> 1152,
@@ -431,7 +433,7 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
     rc = blast_ymixw_launch(x, ldx, V, S, Z, M, in_f, b, r, si, sj, sr, s_layout, dtype, Y, ybytes, st);
   if (rc < 0) return rc;
   if (rc == 1 && !mixu && !y_out && !sat8 && fused >= 0 && (fused == 1 || P <= fuse_max_p))
-    rc = blast_ymix_launch(x, ldx, V, S, Z, M, in_f, b, r, si, sj, sr, s_layout, dtype, Y, ybytes, st);   // (the unused room of Y holds S transposed)
+    rc = blast_ymix_launch(x, ldx, V, S, Z, M, in_f, b, r, si, sj, sr, dtype, Y, ybytes, st);   // (the unused room of Y holds S as (r, i, j) if it has to)
   if (rc < 0) return rc;
   if (rc == 1 && fused == 1) { set_error("blast: the fused kernel does not take this shape (b even and <= 16, block width and rank multiples of 8, f16/bf16)"); return BLR_ERR_UNSUPPORTED; }
   if (rc == 1) {

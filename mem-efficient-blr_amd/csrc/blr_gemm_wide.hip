@@ -38,10 +38,6 @@ constexpr int min2(int a, int b) { return a < b ? a : b; }
 __device__ __forceinline__ void ring_load_lds_if(const void* base, uint32_t off, uint32_t lds, int go) {
   asm volatile("s_cmp_eq_u32 %3, 0\n\ts_cbranch_scc1 .Lskip%=\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n.Lskip%=:" ::"s"(lds), "v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(go)) : "memory", "scc");
 }
-// s_waitcnt vmcnt(N) where some is not zero, vmcnt(0) where it is
-template <int N> __device__ __forceinline__ void wait_loads(int some) {
-  asm volatile("s_cmp_eq_u32 %0, 0\n\ts_cbranch_scc1 .Lall%=\n\ts_waitcnt vmcnt(%1)\n\ts_branch .Lend%=\n.Lall%=:\n\ts_waitcnt vmcnt(0)\n.Lend%=:" ::"s"(__builtin_amdgcn_readfirstlane(some)), "n"(N) : "memory", "scc");
-}
 
 constexpr int WIDE_BM = 256;
 // (k, n) stage: chunk c of row k lies at position c ^ wide_swz(k).  A transposing read takes 32 bytes of each of rows 8 g .. 8 g + 3, g = 0 .. 3: the four
@@ -172,7 +168,7 @@ __global__ __launch_bounds__(512, 2) void gemm_wide_kernel(GemmArgs g, int tiles
   };
   auto handover = [&](int stores) {                    // this stage is in registers, the next one has landed
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    wait_loads<2 * TN>(stores);
+    ring_wait_loads<2 * TN>(stores);
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };

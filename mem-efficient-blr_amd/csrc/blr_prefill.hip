@@ -1,29 +1,10 @@
-// BLAST at more than 16 rows, first half: Z = mix(S, x V) in one launch, with Y = x V never leaving the compute unit.
+// BLAST above 16 rows: the kernels around the products.
 //
-//   Z[i][m][r] = sum_j S(i, j, r) * Y_j[m][r],      Y_j = x_j V_j   (x_j: columns j P .. (j+1) P of x, V_j (P, R))
+//   Z[i][m][r] = sum_j S(i, j, r) * Y_j[m][r],      Y_j = x_j V_j   (x_j: columns j P .. (j+1) P of x, V_j (P, R)),      out_i = Z_i U_i
 //
-// The unfused path writes Y (b, M, R) to memory, reads it back in a mix kernel and writes Z: three passes over an
-// intermediate that is larger than every operand.  Here a workgroup owns a tile of 32 rows x up to 128 ranks for ALL
-// input blocks j and ALL output blocks i:
-//   phase 1  each of the eight waves computes Y_j of the tile for two input blocks on the matrix cores.  V is row-major
-//            (rank contiguous) and the matrix cores want eight consecutive k of one column per lane, so a lane loads its
-//            16-byte piece of eight rows and product e takes element e of each (byte permutes; the column slots of
-//            product e are the ranks 8 n + e).  Loads go straight to registers, two k-steps in flight.  The two Y_j of a
-//            wave leave as (Y_2w, Y_2w+1) pairs of T, one dword per (m, r), into LDS.
-//   phase 2  for one rank r the mix is a 16 x 16 matrix product over the input blocks, Z_r (i, m) = S_r (i, j) Y_r (j, m),
-//            i.e. one matrix-core instruction per rank and 16 rows.  Its operands want four consecutive j per lane: Y
-//            gives them as two of its pair dwords from LDS, S as eight contiguous bytes when it is stored (r, i, j) -
-//            the layout of the bmm names; any other layout is transposed once per call into scratch by a small kernel.
-//            A wave takes 16 ranks of the tile, keeps the products of eight ranks in registers and stores 16 bytes of
-//            Z per (i, m).  Z leaves as T.
-// Phase 1 is bound by the address path (60 loads a wave at 72 columns per block), phase 2 by LDS and by the rate at which the chip
-// takes Z, and Y leaves no LDS for a second workgroup.  So with more tiles than compute units a workgroup walks several (WALK): the next
-// tile's first step is asked for before this one is mixed, the stores of Z drain under the next phase 1, and S is loaded once per
-// rank tile.  4096 rows, fp16, 16 blocks of 72, r = 576 and 288, mean of the two: 41.5 -> 37.5 us; whole calls, together with
-// what the choice of ranks per tile gave, 1152 -> 4608 87.9 -> 84.7, 1152 -> 3456 54.3 -> 51.9, 1024 -> 8192 with r = 512 109.6 -> 94.7, 768 -> 3072 with r = 1000
-// 131.6 -> 115.6, 512 -> 4096 in 8 blocks with r = 1024 at 2000 rows 46.8 -> 45.0 (factors from memory, one run; cards differ by a few per cent).
-// With one tile each there is nothing to walk, and the addresses kept for it cost 2 %: a kernel of its own.
-// What follows is an ordinary batched GEMM out_i = Z_i U_i.
+// For one rank r the mix is a 16 x 16 product over the input blocks, Z_r (i, m) = S_r (i, j) Y_r (j, m): one matrix instruction per rank and 16
+// rows.  blast_mixm_kernel is the mix alone, blast_ymix_kernel forms Y_j in the compute unit for narrow input blocks, blast_ymixw_kernel for
+// wide ones, blast_mixu_kernel continues with the product with U where output blocks are narrow, and blast_one_kernel does all three.
 #include <hip/hip_runtime.h>
 #include <cmath>
 #include <type_traits>
@@ -34,8 +15,6 @@
 namespace blr {
 
 namespace {
-constexpr int YM_NT = 512;
-constexpr int YM_BM = 32;
 constexpr uint32_t YM_OOB = 0x80000000u;
 }  // namespace
 
@@ -45,17 +24,6 @@ __device__ unsigned long long g_trace6[1024 * 16];
 #else
 #define TR6(i) do {} while (0)
 #endif
-
-struct YmixParams {
-  const void* x; int64_t ldx; uint32_t x_bytes;
-  const void* V; const void* S; void* Z;
-  int M, b, P, R;
-  int npc;                      // 16-byte rank pieces of a tile (1..16): the tile spans BR = 8 npc ranks
-  int ksteps;                   // 32-row k-steps that cover P
-  FastDiv nmt;                  // row tiles
-  int items;                    // rank tiles x row tiles
-  const void* St;               // S as (r, i, j), the input block contiguous
-};
 
 template <typename T> struct YmDot;
 template <> struct YmDot<f16> {
@@ -85,223 +53,6 @@ __device__ __forceinline__ uint32_t ym_pack(float lo, float hi) {
 
 // a barrier that orders LDS and leaves loads and stores of memory in flight
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-template <typename T, bool STAGE, bool WALK>
-__global__ __launch_bounds__(YM_NT) void blast_ymix_kernel(YmixParams p) {
-  extern __shared__ __attribute__((aligned(16))) uint32_t ym_lds[];
-  int tid = threadIdx.x;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int n = tid & 15, g = (tid >> 4) & 3;
-  const int b = p.b, P = p.P, R = p.R, M = p.M, BR = p.npc * 8, JP = b >> 1;
-  // Y pairs (Y_2jp, Y_2jp+1) as [jp][m][r]: rows padded by 4 dwords and input-block planes by 16, so that the 16-byte
-  // writes of phase 1 stay aligned and the reads of phase 2 (16 rows x 4 planes of one rank) spread over the banks
-  const int RS = BR + 4, JS = YM_BM * RS + 16;
-  uint32_t* y_s = ym_lds;
-  // A workgroup walks a run of tiles.  Tiles of one rank tile follow each other, within a run and within an XCD: its slice of V stays in
-  // that L2 while the rows stream, and S in the registers.
-  const uint32_t wg = xcd_item(blockIdx.x, gridDim.x), G = gridDim.x;
-  uint32_t item = (uint32_t)((uint64_t)wg * (uint32_t)p.items / G);
-  const uint32_t item_end = (uint32_t)((uint64_t)(wg + 1) * (uint32_t)p.items / G);
-  uint32_t rt = fd_div(item, p.nmt);
-  int m0 = (int)(item - rt * p.nmt.d) * YM_BM, r0 = (int)rt * BR;
-  TR6(0);
-  // the mix's S operands depend on nothing and are used after phase 1: asked for behind the first loads of phase 1 (the
-  // memory pipeline takes an instruction every 16 cycles, and the products can only start on those first loads).  Lane (n, g)
-  // of wave wv: S_r(i = n, j = 4 g .. 4 g + 3) for the wave's 16 ranks r0 + 16 wv ..; waves without ranks in the tile ask nothing
-  const __amdgpu_buffer_rsrc_t sbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.St), 0, (uint32_t)((int64_t)b * b * R * 2), 0x00020000);
-  const int rw = wv * 16;
-  u32x2 sa[16];
-  auto load_sa = [&]() {
-    const bool a_ok = n < b && 4 * g < b;
-    if (rw < BR) {
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int r = r0 + rw + q;
-        const uint32_t off = (a_ok && rw + q < BR && r < R) ? (uint32_t)(((int64_t)r * b + n) * b + 4 * g) * 2u : YM_OOB;
-        sa[q] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(sbuf, off, 0, 0));
-      }
-    }
-  };
-
-  // ---------------------------------------------- phase 1: Y pairs into LDS ----------------------------------------------
-  // One pipeline over the k-steps of the wave's two input blocks (no drain between them): step q < KS belongs to block
-  // 2 wv, step q >= KS to block 2 wv + 1; the accumulators of the first block are packed away at the boundary.
-  // step s of a block covers k = 32 s .. 32 s + 31; this lane holds k = 32 s + 8 g .. + 7 of row 16 mg + n (x) and of its
-  // rank piece (V).  No branch around the loads (the compiler then waits for exactly the step it needs): what lies
-  // outside - rows past M, k past P, lanes without a rank piece - asks for an offset out of bounds and reads zeros.
-  const int KS = p.ksteps;                                   // 32-row steps per input block
-  const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, p.x_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t vbuf = wbuf(reinterpret_cast<const T*>(p.V) + (int64_t)(2 * (wv < JP ? wv : 0)) * P * R, (uint32_t)((int64_t)2 * P * R * 2));
-  u32x4 a0[2], a1[2], b0[8], b1[8];
-  auto load_ab = [&](u32x4 (&a)[2], u32x4 (&bb)[8], int q) {
-    const int jj = q >= KS ? 1 : 0, sst = q - jj * KS;
-    const int k = 32 * sst + 8 * g;
-    const bool kin = k < P, live = n < p.npc && r0 + n * 8 < R;
-#pragma unroll
-    for (int mg = 0; mg < 2; ++mg) {
-      const int m = m0 + 16 * mg + n;
-      const uint32_t off = (m < M && kin) ? (uint32_t)((int64_t)m * p.ldx + (int64_t)(2 * wv + jj) * P + k) * 2u : YM_OOB;
-      a[mg] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xbuf, off, 0, 0));
-    }
-    const uint32_t base = (live && kin) ? (uint32_t)((jj * P + k) * R + r0 + n * 8) * 2u : YM_OOB;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) bb[t] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vbuf, base + (uint32_t)(t * R) * 2u, 0, 0));
-  };
-  if (wv < JP) load_ab(a0, b0, 0);
-  load_sa();
-  TR6(1);
-  for (;;) {
-    if (WALK) asm volatile("" : "+v"(tid), "+v"(n), "+v"(g));         // addresses are formed again for each tile: kept, they would not fit beside the operands
-    if (wv < JP) {
-      uint32_t h0[2][4][4];                                   // Y of the wave's first input block, packed two ranks to a dword
-      f32x4 acc[2][8];
-#pragma unroll
-      for (int mg = 0; mg < 2; ++mg)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[mg][e] = f32x4{0.f, 0.f, 0.f, 0.f};
-      auto step = [&](const u32x4 (&a)[2], const u32x4 (&bb)[8]) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
-          u32x4 bv;
-#pragma unroll
-          for (int h = 0; h < 4; ++h) bv[h] = __builtin_amdgcn_perm(bb[2 * h + 1][e >> 1], bb[2 * h][e >> 1], sel);
-#pragma unroll
-          for (int mg = 0; mg < 2; ++mg) acc[mg][e] = YmDot<T>::mfma(a[mg], bv, acc[mg][e]);
-        }
-      };
-      auto next_block = [&]() {                                // pack away the first block's Y, start the second from zero
-#pragma unroll
-        for (int mg = 0; mg < 2; ++mg)
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) h0[mg][t][q] = ym_pack<T>(acc[mg][2 * q][t], acc[mg][2 * q + 1][t]);
-#pragma unroll
-        for (int mg = 0; mg < 2; ++mg)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) acc[mg][e] = f32x4{0.f, 0.f, 0.f, 0.f};
-      };
-      int q = 0;
-      for (; q + 2 < 2 * KS; q += 2) {                         // two steps per trip (the two register sets take turns)
-        if (q == KS) next_block();
-        load_ab(a1, b1, q + 1);
-        step(a0, b0);
-        if (q + 1 == KS) next_block();
-        load_ab(a0, b0, q + 2);
-        step(a1, b1);
-      }
-      // the last trip on its own: nothing is left to ask for behind it (ten loads that would all be out of bounds still cost
-      // their turns in the memory pipeline)
-      if (q == KS) next_block();
-      load_ab(a1, b1, q + 1);
-      step(a0, b0);
-      if (q + 1 == KS) next_block();
-      step(a1, b1);
-      TR6(2);
-      // acc[mg][e][t] is Y of block 2 wv + 1 at [m0 + 16 mg + 4 g + t][r0 + 8 n + e]; h0 holds block 2 wv
-      if (n < p.npc) {
-#pragma unroll
-        for (int mg = 0; mg < 2; ++mg)
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            uint32_t pr[8];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const uint32_t h1 = ym_pack<T>(acc[mg][2 * q][t], acc[mg][2 * q + 1][t]);
-              pr[2 * q] = __builtin_amdgcn_perm(h1, h0[mg][t][q], 0x05040100u);          // rank 8 n + 2 q:     (Y_2w, Y_2w+1)
-              pr[2 * q + 1] = __builtin_amdgcn_perm(h1, h0[mg][t][q], 0x07060302u);      // rank 8 n + 2 q + 1
-            }
-            uint32_t* dst = &y_s[wv * JS + (16 * mg + 4 * g + t) * RS + n * 8];
-            *reinterpret_cast<u32x4*>(dst) = u32x4{pr[0], pr[1], pr[2], pr[3]};
-            *reinterpret_cast<u32x4*>(dst + 4) = u32x4{pr[4], pr[5], pr[6], pr[7]};
-          }
-      }
-    }
-    TR6(3);
-    // the next tile's first step flies while this one is mixed and stored: phase 1 is bound by the address path, phase 2 by LDS and by
-    // the chip's write rate, and one workgroup's LDS leaves no room for a second one whose phases would fill the gaps
-    const int mt0 = m0, rt0 = r0;                              // this tile's origin
-    const bool more = WALK && ++item < item_end;
-    const uint32_t rt_next = more ? fd_div(item, p.nmt) : rt;
-#pragma unroll
-    for (int q = 0; WALK && q < 16; ++q) asm volatile("" : "+v"(sa[q]));    // S has arrived by now: said here, or the products of phase 2 wait for the next tile's loads with it
-    if (more) {
-      m0 = (int)(item - rt_next * p.nmt.d) * YM_BM;
-      r0 = (int)rt_next * BR;
-      if (wv < JP) load_ab(a0, b0, 0);
-    }
-    lds_barrier();
-    TR6(4);
-
-    // ---------------------------------------------- phase 2: the mix ----------------------------------------------------------
-    // lane (n, g): operand A = S_r(i = n, j = 4 g .. 4 g + 3), operand B = Y_r(j = 4 g .. 4 g + 3, m = 16 mg + n); the
-    // product's lane holds Z_r(i = 4 g + t, m = 16 mg + n), t = 0..3
-    // A lane's 16 bytes of Z belong to a row (i, m) of their own: stored from here, an instruction touches 64 cache lines and
-    // holds the memory pipeline eight times as long as one that writes whole rows (5.3 of a workgroup's 15 us were these
-    // stores).  STAGE: the 16 rows of a product group go through LDS behind Y ([i][m][rank], 16 lanes per row) and leave as
-    // runs of BR ranks; without (the tile's Y leaves no room for that) the lanes store their pieces themselves.
-    const bool b_ok = 2 * g < JP;
-    const int ZRS = BR / 2 + 4;                                // dwords per staged row
-    uint32_t* const z_st = ym_lds + JP * JS;
-#pragma unroll
-    for (int mg = 0; mg < 2; ++mg) {
-      if (STAGE && mg == 1) lds_barrier();     // the first group's rows have been read
-      if (rw < BR) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {                          // eight ranks at a time
-          if (rw + 8 * h < BR) {
-            f32x4 d[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-              const int rr = rw + 8 * h + q;
-              u32x2 yb = {0u, 0u};
-              if (b_ok) {
-                const uint32_t* src = &y_s[(2 * g) * JS + (16 * mg + n) * RS + rr];
-                yb[0] = src[0]; yb[1] = src[JS];
-              }
-              d[q] = YmDot<T>::mfma16(sa[8 * h + q], yb, f32x4{0.f, 0.f, 0.f, 0.f});
-            }
-            const int m = mt0 + 16 * mg + n, r = rt0 + rw + 8 * h;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              const int i = 4 * g + t;
-              u32x4 o;
-#pragma unroll
-              for (int q = 0; q < 4; ++q) o[q] = ym_pack<T>(d[2 * q][t], d[2 * q + 1][t]);
-              if (STAGE) {
-                if (i < b) *reinterpret_cast<u32x4*>(&z_st[(i * 16 + n) * ZRS + (rw + 8 * h) / 2]) = o;
-              } else if (m < M && r < R && i < b) {
-                *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.Z) + ((int64_t)i * M + m) * R + r) = o;
-              }
-            }
-          }
-        }
-      }
-      if (STAGE) {
-        lds_barrier();
-        const int pc = tid & 15, r = rt0 + pc * 8;
-        if (pc < p.npc && r < R) {                           // 32 rows per pass: output blocks 2 it, 2 it + 1
-          const int rr = tid >> 4, m = mt0 + 16 * mg + (rr & 15);
-          u32x4 v[8];
-#pragma unroll
-          for (int it = 0; it < 8; ++it)
-            if (2 * it < b) v[it] = *reinterpret_cast<const u32x4*>(&z_st[(rr + 32 * it) * ZRS + pc * 4]);
-          if (m < M) {
-#pragma unroll
-            for (int it = 0; it < 8; ++it)
-              if (2 * it + (rr >> 4) < b) *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.Z) + ((int64_t)(2 * it + (rr >> 4)) * M + m) * R + r) = v[it];
-          }
-        }
-      }
-    }
-    if (!more) break;
-    // Y is free for the next tile: its last reads lie before the barrier in front of the last stores (STAGE), or before this one
-    if (!STAGE) lds_barrier();
-    if (rt_next != rt) { rt = rt_next; load_sa(); }
-  }
-  TR6(14);
-}
 
 // ---- the mix on its own: Z_i = sum_j S(i, j, r) Y_j for two-byte types, 4 / 8 / 12 / 16 blocks, ranks in pieces of eight -------------------------
 // For one rank the mix is a b x b product with the rows: one 16 x 16 x 16 matrix instruction per rank and 16 rows, as in the kernels around it, which
@@ -434,6 +185,218 @@ int blast_mixm_launch(const void* Y, const void* S, void* Z, int M, int b, int R
   return BLR_OK;
 }
 
+// ---- Z = mix(S, x V) in one launch for narrow input blocks ----------------------------------------------------------------------------------------
+// The tile and the mix of blast_mixm_kernel, with Y made on the spot: 32 rows x 64 ranks of all blocks.  Four waves, wave w makes Y_j for j = w, w + 4, ..:
+// the block's 32 rows of x and its rows of V, at most 96 columns of the block at a time, come as whole lines into a piece of LDS of the wave's
+// own and from there - V through transposing reads - into registers, whereupon the next block's loads go out under the products.  Nothing waits for
+// another wave until all of Y is in registers (16 per block); then Y goes to LDS, over what the blocks came through, and the mix and the way out are
+// those of blast_mixm_kernel.  64 - 80 KB of LDS: two workgroups share a compute unit and fill each other's waits.
+// What bounds it: a wave's chain of trips to the L2, one per block, and the chip's write rate (4096 rows, 16 blocks of 72, r = 576: 75 MB out).  Before, a
+// workgroup of eight waves held 32 rows x 96 - 128 ranks in 150 KB of LDS, read x and V straight into registers, 60 loads of half lines a
+// wave and tile, and had its compute unit to itself.  Whole calls, before -> now: 1152 -> 4608, r = 576 at 2000 / 4096 rows 43.0 / 69.5 -> 38.4 / 63.4 us,
+// 1024 -> 8192, r = 512 45.0 / 74.8 -> 37.4 / 64.0, 2048 -> 8192, r = 768 at 4096 127.1 -> 113.9, 768 -> 3072, r = 1000 99.4 -> 86.8, 512 -> 2048 in 4 blocks, r = 512
+// 32.5 -> 28.2; 0.93 x in the mean over 49 calls of 12 layers at 150 .. 4096 rows, 1.05 x at worst (768 -> 3072, r = 1000 at 600 rows).
+struct YmixParams {
+  MixmParams m;                 // Y not used
+  const void* x; int64_t ldx; const void* V;
+  int P, PP;                    // columns of a block, and of a piece of it (a multiple of 8, at most 96)
+  int slot;                     // bytes of LDS of a wave
+  FastDiv cl;                   // chunks of a row of x in LDS
+};
+template <typename T, bool RIJ, int NB, int KS>        // NB = b / 4; KS: steps of 32 columns that cover a piece
+__global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char ym_lds[];
+  using V8 = typename TypeTraits<T>::vec8;
+  constexpr int b = 4 * NB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int n = lane & 15, g = lane >> 4;
+  const int M = p.m.M, R = p.m.R, P = p.P, PP = p.PP;
+  const uint32_t wg = xcd_item(blockIdx.x, gridDim.x), G = gridDim.x;
+  uint32_t item = (uint32_t)((uint64_t)wg * (uint32_t)p.m.items / G);
+  const uint32_t item_end = (uint32_t)((uint64_t)(wg + 1) * (uint32_t)p.m.items / G);
+  int r8 = lane >> 3;
+  const bool live = g < NB;
+  // x of a block: 32 rows of cl chunks of 16 bytes, cl odd (16 rows' chunks of one number then lie in different banks); V behind it as it lies,
+  // chunk c of row k at c ^ (k & 2) << 1 ^ (k & 8) >> 2 (see the (k, n) stages of blr_gemm_wide.hip)
+  const int cl = (PP / 8) | 1, xi = (cl + 1) / 2;      // 32 cl chunks are cl / 2 KiB
+  unsigned char* const own = ym_lds + wave * p.slot;
+  const uint32_t own0 = ring_lds_addr(own), lds0 = ring_lds_addr(ym_lds);
+  u32x2 sa[2][8];
+  uint32_t rt_have = ~0u;
+  int m0, r0;
+  constexpr int XI = 2 * KS + 1;                       // (at most: 32 (4 KS + 1) chunks)
+  uint32_t v_off[2], x_off[XI];                        // v_off: rows 0 .. 7 of an even and of an odd group of eight
+  auto ask = [&](int j, int k0) {                      // columns k0 .. k0 + PP - 1 of block j
+    const char* xb = reinterpret_cast<const char*>(p.x) + ((int64_t)m0 * p.ldx + (int64_t)j * P + k0) * 2;
+    const char* vb = reinterpret_cast<const char*>(p.V) + ((int64_t)j * P + k0) * R * 2;
+#pragma unroll
+    for (int i = 0; i < XI; ++i)
+      if (i < xi) ring_load_lds(xb, x_off[i], own0 + i * 1024);
+#pragma clang loop unroll(disable)
+    for (int i = 0; i * 8 < PP; ++i) ring_load_lds(vb + (int64_t)i * 16 * R, v_off[i & 1], own0 + (xi + i) * 1024);
+  };
+  auto begin = [&]() {                                 // a tile: S if its ranks are new, and the wave's first piece is asked for
+    asm volatile("" : "+v"(n), "+v"(g), "+v"(r8));   // addresses are formed again for each tile: kept, they would not fit beside Y
+    const uint32_t rt = fd_div(item, p.m.nmt);
+    m0 = (int)(item - rt * p.m.nmt.d) * 32;
+    r0 = (int)rt * 64;
+    if (rt != rt_have) {
+      rt_have = rt;
+      if constexpr (RIJ) {
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            const int r = r0 + (wave + 4 * cc) * 8 + q;
+            sa[cc][q] = u32x2{0u, 0u};
+            if (live && n < b && r < R) sa[cc][q] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const T*>(p.m.S) + ((int64_t)r * b + n) * b + 4 * g);
+          }
+      } else {
+        for (int k = wave; k * 8 < b * b; k += 4) {
+          const int row = k * 8 + r8, i = row / b, j = row - i * b, c = (lane & 7) ^ ((row >> 1) & 7);
+          ring_load_lds(p.m.S, (uint32_t)((i * p.m.s_si + j * p.m.s_sj + min(r0 + c * 8, R - 8)) * 2), lds0 + k * 1024);
+        }
+        __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));
+        lds_barrier();
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc) {
+          u32x4 v[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const int row = n * b + 4 * g + t;
+            v[t] = u32x4{0u, 0u, 0u, 0u};
+            if (live && n < b) v[t] = *reinterpret_cast<const u32x4*>(ym_lds + row * 128 + (((wave + 4 * cc) ^ ((row >> 1) & 7)) << 4));
+          }
+          mixm_turn(v, sa[cc]);
+        }
+        lds_barrier();
+      }
+    }
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+      const int c = (lane & 7) ^ ((r8 & 2) << 1 | o << 1);
+      v_off[o] = (uint32_t)((r8 * R + min(r0 + c * 8, R - 8)) * 2);
+    }
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+      const uint32_t L = min(i * 64 + r8 * 8 + (int)(lane & 7), 32 * cl - 1), row = fd_div(L, p.cl);
+      x_off[i] = (uint32_t)min((int)row, M - 1 - m0) * (uint32_t)(p.ldx * 2) + min(L - row * cl, (uint32_t)PP / 8 - 1) * 16;
+      asm volatile("" : "+v"(x_off[i]));
+    }
+    ask(wave, 0);
+  };
+  if (item >= item_end) return;
+  begin();
+  int stores = 0;                                      // whether 4 NB stores of the tile before are younger than the loads
+  for (;;) {
+    u32x2 y[NB][4][2];
+#pragma unroll
+    for (int jb = 0; jb < NB; ++jb) {
+      f32x4 acc[4][2];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c][0] = acc[c][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma clang loop unroll(disable)
+      for (int at = 0; at < P; at += PP) {             // a last piece that would end past the block begins earlier: what the one before had of it is zero
+        asm volatile("" : "+v"(n), "+v"(g));
+        const int skip = max(at + PP - P, 0);
+        V8 xf[KS][2], vf[KS][4];
+        ring_wait_loads<4 * NB>(stores);
+        stores = 0;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          const int kc = min(4 * s + g, PP / 8 - 1);                               // the lane's eight k, or the last ones there are
+#pragma unroll
+          for (int x = 0; x < 2; ++x) xf[s][x] = *reinterpret_cast<const V8*>(own + ((16 * x + n) * cl + kc) * 16);
+          const int k = 8 * kc + (n >> 2), swz = (k & 2) << 1 | (k & 8) >> 2;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            union { V8 v; s16x4 h[2]; } w;
+            const unsigned char* src = own + xi * 1024 + k * 128 + (((2 * c + ((n & 3) >> 1)) ^ swz) << 4) + (n & 1) * 8;
+            w.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(src));
+            w.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(src + 512));
+            vf[s][c] = w.v;
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        {                                              // the piece is in registers: the next one may come
+          const int j = at + PP < P ? wave + 4 * jb : wave + 4 * (jb + 1);
+          if (j < b) ask(j, at + PP < P ? min(at + PP, P - PP) : 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+          if (32 * s + 8 * g >= PP || 32 * s + 8 * g < skip) {                     // zero on both sides
+            xf[s][0] = xf[s][1] = V8{};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) vf[s][c] = V8{};
+          }
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int x = 0; x < 2; ++x) acc[c][x] = TypeTraits<T>::mfma16(vf[s][c], xf[s][x], acc[c][x]);
+        }
+      }
+      // acc[c][x]: row 16 x + n, ranks 16 c + 4 g .. + 3
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int x = 0; x < 2; ++x) y[jb][c][x] = u32x2{ym_pack<T>(acc[c][x][0], acc[c][x][1]), ym_pack<T>(acc[c][x][2], acc[c][x][3])};
+    }
+    lds_barrier();                                     // nobody reads x and V any more
+#pragma unroll
+    for (int jb = 0; jb < NB; ++jb)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          const int m = 16 * x + n;
+          *reinterpret_cast<u32x2*>(ym_lds + (wave + 4 * jb) * 4096 + m * 128 + (((2 * c + (g >> 1)) ^ ((m >> 1) & 7)) << 4) + (g & 1) * 8) = y[jb][c][x];
+        }
+    lds_barrier();
+    // ---- the mix and the way out, as above, with two pieces of eight ranks a wave ----
+#pragma unroll
+    for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+      for (int mg = 0; mg < 2; ++mg) {
+        __builtin_amdgcn_sched_barrier(0);
+        unsigned char* const at = ym_lds + 4 * g * 4096 + (mg * 16 + n) * 128 + (((wave + 4 * cc) ^ ((n >> 1) & 7)) << 4);
+        u32x4 v[4];
+        u32x2 yb[8];
+        f32x4 d[8];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          v[t] = u32x4{0u, 0u, 0u, 0u};
+          if (live) v[t] = *reinterpret_cast<const u32x4*>(at + t * 4096);
+        }
+        mixm_turn(v, yb);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) d[q] = YmDot<T>::mfma16(sa[cc][q], yb[q], f32x4{0.f, 0.f, 0.f, 0.f});
+        if (live) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            *reinterpret_cast<u32x4*>(at + t * 4096) = u32x4{ym_pack<T>(d[0][t], d[1][t]), ym_pack<T>(d[2][t], d[3][t]), ym_pack<T>(d[4][t], d[5][t]), ym_pack<T>(d[6][t], d[7][t])};
+        }
+      }
+    lds_barrier();
+    // the rows leave through registers, so that the next tile's first pieces are on their way before them
+    u32x4 z[4 * NB];
+#pragma unroll
+    for (int i = 0; i < 4 * NB; ++i) z[i] = *reinterpret_cast<const u32x4*>(ym_lds + (wave + 4 * i) * 1024 + lane * 16);
+    lds_barrier();
+    const int om0 = m0, or0 = r0;
+    const bool more = ++item < item_end;
+    if (more) begin();
+#pragma unroll
+    for (int i = 0; i < 4 * NB; ++i) {                 // (wave + 4 i) & 3 = wave: the wave's rows are the same in every block
+      const int row = wave * 8 + r8, c = (lane & 7) ^ ((row >> 1) & 7);
+      if (om0 + row < M && or0 + c * 8 < R) *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.m.Z) + ((int64_t)i * M + om0 + row) * R + or0 + c * 8) = z[i];
+    }
+    if (!more) break;
+    stores = om0 + 32 <= M && or0 + 64 <= R;
+  }
+}
+
 // S(i, j, r) with any strides -> St[(r b + i) b + j]: one thread per (i, r), neighbouring threads on neighbouring ranks.
 template <typename T>
 __global__ __launch_bounds__(256) void ym_s_transpose_kernel(const T* __restrict__ S, T* __restrict__ St, int b, int R,
@@ -444,73 +407,60 @@ __global__ __launch_bounds__(256) void ym_s_transpose_kernel(const T* __restrict
   for (int j = 0; j < b; ++j) St[((int64_t)r * b + i) * b + j] = S[(int64_t)i * s_si + (int64_t)j * s_sj + (int64_t)r * s_sr];
 }
 
-// Z (b, M, R) of dtype = mix(S, x V).  scratch: room for S transposed to (r, i, j) (b b R elements), used unless S already
-// has that layout.  Returns BLR_OK, a negative blr_status, or 1 when the shape is not for this kernel (b not a multiple of
+// Z (b, M, R) of dtype = mix(S, x V).  scratch: room for S as (r, i, j) (b b R elements), used where S has neither that order nor its ranks
+// contiguous on 16 bytes.  Returns BLR_OK, a negative blr_status, or 1 when the shape is not for this kernel (b not a multiple of
 // 4 or above 16, rank or block width not a multiple of 8, unaligned operands, fp32, scratch too small).
 int blast_ymix_launch(const void* x, int64_t ldx, const void* V, const void* S, void* Z, int M, int in_f, int b, int R,
-                      int64_t s_si, int64_t s_sj, int64_t s_sr, int s_layout, int dtype, void* scratch, size_t scratch_bytes,
-                      hipStream_t st) {
-  if (dtype != BLR_F16 && dtype != BLR_BF16) return 1;
-  if (b < 4 || b > 16 || (b & 3) || in_f % b) return 1;
-  const int P = in_f / b;
-  if (P % 8 || R % 8 || ldx % 8 || !aligned(x, 16) || !aligned(V, 16) || !aligned(Z, 16)) return 1;
-  const int64_t x_elems = (int64_t)(M - 1) * ldx + in_f;
-  if (x_elems * 2 >= (int64_t)YM_OOB || (int64_t)P * R * 2 >= (int64_t)YM_OOB || (int64_t)b * b * R * 2 >= (int64_t)YM_OOB) return 1;
-  YmixParams p = {};
-  p.x = x; p.ldx = ldx; p.x_bytes = (uint32_t)(x_elems * 2); p.V = V; p.S = S; p.Z = Z;
-  p.M = M; p.b = b; p.P = P; p.R = R;
-  // Rank pieces per tile.  One workgroup per compute unit at a time.  A tile costs about 27 + npc units of 0.33 us, a third more where Z's rows
-  // do not fit LDS behind Y and 4 % more where its runs of Z end inside 64 bytes; a last round that is not full costs about half of what it
-  // leaves empty, the first one all of it.  Measured over 6 to 16 pieces, whole calls, at 4096 rows: 1152 -> 4608, r = 576: 6 / 8 / 9 / 11 / 12 / 13 / 16
-  // pieces (6 / 4.5 / 4 / 3.5 / 3 / 3 / 2.5 rounds) 104 / 90 / 88 / 90 / 78 / 93 / 86 us; 1152 -> 3456, r = 288: 6 / 9 / 12 / 13 / 16
-  // (3 / 2 / 1.5 / 1.5 / 1.5) 56 / 49 / 46 / 52 / 53; 768 -> 3072, r = 1000: 8 / 12 / 14 / 16 pieces 116 / 112 / 121 / 118.
-  const int pieces = R / 8;
-  const int cus = device_cus() > 0 ? device_cus() : 256;
-  const auto lds_y_of = [&](int npc) { return (size_t)(b / 2) * (YM_BM * (npc * 8 + 4) + 16) * 4; };
-  const auto lds_z_of = [&](int npc) { return (size_t)b * 16 * (npc * 4 + 4) * 4; };      // the rows of one product group on their way out
-  const auto staged = [&](int npc) { return lds_y_of(npc) + lds_z_of(npc) <= 160 * 1024; };
-  int best_npc = 16; double best_cost = -1.0;
-  for (int npc = 16; npc >= 4; --npc) {
-    const double x = (double)(cdiv(pieces, npc) * cdiv(M, YM_BM)) / cus;
-    const double cost = (x <= 1.0 ? 1.0 : 0.5 * (std::ceil(x) + x)) * (27 + npc) * (staged(npc) ? 1.0 : 1.35) * (npc % 4 ? 1.04 : 1.0);
-    if (best_cost < 0 || cost < best_cost - 1e-9) { best_cost = cost; best_npc = npc; }
-  }
-  p.npc = best_npc;
-  const int nrt = (int)cdiv(pieces, p.npc), nmt = (int)cdiv(M, YM_BM);
+                      int64_t s_si, int64_t s_sj, int64_t s_sr, int dtype, void* scratch, size_t scratch_bytes, hipStream_t st) {
+  if ((dtype != BLR_F16 && dtype != BLR_BF16) || b < 4 || b > 16 || b % 4 || R % 8 || in_f % b || (in_f / b) % 8) return 1;
+  if (ldx % 8 || !aligned(x, 16) || !aligned(V, 16) || !aligned(Z, 16)) return 1;
+  const int64_t lim = (int64_t)1 << 31;
+  if (31 * ldx * 2 + 256 >= lim || (int64_t)8 * R * 2 >= lim) return 1;
+  const int nrt = (int)cdiv(R, 64), nmt = (int)cdiv(M, 32);
   if ((int64_t)nrt * nmt >= 65536 || nmt >= 65536) return 1;
-  p.nmt = fd_make((uint32_t)nmt);
-  p.items = nrt * nmt;
-  p.ksteps = (int)cdiv(P, 32);
-  if (s_layout == BLR_S_RIJ && aligned(S, 8)) {
-    p.St = S;
-  } else {
+  bool rij = s_sj == 1 && s_si == b && s_sr == (int64_t)b * b && aligned(S, 8);
+  const bool run = s_sr == 1 && s_si % 8 == 0 && s_sj % 8 == 0 && s_si >= 0 && s_sj >= 0 && aligned(S, 16) && ((b - 1) * (s_si + s_sj) + R) * 2 < lim;
+  if (!rij && !run) {
     if (!scratch || scratch_bytes < (size_t)b * b * R * 2 || !aligned(scratch, 8)) return 1;
     const unsigned tg = (unsigned)cdiv((int64_t)b * R, 256);
     if (dtype == BLR_F16) hipLaunchKernelGGL(ym_s_transpose_kernel<f16>, dim3(tg), dim3(256), 0, st, (const f16*)S, (f16*)scratch, b, R, s_si, s_sj, s_sr);
     else hipLaunchKernelGGL(ym_s_transpose_kernel<bf16>, dim3(tg), dim3(256), 0, st, (const bf16*)S, (bf16*)scratch, b, R, s_si, s_sj, s_sr);
     BLR_CHECK_LAUNCH("ym_s_transpose");
-    p.St = scratch;
+    S = scratch;
+    rij = true;
   }
-  const bool stage = staged(p.npc);
-  const size_t lds = lds_y_of(p.npc) + (stage ? lds_z_of(p.npc) : 0);
-  const bool walk = p.items > cus;
-  const int fi = (dtype == BLR_F16 ? 0 : 4) + (stage ? 2 : 0) + (walk ? 1 : 0);
-  void* const fns[8] = {(void*)blast_ymix_kernel<f16, false, false>, (void*)blast_ymix_kernel<f16, false, true>,
-                        (void*)blast_ymix_kernel<f16, true, false>, (void*)blast_ymix_kernel<f16, true, true>,
-                        (void*)blast_ymix_kernel<bf16, false, false>, (void*)blast_ymix_kernel<bf16, false, true>,
-                        (void*)blast_ymix_kernel<bf16, true, false>, (void*)blast_ymix_kernel<bf16, true, true>};
-  static bool attr_set[8] = {};
+  YmixParams p = {};
+  p.m.S = S; p.m.Z = Z; p.m.M = M; p.m.b = b; p.m.R = R; p.m.s_si = s_si; p.m.s_sj = s_sj;
+  p.x = x; p.ldx = ldx; p.V = V;
+  p.P = in_f / b;
+  const int pieces = (int)cdiv(p.P, 96);
+  p.PP = (int)cdiv(p.P / 8, pieces) * 8;
+  const int cl = (p.PP / 8) | 1;
+  p.cl = fd_make((uint32_t)cl);
+  p.slot = (cl + 1) / 2 * 1024 + p.PP * 128;
+  p.m.nmt = fd_make((uint32_t)nmt);
+  p.m.items = nrt * nmt;
+  size_t lds = (size_t)4 * p.slot;
+  if (lds < (size_t)b * 4096) lds = (size_t)b * 4096;
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  const unsigned grid = (unsigned)(p.m.items < 2 * cus ? p.m.items : 2 * cus);
+  const int ks = (int)cdiv(p.PP, 32), fi = (((dtype == BLR_F16 ? 0 : 1) * 2 + (rij ? 0 : 1)) * 4 + b / 4 - 1) * 3 + ks - 1;
+#define YN3(T, RIJ, NB) (void*)blast_ymix_kernel<T, RIJ, NB, 1>, (void*)blast_ymix_kernel<T, RIJ, NB, 2>, (void*)blast_ymix_kernel<T, RIJ, NB, 3>
+#define YN(T, RIJ) YN3(T, RIJ, 1), YN3(T, RIJ, 2), YN3(T, RIJ, 3), YN3(T, RIJ, 4)
+  void* const fns[48] = {YN(f16, true), YN(f16, false), YN(bf16, true), YN(bf16, false)};
+#undef YN
+#undef YN3
+  static bool attr_set[48] = {};
   if (!attr_set[fi]) {
-    hipError_t e = hipFuncSetAttribute(fns[fi], hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    const hipError_t e = hipFuncSetAttribute(fns[fi], hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
     if (e != hipSuccess) { set_error("blast_ymix: cannot raise the LDS limit: %s", hipGetErrorString(e)); return BLR_ERR_LAUNCH; }
     attr_set[fi] = true;
   }
   void* args[] = {&p};
-  hipError_t e = hipLaunchKernel(fns[fi], dim3((unsigned)(walk ? cus : p.items)), dim3(YM_NT), args, lds, st);
+  const hipError_t e = hipLaunchKernel(fns[fi], dim3(grid), dim3(256), args, lds, st);
   if (e != hipSuccess) { set_error("blast_ymix: launch failed: %s", hipGetErrorString(e)); return BLR_ERR_LAUNCH; }
   return BLR_OK;
 }
-
 
 // ---- the same first half for wide input blocks: x V as one GEMM over all of x's columns, Y held in registers -------------------
 //

@@ -15,4 +15,9 @@ __device__ __forceinline__ uint32_t ring_lds_addr(const void* p) {
   return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)((void __attribute__((address_space(3)))*)(p)));
 }
 
+// s_waitcnt vmcnt(N) where some (wave-uniform) is not zero, vmcnt(0) where it is
+template <int N> __device__ __forceinline__ void ring_wait_loads(int some) {
+  asm volatile("s_cmp_eq_u32 %0, 0\n\ts_cbranch_scc1 .Lall%=\n\ts_waitcnt vmcnt(%1)\n\ts_branch .Lend%=\n.Lall%=:\n\ts_waitcnt vmcnt(0)\n.Lend%=:" ::"s"(__builtin_amdgcn_readfirstlane(some)), "n"(N) : "memory", "scc");
+}
+
 }  // namespace blr

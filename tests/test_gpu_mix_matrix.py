@@ -1,5 +1,5 @@
-"""GPU parity of the mix on the matrix cores (blast_mixm_kernel): Z_i = sum_j S(i, j, r) Y_j as a launch of its own, which BLAST calls above 16 rows take
-whose input blocks are too wide for a fused first half.  Edges: rows and ranks that end inside a tile of 32 x 64, 4 to 16 blocks, both
+"""GPU parity of the mix on the matrix cores: Z_i = sum_j S(i, j, r) Y_j as a launch of its own (blast_mixm_kernel), which BLAST calls above 16 rows take
+whose input blocks are too wide for a fused first half, and that first half (blast_ymix_kernel).  Edges: rows and ranks that end inside a tile of 32 x 64, 4 to 16 blocks, both
 orders of S, workgroups that walk several tiles and change the rank tile on the way."""
 import numpy as np
 import pytest
@@ -40,7 +40,6 @@ def test_mix_element_by_element(b, order):
     z, y = (torch.full((b, m, r), float("nan"), device="cuda", dtype=dtype) for _ in range(2))
     out = torch.empty(m, b * q, device="cuda", dtype=dtype)
     lib = L.lib()
-    lay = {"ijr": 0, "jir": 0, "rij": 0}
     lay = {"rij": L.S_RIJ, "jir": L.S_JIR, "ijr": L.S_IJR}[order]
     say(f"[case] mix elements b={b} S ({order})")
     ws = torch.empty(lib.blr_blast_workspace_bytes(m, b * p, b * q, b, r, L.BF16, 2), dtype=torch.uint8, device="cuda")
@@ -58,3 +57,37 @@ def test_mix_element_by_element(b, order):
     err = (z.double() - ref).abs().cpu().numpy()
     bound = 0.5 * ulp(ref.cpu().numpy(), dtype) * (1 + 2.0 ** -7) + 16 * 2.0 ** -24 * mag.cpu().numpy()
     assert (err <= bound).all(), f"{np.max(err / bound):.3f} of the bound"
+
+
+FUSED = {"algo": 3}
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_bmm_fp16"])
+@pytest.mark.parametrize("b,p,r,m", [(16, 72, 288, 300), (16, 8, 8, 17), (16, 96, 72, 33), (12, 40, 136, 64), (8, 184, 200, 257), (4, 104, 72, 31),
+                                     (4, 200, 64, 130), (8, 64, 328, 1500), (4, 24, 1000, 2100), (16, 136, 64, 95)])
+def test_fused_first_half(b, p, r, m, name, dtype):
+    """Blocks of one, two and three pieces of columns (the last one overlapping the one before), ranks and rows that end inside a tile, workgroups
+    that walk several tiles."""
+    from triton_funcs import blast_kernels as K, _lib as L
+    q = 16
+    x, U, Vt, S = blast_inputs(b, p, q, r, (m,), seed=b + r + m)
+    Uk, Vk, Sk = (O.blast_to_bmm_layout if "bmm" in name else O.blast_to_partial_layout)(U, Vt, S)
+    say(f"[case] fused {name} b={b} p={p} r={r} m={m} {dtype}")
+    with L.options(BLR_BLAST_YMIXW=0):
+        out = getattr(K, name)(dev(x, dtype), dev(Uk, dtype), dev(Vk, dtype), dev(Sk, dtype), FUSED)
+    assert_close(out, O.blast_forward(rounded(x, dtype), rounded(U, dtype), rounded(Vt, dtype), rounded(S, dtype))[0], dtype, name)
+
+
+@pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_bmm_fp16"])
+def test_fused_first_half_with_s_off_its_boundary(name):
+    from triton_funcs import blast_kernels as K
+    dtype, b, p, q, r, m = torch.float16, 8, 56, 24, 88, 150
+    x, U, Vt, S = blast_inputs(b, p, q, r, (m,), seed=1)
+    Uk, Vk, Sk = (O.blast_to_bmm_layout if "bmm" in name else O.blast_to_partial_layout)(U, Vt, S)
+    flat = torch.empty(Sk.size + 1, device="cuda", dtype=dtype)
+    s = flat[1:].view(Sk.shape)
+    s.copy_(dev(Sk, dtype))
+    say(f"[case] fused {name}, S one element off")
+    out = getattr(K, name)(dev(x, dtype), dev(Uk, dtype), dev(Vk, dtype), s, FUSED)
+    assert_close(out, O.blast_forward(rounded(x, dtype), rounded(U, dtype), rounded(Vt, dtype), rounded(S, dtype))[0], dtype, name)
