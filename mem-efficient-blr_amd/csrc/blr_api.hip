@@ -355,25 +355,29 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
   else { si = (int64_t)b * r; sj = r; sr = 1; }
   int rc = 1;
   int mixu_prepared = 0;
+  // Nobody asked for Y: x V and the mix can run as one launch with Y kept inside the compute units (BLR_ALGO_FUSED).  Chosen
+  // by itself only for narrow input blocks: the fused kernel re-reads V once per 32 rows, and that must cost less than the round trip of Y that
+  // it saves.  Whole calls, fused against the product on wide tiles and the mix alone: 2048 -> 8192 in 16 blocks of 128, r = 768 at 2000 / 4096 rows
+  // 60.6 / 113.9 and 60.9 / 120.7 us, 1152 -> 4608 in 16 of 72, r = 576 38.4 / 63.4 and 43.5 / 73.7; but 3072 -> 3072 in 16 of 192, r = 768 61.1 / 105.2
+  // and 53.3 / 101.0.  With fewer blocks Y is smaller beside V's rows: 1536 -> 3072 in 8 of 192, r = 256 23.2 / 31.7 and 27.9 / 34.1, 640 -> 2560 in 4 of 160,
+  // r = 256 17.4 / 24.5 and 20.4 / 28.6, 1024 -> 4096 in 4 of 256, r = 512 27.5 / 44.8 and 31.5 / 42.2.
+  const int fuse_max_p = b <= 8 ? 192 : 128;
   // Few rows and small ranks: both products on the kernels for problems that do not fill the chip, which give a
-  // 16-block layer of a thousand columns one to several hundred small workgroups where the fused kernels below have 4 .. 32, and
-  // the mix as a launch of its own in between.  The cost of that launch goes with M r; up to where it lies below what the fused
-  // kernel of the shape gains by not having it, measured over the layers of the configurations at 17 .. 1024 rows:
-  //   17 .. 128 rows, any rank: 1152 -> 3456, r = 288 at 17 / 61 / 128 rows 20.4 / 21.3 / 22.6 us (fused) and 13.8 / 19.2 / 28.1
-  //   (tiles of 16 rows, as with codes) against 9.9 / 11.5 / 12.3; 4096 -> 22016, r = 1024 22.8 / 31.7 / 43.7 against 21.4 / 22.2 / 28.3;
-  //   S with the rank contiguous: to M r = 2^18 (2048 -> 8192, r = 512 at 512 rows 34.9 against 31.1 us, at 768 rows 39.4 against 42.4),
-  //   3/4 of that where output blocks are narrow (1152 -> 1152, r = 288 at 512 rows 27.3 against 23.4, at 768 rows 27.1 against 28.0);
-  //   S (r, i, j): the same, but with input blocks that the fused first half takes as they are 80 x 1024 (1152 -> 3456, r = 288 at
-  //   256 rows 18.3 against 17.0, at 384 rows 19.6 against 21.3; 2048 -> 8192, r = 768 at 144 rows 23.6 against 24.7), and not with 9 .. 15
-  //   blocks: that line is older than the mix kernel that such calls have now and lies too low for most of them (fused, or for an odd number of blocks
-  //   GEMM and mix, against three launches: 1536 -> 1536, b = 12, r = 256 at 129 / 260 / 400 / 600 rows 16.1 / 16.4 / 17.2 / 18.0 against 13.8 / 15.6 / 18.3 / 21.1;
-  //   1152 -> 6912, b = 9, r = 256 at 129 / 600 / 1000 rows 19.9 / 27.0 / 31.1 against 13.1 / 24.2 / 30.4; 1040 -> 1040, b = 10, r = 192 at 129 / 1000 rows 19.9 / 25.0
-  //   against 11.1 / 21.6; but 768 -> 3072, b = 12, r = 384 at 129 / 260 rows 14.1 / 15.5 against 14.9 / 18.9); as many blocks
-  //   of that width with the rank contiguous: 5 x 2^15 (1152 -> 2304, b = 12, r = 128 at 1500 / 2000 rows 28.3 / 32.5 against 25.2 / 27.1).
-  // Longer calls of tiny ranks are left to the fused kernels, which were fitted there.
+  // 16-block layer of a thousand columns one to several hundred small workgroups, and the mix as a launch of its own in between.  What
+  // the kernels of many rows save goes with M r; where the lines lie, above 128 rows (three launches against the kernels of many rows, us of GPU time):
+  //   * blocks by fours that the fused first half takes: 80 x 1024 (1152 -> 3456, b = 16, r = 288 with the rank contiguous at 128 / 300 / 800 rows 13.0 / 19.9 / 31.1 and
+  //     14.7 / 17.1 / 22.2; 1024 -> 1024, b = 8, r = 192 at 300 / 800 rows 10.5 / 14.6 and 11.7 / 12.9; 1536 -> 1536, b = 12, r = 256 at 200 / 800 rows
+  //     12.4 / 26.4 and 14.1 / 19.0; 256 -> 1024, b = 4, r = 512 at 128 / 300 rows 10.2 / 11.9 and 9.8 / 10.4; 2048 -> 8192, b = 16, r = 512 at 300 / 800 rows 26.9 / 40.4 and
+  //     24.1 / 31.2), twice that above 128 columns per block (768 -> 3072, b = 4, r = 128 at 800 rows 12.4 and 13.1);
+  //   * 16 wider blocks: 80 x 1024 (4096 -> 4096, r = 512 at 128 / 200 / 800 rows 16.3 / 22.4 / 54.8 and 16.8 / 18.8 / 30.8);
+  //   * narrow output blocks (the kernels that keep Z on chip): 3 x 2^16 (1152 -> 1152, r = 288 at 128 / 400 rows 14.8 / 22.2 and 26.4 / 25.9);
+  //   * the others: 2^18 (1024 -> 4096, b = 4, r = 256 at 800 rows 16.0 and 17.3), 80 x 1024 with S (r, i, j) and narrow blocks, none of them with 9 .. 15
+  //     blocks in that order and 5 x 2^15 in the other (768 -> 2304, b = 6, r = 192 at 200 / 800 rows 12.8 / 16.0 and 16.0 / 17.3; 1152 -> 6912, b = 9, r = 256
+  //     with the rank contiguous at 400 rows 18.2 and 22.3).
   const bool narrow_out = b == 16 && Q % 8 == 0 && Q <= 80 && r % 32 == 0 && !silu_mul_armed();
-  const bool odd_blocks = b > 8 && b != 16;
-  const int64_t by_three = narrow_out ? 3 << 16 : P > 128 ? 1 << 18 : sr != 1 ? (odd_blocks ? 0 : 80 << 10) : odd_blocks ? 5 << 15 : 1 << 18;
+  const bool odd_blocks = b > 8 && b != 16, fours = b % 4 == 0 && b <= 16 && P % 8 == 0 && r % 8 == 0;
+  const int64_t by_three = narrow_out ? 3 << 16 : odd_blocks && sr != 1 && P <= 128 ? 0 : fours && P <= fuse_max_p ? (P > 128 ? 160 << 10 : 80 << 10) : fours && b == 16 ? 80 << 10
+                           : P > 128 ? 1 << 18 : sr != 1 ? 80 << 10 : odd_blocks ? 5 << 15 : 1 << 18;
   const bool few = M <= 128 || (M <= 2048 && (int64_t)M * r <= by_three);
   if (few && !y_out && !z_out && !sat8 && fused <= 0 && dtype != BLR_F32 && option_value(OPT_DECODE_ROWS, 1)) {
     if (M > 16) {
@@ -399,13 +403,6 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
     }
     rc = 1;
   }
-  // Nobody asked for Y: x V and the mix can run as one launch with Y kept inside the compute units (BLR_ALGO_FUSED).  Chosen
-  // by itself only for narrow input blocks: the fused kernel re-reads V once per 32 rows, and that must cost less than the round trip of Y that
-  // it saves.  Whole calls, fused against the product on wide tiles and the mix alone: 2048 -> 8192 in 16 blocks of 128, r = 768 at 2000 / 4096 rows
-  // 60.6 / 113.9 and 60.9 / 120.7 us, 1152 -> 4608 in 16 of 72, r = 576 38.4 / 63.4 and 43.5 / 73.7; but 3072 -> 3072 in 16 of 192, r = 768 61.1 / 105.2
-  // and 53.3 / 101.0.  With fewer blocks Y is smaller beside V's rows: 1536 -> 3072 in 8 of 192, r = 256 23.2 / 31.7 and 27.9 / 34.1, 640 -> 2560 in 4 of 160,
-  // r = 256 17.4 / 24.5 and 20.4 / 28.6, 1024 -> 4096 in 4 of 256, r = 512 27.5 / 44.8 and 31.5 / 42.2.
-  const int fuse_max_p = b <= 8 ? 192 : 128;
   // Narrow output blocks (either layout of U: it is re-laid for the kernel anyway): the mix and the product with U run as one launch that reads Y once and
   // never writes Z (blast_mixu_kernel); the first half is then the plain GEMM, which leaves Y.  Measured at 4096 rows against the
   // mix kernel + batched GEMM: 4608 -> 1152, r = 576: 90 against 122 us; against the fused first half + batched GEMM: 1152 -> 1152,
