@@ -97,10 +97,11 @@ __global__ __launch_bounds__(256, 2) void attention_kernel(const T* __restrict__
   __shared__ __align__(16) T ks[KT * KS];
   __shared__ __align__(16) T vt[DT * 32 * VS];     // (rows past D are read into results that nobody stores)
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
-  const int64_t wg = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (wg >= total) return;
-  const int qt = (int)(wg % q_tiles), h = (int)(wg / q_tiles % H), img = (int)(wg / q_tiles / H);
-  const int q0 = qt * 128 + (tid >> 6) * 32;
+  const unsigned wg = (blockIdx.x & 7) * (unsigned)per_xcd + (blockIdx.x >> 3);
+  if (wg >= (unsigned)total) return;
+  const unsigned qt = wg % (unsigned)q_tiles, head = wg / (unsigned)q_tiles;
+  const int h = (int)(head % (unsigned)H), img = (int)(head / (unsigned)H);
+  const int q0 = (int)qt * 128 + (tid >> 6) * 32;
   const int64_t ld = (int64_t)3 * H * D;
   const T* base = qkv + (int64_t)img * N * ld + (int64_t)h * D;
   const bool live = q0 < N;                        // waves past the last query only help to load
