@@ -186,7 +186,7 @@ int blast_mixm_launch(const void* Y, const void* S, void* Z, int M, int b, int R
 }
 
 // ---- Z = mix(S, x V) in one launch for narrow input blocks ----------------------------------------------------------------------------------------
-// The tile and the mix of blast_mixm_kernel, with Y made on the spot: 32 rows x 64 ranks of all blocks.  Four waves, wave w makes Y_j for j = w, w + 4, ..:
+// The tile and the mix of blast_mixm_kernel, with Y made on the spot: 32 rows (16 where that leaves compute units idle) x 64 ranks of all blocks.  Four waves, wave w makes Y_j for j = w, w + 4, ..:
 // the block's 32 rows of x and its rows of V, at most 96 columns of the block at a time, come as whole lines into a piece of LDS of the wave's
 // own and from there - V through transposing reads - into registers, whereupon the next block's loads go out under the products.  Nothing waits for
 // another wave until all of Y is in registers (16 per block); then Y goes to LDS, over what the blocks came through, and the mix and the way out are
@@ -203,11 +203,11 @@ struct YmixParams {
   int slot;                     // bytes of LDS of a wave
   FastDiv cl;                   // chunks of a row of x in LDS
 };
-template <typename T, bool RIJ, int NB, int KS>        // NB = b / 4; KS: steps of 32 columns that cover a piece
+template <typename T, bool RIJ, int NB, int KS, int RX>   // NB = b / 4; KS: steps of 32 columns that cover a piece; RX: tiles of 16 RX rows
 __global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char ym_lds[];
   using V8 = typename TypeTraits<T>::vec8;
-  constexpr int b = 4 * NB;
+  constexpr int b = 4 * NB, ROWS = 16 * RX, PLANE = ROWS * 128, NZ = 2 * RX * NB;   // PLANE: a block's Y in LDS; NZ: the pieces of Z that a wave stores
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int n = lane & 15, g = lane >> 4;
   const int M = p.m.M, R = p.m.R, P = p.P, PP = p.PP;
@@ -216,15 +216,15 @@ __global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
   const uint32_t item_end = (uint32_t)((uint64_t)(wg + 1) * (uint32_t)p.m.items / G);
   int r8 = lane >> 3;
   const bool live = g < NB;
-  // x of a block: 32 rows of cl chunks of 16 bytes, cl odd (16 rows' chunks of one number then lie in different banks); V behind it as it lies,
+  // x of a block: the rows' cl chunks of 16 bytes, cl odd (16 rows' chunks of one number then lie in different banks); V behind it as it lies,
   // chunk c of row k at c ^ (k & 2) << 1 ^ (k & 8) >> 2 (see the (k, n) stages of blr_gemm_wide.hip)
-  const int cl = (PP / 8) | 1, xi = (cl + 1) / 2;      // 32 cl chunks are cl / 2 KiB
+  const int cl = (PP / 8) | 1, xi = (RX * cl + 3) / 4;      // 16 RX cl chunks, in KiB
   unsigned char* const own = ym_lds + wave * p.slot;
   const uint32_t own0 = ring_lds_addr(own), lds0 = ring_lds_addr(ym_lds);
   u32x2 sa[2][8];
   uint32_t rt_have = ~0u;
   int m0, r0;
-  constexpr int XI = 2 * KS + 1;                       // (at most: 32 (4 KS + 1) chunks)
+  constexpr int XI = RX * KS + 1;                      // (at most: 16 RX (4 KS + 1) chunks)
   uint32_t v_off[2], x_off[XI];                        // v_off: rows 0 .. 7 of an even and of an odd group of eight
   auto ask = [&](int j, int k0) {                      // columns k0 .. k0 + PP - 1 of block j
     const char* xb = reinterpret_cast<const char*>(p.x) + ((int64_t)m0 * p.ldx + (int64_t)j * P + k0) * 2;
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
   auto begin = [&]() {                                 // a tile: S if its ranks are new, and the wave's first piece is asked for
     asm volatile("" : "+v"(n), "+v"(g), "+v"(r8));   // addresses are formed again for each tile: kept, they would not fit beside Y
     const uint32_t rt = fd_div(item, p.m.nmt);
-    m0 = (int)(item - rt * p.m.nmt.d) * 32;
+    m0 = (int)(item - rt * p.m.nmt.d) * ROWS;
     r0 = (int)rt * 64;
     if (rt != rt_have) {
       rt_have = rt;
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
     }
 #pragma unroll
     for (int i = 0; i < XI; ++i) {
-      const uint32_t L = min(i * 64 + r8 * 8 + (int)(lane & 7), 32 * cl - 1), row = fd_div(L, p.cl);
+      const uint32_t L = min(i * 64 + r8 * 8 + (int)(lane & 7), ROWS * cl - 1), row = fd_div(L, p.cl);
       x_off[i] = (uint32_t)min((int)row, M - 1 - m0) * (uint32_t)(p.ldx * 2) + min(L - row * cl, (uint32_t)PP / 8 - 1) * 16;
       asm volatile("" : "+v"(x_off[i]));
     }
@@ -287,26 +287,28 @@ __global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
   };
   if (item >= item_end) return;
   begin();
-  int stores = 0;                                      // whether 4 NB stores of the tile before are younger than the loads
+  int stores = 0;                                      // whether the NZ stores of the tile before are younger than the loads
   for (;;) {
-    u32x2 y[NB][4][2];
+    u32x2 y[NB][4][RX];
 #pragma unroll
     for (int jb = 0; jb < NB; ++jb) {
-      f32x4 acc[4][2];
+      f32x4 acc[4][RX];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) acc[c][0] = acc[c][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int x = 0; x < RX; ++x) acc[c][x] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma clang loop unroll(disable)
       for (int at = 0; at < P; at += PP) {             // a last piece that would end past the block begins earlier: what the one before had of it is zero
         asm volatile("" : "+v"(n), "+v"(g));
         const int skip = max(at + PP - P, 0);
-        V8 xf[KS][2], vf[KS][4];
-        ring_wait_loads<4 * NB>(stores);
+        V8 xf[KS][RX], vf[KS][4];
+        ring_wait_loads<NZ>(stores);
         stores = 0;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
           const int kc = min(4 * s + g, PP / 8 - 1);                               // the lane's eight k, or the last ones there are
 #pragma unroll
-          for (int x = 0; x < 2; ++x) xf[s][x] = *reinterpret_cast<const V8*>(own + ((16 * x + n) * cl + kc) * 16);
+          for (int x = 0; x < RX; ++x) xf[s][x] = *reinterpret_cast<const V8*>(own + ((16 * x + n) * cl + kc) * 16);
           const int k = 8 * kc + (n >> 2), swz = (k & 2) << 1 | (k & 8) >> 2;
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
@@ -327,21 +329,22 @@ __global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
           if (32 * s + 8 * g >= PP || 32 * s + 8 * g < skip) {                     // zero on both sides
-            xf[s][0] = xf[s][1] = V8{};
+#pragma unroll
+            for (int x = 0; x < RX; ++x) xf[s][x] = V8{};
 #pragma unroll
             for (int c = 0; c < 4; ++c) vf[s][c] = V8{};
           }
 #pragma unroll
           for (int c = 0; c < 4; ++c)
 #pragma unroll
-            for (int x = 0; x < 2; ++x) acc[c][x] = TypeTraits<T>::mfma16(vf[s][c], xf[s][x], acc[c][x]);
+            for (int x = 0; x < RX; ++x) acc[c][x] = TypeTraits<T>::mfma16(vf[s][c], xf[s][x], acc[c][x]);
         }
       }
       // acc[c][x]: row 16 x + n, ranks 16 c + 4 g .. + 3
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int x = 0; x < 2; ++x) y[jb][c][x] = u32x2{ym_pack<T>(acc[c][x][0], acc[c][x][1]), ym_pack<T>(acc[c][x][2], acc[c][x][3])};
+        for (int x = 0; x < RX; ++x) y[jb][c][x] = u32x2{ym_pack<T>(acc[c][x][0], acc[c][x][1]), ym_pack<T>(acc[c][x][2], acc[c][x][3])};
     }
     lds_barrier();                                     // nobody reads x and V any more
 #pragma unroll
@@ -349,25 +352,25 @@ __global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
 #pragma unroll
       for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
+        for (int x = 0; x < RX; ++x) {
           const int m = 16 * x + n;
-          *reinterpret_cast<u32x2*>(ym_lds + (wave + 4 * jb) * 4096 + m * 128 + (((2 * c + (g >> 1)) ^ ((m >> 1) & 7)) << 4) + (g & 1) * 8) = y[jb][c][x];
+          *reinterpret_cast<u32x2*>(ym_lds + (wave + 4 * jb) * PLANE + m * 128 + (((2 * c + (g >> 1)) ^ ((m >> 1) & 7)) << 4) + (g & 1) * 8) = y[jb][c][x];
         }
     lds_barrier();
     // ---- the mix and the way out, as above, with two pieces of eight ranks a wave ----
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
-      for (int mg = 0; mg < 2; ++mg) {
+      for (int mg = 0; mg < RX; ++mg) {
         __builtin_amdgcn_sched_barrier(0);
-        unsigned char* const at = ym_lds + 4 * g * 4096 + (mg * 16 + n) * 128 + (((wave + 4 * cc) ^ ((n >> 1) & 7)) << 4);
+        unsigned char* const at = ym_lds + 4 * g * PLANE + (mg * 16 + n) * 128 + (((wave + 4 * cc) ^ ((n >> 1) & 7)) << 4);
         u32x4 v[4];
         u32x2 yb[8];
         f32x4 d[8];
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           v[t] = u32x4{0u, 0u, 0u, 0u};
-          if (live) v[t] = *reinterpret_cast<const u32x4*>(at + t * 4096);
+          if (live) v[t] = *reinterpret_cast<const u32x4*>(at + t * PLANE);
         }
         mixm_turn(v, yb);
 #pragma unroll
@@ -375,25 +378,25 @@ __global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
         if (live) {
 #pragma unroll
           for (int t = 0; t < 4; ++t)
-            *reinterpret_cast<u32x4*>(at + t * 4096) = u32x4{ym_pack<T>(d[0][t], d[1][t]), ym_pack<T>(d[2][t], d[3][t]), ym_pack<T>(d[4][t], d[5][t]), ym_pack<T>(d[6][t], d[7][t])};
+            *reinterpret_cast<u32x4*>(at + t * PLANE) = u32x4{ym_pack<T>(d[0][t], d[1][t]), ym_pack<T>(d[2][t], d[3][t]), ym_pack<T>(d[4][t], d[5][t]), ym_pack<T>(d[6][t], d[7][t])};
         }
       }
     lds_barrier();
     // the rows leave through registers, so that the next tile's first pieces are on their way before them
-    u32x4 z[4 * NB];
+    u32x4 z[NZ];
 #pragma unroll
-    for (int i = 0; i < 4 * NB; ++i) z[i] = *reinterpret_cast<const u32x4*>(ym_lds + (wave + 4 * i) * 1024 + lane * 16);
+    for (int i = 0; i < NZ; ++i) z[i] = *reinterpret_cast<const u32x4*>(ym_lds + (wave + 4 * i) * 1024 + lane * 16);
     lds_barrier();
     const int om0 = m0, or0 = r0;
     const bool more = ++item < item_end;
     if (more) begin();
 #pragma unroll
-    for (int i = 0; i < 4 * NB; ++i) {                 // (wave + 4 i) & 3 = wave: the wave's rows are the same in every block
-      const int row = wave * 8 + r8, c = (lane & 7) ^ ((row >> 1) & 7);
-      if (om0 + row < M && or0 + c * 8 < R) *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.m.Z) + ((int64_t)i * M + om0 + row) * R + or0 + c * 8) = z[i];
+    for (int i = 0; i < NZ; ++i) {                     // piece wave + 4 i: eight rows of block (wave + 4 i) / 2 RX
+      const int row = (wave & (2 * RX - 1)) * 8 + r8, j = (wave + 4 * i) / (2 * RX), c = (lane & 7) ^ ((row >> 1) & 7);
+      if (om0 + row < M && or0 + c * 8 < R) *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.m.Z) + ((int64_t)j * M + om0 + row) * R + or0 + c * 8) = z[i];
     }
     if (!more) break;
-    stores = om0 + 32 <= M && or0 + 64 <= R;
+    stores = om0 + ROWS <= M && or0 + 64 <= R;
   }
 }
 
@@ -416,7 +419,8 @@ int blast_ymix_launch(const void* x, int64_t ldx, const void* V, const void* S, 
   if (ldx % 8 || !aligned(x, 16) || !aligned(V, 16) || !aligned(Z, 16)) return 1;
   const int64_t lim = (int64_t)1 << 31;
   if (31 * ldx * 2 + 256 >= lim || (int64_t)8 * R * 2 >= lim) return 1;
-  const int nrt = (int)cdiv(R, 64), nmt = (int)cdiv(M, 32);
+  const int nrt = (int)cdiv(R, 64);
+  int nmt = (int)cdiv(M, 32);
   if ((int64_t)nrt * nmt >= 65536 || nmt >= 65536) return 1;
   bool rij = s_sj == 1 && s_si == b && s_sr == (int64_t)b * b && aligned(S, 8);
   const bool run = s_sr == 1 && s_si % 8 == 0 && s_sj % 8 == 0 && s_si >= 0 && s_sj >= 0 && aligned(S, 16) && ((b - 1) * (s_si + s_sj) + R) * 2 < lim;
@@ -437,20 +441,28 @@ int blast_ymix_launch(const void* x, int64_t ldx, const void* V, const void* S, 
   p.PP = (int)cdiv(p.P / 8, pieces) * 8;
   const int cl = (p.PP / 8) | 1;
   p.cl = fd_make((uint32_t)cl);
-  p.slot = (cl + 1) / 2 * 1024 + p.PP * 128;
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  // Tiles of 16 rows where those of 32 give a compute unit at most one: twice the workgroups, each with half the products and the way out of half
+  // the rows.  32 / 16 rows, whole calls: 2048 -> 2048 in 16 blocks, r = 256 at 500 / 1000 / 2048 rows 19.6 / 22.2 / 26.3 and 17.5 / 20.6 / 24.3 us, 512 -> 2048 in 4,
+  // r = 512 at 500 / 1000 13.1 / 17.6 and 12.0 / 17.0; but past the line V is read twice as often for nothing: 1536 -> 3072 in 8, r = 256 at 3000 rows 28.8 and
+  // 32.4, 2048 -> 8192, r = 512 at 2048 47.8 and 54.6.
+  const int rx = nrt * nmt <= cus ? 1 : 2;
+  if (rx == 1) nmt = (int)cdiv(M, 16);
+  p.slot = (rx * cl + 3) / 4 * 1024 + p.PP * 128;
   p.m.nmt = fd_make((uint32_t)nmt);
   p.m.items = nrt * nmt;
   size_t lds = (size_t)4 * p.slot;
-  if (lds < (size_t)b * 4096) lds = (size_t)b * 4096;
-  const int cus = device_cus() > 0 ? device_cus() : 256;
+  if (lds < (size_t)b * 2048 * rx) lds = (size_t)b * 2048 * rx;
   const unsigned grid = (unsigned)(p.m.items < 2 * cus ? p.m.items : 2 * cus);
-  const int ks = (int)cdiv(p.PP, 32), fi = (((dtype == BLR_F16 ? 0 : 1) * 2 + (rij ? 0 : 1)) * 4 + b / 4 - 1) * 3 + ks - 1;
-#define YN3(T, RIJ, NB) (void*)blast_ymix_kernel<T, RIJ, NB, 1>, (void*)blast_ymix_kernel<T, RIJ, NB, 2>, (void*)blast_ymix_kernel<T, RIJ, NB, 3>
+  const int ks = (int)cdiv(p.PP, 32), fi = ((((dtype == BLR_F16 ? 0 : 1) * 2 + (rij ? 0 : 1)) * 4 + b / 4 - 1) * 3 + ks - 1) * 2 + rx - 1;
+#define YN1(T, RIJ, NB, KS) (void*)blast_ymix_kernel<T, RIJ, NB, KS, 1>, (void*)blast_ymix_kernel<T, RIJ, NB, KS, 2>
+#define YN3(T, RIJ, NB) YN1(T, RIJ, NB, 1), YN1(T, RIJ, NB, 2), YN1(T, RIJ, NB, 3)
 #define YN(T, RIJ) YN3(T, RIJ, 1), YN3(T, RIJ, 2), YN3(T, RIJ, 3), YN3(T, RIJ, 4)
-  void* const fns[48] = {YN(f16, true), YN(f16, false), YN(bf16, true), YN(bf16, false)};
+  void* const fns[96] = {YN(f16, true), YN(f16, false), YN(bf16, true), YN(bf16, false)};
 #undef YN
 #undef YN3
-  static bool attr_set[48] = {};
+#undef YN1
+  static bool attr_set[96] = {};
   if (!attr_set[fi]) {
     const hipError_t e = hipFuncSetAttribute(fns[fi], hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
     if (e != hipSuccess) { set_error("blast_ymix: cannot raise the LDS limit: %s", hipGetErrorString(e)); return BLR_ERR_LAUNCH; }

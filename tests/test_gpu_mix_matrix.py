@@ -65,10 +65,11 @@ FUSED = {"algo": 3}
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_bmm_fp16"])
 @pytest.mark.parametrize("b,p,r,m", [(16, 72, 288, 300), (16, 8, 8, 17), (16, 96, 72, 33), (12, 40, 136, 64), (8, 184, 200, 257), (4, 104, 72, 31),
-                                     (4, 200, 64, 130), (8, 64, 328, 1500), (4, 24, 1000, 2100), (16, 136, 64, 95)])
+                                     (4, 200, 64, 130), (8, 64, 328, 1500), (4, 24, 1000, 2100), (16, 136, 64, 95),
+                                     (16, 72, 264, 1650), (12, 40, 520, 929), (16, 136, 1000, 545), (4, 72, 64, 128 * 32), (4, 72, 64, 256 * 32 + 1)])
 def test_fused_first_half(b, p, r, m, name, dtype):
-    """Blocks of one, two and three pieces of columns (the last one overlapping the one before), ranks and rows that end inside a tile, workgroups
-    that walk several tiles."""
+    """Blocks of one, two and three pieces of columns (the last one overlapping the one before), ranks and rows that end inside a tile of 16 rows
+    (problems of at most 256 tiles of 32) and of 32, workgroups that walk several tiles."""
     from triton_funcs import blast_kernels as K, _lib as L
     q = 16
     x, U, Vt, S = blast_inputs(b, p, q, r, (m,), seed=b + r + m)
