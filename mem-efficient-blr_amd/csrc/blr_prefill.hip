@@ -237,7 +237,7 @@ __global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
   };
   auto begin = [&]() {                                 // a tile: S if its ranks are new, and the wave's first piece is asked for
     asm volatile("" : "+v"(n), "+v"(g), "+v"(r8));   // addresses are formed again for each tile: kept, they would not fit beside Y
-    const uint32_t rt = fd_div(item, p.m.nmt);
+    const uint32_t rt = item / p.m.nmt.d;                                    // (once a tile: any number of tiles, where the quick division has a limit)
     m0 = (int)(item - rt * p.m.nmt.d) * ROWS;
     r0 = (int)rt * 64;
     if (rt != rt_have) {
@@ -418,10 +418,10 @@ int blast_ymix_launch(const void* x, int64_t ldx, const void* V, const void* S, 
   if ((dtype != BLR_F16 && dtype != BLR_BF16) || b < 4 || b > 16 || b % 4 || R % 8 || in_f % b || (in_f / b) % 8) return 1;
   if (ldx % 8 || !aligned(x, 16) || !aligned(V, 16) || !aligned(Z, 16)) return 1;
   const int64_t lim = (int64_t)1 << 31;
-  if (31 * ldx * 2 + 256 >= lim || (int64_t)8 * R * 2 >= lim) return 1;
+  if ((M < 32 ? M - 1 : 31) * ldx * 2 + 256 >= lim * 2 || (int64_t)8 * R * 2 >= lim) return 1;
   const int nrt = (int)cdiv(R, 64);
   int nmt = (int)cdiv(M, 32);
-  if ((int64_t)nrt * nmt >= 65536 || nmt >= 65536) return 1;
+  if ((int64_t)nrt * nmt >= lim) return 1;
   bool rij = s_sj == 1 && s_si == b && s_sr == (int64_t)b * b && aligned(S, 8);
   const bool run = s_sr == 1 && s_si % 8 == 0 && s_sj % 8 == 0 && s_si >= 0 && s_sj >= 0 && aligned(S, 16) && ((b - 1) * (s_si + s_sj) + R) * 2 < lim;
   if (!rij && !run) {
