@@ -296,7 +296,7 @@ def main():
     del g_gu, step_graphs, round_graph, sets, gu_built, gu
     torch.cuda.empty_cache()
 
-    # second roofline object: the dominant kernel at M = 2048, the ring GEMM (one launch = the dense gate_up layer), MFMA bound
+    # second roofline object: the dominant kernel at M = 2048, the GEMM (one launch = the dense gate_up layer), MFMA bound
     i_f, o_f, _ = LAYERS["gate_up"]
     # (48 launches per replay over four copies, as in the layer table: the card takes some milliseconds of matrix work to settle
     # on the clock its power limit allows, and a replay of a dozen launches read 6 % slower than the table's row of the same kernel)
@@ -304,7 +304,7 @@ def main():
     g_dn = graph_of([dn[i % 4][0] for i in range(48)])
     dn_us = time_graph(g_dn, 48)
     dn_flops = 2.0 * 2048 * i_f * o_f
-    roofline_prefill = {"bound": "mfma", "kernel": "gemm_ring64_kernel<f16, 256x256, 8 waves, stages of 64 k> (dense gate_up 4096->22016, M=2048: one launch)",
+    roofline_prefill = {"bound": "mfma", "kernel": "gemm_wide_kernel<f16, 256x352, 8 waves, stages of 64 k> (dense gate_up 4096->22016, M=2048: one launch)",
                         "achieved": round(dn_flops / (dn_us * 1e-6) / 1e12, 1), "peak": MFMA_PEAK / 1e12, "unit": "TFLOP/s",
                         "frac": round(dn_flops / (dn_us * 1e-6) / MFMA_PEAK, 4), "us_per_launch": round(dn_us, 2),
                         "algorithmic_flops": dn_flops, "algorithmic_bytes": 2 * (2048 * i_f + i_f * o_f + 2048 * o_f),
@@ -320,7 +320,7 @@ def main():
     g_bp = graph_of([bp[i % 4][0] for i in range(48)])
     bp_us = time_graph(g_bp, 48)
     bp_bytes, bp_flops = blast_bytes_flops(2048, i_f, r_gu, o_f)
-    roofline_blast_prefill = {"bound": "mfma", "kernel": "BLAST gate_up 4096->22016 r=1024 b=16, M=2048: blast_ymixw_kernel (x V and the mix) + gemm_ring64_kernel (Z U)",
+    roofline_blast_prefill = {"bound": "mfma", "kernel": "BLAST gate_up 4096->22016 r=1024 b=16, M=2048: gemm_wide_kernel (x V), blast_mixm_kernel (the mix), gemm_wide_kernel (Z U)",
                               "achieved": round(bp_flops / (bp_us * 1e-6) / 1e12, 1), "peak": MFMA_PEAK / 1e12, "unit": "TFLOP/s",
                               "frac": round(bp_flops / (bp_us * 1e-6) / MFMA_PEAK, 4), "us_per_call": round(bp_us, 2),
                               "algorithmic_flops": bp_flops, "algorithmic_bytes": bp_bytes,
