@@ -62,13 +62,15 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // stores.  Wave w owns ranks 8 w .. 8 w + 7.  Lane (n, g) reads Y_j, j = 4 g .. 4 g + 3, of row n - 16 bytes are its eight ranks -, turns them
 // into one operand per rank (byte permutes), and its products are Z_i, i = 4 g .. 4 g + 3, of the same row and ranks: they go back where
 // the lane read Y.  Nothing crosses waves but the loads and the stores of whole rows on either side.  S is kept in registers along the row tiles
-// that a workgroup walks; with the rank contiguous it comes through the same LDS, as (r, i, j) straight in operand order.
+// that a workgroup walks; with the rank contiguous it comes through the same LDS, as (r, i, j) straight in operand order, and in any other order or off its
+// boundary (MIXM_ANY) through LDS as well, an element at a time - once per rank tile.  Every size and every S is taken, so the sums are fp32 for all of them (the kernels in blr_gemm.hip sum in fp16 for fp16): whole calls
+// with S one element off, there -> here, 4096 -> 4096, r = 512 at 1000 / 2048 rows 58.5 / 72.1 -> 35.6 / 53.8 us, 4096 -> 22016, r = 1024 in bf16 224 -> 152.
 // 16 blocks, r = 1024 at 2048 rows (134 MB in and out): 32.9 -> 24.4 us = 5.5 TB/s, the rate of a device copy; bf16 24.6.
 struct MixmParams {
   const void* Y; const void* S; void* Z;
   int M, b, R;
-  int64_t s_si, s_sj;           // strides of S where the rank is contiguous (RIJ: not used)
-  FastDiv nmt;                  // row tiles
+  int64_t s_si, s_sj, s_sr;     // strides of S (RIJ: not used)
+  int nmt;                      // row tiles
   int items;                    // rank tiles x row tiles
 };
 // eight ranks x four blocks: v[t] = 8 ranks of block t -> one operand (four blocks) per rank
@@ -80,7 +82,8 @@ __device__ __forceinline__ void mixm_turn(const u32x4 (&v)[4], u32x2 (&o)[8]) {
     o[q][1] = __builtin_amdgcn_perm(v[3][q >> 1], v[2][q >> 1], sel);
   }
 }
-template <typename T, bool RIJ>
+enum { MIXM_RIJ = 0, MIXM_RUN, MIXM_ANY };
+template <typename T, int ORDER>
 __global__ __launch_bounds__(512, 4) void blast_mixm_kernel(MixmParams p) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char mx_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -93,14 +96,13 @@ __global__ __launch_bounds__(512, 4) void blast_mixm_kernel(MixmParams p) {
   const int r8 = lane >> 3;                            // a load or store instruction of a wave: eight rows, eight lanes each
   const bool live = 4 * g < b;                         // (4 g + 3 < b as well: b is a multiple of four)
   u32x2 sa[8];
-  uint32_t rt_have = ~0u;
+  bool fresh = true;                                   // S of this rank tile is not in registers yet
+  int rt = (int)(item / (uint32_t)p.nmt), mt = (int)(item - (uint32_t)rt * (uint32_t)p.nmt);
   for (; item < item_end; ++item) {
-    const uint32_t rt = fd_div(item, p.nmt);
-    const int m0 = (int)(item - rt * p.nmt.d) * 32, r0 = (int)rt * 64;
+    const int m0 = mt * 32, r0 = rt * 64;
     const int piece = r0 + wave * 8;
-    if (rt != rt_have) {
-      rt_have = rt;
-      if constexpr (RIJ) {
+    if (fresh) {
+      if constexpr (ORDER == MIXM_RIJ) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
           sa[q] = u32x2{0u, 0u};
@@ -109,7 +111,15 @@ __global__ __launch_bounds__(512, 4) void blast_mixm_kernel(MixmParams p) {
       } else {                                         // rows (i, j) of the tile's 64 ranks, i b + j; b b is a multiple of 16
         for (int k = wave; k * 8 < b * b; k += 8) {
           const int row = k * 8 + r8, i = row / b, j = row - i * b, c = (lane & 7) ^ ((row >> 1) & 7);
-          ring_load_lds(p.S, (uint32_t)((i * p.s_si + j * p.s_sj + min(r0 + c * 8, R - 8)) * 2), lds0 + k * 1024);
+          if constexpr (ORDER == MIXM_ANY) {
+            const T* src = reinterpret_cast<const T*>(p.S) + i * p.s_si + j * p.s_sj + min(r0 + c * 8, R - 8) * p.s_sr;
+            typename TypeTraits<T>::vec8 v;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = src[e * p.s_sr];
+            *reinterpret_cast<typename TypeTraits<T>::vec8*>(mx_lds + k * 1024 + lane * 16) = v;
+          } else {
+            ring_load_lds(p.S, (uint32_t)((i * p.s_si + j * p.s_sj + min(r0 + c * 8, R - 8)) * 2), lds0 + k * 1024);
+          }
         }
         __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));
         lds_barrier();
@@ -124,10 +134,12 @@ __global__ __launch_bounds__(512, 4) void blast_mixm_kernel(MixmParams p) {
         lds_barrier();                                 // read by every wave
       }
     }
-    // in: plane j, rows 8 k .. 8 k + 7 (four instructions a plane)
-    for (int k = wave; k < 4 * b; k += 8) {
-      const int row = (k & 3) * 8 + r8, c = (lane & 7) ^ ((row >> 1) & 7);
-      ring_load_lds(p.Y, (uint32_t)(((int64_t)(k >> 2) * M + min(m0 + row, M - 1)) * R + min(r0 + c * 8, R - 8)) * 2u, lds0 + k * 1024);
+    // in: four instructions a plane, a wave the same eight rows of every second plane
+    {
+      const int row = (wave & 3) * 8 + r8, c = (lane & 7) ^ ((row >> 1) & 7);
+      const uint32_t off = (uint32_t)(min(row, M - 1 - m0) * R + min(c * 8, R - 8 - r0)) * 2u;
+      const T* y = reinterpret_cast<const T*>(p.Y) + ((int64_t)(wave >> 2) * M + m0) * R + r0;
+      for (int k = wave; k < 4 * b; k += 8, y += (int64_t)2 * M * R) ring_load_lds(y, off, lds0 + k * 1024);
     }
     __builtin_amdgcn_s_waitcnt(ring_vmcnt(0));         // (S of this tile as well)
     lds_barrier();
@@ -158,6 +170,8 @@ __global__ __launch_bounds__(512, 4) void blast_mixm_kernel(MixmParams p) {
       if (m0 + row < M && r0 + c * 8 < R) *reinterpret_cast<u32x4*>(reinterpret_cast<T*>(p.Z) + ((int64_t)(k >> 2) * M + m0 + row) * R + r0 + c * 8) = z;
     }
     lds_barrier();                                     // the rows have been read: the next tile may land
+    fresh = ++mt == p.nmt;
+    if (fresh) { mt = 0; ++rt; }
   }
 }
 
@@ -165,22 +179,20 @@ __global__ __launch_bounds__(512, 4) void blast_mixm_kernel(MixmParams p) {
 int blast_mixm_launch(const void* Y, const void* S, void* Z, int M, int b, int R, int64_t s_si, int64_t s_sj, int64_t s_sr, int dtype, hipStream_t st) {
   if ((dtype != BLR_F16 && dtype != BLR_BF16) || b < 4 || b > 16 || b % 4 || R % 8 || !aligned(Y, 16) || !aligned(Z, 16)) return 1;
   const int64_t lim = (int64_t)1 << 31;
-  if ((int64_t)b * M * R * 2 >= lim) return 1;
+  const int nrt = (int)cdiv(R, 64), nmt = (int)cdiv(M, 32);
+  if (R >= 1 << 25 || (int64_t)nrt * nmt >= lim) return 1;                         // (the rows of a tile lie within 32 bits)
   const bool rij = s_sj == 1 && s_si == b && s_sr == (int64_t)b * b && aligned(S, 8);
   const bool run = s_sr == 1 && s_si % 8 == 0 && s_sj % 8 == 0 && s_si >= 0 && s_sj >= 0 && aligned(S, 16) && ((b - 1) * (s_si + s_sj) + R) * 2 < lim;
-  if (!rij && !run) return 1;
   MixmParams p = {};
-  p.Y = Y; p.S = S; p.Z = Z; p.M = M; p.b = b; p.R = R; p.s_si = s_si; p.s_sj = s_sj;
-  const int nrt = (int)cdiv(R, 64), nmt = (int)cdiv(M, 32);
-  if ((int64_t)nrt * nmt >= 65536 || nmt >= 65536) return 1;
-  p.nmt = fd_make((uint32_t)nmt);
+  p.Y = Y; p.S = S; p.Z = Z; p.M = M; p.b = b; p.R = R; p.s_si = s_si; p.s_sj = s_sj; p.s_sr = s_sr;
+  p.nmt = nmt;
   p.items = nrt * nmt;
   const int cus = device_cus() > 0 ? device_cus() : 256;
   const unsigned grid = (unsigned)(p.items < 2 * cus ? p.items : 2 * cus);
-  void* const fn = dtype == BLR_F16 ? (rij ? (void*)blast_mixm_kernel<f16, true> : (void*)blast_mixm_kernel<f16, false>)
-                                    : (rij ? (void*)blast_mixm_kernel<bf16, true> : (void*)blast_mixm_kernel<bf16, false>);
+  void* const fns[6] = {(void*)blast_mixm_kernel<f16, MIXM_RIJ>, (void*)blast_mixm_kernel<f16, MIXM_RUN>, (void*)blast_mixm_kernel<f16, MIXM_ANY>,
+                        (void*)blast_mixm_kernel<bf16, MIXM_RIJ>, (void*)blast_mixm_kernel<bf16, MIXM_RUN>, (void*)blast_mixm_kernel<bf16, MIXM_ANY>};
   void* args[] = {&p};
-  const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(512), args, (size_t)b * 4096, st);
+  const hipError_t e = hipLaunchKernel(fns[(dtype == BLR_F16 ? 0 : 3) + (rij ? MIXM_RIJ : run ? MIXM_RUN : MIXM_ANY)], dim3(grid), dim3(512), args, (size_t)b * 4096, st);
   if (e != hipSuccess) { set_error("blast_mixm: launch failed: %s", hipGetErrorString(e)); return BLR_ERR_LAUNCH; }
   return BLR_OK;
 }
@@ -237,8 +249,8 @@ __global__ __launch_bounds__(256, 2) void blast_ymix_kernel(YmixParams p) {
   };
   auto begin = [&]() {                                 // a tile: S if its ranks are new, and the wave's first piece is asked for
     asm volatile("" : "+v"(n), "+v"(g), "+v"(r8));   // addresses are formed again for each tile: kept, they would not fit beside Y
-    const uint32_t rt = item / p.m.nmt.d;                                    // (once a tile: any number of tiles, where the quick division has a limit)
-    m0 = (int)(item - rt * p.m.nmt.d) * ROWS;
+    const uint32_t rt = item / (uint32_t)p.m.nmt;                            // (once a tile: any number of tiles, where the quick division has a limit)
+    m0 = (int)(item - rt * (uint32_t)p.m.nmt) * ROWS;
     r0 = (int)rt * 64;
     if (rt != rt_have) {
       rt_have = rt;
@@ -449,7 +461,7 @@ int blast_ymix_launch(const void* x, int64_t ldx, const void* V, const void* S, 
   const int rx = nrt * nmt <= cus ? 1 : 2;
   if (rx == 1) nmt = (int)cdiv(M, 16);
   p.slot = (rx * cl + 3) / 4 * 1024 + p.PP * 128;
-  p.m.nmt = fd_make((uint32_t)nmt);
+  p.m.nmt = nmt;
   p.m.items = nrt * nmt;
   size_t lds = (size_t)4 * p.slot;
   if (lds < (size_t)b * 2048 * rx) lds = (size_t)b * 2048 * rx;

@@ -59,6 +59,51 @@ def test_mix_element_by_element(b, order):
     assert (err <= bound).all(), f"{np.max(err / bound):.3f} of the bound"
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_bmm_fp16"])
+@pytest.mark.parametrize("b,p,r,m", [(16, 192, 128, 1100), (16, 136, 64, 1300), (12, 208, 136, 300), (8, 200, 72, 131), (4, 200, 200, 2100)])
+def test_s_off_its_boundary_mixes_to_the_same_bits(b, p, r, m, name, dtype):
+    """S one element off the 16 bytes (or the 8 of (r, i, j)): the same kernel and sums, so the same bits; in fp16 the kernels that it went to otherwise sum in fp16."""
+    from triton_funcs import blast_kernels as K, _lib as L
+    x, U, Vt, S = blast_inputs(b, p, 24, r, (m,), seed=b + r)
+    Uk, Vk, Sk = (O.blast_to_bmm_layout if "bmm" in name else O.blast_to_partial_layout)(U, Vt, S)
+    xd, ud, vd, sd = dev(x, dtype), dev(Uk, dtype), dev(Vk, dtype), dev(Sk, dtype)
+    off = torch.empty(sd.numel() + 1, device="cuda", dtype=dtype)[1:].view(sd.shape)
+    off.copy_(sd)
+    say(f"[case] mix {name} b={b} p={p} r={r} m={m} {dtype}, S one element off")
+    with L.options(BLR_BLAST_MIXU=0, BLR_DECODE_ROWS=0):
+        out, ref = (getattr(K, name)(xd, ud, vd, s, TILED) for s in (off, sd))
+    assert torch.equal(out, ref)
+
+
+def test_mix_past_two_gib_and_65536_tiles():
+    """Y of more than 2 GiB (its offsets no longer fit 31 bits) in more than 65536 tiles of 32 x 64: sums in fp32 as at every other size, looked at in rows of the first
+    tiles, about the middle, and of the last, ragged ones."""
+    import ctypes
+    from triton_funcs import _lib as L
+    dtype, b, m, r, p, q = torch.float16, 16, 131072 + 4096 + 21, 1032, 8, 8
+    g = torch.Generator("cuda").manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
+    x, V, U, S = rnd(m, b * p), rnd(b, p, r), rnd(b, r, q), rnd(b, b, r)
+    z, y = (torch.empty(b, m, r, device="cuda", dtype=dtype) for _ in range(2))
+    out = torch.empty(m, b * q, device="cuda", dtype=dtype)
+    lib = L.lib()
+    say(f"[case] mix of Y with {y.numel() * 2} bytes")
+    ws = torch.empty(lib.blr_blast_workspace_bytes(m, b * p, b * q, b, r, L.F16, 2), dtype=torch.uint8, device="cuda")
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    rc = lib.blr_blast_fwd(ptr(x), b * p, ptr(U), ptr(V), ptr(S), ptr(out), b * q, ptr(z), ptr(y), m, b * p, b * q, b, r, L.F16, L.U_RQ, L.S_IJR, 2,
+                           ptr(ws), ws.numel(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, lib.blr_last_error()
+    for rows in (slice(0, 70), slice(m // 2, m // 2 + 70), slice(m - 70, m)):
+        yd, sd = y[:, rows].double(), S.double()
+        assert torch.allclose(yd[3], x[rows, 3 * p:4 * p].double() @ V[3].double(), rtol=1e-3, atol=1e-2)
+        ref = torch.stack([(sd[i][:, None] * yd).sum(0) for i in range(b)])
+        mag = torch.stack([(sd[i][:, None] * yd).abs().sum(0) for i in range(b)])
+        err = (z[:, rows].double() - ref).abs().cpu().numpy()
+        bound = 0.5 * ulp(ref.cpu().numpy(), dtype) * (1 + 2.0 ** -10) + 16 * 2.0 ** -24 * mag.cpu().numpy()
+        assert (err <= bound).all(), f"{np.max(err / bound):.3f} of the bound"
+
+
 FUSED = {"algo": 3}
 
 
