@@ -201,9 +201,10 @@ int gemm_mid_launch(const GemmArgs& a, int kind, bool partial, int dtype, hipStr
 int gemm_mid_f32_slices(int M, int N, int K);   // slices that the reduction of a single fp32 product is worth cutting into
 int gemm_mid_f32_launch(const GemmArgs& a, bool partial, hipStream_t st);
 // Kernels for products of more tiles than compute units, on tiles of 256 x 32 tn (blr_gemm_wide.hip): whether they take the operands, the tn
-// (3 .. 11) for the shape - or, where ring64, 0 .. 2 for a ring kernel that is faster -, and the launch.
+// (3 .. 11) for the shape - or, where the ring kernels take the operands too (ring), 0 .. 2 for one with stages of 64 k that is faster, -1 for their own rules -,
+// and the launch.
 bool gemm_wide_ok(const GemmArgs& a);
-int gemm_wide_plan(const GemmArgs& a, bool ring64);
+int gemm_wide_plan(const GemmArgs& a, bool ring);
 int gemm_wide_launch(const GemmArgs& a, int tn, int dtype, hipStream_t st);
 // Scratch a plain single GEMM M x N x K of dtype wants in GemmArgs::splitk_ws so that a problem with few output tiles and
 // a long reduction can be cut along K to fill the chip (fp32 partial results, summed in a fixed order).  0: no split.

@@ -1360,14 +1360,17 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
     if (pl.kind == MID_RING_128_TWO) return launch_ring64<T, 128, 128, 4, 2, 2>(g, st);
     if (pl.kind >= 0) return gemm_mid_launch(g, pl.kind, false, dt, st);
   }
-  // More tiles than compute units: the width of the tile, or one of the ring kernels with stages of 64 k, by the estimates of blr_gemm_wide.hip
+  // More tiles than compute units: the width of the tile, one of the ring kernels with stages of 64 k, or the rules below, by the estimates of blr_gemm_wide.hip
   // (BLR_GEMM_WIDE: 0 never, 1 by this rule, 3 .. 11 tiles of that many times 32 columns for every product that the kernels take).
   const int wide = option_value(OPT_GEMM_WIDE, 1);
   const bool ring_asked = ring != 1 || option_value(OPT_GEMM_RING_TILE, 0) || option_value(OPT_GEMM_RING_PER_CU, 0) || option_value(OPT_GEMM_RING_WAVES, 0) || option_value(OPT_GEMM_RING_BK, 0);
   if (wide && (wide > 1 || !ring_asked) && gemm_wide_ok(g)) {
-    const int w = wide > 1 ? wide : gemm_wide_plan(g, ring_ok(g) && g.epi == EPI_PLAIN);
+    // (a scatter that the kernels take is in whole 16-byte pieces: the ring kernels take it as well)
+    const int w = wide > 1 ? wide : gemm_wide_plan(g, g.M >= 96 && ring_ok(g));
     if (w >= 3) return gemm_wide_launch(g, w, std::is_same<T, f16>::value ? BLR_F16 : BLR_BF16, st);
-    return w == 0 ? launch_ring64<T, 128, 128, 4, 2, 2>(g, st) : w == 1 ? launch_ring64<T, 256, 128, 8, 3, 1>(g, st) : launch_ring64<T, 256, 256, 8, 2, 1>(g, st);
+    if (w == 0) return launch_ring64<T, 128, 128, 4, 2, 2>(g, st);
+    if (w == 1) return launch_ring64<T, 256, 128, 8, 3, 1>(g, st);
+    if (w == 2) return launch_ring64<T, 256, 256, 8, 2, 1>(g, st);
   }
   if (g.pair && (!ring_ok(g) || g.epi != EPI_PLAIN || g.cn != 1 || g.sat8 || g.gate || g.resid || g.pair_dA % 8 || g.pair_dB % 8 || g.pair_dbias % 8 || !aligned(g.C, 16))) {
     set_error("gemm: a pair of tiles (SiLU-gated halves) needs 16-byte aligned operands, K and the half width multiples of 8, a plain row-major output");

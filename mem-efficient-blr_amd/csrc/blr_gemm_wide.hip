@@ -15,8 +15,8 @@
 //   * a workgroup walks its tiles: the last two steps of one load the first two stages of the next, and the way out needs no barrier
 //     (a wave turns its own blocks in a piece of LDS beside the ring), so that the next tile's loads land under it: 4096 x 576 x 288 in 16
 //     batches 46.8 -> 43.2 us.
-// Measured against the 32-k and 64-k ring kernels with their old rules, 420 products of 260 .. 4096 rows, 64 .. 22000 columns, 72 .. 11000 k, 1 .. 16
-// batches: 0.80 x the time in the mean (geometric), 0.55 at best, 1.07 - 1.11 at worst (three long dense reductions).  4096 x 288 x 576 in 16
+// Measured against the 32-k and 64-k ring kernels with their rules, 1818 products of 260 .. 4096 rows, 64 .. 22000 columns, 72 .. 11008 k, 1 .. 16
+// batches, weights from memory: 0.83 x the time in the mean (geometric), 0.5 at best, 1.17 at worst (gemm_wide_plan has more).  4096 x 288 x 576 in 16
 // batches 49.4 -> 32.6 us (668 TFLOP/s), 2048 x 1024 x 2136 in 3 132.8 -> 76.9, 4096 x 576 x 1000 in 16 60.7 -> 41.4.
 #include <mutex>
 #include <set>
@@ -413,10 +413,9 @@ int wide_width_launch(const GemmArgs& g, int tn, hipStream_t st) {
 }
 
 // What a launch takes, in microseconds: t = c0 + (c1 R + c3 f) w + (c2 R + c4 f) w k, with k = stages of 64, w = the tile's size in units of
-// 256 x 32, f = tiles / what the chip holds at a time, R = f rounded up.  Fitted (non-negative, on relative errors) to eager launches, 24 in a row, of
-// 870 products of 129 .. 4096 rows, 64 .. 22000 columns, 72 .. 11008 k and 1 .. 16 batches on every kind: 7 - 12 % rms each.  On 200 products
-// outside the fit the kind with the smallest estimate takes 0.825 x the time of the rules before (the best kind 0.819 x), three of them
-// more than 3 % longer (8 % at worst); of 200 reductions of 1000 .. 11008 k 0.86 x, eight of them 7 - 15 % longer, one 32 %.
+// 256 x 32, f = tiles / what the chip holds at a time, R = f rounded up.  Fitted (non-negative, on relative errors) to eager launches, 24 in a row over two copies of
+// the operands, of 870 plain products of 129 .. 4096 rows, 64 .. 22000 columns, 72 .. 11008 k and 1 .. 16 batches on every kind: 7 - 12 % rms each.  An output stage
+// costs every kind about the same: with bias and GELU 259 products chosen by these estimates take 0.82 x the time of the ring rules, 1.04 x at worst but for one.
 struct WideModel { int bm, bn, occ; float c[5]; };
 const WideModel kWideModel[12] = {
     {128, 128, 2, {3.424f, 0.050f, 0.202f, 2.019f, 0.406f}},           // the ring kernels with stages of 64 k
@@ -447,21 +446,32 @@ bool gemm_wide_ok(const GemmArgs& g) {
          32 * g.ldc + g.N < lim / 2;
 }
 
-// Columns of the tile in units of 32, or 0, 1, 2 for the ring kernels with stages of 64 k on tiles of 128 x 128, 256 x 128 and 256 x 256, which keep the
-// products that they are estimated to be faster on: mostly reductions of a thousand and more whose tiles of 256 x 128 make whole rounds
-// (2048 x 4096 x 11008: 172 us there, 211 on the best of these tiles).
-int gemm_wide_plan(const GemmArgs& g, bool ring64) {
+// Columns of the tile in units of 32, or 0, 1, 2 for the ring kernels with stages of 64 k on tiles of 128 x 128, 256 x 128 and 256 x 256, or -1 for the ring
+// kernels by their own rules.  The estimates decide for short reductions.  For long ones they are too kind to the tiles here, whose ring is two stages deep, as soon
+// as operands come from memory (they were fitted to warm ones): 4096 x 4096 x 11008 takes 287 us in 256 x 256 tiles of the ring kernel and 321 here, 2048 x 1024 x 2752
+// in 4 batches with Monarch's scatter 49 and 52 - 59 (256 x 128).  So from 1536 k on a single product comes here where its estimate is 5 % better and one of
+// several batches where it is 8 % better, and the others of several batches keep the rules that they had (2048 x 176 x 2088 in 16: 53 us, and 61 on the best of these
+// tiles).  The 8 % are asked from 1024 k on where the batches share the rows of A, which then is the input of a call and not what the launch before left in the
+// caches: Monarch 4096 -> 22016 at 2048 rows 168.7 -> 164.1 us, while Z U of BLAST 11008 -> 4096 stays (the call 113 us, 115 with the ring kernel).  A pair in four
+// batches and more with less than 200 k and results for several rounds is two ways out for hardly any products: 2833 x 1952 x 120 in 4 43.5 us there, 51.0 here,
+// 1548 x 832 x 192 in 8 26.4 and 28.0 (3838 x 584 x 144 the other way, 50.5 and 43.4).
+// With weights from memory, against the ring rules alone: 660 products of 1024 .. 11008 k 0.866 x the time in the mean, nine 3 - 8 % longer (most of them the same kernel,
+// timed twice); 1158 shorter ones, with scatter, output stage and pairs among them, 0.813 x, eight 4 - 17 % longer (the worst: 1528 x 768 x 88 in 16, scattered).
+int gemm_wide_plan(const GemmArgs& g, bool ring) {
   const int cus = device_cus() > 0 ? device_cus() : 256, K = g.pair ? 2 * g.K : g.K;
-  int best = 3;
-  float t_best = 1e30f;
-  for (int i = ring64 ? 0 : 3; i < 12; ++i) {
+  if (ring && g.pair && g.batch >= 4 && g.K < 200 && (int64_t)g.M * g.N * g.batch >= (int64_t)32768 * cus) return -1;
+  int best[2] = {0, 3};                              // ring, wide
+  float t_best[2] = {1e30f, 1e30f};
+  for (int i = ring ? 0 : 3; i < 12; ++i) {
     const WideModel& m = kWideModel[i];
     const int64_t tiles = cdiv(g.M, m.bm) * cdiv(g.N, m.bn) * g.batch, holds = (int64_t)cus * m.occ;
     const float f = (float)tiles / holds, R = (float)cdiv(tiles, holds), w = (float)m.bm * m.bn / 8192.f, k = (float)K / 64.f;
     const float t = m.c[0] + (m.c[1] * R + m.c[3] * f) * w + (m.c[2] * R + m.c[4] * f) * w * k;
-    if (t < t_best) { t_best = t; best = i; }
+    if (t < t_best[i >= 3]) { t_best[i >= 3] = t; best[i >= 3] = i; }
   }
-  return best;
+  const bool deep = g.K >= 1536, apart = g.K >= 1024 && g.batch > 1 && g.lda > g.K;
+  if (t_best[1] < (!deep && !apart ? 1.0f : g.batch > 1 ? 0.92f : 0.95f) * t_best[0]) return best[1];
+  return deep && g.batch > 1 ? -1 : best[0];
 }
 
 int gemm_wide_launch(const GemmArgs& g, int tn, int dtype, hipStream_t st) {

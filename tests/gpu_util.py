@@ -1,4 +1,5 @@
-"""Shared helpers of the GPU parity tests (seeded inputs, oracle comparison)."""
+"""Shared helpers of the GPU parity tests (seeded inputs, oracle comparison, which kernels a call launches)."""
+import ctypes
 import sys
 
 import numpy as np
@@ -50,3 +51,31 @@ def ulp(ref, dtype):
     """Spacing of dtype's numbers at |ref| (float64 numpy): 2^(e - 10) for fp16, 2^(e - 7) for bf16, normal range."""
     a = np.maximum(np.abs(np.asarray(ref, dtype=np.float64)), 2.0 ** -14)
     return 2.0 ** (np.floor(np.log2(a)) - {torch.float16: 10, torch.bfloat16: 7}[dtype])
+
+
+class _KernelNode(ctypes.Structure):                 # hipKernelNodeParams
+    _fields_ = [("block", ctypes.c_uint32 * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint32 * 3), ("params", ctypes.c_void_p),
+                ("lds", ctypes.c_uint32)]
+
+
+def launches(call):
+    """(host function, grid, block, dynamic LDS) of every kernel that call(stream) launches on the stream that it is handed: captured into a graph that is looked at and
+    not run.  call allocates nothing."""
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    stream, graph, n = torch.cuda.Stream(), ctypes.c_void_p(), ctypes.c_size_t()
+    torch.cuda.synchronize()
+    assert hip.hipStreamBeginCapture(ctypes.c_void_p(stream.cuda_stream), 2) == 0          # relaxed
+    call(stream.cuda_stream)
+    assert hip.hipStreamEndCapture(ctypes.c_void_p(stream.cuda_stream), ctypes.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)) == 0
+    out = []
+    for node in nodes:
+        kind, k = ctypes.c_int(), _KernelNode()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0 and kind.value == 0, "a node that is no kernel"
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(k)) == 0
+        out.append((k.func, tuple(k.grid), tuple(k.block), k.lds))
+    assert hip.hipGraphDestroy(graph) == 0
+    return out

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from oracle import blr_oracle as O
-from gpu_util import assert_close, blast_inputs, dev, rounded, say, ulp
+from gpu_util import assert_close, blast_inputs, dev, launches, rounded, say, ulp
 
 pytestmark = pytest.mark.gpu
 
@@ -122,3 +122,90 @@ def test_infinite_weights_stay_infinite(k):
     with L.options(BLR_GEMM_WIDE=3):
         out = K.triton_dense_fp16(dev(x, torch.float16), dev(w, torch.float16), TILED).double().cpu().numpy()
     assert (out == x @ w).all()
+
+
+def _three_ways(call, ring, wide):
+    """What a call launches by the rules, with a ring kernel asked for by name, and with tiles of 32 wide columns."""
+    from triton_funcs import _lib as L
+    with L.options(BLR_GEMM_RING_TILE=ring, BLR_GEMM_RING_BK=64, BLR_GEMM_RING_WAVES=8, BLR_GEMM_RING_PER_CU=2 if ring == 128128 else 0):
+        by_name = launches(call)
+    with L.options(BLR_GEMM_WIDE=wide):
+        on_wide = launches(call)
+    return launches(call), by_name, on_wide
+
+
+# (columns per input block, rank, rows, tile of the ring kernel, the wide tile that would be next): long reductions whose rows of x lie far apart
+@pytest.mark.parametrize("p,rank,m,ring,wide", [(2752, 1024, 2048, 256128, 4), (1024, 1024, 2048, 256128, 4), (2752, 1024, 4096, 256256, 8)])
+def test_monarch_of_long_blocks_stays_with_the_ring_kernels(p, rank, m, ring, wide):
+    from triton_funcs import _lib as L
+    b, s, dtype = 4, 64, torch.float16
+    g = torch.Generator("cuda").manual_seed(p + m)
+    rnd = lambda *sh: torch.randn(*sh, device="cuda", generator=g).to(dtype)
+    x, w1, w2 = rnd(m, b * p), (rnd(b, p, rank).float() / p ** 0.5).to(dtype), rnd(b, rank, s)
+    mid, out = torch.full((b, m, rank), float("nan"), device="cuda", dtype=dtype), torch.empty(m, b * s, device="cuda", dtype=dtype)
+
+    def call(stream):
+        L.check(L.lib().blr_monarch_fwd(x.data_ptr(), b * p, w1.data_ptr(), w2.data_ptr(), out.data_ptr(), b * s, mid.data_ptr(), m, b * p, b * s, b, rank, L.F16, L.W2_RS,
+                                        L.OUT_BLOCKED, 2, None, 0, stream), "blr_monarch_fwd")
+
+    say(f"[case] monarch, first product {m}x{rank}x{p} in {b}")
+    auto, by_name, on_wide = _three_ways(call, ring, wide)
+    assert auto[0] == by_name[0] != on_wide[0]
+    call(L.stream_ptr(x.device))
+    y = torch.stack([x[:, k * p:(k + 1) * p].float() @ w1[k].float() for k in range(b)])          # column c of block k -> block c / per, column k per + c % per
+    per = rank // b
+    ref = y.view(b, m, b, per).permute(2, 1, 0, 3).reshape(b, m, rank)
+    assert_close(mid, ref.double().cpu().numpy(), dtype, "first product", scale=0.5)
+
+
+@pytest.mark.parametrize("m,n,k,act,ring,wide", [(4096, 4096, 11008, "", 256256, 8), (1000, 6912, 1152, "gelu_tanh", 256128, 4), (2048, 2304, 2048, "gelu_tanh", 256128, 4),
+                                                 (1043, 6328, 1992, "silu_mul", 256128, 4)])
+def test_dense_products_that_the_ring_kernels_keep(m, n, k, act, ring, wide):
+    """Plain, with bias and activation, and gated halves."""
+    from triton_funcs import _lib as L
+    dtype, h = torch.float16, 2 if act == "silu_mul" else 1
+    g = torch.Generator("cuda").manual_seed(m)
+    rnd = lambda *sh: torch.randn(*sh, device="cuda", generator=g).to(dtype)
+    x, w, bias, out = rnd(m, k), (rnd(k, h * n).float() / k ** 0.5).to(dtype), rnd(h * n), torch.full((m, n), float("nan"), device="cuda", dtype=dtype)
+    code = {"": 0, "gelu_tanh": 1, "silu_mul": 3}[act]
+
+    def call(stream):
+        L.check(L.lib().blr_dense_fwd_ep(x.data_ptr(), k, w.data_ptr(), out.data_ptr(), n, m, k, h * n, L.F16, 2, None, 0, stream, bias.data_ptr() if act else None, code), "dense")
+
+    say(f"[case] dense {m}x{n}x{k} {act}")
+    auto, by_name, on_wide = _three_ways(call, ring, wide)
+    assert auto == by_name and auto != on_wide
+    call(L.stream_ptr(x.device))
+    y = x.float() @ w.float()
+    if act:
+        y = y + bias.float()
+        y = torch.nn.functional.gelu(y, approximate="tanh") if h == 1 else torch.nn.functional.silu(y[:, :n]) * y[:, n:]
+    assert_close(out, y.double().cpu().numpy(), dtype, "dense")
+
+
+@pytest.mark.parametrize("q,r,m,kept", [(1952, 120, 2833, True), (832, 192, 2600, True), (1952, 208, 2833, False), (1000, 120, 1900, False)])
+def test_gated_halves_of_short_reductions(q, r, m, kept):
+    """Eight blocks as four pairs, less than 200 k: with results for several rounds the ring kernels' rules, otherwise tiles of this kernel."""
+    from triton_funcs import _lib as L
+    b, p, dtype = 8, 40, torch.float16
+    g = torch.Generator("cuda").manual_seed(q)
+    rnd = lambda *sh: torch.randn(*sh, device="cuda", generator=g).to(dtype)
+    x, U, V, S, bias = rnd(m, b * p), (rnd(b, q, r).float() / r ** 0.5).to(dtype), (rnd(b, p, r).float() / p ** 0.5).to(dtype), rnd(r, b, b), rnd(b * q)
+    out = torch.full((m, b * q // 2), float("nan"), device="cuda", dtype=dtype)
+    lib = L.lib()
+    ws = torch.empty(lib.blr_blast_workspace_bytes(m, b * p, b * q, b, r, L.F16, 2), dtype=torch.uint8, device="cuda")
+
+    def call(stream):
+        L.check(lib.blr_blast_fwd_ep(x.data_ptr(), b * p, U.data_ptr(), V.data_ptr(), S.data_ptr(), out.data_ptr(), b * q // 2, m, b * p, b * q, b, r, L.F16, L.U_QR, L.S_RIJ, 2,
+                                     ws.data_ptr(), ws.numel(), stream, bias.data_ptr(), 3), "blr_blast_fwd_ep")
+
+    say(f"[case] gated halves q={q} r={r} m={m}")
+    auto = launches(call)
+    with L.options(BLR_GEMM_WIDE=0):
+        ring = launches(call)
+    assert (auto[-1] == ring[-1]) == kept
+    call(L.stream_ptr(x.device))
+    Y = torch.bmm(x.float().view(m, b, p).transpose(0, 1).contiguous(), V.float()).half().float()
+    y = torch.cat([(Y * S[:, i].float().t()[:, None]).sum(0).half().float() @ U[i].float().t().contiguous() for i in range(b)], 1).half().float() + bias.float()
+    h = b * q // 2
+    assert_close(out, (torch.nn.functional.silu(y[:, :h]) * y[:, h:]).double().cpu().numpy(), dtype, "gated halves")
