@@ -1547,29 +1547,16 @@ static void mix_dispatch(dim3 grid, size_t lds, hipStream_t st, const void* Y, c
 template <typename T> constexpr int mix_vw = 16 / (int)sizeof(T);      // ranks per 16-byte piece
 template <typename T> constexpr int mix_ch = 8 * mix_vw<T>;            // ranks of a chunk
 template <typename T> constexpr int mix_ldr = 9 * mix_vw<T>;
-enum { MIX_S_ANY = 0, MIX_S_R = 1, MIX_S_RIJ = 2, MIX_S_ROW = 3 };     // element by element; 16-byte pieces along r; pieces of the run of (r, i, j), each inside a row (r, i)
+enum { MIX_S_ANY = 0, MIX_S_R = 1, MIX_S_RIJ = 2 };     // element by element; 16-byte pieces along r; pieces of the run of (r, i, j)
 // MIX_S_RIJ reads the chunk as the one contiguous run that it is and lets each element find its place (element by element, a wave's
-// lanes lay 2 b^2 bytes apart; the three linears of a GPT-2 block, 4 and 6 blocks, at 1158 rows 60.7 -> 56.6 us).  Where a row is whole pieces nothing has to be found
-// (ROW, kernels of their own for fp16: one branch more beside the others slows those by 2 %): 16 blocks, whole calls, 5632 -> 1664, r = 864 at 1462 rows 69.3 -> 67.5 us,
-// 2944 -> 6912, r = 320 at 1215 rows 46.5 -> 44.8, 2176 -> 2176, r = 128 at 4096 rows 44.0 -> 42.3.  In bf16, whose kernel is bound by its arithmetic, it is ahead by 2 % on
-// the first, level on the second and behind by 3 % on the third, and is not used.
-template <typename T, bool ROW>
+// lanes lay 2 b^2 bytes apart; the three linears of a GPT-2 block at 1158 rows, whose 6 blocks come here, 60.7 -> 56.6 us).
+template <typename T>
 __device__ __forceinline__ void mix_stage_s(const T* __restrict__ S, T* s_t, int b, int R, int r0,
                                             int64_t s_si, int64_t s_sj, int64_t s_sr, int s_order) {
   constexpr int VW = mix_vw<T>, CH = mix_ch<T>, LDR = mix_ldr<T>;
   typedef T V8 __attribute__((ext_vector_type(VW)));
   const int tid = threadIdx.x;
-  if constexpr (ROW) {
-    const int jv = b / VW;
-    for (int idx = tid; idx < CH * b * jv; idx += 256) {
-      const int j0 = (idx % jv) * VW, t = idx / jv;
-      const int i = t % b, r = t / b;
-      V8 v = (T)0.0f;
-      if (r0 + r < R) v = *reinterpret_cast<const V8*>(&S[(int64_t)(r0 + r) * s_sr + (int64_t)i * s_si + j0]);
-#pragma unroll
-      for (int e = 0; e < VW; ++e) s_t[((j0 + e) * b + i) * LDR + r] = v[e];
-    }
-  } else if (s_order == MIX_S_R) {                             // (j, i, r) or (i, j, r): r contiguous
+  if (s_order == MIX_S_R) {                             // (j, i, r) or (i, j, r): r contiguous
     for (int idx = tid; idx < b * b * 8; idx += 256) {
       const int r8 = (idx & 7) * VW, ji = idx >> 3;
       const int j = ji / b, i = ji - j * b;
@@ -1615,7 +1602,7 @@ __global__ __launch_bounds__(256) void blast_mix_vec_kernel(const T* __restrict_
   T* s_t = reinterpret_cast<T*>(s_lds);      // [b][b][chunk]  (j, i, r)
   const int tid = threadIdx.x;
   const int r0 = blockIdx.x * mix_ch<T>;
-  mix_stage_s<T, false>(S, s_t, b, R, r0, s_si, s_sj, s_sr, s_order);
+  mix_stage_s<T>(S, s_t, b, R, r0, s_si, s_sj, s_sr, s_order);
   __syncthreads();
   const int rl = tid & 7, ms = tid >> 3;     // 8 r-vectors x 32 m slots
   const int r = r0 + rl * VW;
@@ -1647,10 +1634,10 @@ __global__ __launch_bounds__(256) void blast_mix_vec_kernel(const T* __restrict_
   }
 }
 
-// fp16 only: the same mix with packed half-precision multiply-adds (two per lane and instruction).
-// The b <= 16 products of one output are accumulated in fp16; Z is stored as fp16 anyway and the
+// fp16 only: the same mix with packed half-precision multiply-adds (two per lane and instruction), for numbers of blocks that are no multiple of four
+// (blast_mixm_kernel takes the others).  The b < 16 products of one output are accumulated in fp16; Z is stored as fp16 anyway and the
 // reference rounds it to 16 bits as well, so this costs about one extra rounding of the result.
-template <bool FULL16, int MB, bool ROW>         // FULL16: b == 16, so no load sits under a condition; MB rows of m per thread
+template <int MB>                                // MB rows of m per thread
 __global__ __launch_bounds__(256) void blast_mix_h2_kernel(const f16* __restrict__ Y, const f16* __restrict__ S,
                                                            f16* __restrict__ Z, int M, int b, int R,
                                                            int64_t s_si, int64_t s_sj, int64_t s_sr, int m_per_wg, int s_order) {
@@ -1660,7 +1647,7 @@ __global__ __launch_bounds__(256) void blast_mix_h2_kernel(const f16* __restrict
   f16* s_t = reinterpret_cast<f16*>(s_lds);      // [b][b][64]  (j, i, r)
   const int tid = threadIdx.x;
   const int r0 = blockIdx.x * 64;
-  mix_stage_s<f16, ROW>(S, s_t, ROW && FULL16 ? 16 : b, R, r0, s_si, s_sj, s_sr, s_order);
+  mix_stage_s<f16>(S, s_t, b, R, r0, s_si, s_sj, s_sr, s_order);
   __syncthreads();
   const int rl = tid & 7, ms = tid >> 3;     // 8 r-vectors x 32 m slots
   const int r = r0 + rl * 8;
@@ -1675,7 +1662,7 @@ __global__ __launch_bounds__(256) void blast_mix_h2_kernel(const f16* __restrict
       const int mu = min(m + 32 * u, M - 1);         // rows past the end are fetched again and not stored
 #pragma unroll
       for (int j = 0; j < 16; ++j)                   // unconditional: planes past b re-read the last one and are not used
-        yv[u][j] = *reinterpret_cast<const H8*>(&Y[((int64_t)(FULL16 ? j : min(j, b - 1)) * M + mu) * R + r]);
+        yv[u][j] = *reinterpret_cast<const H8*>(&Y[((int64_t)min(j, b - 1) * M + mu) * R + r]);
     }
     for (int i = 0; i < b; ++i) {
       H8 acc[MB];
@@ -1685,7 +1672,7 @@ __global__ __launch_bounds__(256) void blast_mix_h2_kernel(const f16* __restrict
         for (int e = 0; e < 4; ++e) acc[u].v[e] = h2{(_Float16)0.0f, (_Float16)0.0f};
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        if (FULL16 || j < b) {
+        if (j < b) {
           const H8 sv = *reinterpret_cast<const H8*>(&s_t[(j * b + i) * mix_ldr<f16> + rl * 8]);
 #pragma unroll
           for (int u = 0; u < MB; ++u)
@@ -1755,17 +1742,14 @@ int blast_mix_launch(const void* Y, const void* S, void* Z, int M, int b, int R,
     const size_t lds = (size_t)b * b * 144;
     const bool use_h2 = dtype == BLR_F16 && !sat8 && M > 16;
     const int s_order = !aligned(S, 16) ? MIX_S_ANY : s_sr == 1 && s_si % vw == 0 && s_sj % vw == 0 ? MIX_S_R
-                        : s_sj == 1 && s_si == b && s_sr == (int64_t)b * b ? (use_h2 && b % vw == 0 ? MIX_S_ROW : MIX_S_RIJ) : MIX_S_ANY;
+                        : s_sj == 1 && s_si == b && s_sr == (int64_t)b * b ? MIX_S_RIJ : MIX_S_ANY;
     const int mb = use_h2 && M >= 64 ? 2 : 1;
     const int m_per_wg = 32 * mb;                  // one pass of the 32 row slots: more, smaller workgroups measured fastest
     dim3 grid(r_chunks, (unsigned)cdiv(M, m_per_wg));
     if (use_h2) {
-      void* const fns[8] = {(void*)blast_mix_h2_kernel<false, 1, false>, (void*)blast_mix_h2_kernel<false, 1, true>, (void*)blast_mix_h2_kernel<false, 2, false>, (void*)blast_mix_h2_kernel<false, 2, true>,
-                            (void*)blast_mix_h2_kernel<true, 1, false>, (void*)blast_mix_h2_kernel<true, 1, true>, (void*)blast_mix_h2_kernel<true, 2, false>, (void*)blast_mix_h2_kernel<true, 2, true>};
-      int m_wg = m_per_wg, order = s_order;
-      void* args[] = {&Y, &S, &Z, &M, &b, &R, &s_si, &s_sj, &s_sr, &m_wg, &order};
-      const hipError_t e = hipLaunchKernel(fns[(b == 16 ? 4 : 0) + (mb == 2 ? 2 : 0) + (s_order == MIX_S_ROW ? 1 : 0)], grid, dim3(256), args, lds, st);
-      if (e != hipSuccess) { set_error("blast_mix: launch failed: %s", hipGetErrorString(e)); return BLR_ERR_LAUNCH; }
+      if (mb == 2) hipLaunchKernelGGL(blast_mix_h2_kernel<2>, grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_order);
+      else hipLaunchKernelGGL(blast_mix_h2_kernel<1>, grid, dim3(256), lds, st, (const f16*)Y, (const f16*)S, (f16*)Z, M, b, R, s_si, s_sj, s_sr, m_per_wg, s_order);
+      BLR_CHECK_LAUNCH("blast_mix_h2");
       return BLR_OK;
     }
     if (dtype == BLR_F16)
