@@ -432,7 +432,7 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
   if (rc == 1 && !mixu && !y_out && !sat8 && fused >= 0 && (fused == 1 || P <= fuse_max_p))
     rc = blast_ymix_launch(x, ldx, V, S, Z, M, in_f, b, r, si, sj, sr, dtype, Y, ybytes, st);   // (the unused room of Y holds S as (r, i, j) if it has to)
   if (rc < 0) return rc;
-  if (rc == 1 && fused == 1) { set_error("blast: the fused kernel does not take this shape (b even and <= 16, block width and rank multiples of 8, f16/bf16)"); return BLR_ERR_UNSUPPORTED; }
+  if (rc == 1 && fused == 1) { set_error("blast: the fused kernel does not take this call (b a multiple of 4 and <= 16, block width and rank multiples of 8, operands on 16 bytes, f16/bf16)"); return BLR_ERR_UNSUPPORTED; }
   if (rc == 1) {
     GemmArgs g1 = {};
     g1.A = x; g1.lda = ldx; g1.sA = P;

@@ -200,9 +200,10 @@ def test_blast_bmm_narrow_output_blocks(shape, dtype):
 
 def test_blast_fused_refuses_what_it_cannot_tile():
     from triton_funcs import _lib as L
-    x, U, Vt, S = blast_inputs(2, 40, 24, 72, (5,), seed=22)              # two blocks: not a multiple of four
-    with pytest.raises(L.BlrError, match="fused"):
-        _run_blast("triton_blast_full_fp16", x, U, Vt, S, torch.float16, "fused")
+    for b, r in ((2, 72), (6, 72), (4, 36)):                              # numbers of blocks that are even and no multiple of four, a rank that is no multiple of eight
+        x, U, Vt, S = blast_inputs(b, 40, 24, r, (5,), seed=22)
+        with pytest.raises(L.BlrError, match="fused.*multiple of 4"):
+            _run_blast("triton_blast_full_fp16", x, U, Vt, S, torch.float16, "fused")
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
