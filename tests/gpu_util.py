@@ -79,3 +79,19 @@ def launches(call):
         out.append((k.func, tuple(k.grid), tuple(k.block), k.lds))
     assert hip.hipGraphDestroy(graph) == 0
     return out
+
+
+def blast_call(name, x, U, V, S, algo):
+    """A call of the C ABI with the layouts of name's functions, for launches() or a stream, and the tensor that it writes."""
+    from triton_funcs import _lib as L
+    bmm = "bmm" in name
+    (b, p, r), m = V.shape, x.shape[0]
+    q = U.shape[1] if bmm else U.shape[2]
+    dt = L.F16 if x.dtype == torch.float16 else L.BF16
+    out = torch.full((m, b * q), float("nan"), device="cuda", dtype=x.dtype)
+    ws = torch.empty(L.lib().blr_blast_workspace_bytes(m, b * p, b * q, b, r, dt, algo), dtype=torch.uint8, device="cuda")
+
+    def call(stream):
+        L.check(L.lib().blr_blast_fwd(x.data_ptr(), b * p, U.data_ptr(), V.data_ptr(), S.data_ptr(), out.data_ptr(), b * q, None, None, m, b * p, b * q, b, r, dt,
+                                      L.U_QR if bmm else L.U_RQ, L.S_RIJ if bmm else L.S_JIR, algo, ws.data_ptr(), ws.numel(), stream), "blr_blast_fwd")
+    return call, out

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from oracle import blr_oracle as O
-from gpu_util import assert_close, back, blast_inputs, dev, rounded, say
+from gpu_util import assert_close, back, blast_call, blast_inputs, dev, launches, rounded, say
 
 pytestmark = pytest.mark.gpu
 
@@ -103,7 +103,7 @@ FUSED_SHAPES = [(16, 64, 72, 128, (96,)), (16, 72, 216, 288, (2, 75)), (4, 48, 2
 @pytest.mark.parametrize("shape", FUSED_SHAPES)
 def test_blast_fused_algorithm(name, shape, dtype):
     """BLR_ALGO_FUSED: x V and the mix in one launch (Y only ever in LDS), then the batched product with U.  Row counts that
-    are not multiples of the 32-row tile, ranks that are not multiples of the 128-rank tile, k past a block's width, 4 to
+    are not multiples of a tile's 16 or 32 rows, ranks that are not multiples of its 64, blocks of one to eight pieces of columns, 4 to
     16 blocks, S in both layouts."""
     b, p, q, r, lead = shape
     say(f"[case] fused {name} b={b} p={p} q={q} r={r} lead={lead} {dtype}")
@@ -116,7 +116,7 @@ def test_blast_fused_algorithm(name, shape, dtype):
 
 
 # more tiles of the fused first half than compute units, so that a workgroup walks several: runs that go from one rank tile to the next, a last
-# tile with few rows and few ranks, one to four 32-column steps, four to sixteen blocks; 128 ranks at 16 blocks (Z's rows do not fit LDS behind Y)
+# tile with few rows and few ranks, blocks of one and two pieces of up to 96 columns, four to sixteen blocks
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("b,p,r,M", [(16, 72, 576, 4101), (16, 72, 296, 2990), (16, 8, 128, 12001), (4, 40, 136, 9001), (12, 32, 200, 5000), (8, 128, 1024, 1500)])
 def test_blast_fused_first_half_walks(b, p, r, M, dtype):
@@ -137,20 +137,24 @@ def test_blast_fused_first_half_walks(b, p, r, M, dtype):
 @pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_bmm_fp16"])
 @pytest.mark.parametrize("shape", [(16, 256, 256, 512, (1100,)), (16, 192, 88, 256, (8, 130))])
 def test_blast_wide_input_blocks_first_half_on_and_off(name, shape, dtype):
-    """Row counts that fill half the chip with 64 x 64 tiles take x V and the mix as one launch by default (16 input blocks of
-    a multiple of 64 columns, Y in registers); BLR_BLAST_YMIXW=0 sends the same call through the batched GEMM and the mix
-    kernel.  Both against the oracle and against each other, S in both layouts (the (j, i, r) one is staged through LDS inside
-    the kernel); row counts that end inside a tile."""
+    """The fused algorithm takes x V and the mix of 16 input blocks of a multiple of 64 columns as one launch (Y in registers);
+    by itself the same call goes through the batched GEMM and the mix kernel.  Both against the oracle and against each other, S in
+    both layouts (the (j, i, r) one is staged through LDS inside the kernel); row counts that end inside a tile."""
     from triton_funcs import _lib as L
     b, p, q, r, lead = shape
     say(f"[case] wide input blocks {name} b={b} p={p} q={q} r={r} lead={lead} {dtype}")
-    x, U, Vt, S = blast_inputs(b, p, q, r, lead, seed=33)
-    out = _run_blast(name, x, U, Vt, S, dtype, "auto")
+    x, U, Vt, S = blast_inputs(b, p, q, r, (int(np.prod(lead)),), seed=33)
     ref = _ref(x, U, Vt, S, dtype)[0]
-    assert_close(out, ref.reshape(tuple(out.shape)), dtype, f"one launch {name}")
-    with L.options(BLR_BLAST_YMIXW=0):
-        off = _run_blast(name, x, U, Vt, S, dtype, "auto")
-    assert_close(off, ref.reshape(tuple(out.shape)), dtype, f"GEMM + mix {name}")
+    args = [dev(t, dtype) for t in (x,) + ((O.blast_to_bmm_layout if "bmm" in name else O.blast_to_partial_layout)(U, Vt, S))]
+    call, out = blast_call(name, *args, ALGO["fused"])
+    first = launches(call)[0]
+    assert first[2] == (256, 1, 1) and first[3] == 160 * 1024             # a workgroup of four waves that has a compute unit's LDS to itself
+    call(L.stream_ptr(out.device))
+    assert_close(out, ref, dtype, f"one launch {name}")
+    call, off = blast_call(name, *args, ALGO["tiled"])
+    assert first[0] not in [k[0] for k in launches(call)]
+    call(L.stream_ptr(off.device))
+    assert_close(off, ref, dtype, f"GEMM + mix {name}")
     assert_close(out, back(off), dtype, f"one launch against GEMM + mix {name}")
 
 
@@ -163,6 +167,12 @@ NARROW_OUT = [(16, 288, 72, 576, (300,)), (16, 136, 40, 64, (129,)), (16, 200, 8
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("shape", NARROW_OUT)
 def test_blast_bmm_narrow_output_blocks(shape, dtype):
+    from triton_funcs import _lib as L
+    with L.options(BLR_DECODE_ROWS=0):                # (few rows times ranks: left to themselves these sizes take three launches of small tiles)
+        _narrow_output_blocks(shape, dtype)
+
+
+def _narrow_output_blocks(shape, dtype):
     """Output blocks of at most 80 columns with the bmm layouts above 128 rows: the mix and the product with U are one launch
     that keeps the results of all 16 output blocks of a 16-row tile in registers (Z is never written); with input blocks of at most
     96 columns that launch forms Y as well and is the whole call.  Row counts that are
@@ -173,6 +183,8 @@ def test_blast_bmm_narrow_output_blocks(shape, dtype):
     say(f"[case] narrow output blocks b={b} p={p} q={q} r={r} lead={lead} {dtype}")
     x, U, Vt, S = blast_inputs(b, p, q, r, lead, seed=23)
     ref = _ref(x, U, Vt, S, dtype)[0]
+    args = [dev(t, dtype) for t in (x.reshape(-1, b * p),) + O.blast_to_bmm_layout(U, Vt, S)]
+    assert len(launches(blast_call("bmm", *args, ALGO["tiled"])[0])) == 2       # x V and what re-lays U and S in one launch, or the latter alone; the rest
     out = _run_blast("triton_blast_bmm_fp16", x, U, Vt, S, dtype, "tiled")
     assert_close(out, ref.reshape(tuple(out.shape)), dtype, "narrow output blocks")
     out = _run_blast("triton_blast_full_fp16", x, U, Vt, S, dtype, "tiled")          # U as (b, r, q), S as (j, i, r): re-laid as well

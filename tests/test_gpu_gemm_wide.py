@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from oracle import blr_oracle as O
-from gpu_util import assert_close, blast_inputs, dev, launches, rounded, say, ulp
+from gpu_util import assert_close, blast_call, blast_inputs, dev, launches, rounded, say, ulp
 
 pytestmark = pytest.mark.gpu
 
@@ -60,9 +60,9 @@ def test_workgroups_that_walk_several_tiles(tn):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("tn", WIDTHS)
 def test_blast_and_low_rank_through_wide_tiles(tn, dtype):
-    """Batches, both orders of the second operand, and a side job of the first product (16 blocks, narrow outputs)."""
+    """Batches, both orders of the second operand; two products of one matrix."""
     from triton_funcs import blast_kernels as K, low_rank_kernels as LR, _lib as L
-    for b, p, q, r, m in ((4, 80, 40, 72, 300), (2, 176, 264, 136, 257), (16, 136, 72, 96, 130)):
+    for b, p, q, r, m in ((4, 80, 40, 72, 300), (2, 176, 264, 136, 257)):
         x, U, Vt, S = blast_inputs(b, p, q, r, (m,), seed=b + m)
         ref = O.blast_forward(rounded(x, dtype), rounded(U, dtype), rounded(Vt, dtype), rounded(S, dtype))[0]
         for name, lay in (("triton_blast_full_fp16", O.blast_to_partial_layout), ("triton_blast_bmm_fp16", O.blast_to_bmm_layout)):
@@ -71,6 +71,49 @@ def test_blast_and_low_rank_through_wide_tiles(tn, dtype):
             with L.options(BLR_GEMM_WIDE=tn):
                 out = getattr(K, name)(dev(x, dtype), dev(Uk, dtype), dev(Vk, dtype), dev(Sk, dtype), TILED)
             assert_close(out, ref, dtype, name)
+    rng = np.random.default_rng(tn)
+    x, A, B = rng.standard_normal((270, 200)), rng.standard_normal((200, 104)) / 104 ** 0.5, rng.standard_normal((104, 296)) / 104 ** 0.5
+    say(f"[case] wide low rank tn={tn} {dtype}")
+    with L.options(BLR_GEMM_WIDE=tn):
+        out = LR.triton_low_rank_fp16(dev(x, dtype), dev(A, dtype), dev(B, dtype), TILED)
+    assert_close(out, rounded(x, dtype) @ rounded(A, dtype) @ rounded(B, dtype), dtype, "low rank")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tn", WIDTHS)
+def test_side_job_of_the_first_product(tn, dtype):
+    """16 blocks of narrow outputs: workgroups of the first product's launch re-lay U and S for the kernel that does the rest, from both orders of either."""
+    from triton_funcs import _lib as L
+    for b, p, q, r, m in ((16, 136, 72, 96, 130), (16, 104, 8, 32, 300), (16, 200, 80, 160, 257)):
+        x, U, Vt, S = blast_inputs(b, p, q, r, (m,), seed=p + m)
+        ref = O.blast_forward(rounded(x, dtype), rounded(U, dtype), rounded(Vt, dtype), rounded(S, dtype))[0]
+        for name, lay in (("full", O.blast_to_partial_layout), ("bmm", O.blast_to_bmm_layout)):
+            call, out = blast_call(name, *(dev(t, dtype) for t in (x,) + lay(U, Vt, S)), 2)
+            say(f"[case] wide, side job {name} tn={tn} p={p} q={q} r={r} m={m} {dtype}")
+            with L.options(BLR_GEMM_WIDE=tn, BLR_DECODE_ROWS=0):
+                first, *rest = launches(call)
+                side = -(-(16 * r // 8 * q + r * 64) // 512)
+                assert len(rest) == 1 and first[2] == (512, 1, 1) and first[1][0] >= -(-side // 8) * 8 + 8
+                call(L.stream_ptr(out.device))
+            assert_close(out, ref, dtype, name)
+
+
+# (rows, rank, columns per input block, the ring kernel's tile): 16 blocks of narrow outputs whose x V the rules give to a ring kernel
+@pytest.mark.parametrize("m,r,p,ring", [(300, 768, 688, 128128), (1000, 320, 1024, 256128)])
+def test_side_job_on_the_ring_kernels(m, r, p, ring):
+    from triton_funcs import _lib as L
+    b, q, dtype = 16, 72, torch.float16
+    g = torch.Generator("cuda").manual_seed(m)
+    rnd = lambda *sh: torch.randn(*sh, device="cuda", generator=g)
+    x, U, V, S = rnd(m, b * p).to(dtype), (rnd(b, q, r) / r ** 0.5).to(dtype), (rnd(b, p, r) / p ** 0.5).to(dtype), rnd(r, b, b).to(dtype)
+    call, out = blast_call("bmm", x, U, V, S, 2)
+    say(f"[case] side job on the ring kernels m={m} r={r} p={p}")
+    auto, by_name, on_wide = _three_ways(call, ring, 4)
+    assert len(auto) == 2 and auto[0] == by_name[0] != on_wide[0]
+    call(L.stream_ptr(out.device))
+    Y = torch.bmm(x.double().view(m, b, p).transpose(0, 1).contiguous(), V.double())
+    ref = torch.cat([(Y * S[:, i].double().t()[:, None]).sum(0) @ U[i].double().t().contiguous() for i in range(b)], 1)
+    assert_close(out, ref.cpu().numpy(), dtype, "side job")
 
 
 @pytest.mark.parametrize("tn", WIDTHS)

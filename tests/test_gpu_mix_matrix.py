@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import blr_oracle as O
-from gpu_util import assert_close, blast_inputs, dev, rounded, say, ulp
+from gpu_util import assert_close, blast_call, blast_inputs, dev, launches, rounded, say, ulp
 
 pytestmark = pytest.mark.gpu
 TILED = {"algo": 2}
@@ -14,25 +14,31 @@ TILED = {"algo": 2}
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_bmm_fp16"])
-@pytest.mark.parametrize("b,r,m", [(4, 8, 17), (4, 72, 33), (8, 64, 130), (8, 200, 300), (12, 136, 95), (16, 8, 31), (16, 56, 257), (16, 192, 64), (16, 328, 1000)])
+@pytest.mark.parametrize("b,r,m", [(4, 8, 17), (4, 72, 33), (8, 64, 130), (8, 200, 300), (12, 136, 95), (12, 8, 17), (16, 8, 17), (16, 72, 33), (16, 8, 31), (16, 56, 257),
+                                   (16, 192, 64), (16, 328, 1000)])
 def test_mix_on_the_matrix_cores(b, r, m, name, dtype):
-    from triton_funcs import blast_kernels as K, _lib as L
-    p, q = 136, 24
+    from triton_funcs import _lib as L
+    p, q = 200, 24                                    # (columns of a block that no fused first half takes)
     x, U, Vt, S = blast_inputs(b, p, q, r, (m,), seed=b + r + m)
     Uk, Vk, Sk = (O.blast_to_bmm_layout if "bmm" in name else O.blast_to_partial_layout)(U, Vt, S)
     say(f"[case] mix {name} b={b} r={r} m={m} {dtype}")
-    with L.options(BLR_BLAST_MIXU=0, BLR_BLAST_YMIXW=0):
-        out = getattr(K, name)(dev(x, dtype), dev(Uk, dtype), dev(Vk, dtype), dev(Sk, dtype), TILED)
+    call, out = blast_call(name, *(dev(t, dtype) for t in (x, Uk, Vk, Sk)), 2)
+    with L.options(BLR_BLAST_MIXU=0, BLR_DECODE_ROWS=0):
+        kernels = launches(call)
+        assert len(kernels) == 3 and kernels[1][2:] == ((512, 1, 1), b * 4096)        # the mix of a tile of 32 x 64 in LDS
+        call(L.stream_ptr(out.device))
     assert_close(out, O.blast_forward(rounded(x, dtype), rounded(U, dtype), rounded(Vt, dtype), rounded(S, dtype))[0], dtype, name)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("order", ["rij", "jir", "ijr"])
 @pytest.mark.parametrize("b", [4, 8, 12, 16])
-def test_mix_element_by_element(b, order):
+def test_mix_element_by_element(b, order, dtype):
     """One rounding of sums in fp32, for a problem of more tiles than two per compute unit holds (rank tiles change inside a run)."""
     import ctypes
     from triton_funcs import _lib as L
-    dtype, m, r, p, q = torch.bfloat16, 40 * 32 + 5, 15 * 64 + 40, 16, 8
+    m, r, p, q = 40 * 32 + 5, 15 * 64 + 40, 16, 8
+    dt = L.F16 if dtype == torch.float16 else L.BF16
     g = torch.Generator("cuda").manual_seed(b)
     rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
     x, V, U, Sc = rnd(m, b * p), rnd(b, p, r), rnd(b, r, q), rnd(b, b, r)
@@ -41,10 +47,10 @@ def test_mix_element_by_element(b, order):
     out = torch.empty(m, b * q, device="cuda", dtype=dtype)
     lib = L.lib()
     lay = {"rij": L.S_RIJ, "jir": L.S_JIR, "ijr": L.S_IJR}[order]
-    say(f"[case] mix elements b={b} S ({order})")
-    ws = torch.empty(lib.blr_blast_workspace_bytes(m, b * p, b * q, b, r, L.BF16, 2), dtype=torch.uint8, device="cuda")
+    say(f"[case] mix elements b={b} S ({order}) {dtype}")
+    ws = torch.empty(lib.blr_blast_workspace_bytes(m, b * p, b * q, b, r, dt, 2), dtype=torch.uint8, device="cuda")
     ptr = lambda t: ctypes.c_void_p(t.data_ptr())
-    rc = lib.blr_blast_fwd(ptr(x), b * p, ptr(U), ptr(V), ptr(S), ptr(out), b * q, ptr(z), ptr(y), m, b * p, b * q, b, r, L.BF16, L.U_RQ, lay, 2,
+    rc = lib.blr_blast_fwd(ptr(x), b * p, ptr(U), ptr(V), ptr(S), ptr(out), b * q, ptr(z), ptr(y), m, b * p, b * q, b, r, dt, L.U_RQ, lay, 2,
                            ptr(ws), ws.numel(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
     assert rc == 0, lib.blr_last_error()
     yd, sd = y.double(), Sc.double()
@@ -55,7 +61,7 @@ def test_mix_element_by_element(b, order):
             ref[i] += t
             mag[i] += t.abs()
     err = (z.double() - ref).abs().cpu().numpy()
-    bound = 0.5 * ulp(ref.cpu().numpy(), dtype) * (1 + 2.0 ** -7) + 16 * 2.0 ** -24 * mag.cpu().numpy()
+    bound = 0.5 * ulp(ref.cpu().numpy(), dtype) * (1 + 2.0 ** (-10 if dtype == torch.float16 else -7)) + 16 * 2.0 ** -24 * mag.cpu().numpy()
     assert (err <= bound).all(), f"{np.max(err / bound):.3f} of the bound"
 
 
