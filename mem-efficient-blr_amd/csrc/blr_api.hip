@@ -424,8 +424,9 @@ static int blast_tiled(const void* x, int64_t ldx, const void* U, const void* V,
   const bool mixu = mixu_shape && (mixu_mode >= 2 || (mixu_mode == 1 && (P > fuse_max_p || fused < 0)));
   // Wide input blocks (16 of them, a multiple of 64 columns each, rank a multiple of 64): x V as one GEMM whose 64 x 64 tile keeps Y of all
   // 16 blocks in registers, then the mix, in one launch (blast_ymixw_kernel).  Only where the caller asks for the fused algorithm: the
-  // product on wide tiles and the mix on the matrix cores take no longer (the six linears of a Llama-7B block at 2048 rows 481 us with it, 450 without; 5120 -> 5120,
-  // r = 640 at 2048 rows 69 and 53, 8192 -> 2048, r = 768 85 and 59, 4096 -> 4096, r = 512 at 3000 rows 68 and 59, at 1000 rows and below level).
+  // product on wide tiles and the mix on the matrix cores take less time but for one row count (whole calls, one launch / two: 4096 -> 4096, r = 512 at 300 / 1000 / 2048 / 4096
+  // rows 32.3 / 35.9 / 46.0 / 88.1 and 24.0 / 31.2 / 46.6 / 81.2 us; 4096 -> 22016, r = 1024 at 512 / 1000 / 2048 rows 58.2 / 82.8 / 161.6 and 55.0 / 81.4 / 148.7; 5120 -> 5120,
+  // r = 640 at 2048 rows 74.2 and 60.5; 8192 -> 2048, r = 768 at 1000 / 2048 rows 47.4 / 86.6 and 37.4 / 67.0).
   if (!mixu && !y_out && !sat8 && fused == 1 && P > fuse_max_p && option_value(OPT_BLAST_YMIXW, 1))
     rc = blast_ymixw_launch(x, ldx, V, S, Z, M, in_f, b, r, si, sj, sr, s_layout, dtype, Y, ybytes, st);
   if (rc < 0) return rc;

@@ -1376,6 +1376,9 @@ static int pick_mfma(const GemmArgs& g, hipStream_t st) {
     set_error("gemm: a pair of tiles (SiLU-gated halves) needs 16-byte aligned operands, K and the half width multiples of 8, a plain row-major output");
     return BLR_ERR_UNSUPPORTED;
   }
+  // What comes here: products that gemm_wide_plan leaves to these rules (long reductions of several batches, pairs of short ones), operands that the wide tiles do
+  // not take (64 k, int8-rounded results, interleaved columns, a scatter of any period) and every product where BLR_GEMM_WIDE is 0 or one of the ring options
+  // is set.  The figures are of the ring kernels against each other; most of the shapes that they name run on wide tiles by now.
   if ((ring > 0 && ring_ok(g)) || g.pair) {
     int rt = option_value(OPT_GEMM_RING_TILE, 0);
     const bool auto_tile = rt == 0, narrow = rt == 256096;

@@ -488,8 +488,8 @@ int blast_ymix_launch(const void* x, int64_t ldx, const void* V, const void* S, 
 
 // ---- the same first half for wide input blocks: x V as one GEMM over all of x's columns, Y held in registers -------------------
 //
-// blast_ymix_kernel reads V once per 32 rows, straight into registers; from about 128 columns per input block on that costs more
-// than the round trip of Y through memory that it saves.  Here a workgroup of four waves (one per SIMD, so a lane may hold some
+// blast_ymix_kernel reads V once per 32 rows; from about 128 columns per input block on that costs more
+// than the round trip of Y through memory that it saves.  (That round trip has become cheaper since: this kernel runs where the fused algorithm is asked for by name.)  Here a workgroup of four waves (one per SIMD, so a lane may hold some
 // 250 registers) owns 64 rows x 64 ranks for all 16 input blocks.  x is (M, 16 P) and V (16 P, R), both contiguous over the
 // blocks, so Y_0 .. Y_15 of the tile are one GEMM with a reduction over all 16 P columns whose accumulator is packed away and
 // cleared every P columns: stages of 64 k of both operands go global -> LDS directly (whole 128-byte lines; the stage layouts
