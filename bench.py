@@ -371,7 +371,7 @@ def main():
                     fl = 2 * m * r * (i_f + o_f + B * B)
                     row(f"blast_int{bits}/{lname}/M{m}", measure(lambda: mk_blast_q(m, i_f, o_f, r, bits), by), by, fl, m)
 
-    # ---- DiT-XL/2 end to end (BASELINE configs[4]): 16 latents [4,32,32], every qkv/proj/fc1/fc2 linear replaced ----
+    # ---- DiT-XL/2 end to end: 16 latents [4,32,32], every qkv/proj/fc1/fc2 linear replaced ----
     dit = None
     if not args.no_table:
         try:
@@ -430,7 +430,7 @@ def main():
         cpu = {"value": round(times[len(times) // 2] * 1e6, 1), "unit": "us/layer-step", "cores": cores, "kind": "port",
                "sample": f"{reps} repetitions (~{t_used:.0f} s) of the full M=1 step (6 BLAST linears) in fp32 with oracle/torch_port.blast"}
 
-    # ---- BASELINE configs[0]: the reference's own CPU-runnable case (GPT-2-small c_fc, fp32) on the host and on the GPU ---------
+    # ---- the reference's own CPU-runnable case (GPT-2-small c_fc, fp32) on the host and on the GPU ---------
     cpu1 = None
     if not args.no_cpu:
         from oracle import torch_port as T

@@ -74,7 +74,7 @@ def test_blast_small_all_algorithms(name, shape, algo, dtype):
 
 
 def test_blast_gpt2_config_fp32_and_fp16():
-    """x [1,128,768], b=4, U [4,768,128], V [4,192,128], S [4,4,128], seed 0."""
+    """GPT-2 c_fc: x [1,128,768], b=4, U [4,768,128], V [4,192,128], S [4,4,128], seed 0."""
     b, p, q, r = 4, 192, 768, 128
     x, U, Vt, S = blast_inputs(b, p, q, r, (1, 128), seed=0)
     say("[case] gpt2 c_fc fp32")
@@ -223,7 +223,7 @@ def test_blast_fused_refuses_what_it_cannot_tile():
 @pytest.mark.parametrize("layer", list(LLAMA))
 @pytest.mark.parametrize("name", ["triton_blast_full_fp16", "triton_blast_partial_grouped_fp16", "triton_blast_bmm_fp16"])
 def test_blast_llama7b_decode(name, layer, M, dtype):
-    """BASELINE config 3 at decode sizes, in fp16 and in bf16 - the type the reference's *_fp16 kernels actually compute in
+    """Llama-7B linears at decode sizes, in fp16 and in bf16 - the type the reference's *_fp16 kernels actually compute in
     (reference triton_funcs/blast_kernels.py:1953-1955, layer.py:282)."""
     p, q, r = LLAMA[layer]
     b = 16

@@ -115,7 +115,7 @@ def test_dit_small_blast_matches_its_dense_assembly():
 
 
 def test_dit_full_depth_graph_replay_is_finite_and_matches_dense_assembly():
-    """BASELINE config 5 at full size - 28 blocks, 16 latents of 256 tokens, every block linear a BLAST layer - run the way the
+    """DiT-XL/2 at full size - 28 blocks, 16 latents of 256 tokens, every block linear a BLAST layer - run the way the
     benchmark runs it (a captured forward, replayed): every replay equals the eager forward bit for bit, the output is finite,
     and it agrees with the same network after each BLAST layer has been replaced by its assembled dense matrix."""
     from models.dit_xl import CustomDiT, capture_forward

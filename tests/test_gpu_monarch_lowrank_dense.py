@@ -109,7 +109,7 @@ LLAMA_IO = {"qkvo": (4096, 4096), "gate_up": (4096, 22016), "down": (11008, 4096
 @pytest.mark.parametrize("M", [1, 16, 2048])
 @pytest.mark.parametrize("layer", list(LLAMA_IO))
 def test_monarch_llama7b(layer, M, dtype):
-    """nblocks = 4, rank 1024 per block; fp16 as the config says and bf16 as the reference's kernels compute
+    """Llama-7B layers: nblocks = 4, rank 1024 per block; fp16 as the layers are quoted and bf16 as the reference's kernels compute
     (reference triton_funcs/monarch_kernels.py:676-677)."""
     in_f, out_f = LLAMA_IO[layer]
     b, rank = 4, 1024
@@ -266,7 +266,7 @@ def test_load_store_probes_move_every_operand_at_hbm_speed(M):
 @pytest.mark.parametrize("M", [1, 16, 2048])
 @pytest.mark.parametrize("layer", list(LLAMA_IO))
 def test_low_rank_and_dense_llama7b(layer, M, dtype):
-    """r = 1024; fp16 as the config says and bf16 as the reference's kernels compute
+    """Llama-7B layers: r = 1024; fp16 as the layers are quoted and bf16 as the reference's kernels compute
     (reference triton_funcs/low_rank_kernels.py:286-288, dense_kernels.py:268-269)."""
     from triton_funcs import low_rank_kernels as K, dense_kernels as D
     in_f, out_f = LLAMA_IO[layer]

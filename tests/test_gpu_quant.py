@@ -142,7 +142,7 @@ def test_blast_q_vs_oracle_on_dequantized(shape, bits, dtype):
 @pytest.mark.parametrize("bits", [8, 4])
 @pytest.mark.parametrize("layer", ["gate_up", "down"])
 def test_blast_q_llama7b(layer, bits, M, dtype):
-    """BASELINE config 4 at full shape (activations and S in fp16 as the config says, and in bf16).  The weight quantizer is
+    """Llama-7B layers at full shape (activations and S in fp16 as the layers are quoted, and in bf16).  The weight quantizer is
     this build's own definition - the reference has none - so "parity" here means: codes and scales bit-exact against the
     numpy restatement of that definition, outputs against the fp64 product of the dequantized factors."""
     from triton_funcs import blast_sym_quant_kernels as Q

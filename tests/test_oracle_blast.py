@@ -135,7 +135,7 @@ def test_low_rank_and_dense_vs_library_gemm():
 
 
 def test_bytes_flops_match_published_table():
-    # BASELINE table: BLAST gate_up r=1024 b=16 M=1 -> 5.405e7 B, 5.40e7 FLOP; qkvo M=2048 -> 4.221e7 B, 1.772e10.
+    # BLAST gate_up r=1024 b=16 M=1 -> 5.405e7 B, 5.40e7 FLOP; qkvo M=2048 -> 4.221e7 B, 1.772e10.
     by, fl = O.blast_bytes_flops(1, 4096, 1024, 22016, 16)
     assert abs(by - 5.405e7) / 5.405e7 < 1e-3 and abs(fl - 5.40e7) / 5.40e7 < 2e-3
     by, fl = O.blast_bytes_flops(2048, 4096, 512, 4096, 16)
